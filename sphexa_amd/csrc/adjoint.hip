@@ -133,7 +133,7 @@ __global__ void __launch_bounds__(kPairWaves * kWave)
                 T d = sqrt(rx * rx + ry * ry + rz * rz);
                 T v = d * hInv;
                 T w, dw;
-                values(kern.fetchWD(v), w, dw);
+                kern.wAndDw(v, w, dw);
                 rho0 += mj[u] * w;
                 sumVdW += mj[u] * v * dw;
                 T c = d > T(0) ? coef * mj[u] * dw / d : T(0);
@@ -216,7 +216,7 @@ __global__ void __launch_bounds__(kPairWaves * kWave)
                 T d = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
                 T v = d * hInv;
                 T w, dw;
-                values(kern.fetchWD(v), w, dw);
+                kern.wAndDw(v, w, dw);
                 T mj   = mjs[u];
                 T rhoj = rhojs[u];
                 T Vj   = mj / rhoj;
@@ -310,8 +310,8 @@ __global__ void __launch_bounds__(kPairWaves * kWave)
             T hjInv3 = hjInv * hjInv * hjInv;
             T v1 = d * hiInv, v2 = d * hjInv;
             T W1, dW1, W2, dW2;
-            values(kern.fetchWD(v1), W1, dW1);
-            values(kern.fetchWD(v2), W2, dW2);
+            kern.wAndDw(v1, W1, dW1);
+            kern.wAndDw(v2, W2, dW2);
             T Wi = hiInv3 * W1, Wj = hjInv3 * W2;
             T Cj[3][3];
             loadC<T>(f, j, Cj);

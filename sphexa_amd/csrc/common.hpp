@@ -186,7 +186,7 @@ struct sphx_workspace
     // kernel tables: W and dW/dv on [0,2], 20000 points, in both precisions, stored per interval
     double                              K = 0, sincIndex = 0;
     // the reference's W and dW/dv tables for the FP64 form (the FP32 form evaluates W directly)
-    sphx::DevBuf<sphx::TabPair<double>> wh64, whd64;
+    sphx::DevBuf<sphx::TabPair<double>> wh64;
     sphx::DevBuf<sphx::TabQuad<double>> whq64;
     bool                   tablesValid = false;
 

@@ -77,7 +77,7 @@ __global__ void __launch_bounds__(kPackThreads) packMomStd(PairArgs a, MomStdFie
 /* xmassJLoop (sph/include/sph/hydro_ve/xmass_kern.hpp:51-79):
  *   xm_i = m_i / (K / h_i^3 * (m_i + sum_j m_j W(r_ij / h_i)))
  * toRho: computeDensity (hydro_std/density.hpp:42-53) stores rho = m / xm instead. */
-template<class T, bool toRho, bool Wide>
+template<class T, bool toRho, int V>
 __global__ void SPHX_LIGHT_LOOP(T)
     xmassKernel(PairArgs a, const RecMass<T>* __restrict__ rec, const T* __restrict__ h, SincKernel<T> kern,
                 T* __restrict__ out, RecGradh<T>* __restrict__ next, RecVol<T>* __restrict__ nextVol)
@@ -90,23 +90,23 @@ __global__ void SPHX_LIGHT_LOOP(T)
     T                hInv  = T(1) / hi;
     T                h3Inv = hInv * hInv * hInv;
     double           r2h   = 2.0 * double(hi);
-    Acc<T>           rho0(ri.m);
-    withFold(recordNeedsFold<T, Wide>(a.box, ri, r2h), [&](auto fold) {
+    const T          hInv2 = hInv * hInv;
+    Acc              rho0(ri.m);
+    withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
         constexpr int                U = kBatchLight<T>;
         NeighborBatch<U, RecMass<T>> nb(t, rec);
         for (unsigned k = 0; k < t.n; k += U)
         {
             nb.load(k);
-            typename SincKernel<T>::FetchW w[U];
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                w[u] = kern.fetchW(pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]).d * hInv);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                rho0.add(nb.live(k, u, value(w[u])) * nb.r[u].m);
+            {
+                const T z = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]).d2 * hInv2;
+                rho0.add(kern.template w<V>(nb.live2(k, u, z)) * double(nb.r[u].m));
+            }
         }
     });
-    double rhoZero = double(rho0.value()) * a.K * double(h3Inv);
+    double rhoZero = rho0.value() * a.K * double(h3Inv);
     T      xmi     = T(double(ri.m) / rhoZero);
     const T outi   = toRho ? T(ri.m / xmi) : xmi;
     out[i]         = outi;
@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(256) eosStdPolytropicKernel(const T* __restric
 }
 
 /* IADJLoopSTD (hydro_std/iad_kern.hpp:11-76): tau_ab = sum_j m_j/rho_j W_ij r_a r_b, inverted */
-template<class T, bool Wide>
+template<class T, int V>
 __global__ void SPHX_LIGHT_LOOP(T)
     iadStdKernel(PairArgs a, const RecVol<T>* __restrict__ rec, const T* __restrict__ h, SincKernel<T> kern,
                  T* c11, T* c12, T* c13, T* c22, T* c23, T* c33, MomStdFields nf, RecMomStd<T>* __restrict__ next)
@@ -171,28 +171,21 @@ __global__ void SPHX_LIGHT_LOOP(T)
     const uint32_t  i     = t.i;
     const RecVol<T> ri    = rec[i];
     T               hi    = h[i];
-    T               hiInv = T(1) / hi;
+    T               hiInv = T(1) / hi, hiInv2 = hiInv * hiInv;
     double          r2h   = 2.0 * double(hi);
     T               t11 = 0, t12 = 0, t13 = 0, t22 = 0, t23 = 0, t33 = 0;
-    withFold(recordNeedsFold<T, Wide>(a.box, ri, r2h), [&](auto fold) {
+    withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
         constexpr int               U = kBatchLight<T>;
         NeighborBatch<U, RecVol<T>> nb(t, rec);
         for (unsigned k = 0; k < t.n; k += U)
         {
             nb.load(k);
-            Sep<T>                    r[U];
-            typename SincKernel<T>::FetchW w[U];
 #pragma unroll
             for (int u = 0; u < U; ++u)
             {
-                r[u] = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]);
-                w[u] = kern.fetchW(r[u].d * hiInv);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                T rx = r[u].x, ry = r[u].y, rz = r[u].z;
-                T vol_w = nb.r[u].vol * nb.live(k, u, value(w[u]));
+                const Sep<T> r = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]);
+                T rx = r.x, ry = r.y, rz = r.z;
+                T vol_w = nb.r[u].vol * T(kern.template w<V>(nb.live2(k, u, r.d2 * hiInv2)));
                 t11 += rx * rx * vol_w;
                 t12 += rx * ry * vol_w;
                 t13 += rx * rz * vol_w;
@@ -216,7 +209,7 @@ __global__ void SPHX_LIGHT_LOOP(T)
 
 /* momentumAndEnergyJLoop, std (hydro_std/momentum_energy_kern.hpp:11-134) + tsKCourant.
  * PerAlpha: AV coefficients alpha_i, alpha_j from f.alpha instead of the constant 1. */
-template<class T, bool PerAlpha, bool Wide>
+template<class T, bool PerAlpha, int V>
 __global__ void SPHX_MOM_LOOP(T)
     momentumStdKernel(PairArgs a, MomStdFields f, const RecMomStd<T>* __restrict__ rec, SincKernel<T> kern,
                       float Kcour, unsigned long long* minDt)
@@ -230,38 +223,31 @@ __global__ void SPHX_MOM_LOOP(T)
         T                  hi     = ld<T>(f.h, i);
         T                  roi    = ld<T>(f.rho, i);
         T                  hiInv  = ri.hInv;
-        T                  hiInv3 = hiInv * hiInv * hiInv;
+        T                  hiInv2 = hiInv * hiInv, hiInv3 = hiInv2 * hiInv;
         T                  pro_i  = fastDiv(ld<T>(f.p, i), roi * roi); // p_i / (gradh_i rho_i^2), gradh_i = 1
         double             r2h    = 2.0 * double(hi);
         const T            alpha_i = PerAlpha ? ld<T>(f.alpha, i) : T(1);
 
         T      maxvs = 0;
         T      momx = 0, momy = 0, momz = 0;
-        Acc<T>       energy;
-        withFold(recordNeedsFold<T, Wide>(a.box, ri, r2h), [&](auto fold) {
+        Acc    energy;
+        withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
             constexpr int                  U = kBatchMom<T>;
             NeighborBatch<U, RecMomStd<T>> nb(t, rec);
             for (unsigned k = 0; k < t.n; k += U)
             {
                 nb.load(k);
-                Sep<T>                    r[U];
-                typename SincKernel<T>::FetchW wi[U], wj[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                {
-                    r[u]  = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]);
-                    wi[u] = kern.fetchW(r[u].d * hiInv);
-                    wj[u] = kern.fetchW(r[u].d * nb.r[u].hInv);
-                }
 #pragma unroll
                 for (int u = 0; u < U; ++u)
                 {
                     const RecMomStd<T>& rj = nb.r[u];
-                    T rx = r[u].x, ry = r[u].y, rz = r[u].z, dist = r[u].d;
+                    const Sep<T>        r  = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, rj);
+                    T rx = r.x, ry = r.y, rz = r.z;
                     T vx_ij = ri.vx - rj.vx, vy_ij = ri.vy - rj.vy, vz_ij = ri.vz - rj.vz;
                     T rv    = rx * vx_ij + ry * vy_ij + rz * vz_ij;
-                    T Wi    = hiInv3 * nb.live(k, u, value(wi[u]));
-                    T Wj    = rj.hInv * rj.hInv * rj.hInv * nb.live(k, u, value(wj[u]));
+                    T hjInv2 = rj.hInv * rj.hInv;
+                    T Wi     = hiInv3 * T(kern.template w<V>(nb.live2(k, u, r.d2 * hiInv2)));
+                    T Wj     = rj.hInv * hjInv2 * T(kern.template w<V>(nb.live2(k, u, r.d2 * hjInv2)));
 
                     T tA1_i = ri.c11 * rx + ri.c12 * ry + ri.c13 * rz;
                     T tA2_i = ri.c12 * rx + ri.c22 * ry + ri.c23 * rz;
@@ -270,7 +256,7 @@ __global__ void SPHX_MOM_LOOP(T)
                     T tA2_j = rj.c12 * rx + rj.c22 * ry + rj.c23 * rz;
                     T tA3_j = rj.c13 * rx + rj.c23 * ry + rj.c33 * rz;
 
-                    T wij  = fastDiv(rv, dist);
+                    T wij  = overDistance(rv, r.d2);
                     T alpha_j = PerAlpha ? ld<T>(f.alpha, nb.j[u]) : T(1);
                     T visc    = T(0.5) * artificialViscosity(alpha_i, alpha_j, ri.c, rj.c, wij);
                     T vsig = ri.c + rj.c - T(3) * wij;
@@ -294,7 +280,7 @@ __global__ void SPHX_MOM_LOOP(T)
                 }
             }
         });
-        f.du[i] = -a.K * 0.5 * double(energy.value());
+        f.du[i] = -a.K * 0.5 * energy.value();
         st<T>(f.ax, i, T(a.K * double(momx)));
         st<T>(f.ay, i, T(a.K * double(momy)));
         st<T>(f.az, i, T(a.K * double(momz)));
@@ -319,13 +305,13 @@ void launchDensity(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f
     RecVol<T>*   nextVol = toRho && chainable(a, p) ? recordBuffer<RecVol<T>>(ws, a.numParticles, 1) : nullptr;
     {
         KernelScope timer(ws, toRho ? "density_std" : "xmass");
-        launchWide<T>(ws->nbWide, [&](auto wide) {
-            constexpr bool W = decltype(wide)::value;
+        launchVariant<T>(ws, [&](auto variant) {
+            constexpr int V = decltype(variant)::value;
             if (toRho)
-                xmassKernel<T, true, W><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_XMASS) : 0, ws->stream>>>(
+                xmassKernel<T, true, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_XMASS) : 0, ws->stream>>>(
                     a, rec, (const T*)f->h, sincKernel<T>(ws), (T*)out, nullptr, nextVol);
             else
-                xmassKernel<T, false, W><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_XMASS) : 0, ws->stream>>>(
+                xmassKernel<T, false, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_XMASS) : 0, ws->stream>>>(
                     a, rec, (const T*)f->h, sincKernel<T>(ws), (T*)out, next, nullptr);
         });
         SPHX_CHECK_LAUNCH();
@@ -355,8 +341,8 @@ void launchIadStd(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f,
                              : nullptr;
     {
         KernelScope timer(ws, "iad_std");
-        launchWide<T>(ws->nbWide, [&](auto wide) {
-            iadStdKernel<T, decltype(wide)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_IAD) : 0, ws->stream>>>(
+        launchVariant<T>(ws, [&](auto variant) {
+            iadStdKernel<T, decltype(variant)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_IAD) : 0, ws->stream>>>(
                 a, rec, (const T*)f->h, sincKernel<T>(ws), (T*)f->c11, (T*)f->c12, (T*)f->c13, (T*)f->c22,
                 (T*)f->c23, (T*)f->c33, nf, next);
         });
@@ -379,13 +365,13 @@ void launchMomentumStd(sphx_workspace* ws, const PairArgs& a, const MomStdFields
         SPHX_CHECK_LAUNCH();
     }
     KernelScope timer(ws, "momentum_std");
-    launchWide<T>(ws->nbWide, [&](auto wide) {
-        constexpr bool W = decltype(wide)::value;
+    launchVariant<T>(ws, [&](auto variant) {
+        constexpr int V = decltype(variant)::value;
         if (perAlpha)
-            momentumStdKernel<T, true, W><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(a, mf, rec, sincKernel<T>(ws),
+            momentumStdKernel<T, true, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(a, mf, rec, sincKernel<T>(ws),
                                                                                         Kcour, dt);
         else
-            momentumStdKernel<T, false, W><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(a, mf, rec,
+            momentumStdKernel<T, false, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(a, mf, rec,
                                                                                          sincKernel<T>(ws), Kcour, dt);
     });
     SPHX_CHECK_LAUNCH();

@@ -24,7 +24,7 @@ __global__ void __launch_bounds__(kPackThreads) packGradh(PairArgs a, const T* _
 }
 
 /* veDefGradhJLoop (hydro_ve/ve_def_gradh_kern.hpp:44-90): kx and the grad-h term */
-template<class T, bool Wide>
+template<class T, int V>
 __global__ void SPHX_LIGHT_LOOP(T)
     veDefGradhKernel(PairArgs a, const RecGradh<T>* __restrict__ rec, const T* __restrict__ h,
                      SincKernel<T> kern, T* __restrict__ kx, T* __restrict__ gradh, RecIadVe<T>* __restrict__ next,
@@ -37,27 +37,24 @@ __global__ void SPHX_LIGHT_LOOP(T)
     T                 hi  = h[i], mi = ri.m, xmi = ri.xm;
     T                 hInv = T(1) / hi;
     double            r2h  = 2.0 * double(hi);
-    Acc<T>            kxs(xmi), wom(-T(3) * xmi), wr0(-T(3) * mi);
-    withFold(recordNeedsFold<T, Wide>(a.box, ri, r2h), [&](auto fold) {
+    const T           hInv2 = hInv * hInv;
+    Acc               kxs(xmi), wom(-3.0 * double(xmi)), wr0(-3.0 * double(mi));
+    withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
         constexpr int                 U = kBatchLight<T>;
         NeighborBatch<U, RecGradh<T>> nb(t, rec);
         for (unsigned k = 0; k < t.n; k += U)
         {
             nb.load(k);
-            typename SincKernel<T>::FetchWD w[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                w[u] = kern.fetchWD(pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]).d * hInv);
 #pragma unroll
             for (int u = 0; u < U; ++u)
             {
-                T wv, dw;
-                values(w[u], wv, dw);
-                wv = nb.live(k, u, wv), dw = nb.live(k, u, dw);
-                T dterh = -(T(3) * wv + w[u].v * dw);
-                kxs.add(wv * nb.r[u].xm);
-                wom.add(dterh * nb.r[u].xm);
-                wr0.add(dterh * nb.r[u].m);
+                const T z = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]).d2 * hInv2;
+                double  wv, vdw;
+                kern.template wAndVdw<V>(nb.live2(k, u, z), wv, vdw);
+                const double dterh = -(3.0 * wv + vdw);
+                kxs.add(wv * double(nb.r[u].xm));
+                wom.add(dterh * double(nb.r[u].xm));
+                wr0.add(dterh * double(nb.r[u].m));
             }
         }
     });
@@ -65,9 +62,9 @@ __global__ void SPHX_LIGHT_LOOP(T)
     T      th3   = hInv * hInv * hInv;
     double dhInv = double(hInv);
     double h3Inv = double(th3);
-    double kxi   = double(kxs.value()) * (a.K * h3Inv);
-    double whom  = double(wom.value()) * (a.K * h3Inv * dhInv);
-    double wrho0 = double(wr0.value()) * (a.K * h3Inv * dhInv);
+    double kxi   = kxs.value() * (a.K * h3Inv);
+    double whom  = wom.value() * (a.K * h3Inv * dhInv);
+    double wrho0 = wr0.value() * (a.K * h3Inv * dhInv);
     whom          = whom * double(mi) / double(xmi) + (kxi - a.K * double(xmi) * h3Inv) * wrho0;
     double rhoi   = kxi * double(mi) / double(xmi);
     double dhdrho = -double(hi) / (rhoi * 3.0);
@@ -197,7 +194,7 @@ __global__ void __launch_bounds__(kPackThreads) packIadVe(PairArgs a, IadVeField
  *   dV_a[b] = sum_j (v_ja - v_ia) xm_j (-(C_i r_ij)_b W_ij) = -sum_c C_i[b][c] M[a][c],
  *   M[a][c] = sum_j (v_ja - v_ia) xm_j W_ij r_ij,c,
  * so the 9 moments M are accumulated alongside tau and combined with C_i after the inversion. */
-template<class T, bool Wide>
+template<class T, int V>
 __global__ void SPHX_LIGHT_LOOP(T)
     iadDivvCurlvKernel(PairArgs a, IadVeFields f, const RecIadVe<T>* __restrict__ rec, SincKernel<T> kern,
                        RecAv<T>* __restrict__ next, const T* __restrict__ cNext)
@@ -207,30 +204,23 @@ __global__ void SPHX_LIGHT_LOOP(T)
     const uint32_t    i     = t.i;
     const RecIadVe<T> ri    = rec[i];
     T                 hi    = ld<T>(f.h, i);
-    T                 hiInv = T(1) / hi;
+    T                 hiInv = T(1) / hi, hiInv2 = hiInv * hiInv;
     double            r2h   = 2.0 * double(hi);
     T                 t11 = 0, t12 = 0, t13 = 0, t22 = 0, t23 = 0, t33 = 0;
     T                 M[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-    withFold(recordNeedsFold<T, Wide>(a.box, ri, r2h), [&](auto fold) {
+    withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
         constexpr int                 U = kBatchLight<T>;
         NeighborBatch<U, RecIadVe<T>> nb(t, rec);
         for (unsigned k = 0; k < t.n; k += U)
         {
             nb.load(k);
-            Sep<T>                    r[U];
-            typename SincKernel<T>::FetchW w[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                r[u] = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]);
-                w[u] = kern.fetchW(r[u].d * hiInv);
-            }
 #pragma unroll
             for (int u = 0; u < U; ++u)
             {
                 const RecIadVe<T>& rj = nb.r[u];
-                T rx = r[u].x, ry = r[u].y, rz = r[u].z;
-                T wv    = nb.live(k, u, value(w[u]));
+                const Sep<T>       r  = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, rj);
+                T rx = r.x, ry = r.y, rz = r.z;
+                T wv    = T(kern.template w<V>(nb.live2(k, u, r.d2 * hiInv2)));
                 T vol_w = rj.vol * wv;
                 t11 += rx * rx * vol_w;
                 t12 += rx * ry * vol_w;
@@ -302,7 +292,7 @@ __global__ void __launch_bounds__(kPackThreads) packAv(PairArgs a, AvFields f, R
 
 /* AVswitchesJLoop (hydro_ve/av_switches_kern.hpp:44-137). grad(div v) is linear in C_i:
  * gd_b = -K/h_i^3 sum_c C_i[b][c] sum_j f_j W_ij r_ij,c with f_j = xm_j/kx_j (divv_i - divv_j). */
-template<class T, bool Wide>
+template<class T, int V>
 __global__ void SPHX_LIGHT_LOOP(T)
     avSwitchesKernel(PairArgs a, AvFields f, const RecAv<T>* __restrict__ rec, SincKernel<T> kern, double dt,
                      T alphamin, T alphamax, T decay, RecMomVe<T>* __restrict__ next)
@@ -312,33 +302,26 @@ __global__ void SPHX_LIGHT_LOOP(T)
     const uint32_t i     = t.i;
     const RecAv<T> ri    = rec[i];
     T              hi    = ld<T>(f.h, i);
-    T              hiInv = T(1) / hi;
+    T              hiInv = T(1) / hi, hiInv2 = hiInv * hiInv;
     double         r2h   = 2.0 * double(hi);
     T              vsig  = T(1.e-40) * ri.c;
     T              S[3]  = {0, 0, 0};
-    withFold(recordNeedsFold<T, Wide>(a.box, ri, r2h), [&](auto fold) {
+    withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
         constexpr int              U = kBatchLight<T>;
         NeighborBatch<U, RecAv<T>> nb(t, rec);
         for (unsigned k = 0; k < t.n; k += U)
         {
             nb.load(k);
-            Sep<T>                    r[U];
-            typename SincKernel<T>::FetchW w[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                r[u] = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]);
-                w[u] = kern.fetchW(r[u].d * hiInv);
-            }
 #pragma unroll
             for (int u = 0; u < U; ++u)
             {
                 const RecAv<T>& rj = nb.r[u];
-                T rx = r[u].x, ry = r[u].y, rz = r[u].z;
+                const Sep<T>    r  = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, rj);
+                T rx = r.x, ry = r.y, rz = r.z;
                 T rv = rx * (ri.vx - rj.vx) + ry * (ri.vy - rj.vy) + rz * (ri.vz - rj.vz);
-                T vs = nb.in(k, u) && rv < T(0) ? ri.c + rj.c - T(3) * fastDiv(rv, r[u].d) : T(0);
+                T vs = nb.in(k, u) && rv < T(0) ? ri.c + rj.c - T(3) * overDistance(rv, r.d2) : T(0);
                 vsig = vsig < vs ? vs : vsig;
-                T fw = rj.vol * (ri.divv - rj.divv) * nb.live(k, u, value(w[u]));
+                T fw = rj.vol * (ri.divv - rj.divv) * T(kern.template w<V>(nb.live2(k, u, r.d2 * hiInv2)));
                 S[0] += fw * rx, S[1] += fw * ry, S[2] += fw * rz;
             }
         }
@@ -436,7 +419,7 @@ __device__ __forceinline__ T ramExp2(T v)
 }
 
 /* momentumAndEnergyJLoop<avClean> (hydro_ve/momentum_energy_kern.hpp:66-222) + tsKCourant */
-template<class T, bool avClean, bool Wide>
+template<class T, bool avClean, int V>
 __global__ void SPHX_MOM_LOOP(T)
     momentumVeKernel(PairArgs a, MomVeFields f, const RecMomVe<T>* __restrict__ rec, SincKernel<T> kern, T Atmin,
                      T Atmax, T ramp, float Kcour, unsigned long long* minDt)
@@ -449,7 +432,7 @@ __global__ void SPHX_MOM_LOOP(T)
         const RecMomVe<T> ri     = rec[i];
         T                 hi     = ld<T>(f.h, i);
         T                 hiInv  = ri.hInv;
-        T                 hiInv3 = hiInv * hiInv * hiInv;
+        T                 hiInv2 = hiInv * hiInv, hiInv3 = hiInv2 * hiInv;
         T                 gradV_i[6] = {0, 0, 0, 0, 0, 0};
         if constexpr (avClean)
         {
@@ -461,33 +444,25 @@ __global__ void SPHX_MOM_LOOP(T)
 
         T      maxvs = 0;
         T      momx = 0, momy = 0, momz = 0;
-        Acc<T>       energy, avEnergy;
-        withFold(recordNeedsFold<T, Wide>(a.box, ri, r2h), [&](auto fold) {
+        Acc    energy, avEnergy;
+        withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
             constexpr int                 U = kBatchMom<T>;
             NeighborBatch<U, RecMomVe<T>> nb(t, rec);
             for (unsigned k = 0; k < t.n; k += U)
             {
               nb.load(k);
-              Sep<T>                    r[U];
-              typename SincKernel<T>::FetchW wi[U], wj[U];
-#pragma unroll
-              for (int u = 0; u < U; ++u)
-              {
-                  r[u]  = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]);
-                  wi[u] = kern.fetchW(r[u].d * hiInv);
-                  wj[u] = kern.fetchW(r[u].d * nb.r[u].hInv);
-              }
 #pragma unroll
               for (int u = 0; u < U; ++u)
               {
                 const uint32_t     j  = nb.j[u];
                 const RecMomVe<T>& rj = nb.r[u];
-                T rx = r[u].x, ry = r[u].y, rz = r[u].z, dist = r[u].d;
+                const Sep<T>       r  = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, rj);
+                T rx = r.x, ry = r.y, rz = r.z;
                 T vx_ij = ri.vx - rj.vx, vy_ij = ri.vy - rj.vy, vz_ij = ri.vz - rj.vz;
-                T v1    = wi[u].v;
-                T v2    = wj[u].v;
-                T Wi    = hiInv3 * nb.live(k, u, value(wi[u]));
-                T Wj    = rj.hInv * rj.hInv * rj.hInv * nb.live(k, u, value(wj[u]));
+                T hjInv2 = rj.hInv * rj.hInv;
+                T z1     = r.d2 * hiInv2, z2 = r.d2 * hjInv2;
+                T Wi     = hiInv3 * T(kern.template w<V>(nb.live2(k, u, z1)));
+                T Wj     = rj.hInv * hjInv2 * T(kern.template w<V>(nb.live2(k, u, z2)));
 
                 T tA1_i = -(ri.c11 * rx + ri.c12 * ry + ri.c13 * rz) * Wi;
                 T tA2_i = -(ri.c12 * rx + ri.c22 * ry + ri.c23 * rz) * Wi;
@@ -501,9 +476,9 @@ __global__ void SPHX_MOM_LOOP(T)
                 {
                     T gradV_j[6] = {ld<T>(f.dV11, j), ld<T>(f.dV12, j), ld<T>(f.dV13, j),
                                     ld<T>(f.dV22, j), ld<T>(f.dV23, j), ld<T>(f.dV33, j)};
-                    rv += avRvCorrection(rx, ry, rz, v1 < v2 ? v1 : v2, eta_crit, gradV_i, gradV_j);
+                    rv += avRvCorrection(rx, ry, rz, fastSqrt(z1 < z2 ? z1 : z2), eta_crit, gradV_i, gradV_j);
                 }
-                T wij  = fastDiv(rv, dist);
+                T wij  = overDistance(rv, r.d2);
                 T visc = artificialViscosity(ri.alpha, rj.alpha, ri.c, rj.c, wij);
                 T vsig = T(0.5) * (ri.c + rj.c) - T(2) * wij;
                 maxvs  = nb.in(k, u) && vsig > maxvs ? vsig : maxvs;
@@ -547,9 +522,9 @@ __global__ void SPHX_MOM_LOOP(T)
               }
             }
         });
-        T avE    = avEnergy.value() > T(0) ? avEnergy.value() : T(0);
-        T eCoeff = f.tdpdTrho ? ld<T>(f.tdpdTrho, i) : ri.prho;
-        f.du[i]  = a.K * double(eCoeff * energy.value() + T(0.5) * avE);
+        double avE    = avEnergy.value() > 0.0 ? avEnergy.value() : 0.0;
+        double eCoeff = f.tdpdTrho ? double(ld<T>(f.tdpdTrho, i)) : double(ri.prho);
+        f.du[i]       = a.K * (eCoeff * energy.value() + 0.5 * avE);
         st<T>(f.ax, i, T(-a.K * double(momx)));
         st<T>(f.ay, i, T(-a.K * double(momy)));
         st<T>(f.az, i, T(-a.K * double(momz)));
@@ -596,8 +571,8 @@ void launchGradh(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f, 
                             : nullptr;
     {
         KernelScope timer(ws, "ve_def_gradh");
-        launchWide<T>(ws->nbWide, [&](auto wide) {
-            veDefGradhKernel<T, decltype(wide)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_GRADH) : 0, ws->stream>>>(
+        launchVariant<T>(ws, [&](auto variant) {
+            veDefGradhKernel<T, decltype(variant)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_GRADH) : 0, ws->stream>>>(
                 a, rec, (const T*)f->h, sincKernel<T>(ws), (T*)f->kx, (T*)f->gradh, next, (const T*)f->vx,
                 (const T*)f->vy, (const T*)f->vz);
         });
@@ -623,8 +598,8 @@ void launchIadVe(sphx_workspace* ws, const PairArgs& a, const IadVeFields& vf, c
     RecAv<T>* next = chainable(a, p) && f->c ? recordBuffer<RecAv<T>>(ws, a.numParticles, 1 - in) : nullptr;
     {
         KernelScope timer(ws, "iad_divv_curlv");
-        launchWide<T>(ws->nbWide, [&](auto wide) {
-            iadDivvCurlvKernel<T, decltype(wide)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_IAD) : 0, ws->stream>>>(
+        launchVariant<T>(ws, [&](auto variant) {
+            iadDivvCurlvKernel<T, decltype(variant)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_IAD) : 0, ws->stream>>>(
                 a, vf, rec, sincKernel<T>(ws), next, (const T*)f->c);
         });
         SPHX_CHECK_LAUNCH();
@@ -650,8 +625,8 @@ void launchAv(sphx_workspace* ws, const PairArgs& a, const AvFields& af, const s
         chainable(a, p) && f->m && f->prho ? recordBuffer<RecMomVe<T>>(ws, a.numParticles, 1 - in) : nullptr;
     {
         KernelScope timer(ws, "av_switches");
-        launchWide<T>(ws->nbWide, [&](auto wide) {
-            avSwitchesKernel<T, decltype(wide)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_AV) : 0, ws->stream>>>(
+        launchVariant<T>(ws, [&](auto variant) {
+            avSwitchesKernel<T, decltype(variant)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_AV) : 0, ws->stream>>>(
                 a, af, rec, sincKernel<T>(ws), p->minDt, T(p->alphamin), T(p->alphamax), T(p->decay_constant), next);
         });
         SPHX_CHECK_LAUNCH();
@@ -673,13 +648,13 @@ void launchMomVe(sphx_workspace* ws, const PairArgs& a, const MomVeFields& mf, c
         SPHX_CHECK_LAUNCH();
     }
     KernelScope timer(ws, "momentum_ve");
-    launchWide<T>(ws->nbWide, [&](auto wide) {
-        constexpr bool W = decltype(wide)::value;
+    launchVariant<T>(ws, [&](auto variant) {
+        constexpr int V = decltype(variant)::value;
         if (avClean)
-            momentumVeKernel<T, true, W><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(
+            momentumVeKernel<T, true, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(
                 a, mf, rec, sincKernel<T>(ws), T(p->Atmin), T(p->Atmax), T(p->ramp), float(p->Kcour), dt);
         else
-            momentumVeKernel<T, false, W><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(
+            momentumVeKernel<T, false, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(
                 a, mf, rec, sincKernel<T>(ws), T(p->Atmin), T(p->Atmax), T(p->ramp), float(p->Kcour), dt);
     });
     SPHX_CHECK_LAUNCH();

@@ -158,25 +158,25 @@ struct XMassSum
     static constexpr int  kBatch     = isMixed<Th> ? 1 : 2; // FP32 evaluates W, no gather to overlap
     SincKernel<Th>        kern;
     Th                    hInv;
-    Acc<Th>               rho0;
-    typename SincKernel<Th>::FetchW w[kBatch];
-    Th                          mj[kBatch];
-    bool                        on[kBatch];
+    Acc                   rho0;
+    double                w[kBatch];
+    Th                    mj[kBatch];
+    bool                  on[kBatch];
 
     __device__ __forceinline__ void stage(int u, bool stored, double dx, double dy, double dz, double m)
     {
         Th rx = Th(dx), ry = Th(dy), rz = Th(dz);
-        Th dist = fastSqrt(rx * rx + ry * ry + rz * rz);
-        on[u]   = stored;
-        mj[u]   = Th(m);
-        w[u]    = kern.fetchW(stored ? dist * hInv : Th(4)); // 4: past the support, W = 0
+        Th z  = (rx * rx + ry * ry + rz * rz) * (hInv * hInv);
+        on[u] = stored;
+        mj[u] = Th(m);
+        w[u]  = kern.template w<kAnyIndex>(stored ? z : Th(4)); // 4: the edge of the support, W = 0
     }
     __device__ __forceinline__ void flush()
     {
 #pragma unroll
         for (int u = 0; u < kBatch; ++u)
         {
-            rho0.addIf(on[u], value(w[u]) * mj[u]);
+            rho0.addIf(on[u], w[u] * double(mj[u]));
         }
     }
 };
@@ -797,9 +797,9 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
         if constexpr (XMass)
         {
             if constexpr (isMixed<Th>) { sink.kern.n = a.sincN, sink.kern.ni = a.sincInt; }
-            else { sink.kern.w = static_cast<const TabPair<double>*>(a.wh); }
+            else { sink.kern.wTab = static_cast<const TabPair<double>*>(a.wh); }
             sink.hInv = Th(1) / hi;
-            sink.rho0 = Acc<Th>(mi);
+            sink.rho0 = Acc(double(mi));
         }
     };
     resetSink();
@@ -840,7 +840,7 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
             // epilogue of xmassKernel: FP64 normalisation with h^-3 rounded in h's type
             const Th hInv    = Th(1) / hi;
             const Th h3Inv   = hInv * hInv * hInv;
-            double   rhoZero = double(sink.rho0.value()) * a.K * double(h3Inv);
+            double   rhoZero = sink.rho0.value() * a.K * double(h3Inv);
             Th       xmi     = Th(double(mi) / rhoZero);
             static_cast<Th*>(a.xmOut)[t.i] = a.toRho ? Th(mi / xmi) : xmi;
         }

@@ -197,6 +197,14 @@ __device__ __forceinline__ T fastSqrt(T a)
     else { return sqrt(a); }
 }
 
+//! a / sqrt(d2)
+template<class T>
+__device__ __forceinline__ T overDistance(T a, T d2)
+{
+    if constexpr (isMixed<T>) { return a * __builtin_amdgcn_rsqf(d2); }
+    else { return a / sqrt(d2); }
+}
+
 /*! Batched walk over one lane's neighbour list.
  *
  * A pair loop visits its neighbours U at a time (U = 1, 2 or a multiple of 4): load(k) makes the records of
@@ -273,95 +281,58 @@ struct NeighborBatch
     //! whether member u of the batch starting at slot k is a real neighbour
     __device__ __forceinline__ bool in(unsigned k, int u) const { return k + u < n; }
 
-    //! a kernel weight of member u, zeroed for a clamped slot. Every pair term of the loops is
-    //! proportional to a kernel weight, so a clamped slot contributes exactly zero without a branch
-    //! (a branch would let the compiler sink that member's loads behind it).
+    //! the argument z = (r/h)^2 of member u's kernel weight, moved to the edge of the support for a
+    //! clamped slot. Every pair term of the loops is proportional to a kernel weight, so a clamped slot
+    //! contributes exactly zero without a branch (a branch would let the compiler sink that member's
+    //! loads behind it).
     template<class T>
-    __device__ __forceinline__ T live(unsigned k, int u, T w) const
+    __device__ __forceinline__ T live2(unsigned k, int u, T z) const
     {
-        return in(k, u) ? w : T(0);
+        return in(k, u) ? z : T(4);
     }
 };
-
-//! table entry of argument v, fetched ahead of its interpolation
-template<class T, class E>
-struct TableFetch
-{
-    E   e;
-    T   v;
-    int idx;
-};
-
-template<class T, class E>
-__device__ __forceinline__ TableFetch<T, E> fetch(const E* __restrict__ table, T v)
-{
-    TableFetch<T, E> f;
-    f.v   = v;
-    f.idx = tableInterval(v);
-    f.e   = table[f.idx];
-    return f;
-}
-
-template<class T>
-__device__ __forceinline__ T value(const TableFetch<T, TabPair<T>>& f)
-{
-    return interpolate(f.e.t0, f.e.t1, f.v, f.idx);
-}
-
-template<class T>
-__device__ __forceinline__ void values(const TableFetch<T, TabQuad<T>>& f, T& w, T& dw)
-{
-    w  = interpolate(f.e.w0, f.e.w1, f.v, f.idx);
-    dw = interpolate(f.e.d0, f.e.d1, f.v, f.idx);
-}
 
 /*! The SPH kernel W(v) = sinc(pi v / 2)^n and dW/dv on [0, 2), zero from v = 2 on.
  *
- * The FP64 form interpolates the reference's 20000-point tables (lookup), so its values are the
- * reference's. The FP32 form evaluates the function itself. A table lookup is a 64-lane gather
- * that touches about one cache line per lane, and the pair loops are bound by that gather
- * traffic, while the ALUs are mostly idle. The evaluation runs in FP64 arithmetic, which on this
- * GPU issues at the FP32 rate (FP32 ops are not packed here), and is rounded once to FP32: its
- * error is the final rounding, below that of the FP32 table (values rounded to FP32, then
- * interpolated in FP32), and its difference from the FP64 table's interpolant is the
- * interpolation error, about 6e-9 of W(0) for n = 6.
+ * Both forms evaluate the kernel as a function of z = v^2, without a square root, a reciprocal or a
+ * table: sinc(pi v / 2) = (1 - z/4) P(z), whose first factor carries the zero at the edge of the
+ * support exactly (so sinc keeps its relative accuracy up to there) and whose second is a polynomial
+ * fitted at Chebyshev nodes of [0, 4]; d sinc/dz is a polynomial of its own. A table lookup is a
+ * 64-lane gather that touches about one cache line per lane, and a separate sine, cosine and
+ * reciprocal cost three times the arithmetic of the polynomial. W = sinc^n by multiplication for an
+ * integer n (the reference's sinc indices); for other n the FP32 form takes FP32 log2 / exp2 and the
+ * FP64 form its tables.
  *
- * With x = pi v / 2: sin x from its Taylor polynomial on [0, pi/2] (to t^13; the remainder is
- * below 7e-10), reached for v > 1 through sin x = sin y, cos x = -cos y, y = (2 - v) pi/2 formed
- * from the exact 2 - v, so sinc keeps its relative accuracy up to the edge of the support;
- * sinc = sin x / x and d sinc/dx = (cos x - sinc) / x (1 and 0 at x = 0), with 1/x from the
- * hardware reciprocal and one Newton step; W = sinc^n by repeated multiplication for an integer
- * n (the reference's sinc indices), else through FP32 log2 / exp2; dW/dv = n sinc^(n-1)
- * d sinc/dx pi/2. */
-struct DirectW
+ * FP32 form: P and d sinc/dz of degree 6, relative error 6e-11, in FP64 arithmetic (which on this GPU
+ * issues at the FP32 rate, since FP32 ops are not packed here), so W is exact to its final rounding.
+ *
+ * FP64 form: the reference interpolates W linearly in a 20000-point table, up to 6e-9 off the function
+ * for n = 6, and the FP64 results are held to that interpolant. With t = the fraction of v / dx,
+ * the interpolant differs from W(v) by
+ *     L(v) - W(v) = 1/2 dx^2 t (1 - t) W''(v + dx (1 - 2t) / 3) + O(dx^4),
+ * so it is formed as W(v) plus that term, with P of degree 9 (2e-17) and d sinc/dz in the
+ * correction of degree 5 (5e-9 of a term below 6e-9). It equals the interpolated table entries to
+ * 2e-15 of W(0) for n = 3, 5, 6 and 9. W'' follows from Y = d sinc/dv = 2 v sinc_z and the equation of the
+ * sinc function, Y' = -(pi/2)^2 sinc - 4 sinc_z. */
+constexpr double kHalfPiSq = 2.4674011002723396547; // (pi/2)^2
+
+/*! The loops are compiled per variant, chosen on the host for a launch (launchVariant):
+ * kCommon: the default sinc index 6, its powers unrolled; in the FP32 form the wrapping fixed-point
+ * separation as well. kWide (FP32 form): the exact separations of boxes a few smoothing lengths wide, any
+ * index. kAnyIndex: any other sinc index. */
+enum Variant
 {
-    float w, v;
+    kCommon,
+    kWide,
+    kAnyIndex
 };
-struct DirectWD
-{
-    float w, dw, v;
-};
+constexpr int kDefaultIndex = 6;
 
-__device__ __forceinline__ float value(const DirectW& f) { return f.w; }
-
-__device__ __forceinline__ void values(const DirectWD& f, float& w, float& dw)
+//! x^k for a small integer k >= 0 (wave-uniform loop)
+__device__ __forceinline__ double sincPower(double x, int k)
 {
-    w  = f.w;
-    dw = f.dw;
-}
-
-//! x^k for a small integer k >= 0 (wave-uniform loop), or 2^(k log2 x) when k is not an integer
-__device__ __forceinline__ double sincPower(double x, float k, int ki)
-{
-    if (ki == 5)
-    {
-        // the default sinc index 6 (sinc^5 here): the products of the loop below, unrolled
-        const double x2 = x * x;
-        return x * (x2 * x2);
-    }
-    if (ki < 0) { return double(__builtin_amdgcn_exp2f(k * __builtin_amdgcn_logf(float(x)))); }
     double r = 1.0, b = x;
-    for (int e = ki; e > 0; e >>= 1)
+    for (int e = k; e > 0; e >>= 1)
     {
         if (e & 1) { r *= b; }
         b *= b;
@@ -369,92 +340,219 @@ __device__ __forceinline__ double sincPower(double x, float k, int ki)
     return r;
 }
 
-template<bool Derivative>
-__device__ __forceinline__ void sincDirect(float vf, float n, int ni, float& w, float& dw)
+//! sinc(pi v / 2) at z = v^2 in [0, 4], relative error 6e-11 (FP32 form)
+__device__ __forceinline__ double sincOfZ6(double z)
 {
-    constexpr double halfPi = 1.57079632679489661923;
-    const double     v      = vf;
-    const bool       upper  = v > 1.0;
-    const double     x      = v * halfPi;
-    const double     y      = upper ? (2.0 - v) * halfPi : x; // in [0, pi/2] on the support
-    const double     y2     = y * y;
-    // sin y = y (1 - y^2/3! + ... - y^12/13!)
-    double sy = -1.0 / 6227020800.0;
-    sy        = sy * y2 + 1.0 / 39916800.0;
-    sy        = sy * y2 - 1.0 / 362880.0;
-    sy        = sy * y2 + 1.0 / 5040.0;
-    sy        = sy * y2 - 1.0 / 120.0;
-    sy        = sy * y2 + 1.0 / 6.0;
-    sy        = y - y * y2 * sy;
-    double xInv = double(__builtin_amdgcn_rcpf(float(x)));
-    xInv        = xInv + xInv * (1.0 - x * xInv);
-    const bool   zero   = vf == 0.0f;
-    const double sinc   = zero ? 1.0 : sy * xInv;
-    const bool   inside = vf < 2.0f;
-    const double pm1    = sincPower(sinc, n - 1.0f, ni - 1); // sinc^(n-1)
-    w                   = inside ? float(pm1 * sinc) : 0.0f;
-    if constexpr (Derivative)
-    {
-        // cos y = 1 - y^2/2! + ... + y^14/14!
-        double cy = -1.0 / 87178291200.0;
-        cy        = cy * y2 + 1.0 / 479001600.0;
-        cy        = cy * y2 - 1.0 / 3628800.0;
-        cy        = cy * y2 + 1.0 / 40320.0;
-        cy        = cy * y2 - 1.0 / 720.0;
-        cy        = cy * y2 + 1.0 / 24.0;
-        cy        = cy * y2 - 0.5;
-        cy        = 1.0 + y2 * cy;
-        const double cx = upper ? -cy : cy;
-        const double ds = zero ? 0.0 : (cx - sinc) * xInv;
-        dw              = inside ? float(double(n) * pm1 * ds * halfPi) : 0.0f;
-    }
+    double p = 1.4453064921222513e-09;
+    p        = p * z - 1.3731223424662021e-07;
+    p        = p * z + 8.607989820798515e-06;
+    p        = p * z - 0.00037411264408295246;
+    p        = p * z + 0.010425519738884937;
+    p        = p * z - 0.161233516047257;
+    p        = p * z + 0.9999999999728735;
+    return p - 0.25 * z * p;
+}
+
+//! d sinc(pi v / 2) / dz, absolute error 6e-11
+__device__ __forceinline__ double sincSlope6(double z)
+{
+    double q = -2.5764109465564327e-09;
+    q        = q * z + 2.152531546520502e-07;
+    q        = q * z - 1.1449615339245935e-05;
+    q        = q * z + 0.00040855196998758054;
+    q        = q * z - 0.0089414863396859;
+    q        = q * z + 0.10146780180875682;
+    return q * z - 0.4112335166569054;
+}
+
+//! sinc(pi v / 2) at z = v^2 in [0, 4] to FP64 rounding
+__device__ __forceinline__ double sincOfZ9(double z)
+{
+    double p = -5.823067516159113e-16;
+    p        = p * z + 1.0839061254289035e-13;
+    p        = p * z - 1.501141501734521e-11;
+    p        = p * z + 1.643032500260312e-09;
+    p        = p * z - 1.3837782504438124e-07;
+    p        = p * z + 8.610867685597616e-06;
+    p        = p * z - 0.0003741166513510571;
+    p        = p * z + 0.010425522402193063;
+    p        = p * z - 0.16123351671205632;
+    p        = p * z + 1.0;
+    return p - 0.25 * z * p;
+}
+
+//! d sinc(pi v / 2) / dz to FP64 rounding
+__device__ __forceinline__ double sincSlope9(double z)
+{
+    double q = 1.4701693771604546e-15;
+    q        = q * z - 2.4939334615094517e-13;
+    q        = q * z + 3.0892145129869457e-11;
+    q        = q * z - 2.9803963653457545e-09;
+    q        = q * z + 2.174249574964597e-07;
+    q        = q * z - 1.1455473771406392e-05;
+    q        = q * z + 0.00040856012212963613;
+    q        = q * z - 0.008941491755716072;
+    q        = q * z + 0.1014678031604184;
+    return q * z - 0.4112335167120566;
+}
+
+//! d sinc(pi v / 2) / dz, absolute error 5e-9 (the interpolation term)
+__device__ __forceinline__ double sincSlope5(double z)
+{
+    double q = 1.843090979760722e-07;
+    q        = q * z - 1.1310217672036537e-05;
+    q        = q * z + 0.0004082624607906118;
+    q        = q * z - 0.00894121445580337;
+    q        = q * z + 0.10146770837624979;
+    return q * z - 0.4112335114493841;
+}
+
+/*! The point where the linear interpolation between table nodes differs from W by weight * W'':
+ * weight = 1/2 dx^2 t (1 - t), at z1 = (v + dx (1 - 2t) / 3)^2 and sinc s1 there. Only t's value to about
+ * 1e-9 matters, so v = sqrt(z) takes one Newton step from the hardware reciprocal root. */
+struct InterpolationPoint
+{
+    double weight, z1, s1, slope;
+    double back; // v over the shifted v
+};
+__device__ __forceinline__ InterpolationPoint interpolationPoint(double z, double s)
+{
+    constexpr double   dx = 2.0 / (kTableSize - 1);
+    const double       zc = z > 1e-280 ? z : 1e-280;
+    const double       rs = __builtin_amdgcn_rsq(zc);
+    double             v  = zc * rs;
+    v                     = v + 0.5 * rs * (zc - v * v);
+    const double       t  = __builtin_amdgcn_fract(v * (1.0 / dx));
+    InterpolationPoint i;
+    i.weight       = (0.5 * dx * dx) * (t - t * t);
+    const double shift = dx / 3.0 - (2.0 / 3.0) * dx * t;
+    const double u     = 2.0 * v * shift; // z1 - z
+    i.z1               = z + u;
+    i.back             = 1.0 - shift * rs;
+    i.slope        = sincSlope5(i.z1);
+    i.s1           = s + u * i.slope;
+    return i;
 }
 
 template<class T>
 struct SincKernel;
 
-//! FP64: the reference's tables (W, dW/dv, and both per interval)
+//! FP64: the reference's interpolant for the default index (see above), its tables for any other
 template<>
 struct SincKernel<double>
 {
-    const TabPair<double>* w;
-    const TabPair<double>* dw;
-    const TabQuad<double>* wq;
-    using FetchW  = TableFetch<double, TabPair<double>>;
-    using FetchWD = TableFetch<double, TabQuad<double>>;
+    const TabPair<double>* wTab;
+    const TabQuad<double>* wqTab;
 
-    __device__ __forceinline__ FetchW  fetchW(double v) const { return fetch(w, v); }
-    __device__ __forceinline__ FetchWD fetchWD(double v) const { return fetch(wq, v); }
-    __device__ __forceinline__ double  W(double v) const { return lookup(w, v); }
-    __device__ __forceinline__ double  dW(double v) const { return lookup(dw, v); }
+    //! W at z = v^2
+    template<int V>
+    __device__ __forceinline__ double w(double z) const
+    {
+        if constexpr (V != kCommon) { return lookup(wTab, sqrt(z)); }
+        else
+        {
+            constexpr double n         = kDefaultIndex;
+            z                          = z < 4.0 ? z : 4.0;
+            const double             s = sincOfZ9(z);
+            const InterpolationPoint i = interpolationPoint(z, s);
+            const double             q = i.s1 * i.s1; // s1^(n-2) = q^2
+            const double yp            = -kHalfPiSq * i.s1 - 4.0 * i.slope;
+            const double w2            = (q * q) * ((n - 1.0) * 4.0 * i.z1 * (i.slope * i.slope) + i.s1 * yp);
+            const double c             = s * s * s;
+            return c * c + (n * i.weight) * w2;
+        }
+    }
+
+    //! W and v dW/dv at z = v^2
+    template<int V>
+    __device__ __forceinline__ void wAndVdw(double z, double& w, double& vdw) const
+    {
+        if constexpr (V != kCommon)
+        {
+            const double v = sqrt(z);
+            double       dw;
+            lookupBoth(wqTab, v, w, dw);
+            vdw = v * dw;
+        }
+        else
+        {
+            constexpr double n          = kDefaultIndex;
+            z                           = z < 4.0 ? z : 4.0;
+            const double             s  = sincOfZ9(z);
+            const InterpolationPoint i  = interpolationPoint(z, s);
+            const double             q  = i.s1 * i.s1, p3 = q * i.s1, p2 = q * q; // s1^(n-3), s1^(n-2)
+            const double             yp = -kHalfPiSq * i.s1 - 4.0 * i.slope;
+            const double             vy = 2.0 * i.z1 * i.slope;
+            const double w2  = p2 * (2.0 * (n - 1.0) * vy * i.slope + i.s1 * yp);
+            const double vw3 = p3 * (2.0 * (n - 1.0) * (n - 2.0)) * (vy * vy) * i.slope +
+                               p2 * (3.0 * (n - 1.0) * vy * yp + i.s1 * (4.0 * i.slope - 2.0 * yp - kHalfPiSq * vy));
+            const double c   = s * s, pm1 = c * c * s;
+            w                = pm1 * s + (n * i.weight) * w2;
+            vdw              = 2.0 * n * z * pm1 * sincSlope9(z) + (n * i.weight * i.back) * vw3;
+            // the reference forms its dW/dv table from cot x - 1/x, whose cancellation leaves an error of
+            // 1e-16 / v in the entries: below v = 1/4 the entries themselves are taken
+            if (z < 1.0 / 16.0)
+            {
+                const double     v = sqrt(z);
+                const int        k = tableInterval(v);
+                const TabQuad<double>* e = wqTab + k;
+                vdw = v * interpolate(e->d0, e->d1, v, k);
+            }
+        }
+    }
+
+    //! W and dW/dv at v from the tables (the adjoints)
+    __device__ __forceinline__ void wAndDw(double v, double& w, double& dw) const { lookupBoth(wqTab, v, w, dw); }
 };
 
-//! FP32: evaluated directly (sincDirect)
+//! FP32: the kernel function itself, in FP64 arithmetic
 template<>
 struct SincKernel<float>
 {
     float n;
-    int   ni; // n when it is an integer, else -1
-    using FetchW  = DirectW;
-    using FetchWD = DirectWD;
+    int   ni; // n when it is an integer >= 2, else -1
 
-    __device__ __forceinline__ FetchW fetchW(float v) const
+    template<int V>
+    __device__ __forceinline__ double index() const
     {
-        FetchW f;
-        float  unused;
-        f.v = v;
-        sincDirect<false>(v, n, ni, f.w, unused);
-        return f;
+        return V == kCommon ? double(kDefaultIndex) : double(n);
     }
-    __device__ __forceinline__ FetchWD fetchWD(float v) const
+    //! s^(n-1), 0 at the edge of the support
+    template<int V>
+    __device__ __forceinline__ double power(double s) const
     {
-        FetchWD f;
-        f.v = v;
-        sincDirect<true>(v, n, ni, f.w, f.dw);
-        return f;
+        if constexpr (V == kCommon)
+        {
+            const double c = s * s;
+            return c * c * s;
+        }
+        else
+        {
+            if (ni > 0) { return sincPower(s, ni - 1); }
+            return s > 0.0 ? double(__builtin_amdgcn_exp2f((n - 1.0f) * __builtin_amdgcn_logf(float(s)))) : 0.0;
+        }
     }
-    __device__ __forceinline__ float W(float v) const { return fetchW(v).w; }
-    __device__ __forceinline__ float dW(float v) const { return fetchWD(v).dw; }
+    template<int V>
+    __device__ __forceinline__ double w(float zf) const
+    {
+        const double s = sincOfZ6(double(fminf(zf, 4.0f)));
+        return power<V>(s) * s;
+    }
+    template<int V>
+    __device__ __forceinline__ void wAndVdw(float zf, double& w, double& vdw) const
+    {
+        const double z = double(fminf(zf, 4.0f));
+        const double s = sincOfZ6(z), p = power<V>(s);
+        w              = p * s;
+        vdw            = (2.0 * index<V>()) * z * p * sincSlope6(z);
+    }
+    __device__ __forceinline__ void wAndDw(float vf, float& w, float& dw) const
+    {
+        const double v = double(fminf(vf, 2.0f)), z = v * v;
+        const double s = sincOfZ6(z), p = power<kAnyIndex>(s);
+        w              = float(p * s);
+        dw             = float((2.0 * double(n)) * v * p * sincSlope6(z));
+    }
 };
 
 /*! Whether a wave must apply the legacy fold (sfc/box.hpp:218-238). The fold changes a separation
@@ -493,11 +591,11 @@ __device__ __forceinline__ void separation(const DevBox& b, double r, double xi,
     rx = T(d[0]), ry = T(d[1]), rz = T(d[2]);
 }
 
-//! separation of a pair and its length
+//! separation of a pair and its squared length
 template<class T>
 struct Sep
 {
-    T x, y, z, d;
+    T x, y, z, d2;
 };
 
 /*! Position of a particle in the neighbour records: FP64 in the plain form; in the FP32 form
@@ -563,35 +661,29 @@ __device__ __forceinline__ Sep<T> pairSeparation(const DevBox& b, double r2h, co
         s.z = float(int32_t(ri.z - rj.z)) * b.fixStep[2];
     }
     else { separation<Fold>(b, r2h, ri.x, ri.y, ri.z, rj.x, rj.y, rj.z, s.x, s.y, s.z); }
-    s.d = fastSqrt(s.x * s.x + s.y * s.y + s.z * s.z);
+    s.d2 = s.x * s.x + s.y * s.y + s.z * s.z;
     return s;
 }
 
-/*! whether the wave of target record ri must fold its FP64 separations; in the FP32 form, Wide: the
+/*! whether the wave of target record ri must fold its FP64 separations; in the FP32 form, kWide: the
  * last search met a target whose support 2h reaches half a box length, where the wrapping 32-bit
  * difference stops standing for the reference's separation (see Coord above), so the loop takes the
- * exact 64-bit difference. Wide is a kernel template argument, chosen on the host (launchWide), so
- * that the common loop carries none of the registers of the exact path. */
-template<class T, bool Wide, class R>
+ * exact 64-bit difference. The variant is a kernel template argument, chosen on the host
+ * (launchVariant), so that the common loop carries none of the registers of the others. */
+template<class T, int V, class R>
 __device__ __forceinline__ bool recordNeedsFold(const DevBox& b, const R& ri, double r2h)
 {
-    if constexpr (isMixed<T>) { return Wide; }
+    if constexpr (isMixed<T>) { return V == kWide; }
     else { return waveNeedsFold(b, ri.x, ri.y, ri.z, r2h); }
 }
 
-//! host: launch(std::bool_constant<Wide>) with Wide = `wide` in the FP32 form, false in the FP64 form
+//! host: launch(std::integral_constant<int, V>) with the loop variant V of this search and sinc index
 template<class T, class F>
-inline void launchWide(bool wide, F&& launch)
+inline void launchVariant(const sphx_workspace* ws, F&& launch)
 {
-    if constexpr (isMixed<T>)
-    {
-        if (wide)
-        {
-            launch(std::true_type{});
-            return;
-        }
-    }
-    launch(std::false_type{});
+    if (isMixed<T> && ws->nbWide) { launch(std::integral_constant<int, kWide>{}); }
+    else if (ws->sincIndex != double(kDefaultIndex)) { launch(std::integral_constant<int, kAnyIndex>{}); }
+    else { launch(std::integral_constant<int, kCommon>{}); }
 }
 
 //! run `loop` with the fold compiled in or out, chosen once per wave
@@ -602,37 +694,17 @@ __device__ __forceinline__ void withFold(bool fold, F&& loop)
     else { loop(std::false_type{}); }
 }
 
-//! compensated accumulator (Kahan) for the FP32 form, plain sum for FP64
-template<class T>
+//! FP64 accumulator of both forms. The FP32 form's density, grad-h and energy sums add their terms in
+//! FP64 (the kernel values come in FP64 anyway): two instructions a term where a compensated FP32 sum
+//! takes four, and no larger error.
 struct Acc
 {
-    T s, c;
-    __device__ __forceinline__ explicit Acc(T init = T(0)) : s(init), c(0) {}
-    __device__ __forceinline__ void add(T v)
-    {
-        if constexpr (isMixed<T>)
-        {
-            T y  = v - c;
-            T t2 = s + y;
-            c    = (t2 - s) - y;
-            s    = t2;
-        }
-        else { s += v; }
-    }
-    //! add(v) where p holds, the state untouched elsewhere (branch-free)
-    __device__ __forceinline__ void addIf(bool p, T v)
-    {
-        if constexpr (isMixed<T>)
-        {
-            T y  = v - c;
-            T t2 = s + y;
-            T c2 = (t2 - s) - y;
-            s    = p ? t2 : s;
-            c    = p ? c2 : c;
-        }
-        else { s = p ? s + v : s; }
-    }
-    __device__ __forceinline__ T value() const { return s; }
+    double s;
+    __device__ __forceinline__ explicit Acc(double init = 0.0) : s(init) {}
+    __device__ __forceinline__ void add(double v) { s += v; }
+    //! add(v) where p holds
+    __device__ __forceinline__ void addIf(bool p, double v) { s = p ? s + v : s; }
+    __device__ __forceinline__ double value() const { return s; }
 };
 
 //! positive-double minimum through the integer order of their bit patterns
@@ -730,14 +802,14 @@ inline SincKernel<T> sincKernel(sphx_workspace* ws)
     SincKernel<T> k;
     if constexpr (isMixed<T>)
     {
-        k.n  = float(ws->sincIndex);
-        k.ni = ws->sincIndex == double(int(ws->sincIndex)) && ws->sincIndex < 64 ? int(ws->sincIndex) : -1;
+        const double n = ws->sincIndex;
+        k.n            = float(n);
+        k.ni           = n == double(int(n)) && n >= 2 && n < 64 ? int(n) : -1;
     }
     else
     {
-        k.w  = ws->wh64.get();
-        k.dw = ws->whd64.get();
-        k.wq = ws->whq64.get();
+        k.wTab  = ws->wh64.get();
+        k.wqTab = ws->whq64.get();
     }
     return k;
 }
