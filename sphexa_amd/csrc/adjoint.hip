@@ -93,10 +93,10 @@ struct DensityVjpArgs
 constexpr int kDensityNq = 3; // neighbour-side record: gx, gy, gz
 
 template<class T>
-__global__ void __launch_bounds__(kPairWaves * kWave)
+__global__ void __launch_bounds__(kVjpWaves * kWave)
     densityStdVjpKernel(PairArgs a, DensityVjpArgs f, SincKernel<T> kern, PairOut<T> out)
 {
-    Lane t = laneTarget(a.L);
+    const Lane t = vjpTarget(a.L);
     if (!t.valid) { return; }
     const uint32_t i    = t.i;
     const T        hi   = ld<T>(f.h, i);
@@ -112,13 +112,10 @@ __global__ void __launch_bounds__(kPairWaves * kWave)
         for (unsigned k0 = 0; k0 < t.n; k0 += U)
         {
             uint32_t j[U], e[U];
+            a.L.lists.quad(t.r, k0, j);
 #pragma unroll
             for (int u = 0; u < U; ++u)
-            {
-                const unsigned kk = min(k0 + u, t.n - 1);
-                j[u]              = t.list[laneSlot(kk)];
-                e[u]              = out.recordOf[ps + kk];
-            }
+                e[u] = out.recordOf[ps + min(k0 + u, t.n - 1)];
             double xj[U], yj[U], zj[U];
             T      mj[U];
 #pragma unroll
@@ -157,10 +154,10 @@ struct IadVjpArgs
 constexpr int kIadNq = 4; // neighbour-side record: gx, gy, gz, grho
 
 template<class T>
-__global__ void __launch_bounds__(kPairWaves * kWave)
+__global__ void __launch_bounds__(kVjpWaves * kWave)
     iadStdVjpKernel(PairArgs a, IadVjpArgs f, SincKernel<T> kern, PairOut<T> out)
 {
-    Lane t = laneTarget(a.L);
+    const Lane t = vjpTarget(a.L);
     if (!t.valid) { return; }
     const uint32_t i    = t.i;
     const T        hi   = ld<T>(f.h, i);
@@ -192,13 +189,10 @@ __global__ void __launch_bounds__(kPairWaves * kWave)
         for (unsigned k0 = 0; k0 < t.n; k0 += U)
         {
             uint32_t j[U], e[U];
+            a.L.lists.quad(t.r, k0, j);
 #pragma unroll
             for (int u = 0; u < U; ++u)
-            {
-                const unsigned kk = min(k0 + u, t.n - 1);
-                j[u]              = t.list[laneSlot(kk)];
-                e[u]              = out.recordOf[ps + kk];
-            }
+                e[u] = out.recordOf[ps + min(k0 + u, t.n - 1)];
             double xj[U], yj[U], zj[U];
             T      mjs[U], rhojs[U];
 #pragma unroll
@@ -273,10 +267,10 @@ __device__ __forceinline__ void symOuter(const T u[3], const T r[3], T out[6])
 constexpr int kMomNq = 13;
 
 template<class T>
-__global__ void __launch_bounds__(kPairWaves * kWave)
+__global__ void __launch_bounds__(kVjpWaves * kWave)
     momentumStdVjpKernel(PairArgs a, MomVjpArgs f, SincKernel<T> kern, PairOut<T> out)
 {
-    Lane t = laneTarget(a.L);
+    const Lane t = vjpTarget(a.L);
     if (!t.valid) { return; }
     const uint32_t i      = t.i;
     const T        hi     = ld<T>(f.h, i);
@@ -298,9 +292,12 @@ __global__ void __launch_bounds__(kPairWaves * kWave)
 
     const uint32_t ps = out.firstPair(i);
     withFold(waveNeedsFold(a.box, xi, yi, zi, r2h), [&](auto fold) {
+        uint32_t jq[4];
         for (unsigned k = 0; k < t.n; ++k)
         {
-            const uint32_t j = t.list[laneSlot(k)];
+            if ((k & 3u) == 0) { a.L.lists.quad(t.r, k, jq); }
+            const uint32_t j = jq[0];
+            jq[0] = jq[1], jq[1] = jq[2], jq[2] = jq[3];
             const uint32_t e = out.recordOf[ps + k];
             T              r[3];
             separation<decltype(fold)::value>(a.box, r2h, xi, yi, zi, a.x[j], a.y[j], a.z[j], r[0], r[1], r[2]);
@@ -413,15 +410,15 @@ __global__ void pairCountKernel(const uint32_t* __restrict__ nc, uint32_t nbFirs
 }
 
 //! key (j << pbits) | p of every stored pair p = pairStart[t] + k, j the neighbour in slot k of target t
-__global__ void pairKeysKernel(const uint32_t* __restrict__ nbrs, const uint32_t* __restrict__ pairStart, uint32_t nt,
-                               uint32_t ngmax4, int pbits, uint64_t* __restrict__ keys)
+__global__ void pairKeysKernel(NeighborLists lists, const uint32_t* __restrict__ pairStart, uint32_t nt, int pbits,
+                               uint64_t* __restrict__ keys)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nt) { return; }
     const uint32_t p0 = pairStart[t], n = pairStart[t + 1] - p0;
     for (uint32_t k = 0; k < n; ++k)
     {
-        const uint32_t j = nbrs[listOffset(t / kGroup, ngmax4, k, t % kGroup)];
+        const uint32_t j = lists.entry(t, k);
         keys[p0 + k]     = (uint64_t(j) << pbits) | uint64_t(p0 + k);
     }
 }
@@ -553,8 +550,8 @@ void buildAdjointPairs(sphx_workspace* ws)
     A.rowStart.reserve(size_t(n) + 1);
     if (pairs > 0)
     {
-        pairKeysKernel<<<ceilDiv(nt, 256), 256, 0, ws->stream>>>(ws->nbrs.get(), A.pairStart.get(), nt,
-                                                                  paddedNgmax(ws->nbNgmax), pbits, A.keys.get());
+        pairKeysKernel<<<ceilDiv(nt, 256), 256, 0, ws->stream>>>(neighborLists(ws), A.pairStart.get(), nt, pbits,
+                                                                 A.keys.get());
         SPHX_CHECK_LAUNCH();
         size_t sortBytes = 0;
         SPHX_HIP(rocprim::radix_sort_keys(nullptr, sortBytes, A.keys.get(), A.sorted.get(), size_t(pairs), 0,
@@ -628,14 +625,14 @@ void densityStdVjp(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f
                "density adjoint needs fields h, m, cotangent rho and gradients x, y, z, h");
     requireConsecutive(a);
     DensityVjpArgs d{f->h, f->m, in->rho, out->x, out->y, out->z, out->h};
-    unsigned       blocks = pairBlocks(a.L);
+    unsigned       blocks = vjpBlocks(a.L);
     if (blocks == 0) { return; }
     buildAdjointPairs(ws);
     void* const g[kDensityNq] = {out->x, out->y, out->z};
     auto        run           = [&](auto zero) {
         using T      = decltype(zero);
         PairOut<T> o = pairOut<T>(ws, kPaddedNq<T, kDensityNq>);
-        densityStdVjpKernel<T><<<blocks, kPairWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), o);
+        densityStdVjpKernel<T><<<blocks, kVjpWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), o);
         SPHX_CHECK_LAUNCH();
         pull<T, kDensityNq>(ws, o, first, last, g);
     };
@@ -662,14 +659,14 @@ void iadStdVjp(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f, co
                  out->h,
                  out->rho};
     requireConsecutive(a);
-    unsigned blocks = pairBlocks(a.L);
+    unsigned blocks = vjpBlocks(a.L);
     if (blocks == 0) { return; }
     buildAdjointPairs(ws);
     void* const g[kIadNq] = {out->x, out->y, out->z, out->rho};
     auto        run       = [&](auto zero) {
         using T      = decltype(zero);
         PairOut<T> o = pairOut<T>(ws, kPaddedNq<T, kIadNq>);
-        iadStdVjpKernel<T><<<blocks, kPairWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), o);
+        iadStdVjpKernel<T><<<blocks, kVjpWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), o);
         SPHX_CHECK_LAUNCH();
         pull<T, kIadNq>(ws, o, first, last, g);
     };
@@ -712,7 +709,7 @@ void momentumEnergyStdVjp(sphx_workspace* ws, const DevBox& box, const sphx_fiel
                  out->alpha,
                  {out->c11, out->c12, out->c13, out->c22, out->c23, out->c33}};
     requireConsecutive(a);
-    unsigned blocks = pairBlocks(a.L);
+    unsigned blocks = vjpBlocks(a.L);
     if (blocks == 0) { return; }
     buildAdjointPairs(ws);
     void* const g[kMomNq] = {out->x,   out->y,   out->z,   out->h,   out->rho, out->p,  out->alpha,
@@ -720,7 +717,7 @@ void momentumEnergyStdVjp(sphx_workspace* ws, const DevBox& box, const sphx_fiel
     auto        run       = [&](auto zero) {
         using T      = decltype(zero);
         PairOut<T> o = pairOut<T>(ws, kPaddedNq<T, kMomNq>);
-        momentumStdVjpKernel<T><<<blocks, kPairWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), o);
+        momentumStdVjpKernel<T><<<blocks, kVjpWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), o);
         SPHX_CHECK_LAUNCH();
         pull<T, kMomNq>(ws, o, first, last, g);
     };

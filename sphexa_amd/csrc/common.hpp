@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -25,21 +26,83 @@ constexpr int      kTableSize = 20000;
 constexpr int      kWave      = 64; // gfx950 wavefront
 constexpr int      kGroup     = 64; // targets per neighbour-search group (one wavefront)
 
-/* Neighbour-list layout. Group g of 64 consecutive targets owns ngmax4 = ngmax rounded up to 4
- * slots per lane; slot k of lane l is at
+/* Neighbour-list layouts. Lists are stored per block of 64 consecutive searched targets.
+ *
+ * Local lists: each target group of the search has a table of the particles that are neighbours of any
+ * of its targets, in visiting order, and a target's list holds 16-bit positions in its group's table (group
+ * r / 64 for the r-th searched target, or owner[r] of a search over other groups than consecutive ones).
+ * Slot k of lane l of block g is the 16-bit word
+ *     (g * ngmax8 + (k & ~7)) * 64 + 8 l + (k & 7),
+ * so each lane's slots come in 16-byte octets and octet o of all 64 lanes is one contiguous kilobyte.
+ * The pair loops stage the table's records in LDS once and read every neighbour from there.
+ *
+ * Global lists (the fused search, a search with a table that would not fit, or over so many groups that their
+ * tables would take too much memory): 32-bit particle indices, slot k of lane l of block g at
  *     (g * ngmax4 + (k & ~3)) * 64 + 4 l + (k & 3),
- * so each lane's slots come in 16-byte quads and quad q of all 64 lanes is one contiguous
- * kilobyte: the search stores a lane's entries a quad at a time, and a pair loop reads four
- * neighbour indices of all its lanes with one coalesced 16-byte-per-lane load. */
+ * in 16-byte quads. ngmax4 and ngmax8 are ngmax rounded up to 4 and 8. */
 __host__ __device__ inline uint32_t paddedNgmax(uint32_t ngmax) { return (ngmax + 3u) & ~3u; }
+__host__ __device__ inline uint32_t paddedNgmax8(uint32_t ngmax) { return (ngmax + 7u) & ~7u; }
 
 __host__ __device__ inline size_t listOffset(uint32_t g, uint32_t ngmax4, uint32_t k, uint32_t lane)
 {
     return (size_t(g) * ngmax4 + (k & ~3u)) * kGroup + 4u * lane + (k & 3u);
 }
+__host__ __device__ inline size_t localOffset(uint32_t g, uint32_t ngmax8, uint32_t k, uint32_t lane)
+{
+    return (size_t(g) * ngmax8 + (k & ~7u)) * kGroup + 8u * lane + (k & 7u);
+}
 
-//! slot k relative to a lane's slot 0
-__host__ __device__ inline size_t laneSlot(uint32_t k) { return size_t(k & ~3u) * kGroup + (k & 3u); }
+/*! particles a group's table holds at most. 64 targets of 90 neighbours fill 450-640 entries on a lattice and
+ * 350-900 on the Evrard sphere; a search that meets a larger table stores global lists instead. */
+constexpr uint32_t kTableCap = 2048;
+//! bins of the table sizes' histogram, kTableBin entries each
+constexpr uint32_t kTableBin  = 64;
+constexpr uint32_t kTableBins = kTableCap / kTableBin;
+
+/*! the stored lists of the last search (see the layouts above) */
+struct NeighborLists
+{
+    const void*     nbrs;
+    const uint32_t* table;      // local lists: kTableCap particles per group ...
+    const uint32_t* tableCount; // ... and how many of them are used; null for global lists
+    const uint32_t* owner;      // the searched targets' groups (kNoGroup: not searched), null: consecutive groups
+    uint32_t        ngmax;
+
+    static constexpr uint32_t kNoGroup = 0xffffffffu;
+
+    //! group whose table the r-th target's list refers to
+    __device__ __forceinline__ uint32_t group(uint32_t r) const { return owner ? owner[r] : r / kGroup; }
+
+    //! particles in slots k..k+3 (k a multiple of 4) of the r-th searched target; slots past its count hold its
+    //! last neighbour again
+    __device__ __forceinline__ void quad(uint32_t r, uint32_t k, uint32_t (&j)[4]) const
+    {
+        const uint32_t g = r / kGroup, lane = r % kGroup;
+        if (tableCount == nullptr)
+        {
+            const uint4 q = *reinterpret_cast<const uint4*>(static_cast<const uint32_t*>(nbrs) +
+                                                            listOffset(g, paddedNgmax(ngmax), k, lane));
+            j[0] = q.x, j[1] = q.y, j[2] = q.z, j[3] = q.w;
+            return;
+        }
+        const uint2     q = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(nbrs) +
+                                                        localOffset(g, paddedNgmax8(ngmax), k, lane));
+        const uint32_t* t = table + size_t(group(r)) * kTableCap;
+        j[0] = t[q.x & 0xffffu], j[1] = t[q.x >> 16], j[2] = t[q.y & 0xffffu], j[3] = t[q.y >> 16];
+    }
+
+    //! particle in slot k of the r-th searched target
+    __device__ __forceinline__ uint32_t entry(uint32_t r, uint32_t k) const
+    {
+        const uint32_t g = r / kGroup, lane = r % kGroup;
+        if (tableCount == nullptr)
+        {
+            return static_cast<const uint32_t*>(nbrs)[listOffset(g, paddedNgmax(ngmax), k, lane)];
+        }
+        return table[size_t(group(r)) * kTableCap +
+                     static_cast<const uint16_t*>(nbrs)[localOffset(g, paddedNgmax8(ngmax), k, lane)]];
+    }
+};
 
 /* ---------------------------------------------------------------------------------------------
  * error handling: every entry point returns an sphx_status and records a message
@@ -192,8 +255,10 @@ struct sphx_workspace
 
     sphx::Tree tree;
 
-    // neighbour lists of the last search: group-interleaved [group][k][lane]
-    sphx::DevBuf<uint32_t> nbrs;
+    // neighbour lists of the last search, and their groups' tables when they are local lists
+    sphx::DevBuf<uint32_t> nbrs, nbTable, nbTableCount, nbOwner;
+    bool                   nbLocal = false, nbOwned = false;
+    uint32_t               nbTableHist[sphx::kTableBins + 1] = {}; // groups by table size; the last bin: over kTableCap
     uint32_t               nbFirst = 0, nbLast = 0, nbNgmax = 0;
     const uint32_t*        nbNc = nullptr; // nc array the lists were built with
     bool                   nbValid = false;
@@ -219,6 +284,7 @@ struct sphx_workspace
     bool                   syncTree   = false; // the workspace tree is that sync's (its counts are of its keys)
     uint32_t               syncBucket = 0;     // its bucket size
     sphx::DevBuf<sphx::Chunk16> records; // packed neighbour records of the current pair loop
+    sphx::DevBuf<sphx::Chunk16> recordsGradV; // AV cleaning: packed velocity gradients
     sphx::DevBuf<sphx::Chunk16> records2; // records a pair loop's epilogue writes for the next loop
 
     // record chaining (SPHX_FLAG_CHAIN): every entry point that may write particle fields or the
@@ -375,12 +441,13 @@ __device__ __forceinline__ void groupRange(const Groups& G, uint32_t g, uint32_t
 /* 64-bit slots of the workspace counters: the search's statistics (stored pairs, maximum count,
  * non-converged targets) in 0-2, the Courant dt of the momentum loops in 3, the device maxima of the
  * time step in 4, the search's wide-support count, candidate tests and oversized groups in 5-7, the
- * largest h of the searched targets (FP64 bits) in 8 */
-constexpr int kCounterSlots  = 9;
+ * largest h of the searched targets (FP64 bits) in 8, the histogram of the table sizes from 9 on */
+constexpr int kCounterSlots  = 9 + (int(kTableBins) + 2) / 2;
 constexpr int kStatWide      = 5;
 constexpr int kStatTests     = 6;
 constexpr int kStatBadGroups = 7;
 constexpr int kStatHMax      = 8;
+constexpr int kStatHist      = 9; // first slot of the 32-bit bins of the table sizes
 
 constexpr unsigned kNumXcd = 8; // MI355X: 8 accelerator complex dies, one L2 each
 
@@ -510,12 +577,18 @@ struct DevBox
     double fixScale[3]; // 2^32 / P
     double fixStepD[3]; // P / 2^32
     float  fixStep[3];  // P / 2^32, rounded to float
+    // the FP32 form's common loops (kCommon) keep separations in units of the fixed point, one for all
+    // dimensions; `unit` is that length there, 1 in every other loop
+    int   raw;
+    float unit;
 };
 
 inline DevBox makeDevBox(const sphx_box_t* b)
 {
     DevBox d;
     d.anyPbc = 0;
+    d.raw    = 0;
+    d.unit   = 1.0f;
     for (int k = 0; k < 3; ++k)
     {
         d.lo[k]   = b->lo[k];
@@ -531,39 +604,51 @@ inline DevBox makeDevBox(const sphx_box_t* b)
     return d;
 }
 
-//! the box of the pair loops; in the FP32 form its fixed point runs over the period len / 2^shift[k]
-//! per dimension (fixedPointShift)
-inline DevBox makePairBox(const sphx_box_t* b, const int shift[3])
+constexpr int kDefaultIndex = 6; // the reference's default sinc index
+
+//! host: the largest shift s <= 16 with len / 2^s >= 8 hMax (see Coord), 0 for wide supports
+inline int fixedPointShift(double len, double hMax, bool wide)
 {
-    DevBox d = makeDevBox(b);
+    int s = 0;
+    while (!wide && s < 16 && std::ldexp(len, -(s + 1)) >= 8.0 * hMax) { ++s; }
+    return s;
+}
+
+/*! host: the box of the pair loops over the last search's lists, with the fixed point of the FP32 form. The
+ * period is a box length over a power of two in a periodic dimension and may be anything of at least
+ * 8 hMax in an open one. When the periodic dimensions have one length, every dimension takes that length's (an open
+ * box: the longest's) period, so that the fixed point has one unit and the common loops need not scale each
+ * component of a separation. */
+inline DevBox pairBox(const sphx_workspace* ws, const sphx_box_t* b)
+{
+    DevBox d      = makeDevBox(b);
+    double common = 0;
+    bool   one    = !ws->nbWide;
+    for (int k = 0; k < 3; ++k)
+        if (d.pbc[k])
+        {
+            one    = one && (common == 0 || common == d.len[k]);
+            common = d.len[k];
+        }
+    if (common == 0) { common = std::max(d.len[0], std::max(d.len[1], d.len[2])); }
     for (int k = 0; k < 3; ++k)
     {
-        const double p = std::ldexp(d.len[k], -shift[k]);
-        d.fixScale[k]  = 4294967296.0 / p;
-        d.fixStepD[k]  = p / 4294967296.0;
-        d.fixStep[k]   = float(d.fixStepD[k]);
+        const double len = one ? common : d.len[k];
+        const double p   = std::ldexp(len, -fixedPointShift(len, ws->nbHMax, ws->nbWide));
+        d.fixScale[k]    = 4294967296.0 / p;
+        d.fixStepD[k]    = p / 4294967296.0;
+        d.fixStep[k]     = float(d.fixStepD[k]);
     }
+    d.raw  = one && ws->sincIndex == double(kDefaultIndex);
+    d.unit = d.raw ? d.fixStep[0] : 1.0f;
     return d;
 }
 
-//! host: the fixed-point shift per dimension for a search whose largest h is hMax (see Coord)
-inline void fixedPointShift(const sphx_box_t* b, double hMax, bool wide, int shift[3])
+//! host: the stored lists of the last search
+inline NeighborLists neighborLists(const sphx_workspace* ws)
 {
-    for (int d = 0; d < 3; ++d)
-    {
-        const double len = b->hi[d] - b->lo[d];
-        int          s   = 0;
-        while (!wide && s < 16 && std::ldexp(len, -(s + 1)) >= 8.0 * hMax) { ++s; }
-        shift[d] = s;
-    }
-}
-
-//! host: the box of the FP32 pair loops over the last search's lists (FP64 form: the plain box)
-inline DevBox pairBox(const sphx_workspace* ws, const sphx_box_t* b)
-{
-    int shift[3];
-    fixedPointShift(b, ws->nbHMax, ws->nbWide, shift);
-    return makePairBox(b, shift);
+    return NeighborLists{ws->nbrs.get(), ws->nbTable.get(), ws->nbLocal ? ws->nbTableCount.get() : nullptr,
+                         ws->nbOwned ? ws->nbOwner.get() : nullptr, ws->nbNgmax};
 }
 
 /* ---------------------------------------------------------------------------------------------

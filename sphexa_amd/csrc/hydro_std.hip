@@ -48,18 +48,21 @@ struct MomStdFields
 /* The std momentum-energy record, built by the pack kernel or by the IAD epilogue under
  * SPHX_FLAG_CHAIN with this one function, so both give the same bits. C = {c11, .., c33}. */
 template<class T>
-__device__ __forceinline__ RecMomStd<T> momStdRecord(Coord<T> x, Coord<T> y, Coord<T> z, T vx, T vy, T vz, T h, T m,
-                                                     T rho, T p, T c, const T C[6])
+__device__ __forceinline__ RecMomStd<T> momStdRecord(const DevBox& b, Coord<T> x, Coord<T> y, Coord<T> z, T vx, T vy, T vz, T h, T m,
+                                                     T rho, T p, T c, T alpha, const T C[6])
 {
     RecMomStd<T> r;
     r.x = x, r.y = y, r.z = z;
     r.vx = vx, r.vy = vy, r.vz = vz;
-    r.hInv = T(1) / h;
-    r.m    = m;
-    r.vol  = fastDiv(m, rho);
-    r.pro  = fastDiv(p, rho); // p_j / (rho_j gradh_j), gradh_j = 1
-    r.c    = c;
-    r.c11 = C[0], r.c12 = C[1], r.c13 = C[2], r.c22 = C[3], r.c23 = C[4], r.c33 = C[5];
+    const T hInv = T(1) / h, unit = unitOf<T>(b);
+    r.scale = kernelScale(b, hInv);
+    r.m     = m;
+    r.vol   = fastDiv(m, rho) * (hInv * hInv * hInv);
+    r.pro   = fastDiv(p, rho); // p_j / (rho_j gradh_j), gradh_j = 1
+    r.c     = c;
+    r.alpha = alpha;
+    r.c11 = C[0] * unit, r.c12 = C[1] * unit, r.c13 = C[2] * unit;
+    r.c22 = C[3] * unit, r.c23 = C[4] * unit, r.c33 = C[5] * unit;
     return r;
 }
 
@@ -69,44 +72,37 @@ __global__ void __launch_bounds__(kPackThreads) packMomStd(PairArgs a, MomStdFie
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.numParticles) { return; }
     const T C[6] = {ld<T>(f.c11, i), ld<T>(f.c12, i), ld<T>(f.c13, i), ld<T>(f.c22, i), ld<T>(f.c23, i), ld<T>(f.c33, i)};
-    rec[i] = momStdRecord<T>(coordOf<T>(a.box, 0, a.x[i]), coordOf<T>(a.box, 1, a.y[i]), coordOf<T>(a.box, 2, a.z[i]),
+    rec[i] = momStdRecord<T>(a.box, coordOf<T>(a.box, 0, a.x[i]), coordOf<T>(a.box, 1, a.y[i]), coordOf<T>(a.box, 2, a.z[i]),
                              ld<T>(f.vx, i), ld<T>(f.vy, i), ld<T>(f.vz, i), ld<T>(f.h, i), ld<T>(f.m, i),
-                             ld<T>(f.rho, i), ld<T>(f.p, i), ld<T>(f.c, i), C);
+                             ld<T>(f.rho, i), ld<T>(f.p, i), ld<T>(f.c, i), f.alpha ? ld<T>(f.alpha, i) : T(1), C);
 }
 
 /* xmassJLoop (sph/include/sph/hydro_ve/xmass_kern.hpp:51-79):
  *   xm_i = m_i / (K / h_i^3 * (m_i + sum_j m_j W(r_ij / h_i)))
  * toRho: computeDensity (hydro_std/density.hpp:42-53) stores rho = m / xm instead. */
 template<class T, bool toRho, int V>
-__global__ void SPHX_LIGHT_LOOP(T)
+__global__ void __launch_bounds__(kLightWaves * kWave)
     xmassKernel(PairArgs a, const RecMass<T>* __restrict__ rec, const T* __restrict__ h, SincKernel<T> kern,
                 T* __restrict__ out, RecGradh<T>* __restrict__ next, RecVol<T>* __restrict__ nextVol)
 {
-    Lane t = laneTarget(a.L);
-    if (!t.valid) { return; }
+    const Lane       t     = groupTarget(a.L, blockGroup());
     const uint32_t   i     = t.i;
     const RecMass<T> ri    = rec[i];
     T                hi    = h[i];
     T                hInv  = T(1) / hi;
     T                h3Inv = hInv * hInv * hInv;
+    const T          scale = kernelScale(a.box, hInv);
     double           r2h   = 2.0 * double(hi);
-    const T          hInv2 = hInv * hInv;
-    Acc              rho0(ri.m);
-    withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
-        constexpr int                U = kBatchLight<T>;
-        NeighborBatch<U, RecMass<T>> nb(t, rec);
-        for (unsigned k = 0; k < t.n; k += U)
-        {
-            nb.load(k);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                const T z = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]).d2 * hInv2;
-                rho0.add(kern.template w<V>(nb.live2(k, u, z)) * double(nb.r[u].m));
-            }
-        }
+    double           sum[1] = {0.0};
+    PairWalk<kLightWaves, isMixed<T> ? 4 : 2, RecMass<T>> walk(a.L, t, rec);
+    withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
+        walk([&](bool live, const RecMass<T>& rj) {
+            const T d2 = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj).d2;
+            sum[0] += kern.template w<V>(kern.clamp(kern.arg(d2, scale), live)) * double(rj.m);
+        }, rec);
     });
-    double rhoZero = rho0.value() * a.K * double(h3Inv);
+    if (!waveSums<kLightWaves>(sum) || !t.valid) { return; }
+    double rhoZero = (double(ri.m) + sum[0]) * a.K * double(h3Inv);
     T      xmi     = T(double(ri.m) / rhoZero);
     const T outi   = toRho ? T(ri.m / xmi) : xmi;
     out[i]         = outi;
@@ -162,138 +158,117 @@ __global__ void __launch_bounds__(256) eosStdPolytropicKernel(const T* __restric
 
 /* IADJLoopSTD (hydro_std/iad_kern.hpp:11-76): tau_ab = sum_j m_j/rho_j W_ij r_a r_b, inverted */
 template<class T, int V>
-__global__ void SPHX_LIGHT_LOOP(T)
+__global__ void __launch_bounds__(kLightWaves * kWave)
     iadStdKernel(PairArgs a, const RecVol<T>* __restrict__ rec, const T* __restrict__ h, SincKernel<T> kern,
                  T* c11, T* c12, T* c13, T* c22, T* c23, T* c33, MomStdFields nf, RecMomStd<T>* __restrict__ next)
 {
-    Lane t = laneTarget(a.L);
-    if (!t.valid) { return; }
+    const Lane      t     = groupTarget(a.L, blockGroup());
     const uint32_t  i     = t.i;
     const RecVol<T> ri    = rec[i];
     T               hi    = h[i];
-    T               hiInv = T(1) / hi, hiInv2 = hiInv * hiInv;
+    T               hiInv = T(1) / hi, scale = kernelScale(a.box, hiInv);
     double          r2h   = 2.0 * double(hi);
     T               t11 = 0, t12 = 0, t13 = 0, t22 = 0, t23 = 0, t33 = 0;
-    withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
-        constexpr int               U = kBatchLight<T>;
-        NeighborBatch<U, RecVol<T>> nb(t, rec);
-        for (unsigned k = 0; k < t.n; k += U)
-        {
-            nb.load(k);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                const Sep<T> r = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]);
-                T rx = r.x, ry = r.y, rz = r.z;
-                T vol_w = nb.r[u].vol * T(kern.template w<V>(nb.live2(k, u, r.d2 * hiInv2)));
-                t11 += rx * rx * vol_w;
-                t12 += rx * ry * vol_w;
-                t13 += rx * rz * vol_w;
-                t22 += ry * ry * vol_w;
-                t23 += ry * rz * vol_w;
-                t33 += rz * rz * vol_w;
-            }
-        }
+    PairWalk<kLightWaves, isMixed<T> ? 4 : 2, RecVol<T>> walk(a.L, t, rec);
+    withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
+        walk([&](bool live, const RecVol<T>& rj) {
+            const Sep<T> r = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj);
+            T rx = r.x, ry = r.y, rz = r.z;
+            T vol_w = rj.vol * T(kern.template w<V>(kern.clamp(kern.arg(r.d2, scale), live)));
+            t11 += rx * rx * vol_w;
+            t12 += rx * ry * vol_w;
+            t13 += rx * rz * vol_w;
+            t22 += ry * ry * vol_w;
+            t23 += ry * rz * vol_w;
+            t33 += rz * rz * vol_w;
+        }, rec);
     });
+    double tau[6] = {t11, t12, t13, t22, t23, t33};
+    if (!waveSums<kLightWaves>(tau) || !t.valid) { return; }
     double cij[6];
-    iadInvert(t11, t12, t13, t22, t23, t33, double(hi), a.K, cij);
+    const double uu = double(unitOf<T>(a.box)) * double(unitOf<T>(a.box));
+    iadInvert(uu * tau[0], uu * tau[1], uu * tau[2], uu * tau[3], uu * tau[4], uu * tau[5], double(hi), a.K, cij);
     const T C[6] = {T(cij[0]), T(cij[1]), T(cij[2]), T(cij[3]), T(cij[4]), T(cij[5])};
     c11[i] = C[0], c12[i] = C[1], c13[i] = C[2];
     c22[i] = C[3], c23[i] = C[4], c33[i] = C[5];
     if (next)
     {
-        next[i] = momStdRecord<T>(ri.x, ri.y, ri.z, ld<T>(nf.vx, i), ld<T>(nf.vy, i), ld<T>(nf.vz, i), hi,
-                                  ld<T>(nf.m, i), ld<T>(nf.rho, i), ld<T>(nf.p, i), ld<T>(nf.c, i), C);
+        next[i] = momStdRecord<T>(a.box, ri.x, ri.y, ri.z, ld<T>(nf.vx, i), ld<T>(nf.vy, i), ld<T>(nf.vz, i), hi,
+                                  ld<T>(nf.m, i), ld<T>(nf.rho, i), ld<T>(nf.p, i), ld<T>(nf.c, i),
+                                  nf.alpha ? ld<T>(nf.alpha, i) : T(1), C);
     }
 }
 
 /* momentumAndEnergyJLoop, std (hydro_std/momentum_energy_kern.hpp:11-134) + tsKCourant.
  * PerAlpha: AV coefficients alpha_i, alpha_j from f.alpha instead of the constant 1. */
 template<class T, bool PerAlpha, int V>
-__global__ void SPHX_MOM_LOOP(T)
+__global__ void __launch_bounds__(kMomWaves<T> * kWave)
     momentumStdKernel(PairArgs a, MomStdFields f, const RecMomStd<T>* __restrict__ rec, SincKernel<T> kern,
                       float Kcour, unsigned long long* minDt)
 {
-    Lane   t      = laneTarget(a.L);
+    const Lane         t      = groupTarget(a.L, blockGroup());
+    const uint32_t     i      = t.i;
+    const RecMomStd<T> ri     = rec[i];
+    T                  hi     = ld<T>(f.h, i);
+    T                  roi    = ld<T>(f.rho, i);
+    T                  pro_i  = fastDiv(ld<T>(f.p, i), roi * roi); // p_i / (gradh_i rho_i^2), gradh_i = 1
+    T                  vol_i  = fastDiv(ri.m, roi);
+    T                  hiInv  = T(1) / hi, hiInv3 = hiInv * hiInv * hiInv;
+    double             r2h    = 2.0 * double(hi);
+
+    T      maxvs = 0;
+    T      momx = 0, momy = 0, momz = 0;
+    double energy = 0.0;
+    PairWalk<kMomWaves<T>, 2, RecMomStd<T>> walk(a.L, t, rec);
+    withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
+        walk([&](bool live, const RecMomStd<T>& rj) {
+            const Sep<T> r = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj);
+            T rx = r.x, ry = r.y, rz = r.z;
+            T vx_ij = ri.vx - rj.vx, vy_ij = ri.vy - rj.vy, vz_ij = ri.vz - rj.vz;
+            T rv    = rx * vx_ij + ry * vy_ij + rz * vz_ij;
+            const T Wi = hiInv3 * T(kern.template w<V>(kern.clamp(kern.arg(r.d2, ri.scale), live)));
+            const T Wj = rj.vol * T(kern.template w<V>(kern.clamp(kern.arg(r.d2, rj.scale), live)));
+
+            // C_i r and C_j r, and their products with v_ij
+            const T ax_i = ri.c11 * rx + ri.c12 * ry + ri.c13 * rz, ax_j = rj.c11 * rx + rj.c12 * ry + rj.c13 * rz;
+            const T ay_i = ri.c12 * rx + ri.c22 * ry + ri.c23 * rz, ay_j = rj.c12 * rx + rj.c22 * ry + rj.c23 * rz;
+            const T az_i = ri.c13 * rx + ri.c23 * ry + ri.c33 * rz, az_j = rj.c13 * rx + rj.c23 * ry + rj.c33 * rz;
+            const T va_i = vx_ij * ax_i + vy_ij * ay_i + vz_ij * az_i, va_j = vx_ij * ax_j + vy_ij * ay_j + vz_ij * az_j;
+
+            const T wij  = overDistance(rv, r.d2);
+            const T cs   = ri.c + rj.c;
+            const T visc = T(0.5) * artificialViscosity(PerAlpha ? ri.alpha : T(1), PerAlpha ? rj.alpha : T(1), cs, wij);
+            const T vsig = cs - T(3) * wij;
+            maxvs        = vsig > maxvs ? vsig : maxvs;
+
+            const T mp = rj.m * pro_i, vv = visc * vol_i;
+            const T aa = Wi * (mp + vv), ae = Wi * (T(2) * mp + vv);
+            const T bb = Wj * (rj.pro + visc), be = Wj * visc;
+            momx += aa * ax_i + bb * ax_j;
+            momy += aa * ay_i + bb * ay_j;
+            momz += aa * az_i + bb * az_j;
+            energy += double(ae * va_i + be * va_j);
+        }, rec);
+    });
+    double sum[5] = {maxvs, momx, momy, momz, energy};
+    if (!waveSums<kMomWaves<T>, 5, 1>(sum)) { return; }
     double dtLane = INFINITY;
     if (t.valid)
     {
-        const uint32_t     i      = t.i;
-        const RecMomStd<T> ri     = rec[i];
-        T                  hi     = ld<T>(f.h, i);
-        T                  roi    = ld<T>(f.rho, i);
-        T                  hiInv  = ri.hInv;
-        T                  hiInv2 = hiInv * hiInv, hiInv3 = hiInv2 * hiInv;
-        T                  pro_i  = fastDiv(ld<T>(f.p, i), roi * roi); // p_i / (gradh_i rho_i^2), gradh_i = 1
-        double             r2h    = 2.0 * double(hi);
-        const T            alpha_i = PerAlpha ? ld<T>(f.alpha, i) : T(1);
-
-        T      maxvs = 0;
-        T      momx = 0, momy = 0, momz = 0;
-        Acc    energy;
-        withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
-            constexpr int                  U = kBatchMom<T>;
-            NeighborBatch<U, RecMomStd<T>> nb(t, rec);
-            for (unsigned k = 0; k < t.n; k += U)
-            {
-                nb.load(k);
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                {
-                    const RecMomStd<T>& rj = nb.r[u];
-                    const Sep<T>        r  = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, rj);
-                    T rx = r.x, ry = r.y, rz = r.z;
-                    T vx_ij = ri.vx - rj.vx, vy_ij = ri.vy - rj.vy, vz_ij = ri.vz - rj.vz;
-                    T rv    = rx * vx_ij + ry * vy_ij + rz * vz_ij;
-                    T hjInv2 = rj.hInv * rj.hInv;
-                    T Wi     = hiInv3 * T(kern.template w<V>(nb.live2(k, u, r.d2 * hiInv2)));
-                    T Wj     = rj.hInv * hjInv2 * T(kern.template w<V>(nb.live2(k, u, r.d2 * hjInv2)));
-
-                    T tA1_i = ri.c11 * rx + ri.c12 * ry + ri.c13 * rz;
-                    T tA2_i = ri.c12 * rx + ri.c22 * ry + ri.c23 * rz;
-                    T tA3_i = ri.c13 * rx + ri.c23 * ry + ri.c33 * rz;
-                    T tA1_j = rj.c11 * rx + rj.c12 * ry + rj.c13 * rz;
-                    T tA2_j = rj.c12 * rx + rj.c22 * ry + rj.c23 * rz;
-                    T tA3_j = rj.c13 * rx + rj.c23 * ry + rj.c33 * rz;
-
-                    T wij  = overDistance(rv, r.d2);
-                    T alpha_j = PerAlpha ? ld<T>(f.alpha, nb.j[u]) : T(1);
-                    T visc    = T(0.5) * artificialViscosity(alpha_i, alpha_j, ri.c, rj.c, wij);
-                    T vsig = ri.c + rj.c - T(3) * wij;
-                    maxvs  = nb.in(k, u) && vsig > maxvs ? vsig : maxvs;
-
-                    T mj_roj_Wj = rj.vol * Wj;
-                    T mj_pro_i  = rj.m * pro_i;
-                    {
-                        T aa = Wi * (mj_pro_i + visc * ri.vol);
-                        T bb = mj_roj_Wj * (rj.pro + visc);
-                        momx += aa * tA1_i + bb * tA1_j;
-                        momy += aa * tA2_i + bb * tA2_j;
-                        momz += aa * tA3_i + bb * tA3_j;
-                    }
-                    {
-                        T aa = Wi * (T(2) * mj_pro_i + visc * ri.vol);
-                        T bb = visc * mj_roj_Wj;
-                        energy.add(vx_ij * (aa * tA1_i + bb * tA1_j) + vy_ij * (aa * tA2_i + bb * tA2_j) +
-                                   vz_ij * (aa * tA3_i + bb * tA3_j));
-                    }
-                }
-            }
-        });
-        f.du[i] = -a.K * 0.5 * energy.value();
-        st<T>(f.ax, i, T(a.K * double(momx)));
-        st<T>(f.ay, i, T(a.K * double(momy)));
-        st<T>(f.az, i, T(a.K * double(momz)));
-        dtLane = courantDt(maxvs, hi, ri.c, Kcour);
+        f.du[i] = -a.K * 0.5 * sum[4];
+        st<T>(f.ax, i, T(a.K * sum[1]));
+        st<T>(f.ay, i, T(a.K * sum[2]));
+        st<T>(f.az, i, T(a.K * sum[3]));
+        dtLane = courantDt(T(sum[0]), hi, ri.c, Kcour);
     }
-    reduceMinDt<T>(minDt, dtLane, a.L.groups);
+    reduceMinDt(minDt, dtLane, a.L.groups);
 }
 
 template<class T>
-void launchDensity(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f, const sphx_params_t* p, bool toRho,
+void launchDensity(sphx_workspace* ws, PairArgs a, const sphx_fields_t* f, const sphx_params_t* p, bool toRho,
                    void* out)
 {
-    unsigned blocks = pairBlocks(a.L);
+    unsigned blocks = a.L.groups.num;
     if (blocks == 0) { return; }
     RecMass<T>* rec = recordBuffer<RecMass<T>>(ws, a.numParticles, 0);
     packMass<T><<<ceilDiv(a.numParticles, kPackThreads), kPackThreads, 0, ws->stream>>>(a.box, a.x, a.y, a.z,
@@ -304,14 +279,16 @@ void launchDensity(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f
     RecGradh<T>* next = !toRho && chainable(a, p) ? recordBuffer<RecGradh<T>>(ws, a.numParticles, 1) : nullptr;
     RecVol<T>*   nextVol = toRho && chainable(a, p) ? recordBuffer<RecVol<T>>(ws, a.numParticles, 1) : nullptr;
     {
+        const PairLaunch run = pairLaunch(ws, sizeof(RecMass<T>), kLightWaves, 1);
+        a.L.stage            = run.stage;
         KernelScope timer(ws, toRho ? "density_std" : "xmass");
-        launchVariant<T>(ws, [&](auto variant) {
+        launchVariant<T>(ws, a.box, [&](auto variant) {
             constexpr int V = decltype(variant)::value;
             if (toRho)
-                xmassKernel<T, true, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_XMASS) : 0, ws->stream>>>(
+                xmassKernel<T, true, V><<<blocks, kLightWaves * kWave, run.lds, ws->stream>>>(
                     a, rec, (const T*)f->h, sincKernel<T>(ws), (T*)out, nullptr, nextVol);
             else
-                xmassKernel<T, false, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_XMASS) : 0, ws->stream>>>(
+                xmassKernel<T, false, V><<<blocks, kLightWaves * kWave, run.lds, ws->stream>>>(
                     a, rec, (const T*)f->h, sincKernel<T>(ws), (T*)out, next, nullptr);
         });
         SPHX_CHECK_LAUNCH();
@@ -321,9 +298,9 @@ void launchDensity(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f
 }
 
 template<class T>
-void launchIadStd(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f, const sphx_params_t* p)
+void launchIadStd(sphx_workspace* ws, PairArgs a, const sphx_fields_t* f, const sphx_params_t* p)
 {
-    unsigned blocks = pairBlocks(a.L);
+    unsigned blocks = a.L.groups.num;
     int      in     = takeChain(ws, kChainVol, a, f, p);
     if (blocks == 0) { return; }
     RecVol<T>* rec = recordBuffer<RecVol<T>>(ws, a.numParticles, in < 0 ? 0 : in);
@@ -336,13 +313,16 @@ void launchIadStd(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f,
     }
     // IAD leaves the momentum-energy records when chaining (it needs v, p and c besides its own fields)
     MomStdFields  nf{f->vx, f->vy, f->vz, f->h, f->m, f->rho, f->p, f->c};
+    nf.alpha = (p->flags & SPHX_FLAG_STD_ALPHA) ? f->alpha : nullptr;
     RecMomStd<T>* next = chainable(a, p) && f->vx && f->vy && f->vz && f->p && f->c
                              ? recordBuffer<RecMomStd<T>>(ws, a.numParticles, 1 - in)
                              : nullptr;
     {
+        const PairLaunch run = pairLaunch(ws, sizeof(RecVol<T>), kLightWaves, 6);
+        a.L.stage            = run.stage;
         KernelScope timer(ws, "iad_std");
-        launchVariant<T>(ws, [&](auto variant) {
-            iadStdKernel<T, decltype(variant)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_IAD) : 0, ws->stream>>>(
+        launchVariant<T>(ws, a.box, [&](auto variant) {
+            iadStdKernel<T, decltype(variant)::value><<<blocks, kLightWaves * kWave, run.lds, ws->stream>>>(
                 a, rec, (const T*)f->h, sincKernel<T>(ws), (T*)f->c11, (T*)f->c12, (T*)f->c13, (T*)f->c22,
                 (T*)f->c23, (T*)f->c33, nf, next);
         });
@@ -352,10 +332,10 @@ void launchIadStd(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f,
 }
 
 template<class T>
-void launchMomentumStd(sphx_workspace* ws, const PairArgs& a, const MomStdFields& mf, const sphx_fields_t* f,
+void launchMomentumStd(sphx_workspace* ws, PairArgs a, const MomStdFields& mf, const sphx_fields_t* f,
                        const sphx_params_t* p, float Kcour, unsigned long long* dt, bool perAlpha)
 {
-    unsigned blocks = pairBlocks(a.L);
+    unsigned blocks = a.L.groups.num;
     int      in     = takeChain(ws, kChainMomStd, a, f, p);
     if (blocks == 0) { return; }
     RecMomStd<T>* rec = recordBuffer<RecMomStd<T>>(ws, a.numParticles, in < 0 ? 0 : in);
@@ -364,14 +344,16 @@ void launchMomentumStd(sphx_workspace* ws, const PairArgs& a, const MomStdFields
         packMomStd<T><<<ceilDiv(a.numParticles, kPackThreads), kPackThreads, 0, ws->stream>>>(a, mf, rec);
         SPHX_CHECK_LAUNCH();
     }
+    const PairLaunch run = pairLaunch(ws, sizeof(RecMomStd<T>), kMomWaves<T>, 5);
+    a.L.stage            = run.stage;
     KernelScope timer(ws, "momentum_std");
-    launchVariant<T>(ws, [&](auto variant) {
+    launchVariant<T>(ws, a.box, [&](auto variant) {
         constexpr int V = decltype(variant)::value;
         if (perAlpha)
-            momentumStdKernel<T, true, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(a, mf, rec, sincKernel<T>(ws),
+            momentumStdKernel<T, true, V><<<blocks, kMomWaves<T> * kWave, run.lds, ws->stream>>>(a, mf, rec, sincKernel<T>(ws),
                                                                                         Kcour, dt);
         else
-            momentumStdKernel<T, false, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(a, mf, rec,
+            momentumStdKernel<T, false, V><<<blocks, kMomWaves<T> * kWave, run.lds, ws->stream>>>(a, mf, rec,
                                                                                          sincKernel<T>(ws), Kcour, dt);
     });
     SPHX_CHECK_LAUNCH();
@@ -465,7 +447,7 @@ double momentumEnergyStd(sphx_workspace* ws, const DevBox& box, const sphx_field
     const bool perAlpha = (p->flags & SPHX_FLAG_STD_ALPHA) != 0;
     SPHX_REQUIRE(!perAlpha || f->alpha, SPHX_ERR_ARG, "SPHX_FLAG_STD_ALPHA set but fields.alpha is NULL");
     MomStdFields mf{f->vx,  f->vy,  f->vz,  f->h,  f->m,  f->rho, f->p,  f->c,  f->c11, f->c12,
-                    f->c13, f->c22, f->c23, f->c33, f->ax, f->ay,  f->az, f->du, f->alpha};
+                    f->c13, f->c22, f->c23, f->c33, f->ax, f->ay,  f->az, f->du, perAlpha ? f->alpha : nullptr};
     if (p->hydro_type == SPHX_F32) launchMomentumStd<float>(ws, a, mf, f, p, float(p->Kcour), dt, perAlpha);
     else launchMomentumStd<double>(ws, a, mf, f, p, float(p->Kcour), dt, perAlpha);
     unsigned long long bits = 0;

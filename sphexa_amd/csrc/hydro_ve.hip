@@ -25,46 +25,39 @@ __global__ void __launch_bounds__(kPackThreads) packGradh(PairArgs a, const T* _
 
 /* veDefGradhJLoop (hydro_ve/ve_def_gradh_kern.hpp:44-90): kx and the grad-h term */
 template<class T, int V>
-__global__ void SPHX_LIGHT_LOOP(T)
+__global__ void __launch_bounds__(kLightWaves * kWave)
     veDefGradhKernel(PairArgs a, const RecGradh<T>* __restrict__ rec, const T* __restrict__ h,
                      SincKernel<T> kern, T* __restrict__ kx, T* __restrict__ gradh, RecIadVe<T>* __restrict__ next,
                      const T* __restrict__ vx, const T* __restrict__ vy, const T* __restrict__ vz)
 {
-    Lane t = laneTarget(a.L);
-    if (!t.valid) { return; }
+    const Lane        t   = groupTarget(a.L, blockGroup());
     const uint32_t    i   = t.i;
     const RecGradh<T> ri  = rec[i];
     T                 hi  = h[i], mi = ri.m, xmi = ri.xm;
     T                 hInv = T(1) / hi;
     double            r2h  = 2.0 * double(hi);
-    const T           hInv2 = hInv * hInv;
-    Acc               kxs(xmi), wom(-3.0 * double(xmi)), wr0(-3.0 * double(mi));
-    withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
-        constexpr int                 U = kBatchLight<T>;
-        NeighborBatch<U, RecGradh<T>> nb(t, rec);
-        for (unsigned k = 0; k < t.n; k += U)
-        {
-            nb.load(k);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                const T z = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, nb.r[u]).d2 * hInv2;
-                double  wv, vdw;
-                kern.template wAndVdw<V>(nb.live2(k, u, z), wv, vdw);
-                const double dterh = -(3.0 * wv + vdw);
-                kxs.add(wv * double(nb.r[u].xm));
-                wom.add(dterh * double(nb.r[u].xm));
-                wr0.add(dterh * double(nb.r[u].m));
-            }
-        }
+    const T           scale = kernelScale(a.box, hInv);
+    double            sum[3] = {0.0, 0.0, 0.0}; // of W xm_j, dterh xm_j, dterh m_j
+    PairWalk<kLightWaves, isMixed<T> ? 4 : 2, RecGradh<T>> walk(a.L, t, rec);
+    withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
+        walk([&](bool live, const RecGradh<T>& rj) {
+            const T d2 = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj).d2;
+            double  wv, vdw;
+            kern.template wAndVdw<V>(kern.clamp(kern.arg(d2, scale), live), wv, vdw);
+            const double dterh = -(3.0 * wv + vdw);
+            sum[0] += wv * double(rj.xm);
+            sum[1] += dterh * double(rj.xm);
+            sum[2] += dterh * double(rj.m);
+        }, rec);
     });
+    if (!waveSums<kLightWaves>(sum) || !t.valid) { return; }
     // per-target epilogue in FP64 following the reference's order; h^-3 is rounded in T as there
     T      th3   = hInv * hInv * hInv;
     double dhInv = double(hInv);
     double h3Inv = double(th3);
-    double kxi   = kxs.value() * (a.K * h3Inv);
-    double whom  = wom.value() * (a.K * h3Inv * dhInv);
-    double wrho0 = wr0.value() * (a.K * h3Inv * dhInv);
+    double kxi   = (double(xmi) + sum[0]) * (a.K * h3Inv);
+    double whom  = (sum[1] - 3.0 * double(xmi)) * (a.K * h3Inv * dhInv);
+    double wrho0 = (sum[2] - 3.0 * double(mi)) * (a.K * h3Inv * dhInv);
     whom          = whom * double(mi) / double(xmi) + (kxi - a.K * double(xmi) * h3Inv) * wrho0;
     double rhoi   = kxi * double(mi) / double(xmi);
     double dhdrho = -double(hi) / (rhoi * 3.0);
@@ -156,21 +149,23 @@ __device__ __forceinline__ RecAv<T> avRecord(Coord<T> x, Coord<T> y, Coord<T> z,
 
 //! C = {c11, c12, c13, c22, c23, c33}
 template<class T>
-__device__ __forceinline__ RecMomVe<T> momVeRecord(Coord<T> x, Coord<T> y, Coord<T> z, T vx, T vy, T vz, T h, T m,
+__device__ __forceinline__ RecMomVe<T> momVeRecord(const DevBox& b, Coord<T> x, Coord<T> y, Coord<T> z, T vx, T vy, T vz, T h, T m,
                                                    T c, T xm, T kx, T alpha, T prho, const T C[6])
 {
     RecMomVe<T> r;
     r.x = x, r.y = y, r.z = z;
     r.vx = vx, r.vy = vy, r.vz = vz;
-    r.hInv  = T(1) / h;
+    const T hInv = T(1) / h, hInv3 = hInv * hInv * hInv, unit = unitOf<T>(b);
+    r.scale = kernelScale(b, hInv);
     r.m     = m;
     r.c     = c;
     r.xm    = xm;
     r.rho   = kx * m / xm;
-    r.vol   = fastDiv(m, r.rho);
+    r.vol   = fastDiv(m, r.rho) * hInv3;
     r.alpha = alpha;
-    r.prho  = prho;
-    r.c11 = C[0], r.c12 = C[1], r.c13 = C[2], r.c22 = C[3], r.c23 = C[4], r.c33 = C[5];
+    r.prho  = prho * hInv3;
+    r.c11 = C[0] * unit, r.c12 = C[1] * unit, r.c13 = C[2] * unit;
+    r.c22 = C[3] * unit, r.c23 = C[4] * unit, r.c33 = C[5] * unit;
     return r;
 }
 
@@ -195,49 +190,46 @@ __global__ void __launch_bounds__(kPackThreads) packIadVe(PairArgs a, IadVeField
  *   M[a][c] = sum_j (v_ja - v_ia) xm_j W_ij r_ij,c,
  * so the 9 moments M are accumulated alongside tau and combined with C_i after the inversion. */
 template<class T, int V>
-__global__ void SPHX_LIGHT_LOOP(T)
+__global__ void __launch_bounds__(kLightWaves * kWave)
     iadDivvCurlvKernel(PairArgs a, IadVeFields f, const RecIadVe<T>* __restrict__ rec, SincKernel<T> kern,
                        RecAv<T>* __restrict__ next, const T* __restrict__ cNext)
 {
-    Lane t = laneTarget(a.L);
-    if (!t.valid) { return; }
+    const Lane        t     = groupTarget(a.L, blockGroup());
     const uint32_t    i     = t.i;
     const RecIadVe<T> ri    = rec[i];
     T                 hi    = ld<T>(f.h, i);
-    T                 hiInv = T(1) / hi, hiInv2 = hiInv * hiInv;
+    T                 hiInv = T(1) / hi, scale = kernelScale(a.box, hiInv);
     double            r2h   = 2.0 * double(hi);
     T                 t11 = 0, t12 = 0, t13 = 0, t22 = 0, t23 = 0, t33 = 0;
-    T                 M[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-    withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
-        constexpr int                 U = kBatchLight<T>;
-        NeighborBatch<U, RecIadVe<T>> nb(t, rec);
-        for (unsigned k = 0; k < t.n; k += U)
-        {
-            nb.load(k);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                const RecIadVe<T>& rj = nb.r[u];
-                const Sep<T>       r  = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, rj);
-                T rx = r.x, ry = r.y, rz = r.z;
-                T wv    = T(kern.template w<V>(nb.live2(k, u, r.d2 * hiInv2)));
-                T vol_w = rj.vol * wv;
-                t11 += rx * rx * vol_w;
-                t12 += rx * ry * vol_w;
-                t13 += rx * rz * vol_w;
-                t22 += ry * ry * vol_w;
-                t23 += ry * rz * vol_w;
-                t33 += rz * rz * vol_w;
-                T xw  = rj.xm * wv;
-                T dvx = (rj.vx - ri.vx) * xw, dvy = (rj.vy - ri.vy) * xw, dvz = (rj.vz - ri.vz) * xw;
-                M[0][0] += dvx * rx, M[0][1] += dvx * ry, M[0][2] += dvx * rz;
-                M[1][0] += dvy * rx, M[1][1] += dvy * ry, M[1][2] += dvy * rz;
-                M[2][0] += dvz * rx, M[2][1] += dvz * ry, M[2][2] += dvz * rz;
-            }
-        }
+    T                 m11 = 0, m12 = 0, m13 = 0, m21 = 0, m22 = 0, m23 = 0, m31 = 0, m32 = 0, m33 = 0;
+    PairWalk<kLightWaves, isMixed<T> ? 4 : 2, RecIadVe<T>> walk(a.L, t, rec);
+    withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
+        walk([&](bool live, const RecIadVe<T>& rj) {
+            const Sep<T> r = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj);
+            T rx = r.x, ry = r.y, rz = r.z;
+            T wv    = T(kern.template w<V>(kern.clamp(kern.arg(r.d2, scale), live)));
+            T vol_w = rj.vol * wv;
+            t11 += rx * rx * vol_w;
+            t12 += rx * ry * vol_w;
+            t13 += rx * rz * vol_w;
+            t22 += ry * ry * vol_w;
+            t23 += ry * rz * vol_w;
+            t33 += rz * rz * vol_w;
+            T xw  = rj.xm * wv;
+            T dvx = (rj.vx - ri.vx) * xw, dvy = (rj.vy - ri.vy) * xw, dvz = (rj.vz - ri.vz) * xw;
+            m11 += dvx * rx, m12 += dvx * ry, m13 += dvx * rz;
+            m21 += dvy * rx, m22 += dvy * ry, m23 += dvy * rz;
+            m31 += dvz * rx, m32 += dvz * ry, m33 += dvz * rz;
+        }, rec);
     });
+    double sum[15] = {t11, t12, t13, t22, t23, t33, m11, m12, m13, m21, m22, m23, m31, m32, m33};
+    if (!waveSums<kLightWaves>(sum) || !t.valid) { return; }
     double cij[6];
-    iadInvert(t11, t12, t13, t22, t23, t33, double(hi), a.K, cij);
+    const double u = double(unitOf<T>(a.box)), uu = u * u;
+    iadInvert(uu * sum[0], uu * sum[1], uu * sum[2], uu * sum[3], uu * sum[4], uu * sum[5], double(hi), a.K, cij);
+    const T M[3][3] = {{T(u * sum[6]), T(u * sum[7]), T(u * sum[8])},
+                       {T(u * sum[9]), T(u * sum[10]), T(u * sum[11])},
+                       {T(u * sum[12]), T(u * sum[13]), T(u * sum[14])}};
     T c[6];
     for (int q = 0; q < 6; ++q)
         c[q] = T(cij[q]);
@@ -293,39 +285,35 @@ __global__ void __launch_bounds__(kPackThreads) packAv(PairArgs a, AvFields f, R
 /* AVswitchesJLoop (hydro_ve/av_switches_kern.hpp:44-137). grad(div v) is linear in C_i:
  * gd_b = -K/h_i^3 sum_c C_i[b][c] sum_j f_j W_ij r_ij,c with f_j = xm_j/kx_j (divv_i - divv_j). */
 template<class T, int V>
-__global__ void SPHX_LIGHT_LOOP(T)
+__global__ void __launch_bounds__(kLightWaves * kWave)
     avSwitchesKernel(PairArgs a, AvFields f, const RecAv<T>* __restrict__ rec, SincKernel<T> kern, double dt,
                      T alphamin, T alphamax, T decay, RecMomVe<T>* __restrict__ next)
 {
-    Lane t = laneTarget(a.L);
-    if (!t.valid) { return; }
+    const Lane     t     = groupTarget(a.L, blockGroup());
     const uint32_t i     = t.i;
     const RecAv<T> ri    = rec[i];
     T              hi    = ld<T>(f.h, i);
-    T              hiInv = T(1) / hi, hiInv2 = hiInv * hiInv;
+    T              hiInv = T(1) / hi, scale = kernelScale(a.box, hiInv);
     double         r2h   = 2.0 * double(hi);
     T              vsig  = T(1.e-40) * ri.c;
-    T              S[3]  = {0, 0, 0};
-    withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
-        constexpr int              U = kBatchLight<T>;
-        NeighborBatch<U, RecAv<T>> nb(t, rec);
-        for (unsigned k = 0; k < t.n; k += U)
-        {
-            nb.load(k);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                const RecAv<T>& rj = nb.r[u];
-                const Sep<T>    r  = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, rj);
-                T rx = r.x, ry = r.y, rz = r.z;
-                T rv = rx * (ri.vx - rj.vx) + ry * (ri.vy - rj.vy) + rz * (ri.vz - rj.vz);
-                T vs = nb.in(k, u) && rv < T(0) ? ri.c + rj.c - T(3) * overDistance(rv, r.d2) : T(0);
-                vsig = vsig < vs ? vs : vsig;
-                T fw = rj.vol * (ri.divv - rj.divv) * T(kern.template w<V>(nb.live2(k, u, r.d2 * hiInv2)));
-                S[0] += fw * rx, S[1] += fw * ry, S[2] += fw * rz;
-            }
-        }
+    T              S0 = 0, S1 = 0, S2 = 0;
+    PairWalk<kLightWaves, isMixed<T> ? 4 : 2, RecAv<T>> walk(a.L, t, rec);
+    withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
+        walk([&](bool live, const RecAv<T>& rj) {
+            const Sep<T> r = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj);
+            T rx = r.x, ry = r.y, rz = r.z;
+            T rv = rx * (ri.vx - rj.vx) + ry * (ri.vy - rj.vy) + rz * (ri.vz - rj.vz);
+            T vs = live && rv < T(0) ? ri.c + rj.c - T(3) * overDistance(rv, r.d2) : T(0);
+            vsig = vsig < vs ? vs : vsig;
+            T fw = rj.vol * (ri.divv - rj.divv) * T(kern.template w<V>(kern.clamp(kern.arg(r.d2, scale), live)));
+            S0 += fw * rx, S1 += fw * ry, S2 += fw * rz;
+        }, rec);
     });
+    double sum[4] = {vsig, S0, S1, S2};
+    if (!waveSums<kLightWaves, 4, 1>(sum) || !t.valid) { return; }
+    vsig         = T(sum[0]);
+    const double u = double(unitOf<T>(a.box));
+    const T S[3] = {T(u * sum[1]), T(u * sum[2]), T(u * sum[3])};
     T c11i = ld<T>(f.c11, i), c12i = ld<T>(f.c12, i), c13i = ld<T>(f.c13, i);
     T c22i = ld<T>(f.c22, i), c23i = ld<T>(f.c23, i), c33i = ld<T>(f.c33, i);
     T kh3  = T(a.K * double(hiInv * hiInv * hiInv));
@@ -353,7 +341,7 @@ __global__ void SPHX_LIGHT_LOOP(T)
     if (next)
     {
         const T C[6] = {c11i, c12i, c13i, c22i, c23i, c33i};
-        next[i] = momVeRecord<T>(ri.x, ri.y, ri.z, ri.vx, ri.vy, ri.vz, hi, ld<T>(f.m, i), ri.c, ld<T>(f.xm, i),
+        next[i] = momVeRecord<T>(a.box, ri.x, ri.y, ri.z, ri.vx, ri.vy, ri.vz, hi, ld<T>(f.m, i), ri.c, ld<T>(f.xm, i),
                                  ld<T>(f.kx, i), alpha_i, ld<T>(f.prho, i), C);
     }
 }
@@ -372,9 +360,20 @@ __global__ void __launch_bounds__(kPackThreads) packMomVe(PairArgs a, MomVeField
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.numParticles) { return; }
     const T C[6] = {ld<T>(f.c11, i), ld<T>(f.c12, i), ld<T>(f.c13, i), ld<T>(f.c22, i), ld<T>(f.c23, i), ld<T>(f.c33, i)};
-    rec[i] = momVeRecord<T>(coordOf<T>(a.box, 0, a.x[i]), coordOf<T>(a.box, 1, a.y[i]), coordOf<T>(a.box, 2, a.z[i]),
+    rec[i] = momVeRecord<T>(a.box, coordOf<T>(a.box, 0, a.x[i]), coordOf<T>(a.box, 1, a.y[i]), coordOf<T>(a.box, 2, a.z[i]),
                             ld<T>(f.vx, i), ld<T>(f.vy, i), ld<T>(f.vz, i), ld<T>(f.h, i), ld<T>(f.m, i),
                             ld<T>(f.c, i), ld<T>(f.xm, i), ld<T>(f.kx, i), ld<T>(f.alpha, i), ld<T>(f.prho, i), C);
+}
+
+//! the AV-cleaning records: the velocity gradients per unit of the separations
+template<class T>
+__global__ void __launch_bounds__(kPackThreads) packGradV(DevBox b, MomVeFields f, RecGradV<T>* __restrict__ rec, uint32_t n)
+{
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) { return; }
+    const T u = unitOf<T>(b);
+    rec[i]    = RecGradV<T>{{u * ld<T>(f.dV11, i), u * ld<T>(f.dV12, i), u * ld<T>(f.dV13, i), u * ld<T>(f.dV22, i),
+                          u * ld<T>(f.dV23, i), u * ld<T>(f.dV33, i)}};
 }
 
 //! avRvCorrection (hydro_ve/momentum_energy_kern.hpp:44-63) with the reference's symv layout
@@ -420,117 +419,108 @@ __device__ __forceinline__ T ramExp2(T v)
 
 /* momentumAndEnergyJLoop<avClean> (hydro_ve/momentum_energy_kern.hpp:66-222) + tsKCourant */
 template<class T, bool avClean, int V>
-__global__ void SPHX_MOM_LOOP(T)
-    momentumVeKernel(PairArgs a, MomVeFields f, const RecMomVe<T>* __restrict__ rec, SincKernel<T> kern, T Atmin,
+__global__ void __launch_bounds__(kMomWaves<T> * kWave)
+    momentumVeKernel(PairArgs a, MomVeFields f, const RecMomVe<T>* __restrict__ rec,
+                     const RecGradV<T>* __restrict__ gradV, SincKernel<T> kern, T Atmin,
                      T Atmax, T ramp, float Kcour, unsigned long long* minDt)
 {
-    Lane   t      = laneTarget(a.L);
+    const Lane        t      = groupTarget(a.L, blockGroup());
+    const uint32_t    i      = t.i;
+    const RecMomVe<T> ri     = rec[i];
+    T                 hi     = ld<T>(f.h, i);
+    const T           rhoInv_i = T(1) / ri.rho, prho_i = ld<T>(f.prho, i);
+    const T           hiInv    = T(1) / hi, hiInv3 = hiInv * hiInv * hiInv;
+    RecGradV<T>       gradV_i{};
+    if constexpr (avClean) { gradV_i = gradV[i]; }
+    T      eta_crit = T(cbrt(32.0 * M_PI / 3.0 / double(t.n + 1)));
+    double r2h      = 2.0 * double(hi);
+
+    T      maxvs = 0;
+    T      momx = 0, momy = 0, momz = 0;
+    double energy = 0.0, avEnergy = 0.0;
+    auto   pairTerms = [&](auto fold, bool live, const RecMomVe<T>& rj, const RecGradV<T>* gradV_j) {
+        const Sep<T> r = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj);
+        T rx = r.x, ry = r.y, rz = r.z;
+        T vx_ij = ri.vx - rj.vx, vy_ij = ri.vy - rj.vy, vz_ij = ri.vz - rj.vz;
+        const T Wi = hiInv3 * T(kern.template w<V>(kern.clamp(kern.arg(r.d2, ri.scale), live)));
+        const T Wj = T(kern.template w<V>(kern.clamp(kern.arg(r.d2, rj.scale), live)));
+
+        // C_i r and C_j r (the reference's gradient terms are these times -W h^-3), and their products with v_ij
+        const T ax_i = ri.c11 * rx + ri.c12 * ry + ri.c13 * rz, ax_j = rj.c11 * rx + rj.c12 * ry + rj.c13 * rz;
+        const T ay_i = ri.c12 * rx + ri.c22 * ry + ri.c23 * rz, ay_j = rj.c12 * rx + rj.c22 * ry + rj.c23 * rz;
+        const T az_i = ri.c13 * rx + ri.c23 * ry + ri.c33 * rz, az_j = rj.c13 * rx + rj.c23 * ry + rj.c33 * rz;
+        const T va_i = vx_ij * ax_i + vy_ij * ay_i + vz_ij * az_i, va_j = vx_ij * ax_j + vy_ij * ay_j + vz_ij * az_j;
+
+        T rv = rx * vx_ij + ry * vy_ij + rz * vz_ij;
+        if constexpr (avClean)
+        {
+            const T zScale = (ri.scale < T(0)) == (ri.scale < rj.scale) ? rj.scale : ri.scale; // of the larger h
+            rv += avRvCorrection(rx, ry, rz, fastSqrt(r.d2 * zScale * (isMixed<T> ? T(-4) : T(1))), eta_crit, gradV_i.g,
+                                 gradV_j->g);
+        }
+        const T wij  = overDistance(rv, r.d2);
+        const T cs   = ri.c + rj.c;
+        const T visc = artificialViscosity(ri.alpha, rj.alpha, cs, wij);
+        const T vsig = T(0.5) * cs - T(2) * wij;
+        maxvs        = vsig > maxvs ? vsig : maxvs;
+
+        // the Atwood number against its bounds without a division, which only the ramp between them needs
+        const T dRho = fabs(ri.rho - rj.rho), sRho = ri.rho + rj.rho;
+        const bool steep = dRho > Atmax * sRho;
+        T a_mom = ri.xm * (steep ? rj.xm : ri.xm);
+        T b_mom = rj.xm * (steep ? ri.xm : rj.xm);
+        if (!steep && dRho >= Atmin * sRho)
+        {
+            // xm_i^(2-s) xm_j^s = xm_i^2 2^(s log2(xm_j/xm_i)), and symmetrically for b:
+            // one logarithm and two exponentials instead of four powers
+            const T sigma = ramp * (fastDiv(dRho, sRho) - Atmin);
+            const T lr    = ramLog2(fastDiv(rj.xm, ri.xm));
+            a_mom         = ri.xm * ri.xm * ramExp2(sigma * lr);
+            b_mom         = rj.xm * rj.xm * ramExp2(-sigma * lr);
+        }
+
+        const T mWi = rj.m * Wi, mWj = rj.m * Wj;
+        const T hv  = T(0.5) * visc;
+        const T vi  = mWi * rhoInv_i * hv, vj = rj.vol * Wj * hv; // viscous weights
+        const T en  = mWi * a_mom;
+        const T ci  = en * prho_i + vi, cj = mWj * b_mom * rj.prho + vj;
+        avEnergy += double(vi * va_i + vj * va_j);
+        energy += double(en * va_i);
+        momx += ci * ax_i + cj * ax_j;
+        momy += ci * ay_i + cj * ay_j;
+        momz += ci * az_i + cj * az_j;
+    };
+    const bool needFold = recordNeedsFold<T, V>(a.box, t, ri, r2h);
+    if constexpr (avClean)
+    {
+        PairWalk<kMomWaves<T>, 2, RecMomVe<T>, RecGradV<T>> walk(a.L, t, rec, gradV);
+        withFold(needFold, [&](auto fold) {
+            walk([&](bool live, const RecMomVe<T>& rj, const RecGradV<T>& gj) { pairTerms(fold, live, rj, &gj); }, rec,
+                 gradV);
+        });
+    }
+    else
+    {
+        PairWalk<kMomWaves<T>, 2, RecMomVe<T>> walk(a.L, t, rec);
+        withFold(needFold, [&](auto fold) {
+            walk([&](bool live, const RecMomVe<T>& rj) { pairTerms(fold, live, rj, nullptr); }, rec);
+        });
+    }
+    double sum[6] = {maxvs, momx, momy, momz, energy, avEnergy};
+    if (!waveSums<kMomWaves<T>, 6, 1>(sum)) { return; }
     double dtLane = INFINITY;
     if (t.valid)
     {
-        const uint32_t    i      = t.i;
-        const RecMomVe<T> ri     = rec[i];
-        T                 hi     = ld<T>(f.h, i);
-        T                 hiInv  = ri.hInv;
-        T                 hiInv2 = hiInv * hiInv, hiInv3 = hiInv2 * hiInv;
-        T                 gradV_i[6] = {0, 0, 0, 0, 0, 0};
-        if constexpr (avClean)
-        {
-            gradV_i[0] = ld<T>(f.dV11, i), gradV_i[1] = ld<T>(f.dV12, i), gradV_i[2] = ld<T>(f.dV13, i);
-            gradV_i[3] = ld<T>(f.dV22, i), gradV_i[4] = ld<T>(f.dV23, i), gradV_i[5] = ld<T>(f.dV33, i);
-        }
-        T      eta_crit = T(cbrt(32.0 * M_PI / 3.0 / double(t.n + 1)));
-        double r2h      = 2.0 * double(hi);
-
-        T      maxvs = 0;
-        T      momx = 0, momy = 0, momz = 0;
-        Acc    energy, avEnergy;
-        withFold(recordNeedsFold<T, V>(a.box, ri, r2h), [&](auto fold) {
-            constexpr int                 U = kBatchMom<T>;
-            NeighborBatch<U, RecMomVe<T>> nb(t, rec);
-            for (unsigned k = 0; k < t.n; k += U)
-            {
-              nb.load(k);
-#pragma unroll
-              for (int u = 0; u < U; ++u)
-              {
-                const uint32_t     j  = nb.j[u];
-                const RecMomVe<T>& rj = nb.r[u];
-                const Sep<T>       r  = pairSeparation<decltype(fold)::value, T>(a.box, r2h, ri, rj);
-                T rx = r.x, ry = r.y, rz = r.z;
-                T vx_ij = ri.vx - rj.vx, vy_ij = ri.vy - rj.vy, vz_ij = ri.vz - rj.vz;
-                T hjInv2 = rj.hInv * rj.hInv;
-                T z1     = r.d2 * hiInv2, z2 = r.d2 * hjInv2;
-                T Wi     = hiInv3 * T(kern.template w<V>(nb.live2(k, u, z1)));
-                T Wj     = rj.hInv * hjInv2 * T(kern.template w<V>(nb.live2(k, u, z2)));
-
-                T tA1_i = -(ri.c11 * rx + ri.c12 * ry + ri.c13 * rz) * Wi;
-                T tA2_i = -(ri.c12 * rx + ri.c22 * ry + ri.c23 * rz) * Wi;
-                T tA3_i = -(ri.c13 * rx + ri.c23 * ry + ri.c33 * rz) * Wi;
-                T tA1_j = -(rj.c11 * rx + rj.c12 * ry + rj.c13 * rz) * Wj;
-                T tA2_j = -(rj.c12 * rx + rj.c22 * ry + rj.c23 * rz) * Wj;
-                T tA3_j = -(rj.c13 * rx + rj.c23 * ry + rj.c33 * rz) * Wj;
-
-                T rv = rx * vx_ij + ry * vy_ij + rz * vz_ij;
-                if constexpr (avClean)
-                {
-                    T gradV_j[6] = {ld<T>(f.dV11, j), ld<T>(f.dV12, j), ld<T>(f.dV13, j),
-                                    ld<T>(f.dV22, j), ld<T>(f.dV23, j), ld<T>(f.dV33, j)};
-                    rv += avRvCorrection(rx, ry, rz, fastSqrt(z1 < z2 ? z1 : z2), eta_crit, gradV_i, gradV_j);
-                }
-                T wij  = overDistance(rv, r.d2);
-                T visc = artificialViscosity(ri.alpha, rj.alpha, ri.c, rj.c, wij);
-                T vsig = T(0.5) * (ri.c + rj.c) - T(2) * wij;
-                maxvs  = nb.in(k, u) && vsig > maxvs ? vsig : maxvs;
-
-                T a_mom, b_mom;
-                T dRho   = ri.rho - rj.rho;
-                T Atwood = fastDiv(dRho < T(0) ? -dRho : dRho, ri.rho + rj.rho);
-                if (Atwood < Atmin)
-                {
-                    a_mom = ri.xm * ri.xm;
-                    b_mom = rj.xm * rj.xm;
-                }
-                else if (Atwood > Atmax)
-                {
-                    a_mom = ri.xm * rj.xm;
-                    b_mom = a_mom;
-                }
-                else
-                {
-                    // xm_i^(2-s) xm_j^s = xm_i^2 2^(s log2(xm_j/xm_i)), and symmetrically for b:
-                    // one logarithm and two exponentials instead of four powers
-                    T sigma = ramp * (Atwood - Atmin);
-                    T lr    = ramLog2(fastDiv(rj.xm, ri.xm));
-                    a_mom   = ri.xm * ri.xm * ramExp2(sigma * lr);
-                    b_mom   = rj.xm * rj.xm * ramExp2(-sigma * lr);
-                }
-
-                T a_visc   = fastDiv(rj.m, ri.rho) * visc;
-                T b_visc   = rj.vol * visc;
-                T a_visc_x = T(0.5) * (a_visc * tA1_i + b_visc * tA1_j);
-                T a_visc_y = T(0.5) * (a_visc * tA2_i + b_visc * tA2_j);
-                T a_visc_z = T(0.5) * (a_visc * tA3_i + b_visc * tA3_j);
-                avEnergy.add(a_visc_x * vx_ij + a_visc_y * vy_ij + a_visc_z * vz_ij);
-                energy.add(rj.m * a_mom * (vx_ij * tA1_i + vy_ij * tA2_i + vz_ij * tA3_i));
-
-                T mom_i = rj.m * ri.prho * a_mom;
-                T mom_j = rj.m * rj.prho * b_mom;
-                momx += mom_i * tA1_i + mom_j * tA1_j + a_visc_x;
-                momy += mom_i * tA2_i + mom_j * tA2_j + a_visc_y;
-                momz += mom_i * tA3_i + mom_j * tA3_j + a_visc_z;
-              }
-            }
-        });
-        double avE    = avEnergy.value() > 0.0 ? avEnergy.value() : 0.0;
-        double eCoeff = f.tdpdTrho ? double(ld<T>(f.tdpdTrho, i)) : double(ri.prho);
-        f.du[i]       = a.K * (eCoeff * energy.value() + 0.5 * avE);
-        st<T>(f.ax, i, T(-a.K * double(momx)));
-        st<T>(f.ay, i, T(-a.K * double(momy)));
-        st<T>(f.az, i, T(-a.K * double(momz)));
-        dtLane = courantDt(maxvs, hi, ri.c, Kcour);
+        // the sums carry the opposite sign of the reference's
+        double avE    = sum[5] < 0.0 ? -sum[5] : 0.0;
+        double eCoeff = f.tdpdTrho ? double(ld<T>(f.tdpdTrho, i)) : double(prho_i);
+        f.du[i]       = a.K * (0.5 * avE - eCoeff * sum[4]);
+        st<T>(f.ax, i, T(a.K * sum[1]));
+        st<T>(f.ay, i, T(a.K * sum[2]));
+        st<T>(f.az, i, T(a.K * sum[3]));
+        dtLane = courantDt(T(sum[0]), hi, ri.c, Kcour);
     }
-    reduceMinDt<T>(minDt, dtLane, a.L.groups);
+    reduceMinDt(minDt, dtLane, a.L.groups);
 }
 
 unsigned long long* resetDt(sphx_workspace* ws)
@@ -552,9 +542,9 @@ double readDt(sphx_workspace* ws, unsigned long long* dt)
 }
 
 template<class T>
-void launchGradh(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f, const sphx_params_t* p)
+void launchGradh(sphx_workspace* ws, PairArgs a, const sphx_fields_t* f, const sphx_params_t* p)
 {
-    unsigned blocks = pairBlocks(a.L);
+    unsigned blocks = a.L.groups.num;
     int      in     = takeChain(ws, kChainGradh, a, f, p);
     if (blocks == 0) { return; }
     RecGradh<T>* rec = recordBuffer<RecGradh<T>>(ws, a.numParticles, in < 0 ? 0 : in);
@@ -570,9 +560,11 @@ void launchGradh(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f, 
                             ? recordBuffer<RecIadVe<T>>(ws, a.numParticles, out)
                             : nullptr;
     {
+        const PairLaunch run = pairLaunch(ws, sizeof(RecGradh<T>), kLightWaves, 3);
+        a.L.stage            = run.stage;
         KernelScope timer(ws, "ve_def_gradh");
-        launchVariant<T>(ws, [&](auto variant) {
-            veDefGradhKernel<T, decltype(variant)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_GRADH) : 0, ws->stream>>>(
+        launchVariant<T>(ws, a.box, [&](auto variant) {
+            veDefGradhKernel<T, decltype(variant)::value><<<blocks, kLightWaves * kWave, run.lds, ws->stream>>>(
                 a, rec, (const T*)f->h, sincKernel<T>(ws), (T*)f->kx, (T*)f->gradh, next, (const T*)f->vx,
                 (const T*)f->vy, (const T*)f->vz);
         });
@@ -582,10 +574,10 @@ void launchGradh(sphx_workspace* ws, const PairArgs& a, const sphx_fields_t* f, 
 }
 
 template<class T>
-void launchIadVe(sphx_workspace* ws, const PairArgs& a, const IadVeFields& vf, const sphx_fields_t* f,
+void launchIadVe(sphx_workspace* ws, PairArgs a, const IadVeFields& vf, const sphx_fields_t* f,
                  const sphx_params_t* p)
 {
-    unsigned blocks = pairBlocks(a.L);
+    unsigned blocks = a.L.groups.num;
     int      in     = takeChain(ws, kChainIadVe, a, f, p);
     if (blocks == 0) { return; }
     RecIadVe<T>* rec = recordBuffer<RecIadVe<T>>(ws, a.numParticles, in < 0 ? 0 : in);
@@ -597,9 +589,11 @@ void launchIadVe(sphx_workspace* ws, const PairArgs& a, const IadVeFields& vf, c
     }
     RecAv<T>* next = chainable(a, p) && f->c ? recordBuffer<RecAv<T>>(ws, a.numParticles, 1 - in) : nullptr;
     {
+        const PairLaunch run = pairLaunch(ws, sizeof(RecIadVe<T>), kLightWaves, 15);
+        a.L.stage            = run.stage;
         KernelScope timer(ws, "iad_divv_curlv");
-        launchVariant<T>(ws, [&](auto variant) {
-            iadDivvCurlvKernel<T, decltype(variant)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_IAD) : 0, ws->stream>>>(
+        launchVariant<T>(ws, a.box, [&](auto variant) {
+            iadDivvCurlvKernel<T, decltype(variant)::value><<<blocks, kLightWaves * kWave, run.lds, ws->stream>>>(
                 a, vf, rec, sincKernel<T>(ws), next, (const T*)f->c);
         });
         SPHX_CHECK_LAUNCH();
@@ -608,10 +602,10 @@ void launchIadVe(sphx_workspace* ws, const PairArgs& a, const IadVeFields& vf, c
 }
 
 template<class T>
-void launchAv(sphx_workspace* ws, const PairArgs& a, const AvFields& af, const sphx_fields_t* f,
+void launchAv(sphx_workspace* ws, PairArgs a, const AvFields& af, const sphx_fields_t* f,
               const sphx_params_t* p)
 {
-    unsigned blocks = pairBlocks(a.L);
+    unsigned blocks = a.L.groups.num;
     int      in     = takeChain(ws, kChainAv, a, f, p);
     if (blocks == 0) { return; }
     RecAv<T>* rec = recordBuffer<RecAv<T>>(ws, a.numParticles, in < 0 ? 0 : in);
@@ -624,9 +618,11 @@ void launchAv(sphx_workspace* ws, const PairArgs& a, const AvFields& af, const s
     RecMomVe<T>* next =
         chainable(a, p) && f->m && f->prho ? recordBuffer<RecMomVe<T>>(ws, a.numParticles, 1 - in) : nullptr;
     {
+        const PairLaunch run = pairLaunch(ws, sizeof(RecAv<T>), kLightWaves, 4);
+        a.L.stage            = run.stage;
         KernelScope timer(ws, "av_switches");
-        launchVariant<T>(ws, [&](auto variant) {
-            avSwitchesKernel<T, decltype(variant)::value><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_AV) : 0, ws->stream>>>(
+        launchVariant<T>(ws, a.box, [&](auto variant) {
+            avSwitchesKernel<T, decltype(variant)::value><<<blocks, kLightWaves * kWave, run.lds, ws->stream>>>(
                 a, af, rec, sincKernel<T>(ws), p->minDt, T(p->alphamin), T(p->alphamax), T(p->decay_constant), next);
         });
         SPHX_CHECK_LAUNCH();
@@ -635,10 +631,10 @@ void launchAv(sphx_workspace* ws, const PairArgs& a, const AvFields& af, const s
 }
 
 template<class T>
-void launchMomVe(sphx_workspace* ws, const PairArgs& a, const MomVeFields& mf, const sphx_fields_t* f,
+void launchMomVe(sphx_workspace* ws, PairArgs a, const MomVeFields& mf, const sphx_fields_t* f,
                  const sphx_params_t* p, bool avClean, unsigned long long* dt)
 {
-    unsigned blocks = pairBlocks(a.L);
+    unsigned blocks = a.L.groups.num;
     int      in     = takeChain(ws, kChainMomVe, a, f, p);
     if (blocks == 0) { return; }
     RecMomVe<T>* rec = recordBuffer<RecMomVe<T>>(ws, a.numParticles, in < 0 ? 0 : in);
@@ -647,15 +643,25 @@ void launchMomVe(sphx_workspace* ws, const PairArgs& a, const MomVeFields& mf, c
         packMomVe<T><<<ceilDiv(a.numParticles, kPackThreads), kPackThreads, 0, ws->stream>>>(a, mf, rec);
         SPHX_CHECK_LAUNCH();
     }
+    RecGradV<T>* gradV = nullptr;
+    if (avClean)
+    {
+        ws->recordsGradV.reserve((size_t(a.numParticles) * sizeof(RecGradV<T>) + 15) / 16);
+        gradV = reinterpret_cast<RecGradV<T>*>(ws->recordsGradV.get());
+        packGradV<T><<<ceilDiv(a.numParticles, kPackThreads), kPackThreads, 0, ws->stream>>>(a.box, mf, gradV, a.numParticles);
+        SPHX_CHECK_LAUNCH();
+    }
+    const PairLaunch run = pairLaunch(ws, sizeof(RecMomVe<T>) + (avClean ? sizeof(RecGradV<T>) : 0), kMomWaves<T>, 6);
+    a.L.stage            = run.stage;
     KernelScope timer(ws, "momentum_ve");
-    launchVariant<T>(ws, [&](auto variant) {
+    launchVariant<T>(ws, a.box, [&](auto variant) {
         constexpr int V = decltype(variant)::value;
         if (avClean)
-            momentumVeKernel<T, true, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(
-                a, mf, rec, sincKernel<T>(ws), T(p->Atmin), T(p->Atmax), T(p->ramp), float(p->Kcour), dt);
+            momentumVeKernel<T, true, V><<<blocks, kMomWaves<T> * kWave, run.lds, ws->stream>>>(
+                a, mf, rec, gradV, sincKernel<T>(ws), T(p->Atmin), T(p->Atmax), T(p->ramp), float(p->Kcour), dt);
         else
-            momentumVeKernel<T, false, V><<<blocks, kPairWaves * kWave, isMixed<T> ? occupancyCap(SPHX_CAP_MOM) : 0, ws->stream>>>(
-                a, mf, rec, sincKernel<T>(ws), T(p->Atmin), T(p->Atmax), T(p->ramp), float(p->Kcour), dt);
+            momentumVeKernel<T, false, V><<<blocks, kMomWaves<T> * kWave, run.lds, ws->stream>>>(
+                a, mf, rec, gradV, sincKernel<T>(ws), T(p->Atmin), T(p->Atmax), T(p->ramp), float(p->Kcour), dt);
     });
     SPHX_CHECK_LAUNCH();
 }

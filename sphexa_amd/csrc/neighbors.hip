@@ -58,10 +58,13 @@ struct SearchArgs
     const double*        sizes;
     DevBox               box;
     double               slack; // absolute enlargement of search radii (rounding margin)
-    uint32_t             first, last, ng0, ngmax, ngmax4;
+    uint32_t             first, last, ng0, ngmax;
     Groups               groups; // target groups, one wavefront each
     int                  iterateH;
-    uint32_t*            nbrs;
+    void*                nbrs;
+    uint32_t*            owner;      // local lists: the targets' groups (null: consecutive groups)
+    uint32_t*            table;      // local lists: the groups' tables ...
+    uint32_t*            tableCount; // ... and their sizes (over kTableCap: the table did not fit)
     uint32_t*            nc;
     unsigned long long*  stats; // [0] stored pairs, [1] max count, [2] non-converged particles, [kStatWide] wide
                                 // support, [kStatTests] candidate distance tests (swept candidates x 64 lanes)
@@ -78,7 +81,7 @@ struct SearchArgs
 
 //! per-wave LDS: traversal stack, candidate leaves, the kept leaves' particle ranges, and the
 //! double-buffered candidate tile (with the candidates' masses for the fused XMass only)
-template<bool Mass>
+template<bool Mass, bool Local>
 struct WaveLds
 {
     int32_t  stack[kStackCap];      // pending nodes, the first in visiting order on top
@@ -90,12 +93,13 @@ struct WaveLds
     double   tx[2][kWave], ty[2][kWave], tz[2][kWave];
     uint32_t tj[2][kWave]; // particle index of each staged candidate
     double   tm[2][Mass ? kWave : 1]; // its mass (fused XMass only)
+    uint32_t self[Local ? kWave : 1]; // local lists: the target's own place in the tile
 };
 
 // sixteen waves of the search share a CU's 160 KB of LDS (the fused search + XMass, with its masses,
 // holds three waves per SIMD by its registers)
-static_assert(sizeof(WaveLds<false>) <= 160 * 1024 / 16, "search LDS must leave room for 16 waves per CU");
-static_assert(sizeof(WaveLds<true>) <= 160 * 1024 / 12, "fused search LDS must leave room for 12 waves per CU");
+static_assert(sizeof(WaveLds<false, true>) <= 160 * 1024 / 16, "search LDS must leave room for 16 waves per CU");
+static_assert(sizeof(WaveLds<true, false>) <= 160 * 1024 / 12, "fused search LDS must leave room for 12 waves per CU");
 
 //! per-target state of a lane
 struct Target
@@ -108,32 +112,40 @@ struct Target
 };
 
 //! A lane's appending writer into its neighbour list: entries collect in a register quad that is
-//! stored (16 bytes) when full and, for the incomplete last quad, by finish(). Slots past the
-//! stored count inside that quad receive don't-care values; readers never use them.
+//! stored (16 bytes) when full and, for the incomplete last one, by finish(). Local lists pack eight
+//! 16-bit table positions into it, global lists four particle indices. Slots past the stored count
+//! inside the last 16 bytes repeat the newest entry.
+template<bool Local>
 struct ListWriter
 {
-    uint32_t* base; // the lane's slot 0
-    uint32_t  q0 = 0, q1 = 0, q2 = 0, q3 = 0; // the last four entries, oldest first
-    uint32_t  swept = 0; // candidates swept by the wave (each tested by all 64 lanes)
+    static constexpr unsigned kRun = Local ? 8 : 4; // entries per 16 bytes
 
-    //! entry k = j: shifted in behind the previous three, stored when it completes a quad
-    __device__ __forceinline__ void put(unsigned k, uint32_t j)
+    char*    base; // the lane's slot 0
+    uint32_t q0 = 0, q1 = 0, q2 = 0, q3 = 0; // the last entries, oldest first
+    uint32_t swept = 0;    // candidates swept by the wave (each tested by all 64 lanes)
+    uint32_t inTable = 0;  // local lists: particles in the group's table (wave-uniform)
+    uint32_t group   = 0;  // the group
+
+    //! entry k = e: shifted in behind the previous ones, stored when it completes 16 bytes
+    __device__ __forceinline__ void put(unsigned k, uint32_t e)
     {
-        q0 = q1, q1 = q2, q2 = q3, q3 = j;
-        if ((k & 3u) == 3u) { store(k, q0, q1, q2, q3); }
+        if constexpr (Local)
+        {
+            q0 = __builtin_amdgcn_alignbit(q1, q0, 16), q1 = __builtin_amdgcn_alignbit(q2, q1, 16);
+            q2 = __builtin_amdgcn_alignbit(q3, q2, 16), q3 = __builtin_amdgcn_alignbit(e, q3, 16);
+        }
+        else { q0 = q1, q1 = q2, q2 = q3, q3 = e; }
+        if ((k & (kRun - 1)) == kRun - 1)
+        {
+            // runs of all 64 lanes interleave: run r starts at r * 64 * 16 bytes
+            *reinterpret_cast<uint4*>(base + size_t(k / kRun) * (kGroup * 16)) = make_uint4(q0, q1, q2, q3);
+        }
     }
-    __device__ __forceinline__ void store(unsigned k, uint32_t a, uint32_t b, uint32_t c, uint32_t d)
-    {
-        *reinterpret_cast<uint4*>(base + laneSlot(k & ~3u)) = make_uint4(a, b, c, d);
-    }
-    //! flush after `stored` entries: the r = stored % 4 last ones (q3 the newest) open the quad;
-    //! its remaining slots (never read) repeat the newest entry
+    //! flush after `stored` entries
     __device__ __forceinline__ void finish(unsigned stored)
     {
-        const unsigned r = stored & 3u;
-        if (r == 1) { store(stored - 1, q3, q3, q3, q3); }
-        else if (r == 2) { store(stored - 1, q2, q3, q3, q3); }
-        else if (r == 3) { store(stored - 1, q1, q2, q3, q3); }
+        const uint32_t last = Local ? q3 >> 16 : q3;
+        while (stored & (kRun - 1)) { put(stored++, last); }
     }
 };
 
@@ -166,10 +178,10 @@ struct XMassSum
     __device__ __forceinline__ void stage(int u, bool stored, double dx, double dy, double dz, double m)
     {
         Th rx = Th(dx), ry = Th(dy), rz = Th(dz);
-        Th z  = (rx * rx + ry * ry + rz * rz) * (hInv * hInv);
+        Th d2 = rx * rx + ry * ry + rz * rz;
         on[u] = stored;
         mj[u] = Th(m);
-        w[u]  = kern.template w<kAnyIndex>(stored ? z : Th(4)); // 4: the edge of the support, W = 0
+        w[u]  = kern.template w<kAnyIndex>(kern.clamp(kern.arg(d2, kernelScale(hInv)), stored));
     }
     __device__ __forceinline__ void flush()
     {
@@ -190,6 +202,18 @@ __device__ __forceinline__ double uniformD(double v)
     return __longlong_as_double((long long)((uint64_t(hi) << 32) | lo));
 }
 
+//! bitwise or over the wave (uniform result): row steps, then the two row broadcasts, total in lane 63
+__device__ __forceinline__ uint32_t waveOr(uint32_t v)
+{
+    v |= __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true); // row_shr:1
+    v |= __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true); // row_shr:2
+    v |= __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true); // row_shr:4
+    v |= __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true); // row_shr:8
+    v |= __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false); // row_bcast:15
+    v |= __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false); // row_bcast:31
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
 enum class Fold
 {
     none,    // all pairs of the tile use the direct image
@@ -200,11 +224,14 @@ enum class Fold
 //! Test the `n` staged candidates against the lane's target. Hits are recorded as bits of a
 //! per-lane mask over the tile's candidates and appended afterwards in candidate order, so the
 //! list keeps the traversal order while the test loop stays free of the divergent append.
-template<Fold mode, class Sink>
+/* Local lists: a target's own bit is cleared (a lane finds its place through `self`), the candidates
+ * that some target keeps take the next positions of the group's table, and their entries of tj become
+ * those positions. */
+template<Fold mode, bool Local, class Sink>
 __device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, const double* tx, const double* ty,
-                                          const double* tz, const uint32_t* tj, const double* tm, uint32_t n,
-                                          double sx, double sy, double sz, unsigned& count, ListWriter& out,
-                                          Sink& sink)
+                                          const double* tz, uint32_t* tj, const double* tm, uint32_t* self,
+                                          uint32_t n, double sx, double sy, double sz, unsigned& count,
+                                          ListWriter<Local>& out, Sink& sink)
 {
 #pragma clang fp contract(off)
     const DevBox&  b     = a.box;
@@ -236,6 +263,28 @@ __device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, 
         uint64_t       m  = test32(c0, min(cn, 32u));
         if (cn > 32u) { m |= uint64_t(test32(c0 + 32u, cn - 32u)) << 32; }
         if (!t.active) { m = 0; }
+        if constexpr (Local)
+        {
+            const unsigned lane = laneId();
+            const uint32_t j    = lane < cn ? tj[c0 + lane] : 0xffffffffu;
+            self[lane]          = kWave;
+            __builtin_amdgcn_wave_barrier();
+            // the wave's targets are consecutive particles from lane 0's on
+            const uint32_t rel = j - (t.i - lane);
+            if (rel < uint32_t(kWave)) { self[rel] = lane; }
+            __builtin_amdgcn_wave_barrier();
+            const uint32_t own = self[lane];
+            if (own < uint32_t(kWave)) { m &= ~(uint64_t(1) << own); }
+            const uint64_t used = uint64_t(waveOr(uint32_t(m))) | uint64_t(waveOr(uint32_t(m >> 32))) << 32;
+            const uint32_t pos  = out.inTable + laneRank(used);
+            if ((used >> lane) & 1u)
+            {
+                if (pos < kTableCap) { a.table[size_t(out.group) * kTableCap + pos] = j; }
+                tj[c0 + lane] = pos;
+            }
+            out.inTable += uint32_t(__popcll(used));
+            __builtin_amdgcn_wave_barrier();
+        }
         while (m)
         {
 #pragma unroll
@@ -244,7 +293,7 @@ __device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, 
                 const bool     have  = m != 0;
                 const uint32_t c     = c0 + (have ? uint32_t(__builtin_ctzll(m)) : 0u);
                 const uint32_t j     = tj[c];
-                const bool     keep  = have && j != t.i;
+                const bool     keep  = have && (Local || j != t.i);
                 const bool     store = keep && count < ngmax;
                 m &= m - 1;
                 if (store) { out.put(count, j); }
@@ -315,9 +364,9 @@ __device__ __forceinline__ double imageShift(const DevBox& b, int code, int d)
 }
 
 //! sweep the first n candidates of tile buffer `buf`, all of image `code`
-template<class Sink, class Lds>
+template<bool Local, class Sink, class Lds>
 __device__ __forceinline__ void sweepBuffer(const SearchArgs& a, const Target& t, Lds& lds, int buf, uint32_t n,
-                                            int code, unsigned& count, ListWriter& out, Sink& sink)
+                                            int code, unsigned& count, ListWriter<Local>& out, Sink& sink)
 {
     __builtin_amdgcn_wave_barrier(); // a wave's LDS accesses complete in order
     out.swept += n;
@@ -325,12 +374,12 @@ __device__ __forceinline__ void sweepBuffer(const SearchArgs& a, const Target& t
     const double* ty = lds.ty[buf];
     const double* tz = lds.tz[buf];
     if (code == kPerPairImage)
-        sweepTile<Fold::perPair>(a, t, tx, ty, tz, lds.tj[buf], lds.tm[buf], n, 0, 0, 0, count, out, sink);
+        sweepTile<Fold::perPair>(a, t, tx, ty, tz, lds.tj[buf], lds.tm[buf], lds.self, n, 0, 0, 0, count, out, sink);
     else if (code != kNoShiftImage)
-        sweepTile<Fold::shifted>(a, t, tx, ty, tz, lds.tj[buf], lds.tm[buf], n, imageShift(a.box, code, 0),
+        sweepTile<Fold::shifted>(a, t, tx, ty, tz, lds.tj[buf], lds.tm[buf], lds.self, n, imageShift(a.box, code, 0),
                                  imageShift(a.box, code, 1), imageShift(a.box, code, 2), count, out, sink);
     else
-        sweepTile<Fold::none>(a, t, tx, ty, tz, lds.tj[buf], lds.tm[buf], n, 0, 0, 0, count, out, sink);
+        sweepTile<Fold::none>(a, t, tx, ty, tz, lds.tj[buf], lds.tm[buf], lds.self, n, 0, 0, 0, count, out, sink);
     __builtin_amdgcn_wave_barrier();
 }
 
@@ -346,10 +395,11 @@ __device__ __forceinline__ void sweepBuffer(const SearchArgs& a, const Target& t
  *    A full tile of 64 (or the last one, or one whose image ends) is swept, while the next
  *    window's loads are in flight. The candidate order is therefore the traversal order, as in
  *    the reference. */
-template<class Sink, class Lds>
+template<bool Local, class Sink, class Lds>
 __device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t, Lds& lds, const int32_t* leaves, int nLeaf,
                             const double gc[3],
-                            const double ge[3], double reach, unsigned& count, ListWriter& out, Sink& sink)
+                            const double ge[3], double reach, unsigned& count, ListWriter<Local>& out,
+                            Sink& sink)
 {
 #pragma clang fp contract(off)
     const DevBox&  b    = a.box;
@@ -591,9 +641,9 @@ __device__ __forceinline__ void sortFoundLeaves(Lds& lds, int n)
  * i.e. it proceeds depth first and adds at most 7 entries per tree level below the popped node
  * (<= 7*20 = 140 < 160) on top of the stack it started from. A single pop adds at most one leaf,
  * the first in order of all, and the buffer is swept whenever it reaches its spare slots. */
-template<class Sink, class Lds>
-__device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const Target& t, double radius, Lds& lds, ListWriter& out,
-                                    Sink& sink)
+template<bool Local, class Sink, class Lds>
+__device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const Target& t, double radius, Lds& lds,
+                                                    ListWriter<Local>& out, Sink& sink)
 {
 #pragma clang fp contract(off)
     const unsigned lane = laneId();
@@ -715,15 +765,13 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
     return count;
 }
 
-//! search of the active lanes' targets into their lists (slot 0 at myList); returns the counts
-template<class Sink, class Lds>
-__device__ __forceinline__ unsigned searchGroup(const SearchArgs& a, const Target& t, double radius, Lds& lds, uint32_t* myList,
-                                Sink& sink, uint32_t& swept)
+//! search of the active lanes' targets into their lists (`out` at slot 0); returns the counts
+template<bool Local, class Sink, class Lds>
+__device__ __forceinline__ unsigned searchGroup(const SearchArgs& a, const Target& t, double radius, Lds& lds,
+                                                ListWriter<Local>& out, Sink& sink)
 {
-    ListWriter out{myList};
-    unsigned   count = searchGroupInto(a, t, radius, lds, out, sink);
+    unsigned count = searchGroupInto(a, t, radius, lds, out, sink);
     if (t.active) { out.finish(min(count, a.ngmax)); }
-    swept += out.swept;
     return count;
 }
 
@@ -759,12 +807,13 @@ __device__ __forceinline__ void setRadius(Target& t, Th hi, double slack)
 #define SPHX_WAVES_SEARCH_F64 4
 #endif
 
-template<class Th, bool XMass>
+template<class Th, bool XMass, bool Local>
 __global__ void __launch_bounds__(kWavesPerBlock * kWave)
 __attribute__((amdgpu_waves_per_eu(XMass ? 1 : isMixed<Th> ? SPHX_WAVES_SEARCH_F32 : SPHX_WAVES_SEARCH_F64)))
 searchKernel(SearchArgs a, Th* __restrict__ h)
 {
-    __shared__ WaveLds<XMass> ldsMem[kWavesPerBlock];
+    static_assert(!(XMass && Local), "the fused XMass stores global lists");
+    __shared__ WaveLds<XMass, Local> ldsMem[kWavesPerBlock];
 
     const unsigned wid  = threadIdx.x / kWave;
     const unsigned lane = laneId();
@@ -775,7 +824,7 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     groupRange(a.groups, g, base, end, oversized);
     base = uniform(base), end = uniform(end);
     if (oversized && lane == 0) { atomicAdd(&a.stats[kStatBadGroups], 1ull); }
-    WaveLds<XMass>& lds = ldsMem[wid];
+    WaveLds<XMass, Local>& lds = ldsMem[wid];
 
     Target t;
     t.i      = base + lane;
@@ -786,8 +835,15 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     t.z      = t.active ? a.z[t.i] : 0.0;
     setRadius(t, hi, a.slack);
     // lists are indexed by particle: target i at group (i - first) / 64, lane (i - first) % 64
-    const uint32_t r      = t.active ? t.i - a.first : 0u;
-    uint32_t*      myList = a.nbrs + listOffset(r / kGroup, a.ngmax4, 0, r % kGroup);
+    const uint32_t    r = t.active ? t.i - a.first : 0u;
+    ListWriter<Local> out;
+    if constexpr (Local)
+    {
+        out.base  = static_cast<char*>(a.nbrs) + 2 * localOffset(r / kGroup, paddedNgmax8(a.ngmax), 0, r % kGroup);
+        out.group = g;
+        if (a.owner && t.active) { a.owner[r] = g; }
+    }
+    else { out.base = static_cast<char*>(a.nbrs) + 4 * listOffset(r / kGroup, paddedNgmax(a.ngmax), 0, r % kGroup); }
 
     using Sink = std::conditional_t<XMass, XMassSum<Th>, ListOnly>;
     Sink      sink;
@@ -805,8 +861,7 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     resetSink();
 
     bool     valid = t.active;
-    uint32_t swept = 0;
-    unsigned count = searchGroup(a, t, double(2) * double(hi), lds, myList, sink, swept);
+    unsigned count = searchGroup(a, t, double(2) * double(hi), lds, out, sink);
     unsigned ncSph = 1 + count;
 
     int      updates = 0;
@@ -825,7 +880,7 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
                 resetSink();
             }
             t.active       = repeat;
-            unsigned again = searchGroup(a, t, double(2) * double(hi), lds, myList, sink, swept);
+            unsigned again = searchGroup(a, t, double(2) * double(hi), lds, out, sink);
             if (repeat) { ncSph = 1 + again; }
         }
     }
@@ -833,8 +888,6 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     {
         if (updates > 0) { h[t.i] = hi; }
         a.nc[t.i] = ncSph;
-        // slot 0 always names a particle: the pair loops read one slot ahead without a branch
-        if (ncSph == 1) { myList[0] = t.i; }
         if constexpr (XMass)
         {
             // epilogue of xmassKernel: FP64 normalisation with h^-3 rounded in h's type
@@ -862,21 +915,36 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
         atomicMax(&a.stats[1], (unsigned long long)mx);
         if (fails) { atomicAdd(&a.stats[2], (unsigned long long)fails); }
         if (wide) { atomicAdd(&a.stats[kStatWide], (unsigned long long)wide); }
-        atomicAdd(&a.stats[kStatTests], (unsigned long long)swept * kWave);
+        atomicAdd(&a.stats[kStatTests], (unsigned long long)out.swept * kWave);
+        if constexpr (Local) { a.tableCount[g] = out.inTable; }
     }
 }
 
-//! row i - first of `out` = stored list of target i; groups count from the searched range's first target
-__global__ void copyListsKernel(const uint32_t* __restrict__ nbrs, const uint32_t* __restrict__ nc,
-                                uint32_t* __restrict__ out, uint32_t searchFirst, uint32_t first, uint32_t last,
-                                uint32_t ngmax)
+//! histogram of the groups' table sizes: bin s / kTableBin, the last one for tables that did not fit
+__global__ void __launch_bounds__(256) tableHistKernel(const uint32_t* __restrict__ tableCount, uint32_t blocks,
+                                                       uint32_t* hist)
+{
+    __shared__ uint32_t part[kTableBins + 1];
+    if (threadIdx.x <= kTableBins) { part[threadIdx.x] = 0; }
+    __syncthreads();
+    for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < blocks; g += gridDim.x * blockDim.x)
+    {
+        const uint32_t s = tableCount[g];
+        atomicAdd(&part[s > kTableCap ? kTableBins : (s == 0 ? 0 : (s - 1) / kTableBin)], 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x <= kTableBins && part[threadIdx.x]) { atomicAdd(&hist[threadIdx.x], part[threadIdx.x]); }
+}
+
+//! row i - first of `out` = stored list of target i
+__global__ void copyListsKernel(NeighborLists lists, const uint32_t* __restrict__ nc, uint32_t* __restrict__ out,
+                                uint32_t searchFirst, uint32_t first, uint32_t last)
 {
     uint32_t i = first + blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= last) { return; }
-    uint32_t r = i - searchFirst, g = r / kGroup, lane = r % kGroup;
-    uint32_t n = min(nc[i] - 1, ngmax);
+    uint32_t n = min(nc[i] - 1, lists.ngmax);
     for (uint32_t k = 0; k < n; ++k)
-        out[size_t(i - first) * ngmax + k] = nbrs[listOffset(g, paddedNgmax(ngmax), k, lane)];
+        out[size_t(i - first) * lists.ngmax + k] = lists.entry(i - searchFirst, k);
 }
 
 } // namespace
@@ -893,11 +961,27 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     const Tree&  t      = ws->tree;
     const Groups grp    = groupsFor(ws, first, last);
     const uint32_t groups = grp.num;
-    // list blocks of 64 consecutive particles from first, whatever the target groups
-    ws->nbrs.reserve(std::max<size_t>(1, size_t(ceilDiv(last - first, kGroup)) * paddedNgmax(p->ngmax) * kGroup));
+    // list blocks of 64 consecutive particles from first, whatever the target groups. Local lists take 2 bytes
+    // a slot and 8 KB of table per group; with more than twice as many groups as blocks the tables
+    // would outgrow the lists, and the search stores global lists (4 bytes a slot)
+    const size_t blocks64    = std::max<size_t>(1, ceilDiv(last - first, kGroup));
+    const bool   tryLocal    = xmassOut == kSearchOnly && groups <= 2 * blocks64 + 64;
+    const bool   owned       = tryLocal && grp.start != nullptr;
+    const size_t localWords  = blocks64 * paddedNgmax8(p->ngmax) * kGroup / 2;
+    const size_t globalWords = blocks64 * paddedNgmax(p->ngmax) * kGroup;
+    ws->nbrs.reserve(tryLocal ? localWords : globalWords);
+    if (tryLocal)
+    {
+        ws->nbTable.reserve(std::max<size_t>(1, groups) * kTableCap);
+        ws->nbTableCount.reserve(std::max<size_t>(1, groups));
+    }
+    if (owned)
+    {
+        const size_t pairs = (size_t(last - first) + 1) / 2; // two owners per 64-bit word
+        ws->nbOwner.reserve(2 * std::max<size_t>(1, pairs));
+        fill64(ws, reinterpret_cast<uint64_t*>(ws->nbOwner.get()), ~uint64_t(0), pairs);
+    }
     ws->counters.reserve(2 * kCounterSlots);
-    fill64(ws, reinterpret_cast<uint64_t*>(ws->counters.get()), 0, 3);
-    fill64(ws, reinterpret_cast<uint64_t*>(ws->counters.get()) + kStatWide, 0, kCounterSlots - kStatWide);
 
     double scale = 0;
     for (int d = 0; d < 3; ++d)
@@ -914,11 +998,14 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     a.sizes          = t.sizes.get();
     a.box            = box;
     a.slack          = 1e-12 * scale;
-    a.first = first, a.last = last, a.ng0 = p->ng0, a.ngmax = p->ngmax, a.ngmax4 = paddedNgmax(p->ngmax);
+    a.first = first, a.last = last, a.ng0 = p->ng0, a.ngmax = p->ngmax;
     a.groups = grp;
     a.iterateH = iterateH ? 1 : 0;
-    a.nbrs     = ws->nbrs.get();
-    a.nc       = f->nc;
+    a.nbrs       = ws->nbrs.get();
+    a.owner      = owned ? ws->nbOwner.get() : nullptr;
+    a.table      = ws->nbTable.get();
+    a.tableCount = ws->nbTableCount.get();
+    a.nc         = f->nc;
     a.stats    = reinterpret_cast<unsigned long long*>(ws->counters.get());
     a.minLen   = std::min(box.len[0], std::min(box.len[1], box.len[2]));
     a.m = nullptr, a.wh = nullptr, a.sincN = 0, a.sincInt = -1, a.K = 0, a.xmOut = nullptr, a.toRho = 0;
@@ -937,32 +1024,66 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
         a.toRho = xmassOut == kSearchRho;
     }
 
-    if (groups > 0)
-    {
-        unsigned    blocks = ceilDiv(groups, kWavesPerBlock);
-        KernelScope timer(ws, "search");
-        const dim3  grid(blocks), block(kWavesPerBlock * kWave);
-        if (xmassOut == kSearchOnly)
-        {
-            if (f32) searchKernel<float, false><<<grid, block, 0, ws->stream>>>(a, static_cast<float*>(f->h));
-            else searchKernel<double, false><<<grid, block, 0, ws->stream>>>(a, static_cast<double*>(f->h));
-        }
-        else
-        {
-            if (f32) searchKernel<float, true><<<grid, block, 0, ws->stream>>>(a, static_cast<float*>(f->h));
-            else searchKernel<double, true><<<grid, block, 0, ws->stream>>>(a, static_cast<double*>(f->h));
-        }
-        SPHX_CHECK_LAUNCH();
-    }
     unsigned long long stats[kCounterSlots];
-    SPHX_HIP(hipMemcpyAsync(stats, ws->counters.get(), sizeof(stats), hipMemcpyDeviceToHost, ws->stream));
-    SPHX_HIP(hipStreamSynchronize(ws->stream));
+    uint32_t           hist[kTableBins + 1];
+    auto               run = [&](bool local)
+    {
+        fill64(ws, reinterpret_cast<uint64_t*>(ws->counters.get()), 0, 3);
+        fill64(ws, reinterpret_cast<uint64_t*>(ws->counters.get()) + kStatWide, 0, kCounterSlots - kStatWide);
+        if (groups > 0)
+        {
+            unsigned    blocks = ceilDiv(groups, kWavesPerBlock);
+            KernelScope timer(ws, "search");
+            const dim3  grid(blocks), block(kWavesPerBlock * kWave);
+            if (local)
+            {
+                if (f32) searchKernel<float, false, true><<<grid, block, 0, ws->stream>>>(a, static_cast<float*>(f->h));
+                else searchKernel<double, false, true><<<grid, block, 0, ws->stream>>>(a, static_cast<double*>(f->h));
+            }
+            else if (xmassOut == kSearchOnly)
+            {
+                if (f32) searchKernel<float, false, false><<<grid, block, 0, ws->stream>>>(a, static_cast<float*>(f->h));
+                else searchKernel<double, false, false><<<grid, block, 0, ws->stream>>>(a, static_cast<double*>(f->h));
+            }
+            else
+            {
+                if (f32) searchKernel<float, true, false><<<grid, block, 0, ws->stream>>>(a, static_cast<float*>(f->h));
+                else searchKernel<double, true, false><<<grid, block, 0, ws->stream>>>(a, static_cast<double*>(f->h));
+            }
+            SPHX_CHECK_LAUNCH();
+            if (local)
+            {
+                tableHistKernel<<<std::min(ceilDiv(groups, 256), 64u), 256, 0, ws->stream>>>(
+                    ws->nbTableCount.get(), groups,
+                    reinterpret_cast<uint32_t*>(ws->counters.get()) + 2 * kStatHist);
+                SPHX_CHECK_LAUNCH();
+            }
+        }
+        SPHX_HIP(hipMemcpyAsync(stats, ws->counters.get(), sizeof(stats), hipMemcpyDeviceToHost, ws->stream));
+        SPHX_HIP(hipStreamSynchronize(ws->stream));
+        std::memcpy(hist, &stats[kStatHist], sizeof(hist));
+    };
+    run(tryLocal);
+    bool                     local = tryLocal;
+    const unsigned long long fails = stats[2];
+    if (local && hist[kTableBins] > 0)
+    {
+        // a table did not fit: the same lists in the global layout, at the h the first run converged to
+        local      = false;
+        a.iterateH = 0;
+        ws->nbrs.reserve(globalWords);
+        a.nbrs = ws->nbrs.get();
+        run(false);
+    }
 
     ws->nbFirst      = first;
     ws->nbLast       = last;
     ws->nbNgmax      = p->ngmax;
     ws->nbNc         = f->nc;
     ws->nbValid      = true;
+    ws->nbLocal      = local;
+    ws->nbOwned      = local && owned;
+    std::memcpy(ws->nbTableHist, hist, sizeof(hist));
     ++ws->searchSerial;
     ws->statSumPairs = stats[0];
     ws->statMaxCount = uint32_t(stats[1]);
@@ -974,7 +1095,7 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
         ws->nbValid = false;
         throw Error{SPHX_ERR_ARG, std::to_string(stats[kStatBadGroups]) + " target groups hold more than 64 particles"};
     }
-    return stats[2] > 0 ? SPHX_ERR_NOT_CONVERGED : SPHX_OK;
+    return fails > 0 ? SPHX_ERR_NOT_CONVERGED : SPHX_OK;
 }
 
 void copyNeighbors(sphx_workspace* ws, uint32_t* out, uint32_t first, uint32_t last)
@@ -995,8 +1116,8 @@ void copyNeighbors(sphx_workspace* ws, uint32_t* out, uint32_t first, uint32_t l
         staging.reserve(len);
         dst = staging.get();
     }
-    copyListsKernel<<<ceilDiv(last - first, 256), 256, 0, ws->stream>>>(ws->nbrs.get(), ws->nbNc, dst, ws->nbFirst, first,
-                                                                          last, ws->nbNgmax);
+    copyListsKernel<<<ceilDiv(last - first, 256), 256, 0, ws->stream>>>(neighborLists(ws), ws->nbNc, dst, ws->nbFirst,
+                                                                        first, last);
     SPHX_CHECK_LAUNCH();
     if (!onDevice)
     {

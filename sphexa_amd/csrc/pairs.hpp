@@ -1,18 +1,32 @@
 // Helpers shared by the SPH pair-loop kernels (std and VE).
 //
-// Launch shape: one wavefront per group of 64 consecutive targets (the neighbour-search group),
-// 4 waves per block, blocks renumbered per XCD (xcdBlock) so that neighbouring groups share an
-// L2. Lane l of wave g owns target first + 64 g + l and walks its own list slots
-// k < min(nc-1, ngmax) in the quad layout of common.hpp (listOffset).
+// Launch shape: one block of W waves (4, or 8 where the records fill a CU's LDS) per group of 64 consecutive targets (the neighbour-search
+// group), blocks renumbered per XCD (xcdBlock) so that neighbouring groups share an L2. Lane l of
+// every wave owns target first + 64 g + l; wave w takes the quads w, w + W, .. of its list, and the
+// waves' partial sums are added at the end in a fixed order (waveSums), so a target's result does
+// not depend on the grouping of the call.
+//
+// The targets of a group share most of their neighbours: about 600 distinct particles against
+// 64 x 91 list entries on a lattice. Read from global memory, each entry costs one tag lookup of the
+// vector cache per lane and 16-byte chunk of its record, about 50 cycles of a CU per chunk, which
+// bound the loops. With local lists (common.hpp) the block first copies the records of the group's
+// table to LDS, chunk c of all records side by side, and every neighbour is read from there
+// (PairWalk). Groups whose table does not fit the launch's LDS, and global lists,
+// read the records from global memory in the same order. Measured (ms; gathers from global memory, then this):
+// mixed VE at 8M particles, XMass 1.27 -> 0.81, grad-h 2.13 -> 1.36, IAD 2.17 -> 1.57, AV switches 2.84 -> 1.78,
+// momentum-energy 4.92 -> 3.24; FP64 VE at 4.1M, 2.35 -> 1.05, 2.90 -> 2.06, 3.26 -> 2.07, 4.06 -> 2.30, 6.76 ->
+// 5.26 (with the kernel evaluated instead of gathered from its table). What bounds them now: the FP32 form
+// the vector ALU (62-86% of its issue slots), the FP64 form the latency of a block's phases at 2-3 waves per SIMD.
 //
 // Two arithmetic forms share each kernel template:
 //  * T = double ("plain" FP64): the reference JLoop formulas in FP64.
 //  * T = float ("mixed"): HydroType fields in float (the reference's SphTypes layout); pair
-//    separations are formed in FP64 from the FP64 positions, folded, then rounded to float;
-//    kernel lookups, gradients and pair terms in FP32; density and energy sums with
-//    compensated (Kahan) summation; the IAD 3x3 inversion in FP64.
+//    separations from 32-bit fixed point, gradients and pair terms in FP32; kernel values and the
+//    density, grad-h and energy sums in FP64; the IAD 3x3 inversion in FP64.
 #pragma once
 
+#include <algorithm>
+#include <tuple>
 #include <type_traits>
 
 #include "common.hpp"
@@ -20,125 +34,63 @@
 namespace sphx
 {
 
-#ifndef SPHX_PAIR_WAVES_PER_BLOCK
-#define SPHX_PAIR_WAVES_PER_BLOCK 4
-#endif
-constexpr int kPairWaves = SPHX_PAIR_WAVES_PER_BLOCK;
-
 template<class T>
 constexpr bool isMixed = std::is_same_v<T, float>;
 
-// neighbours per batch (NeighborBatch) of the light loops (XMass, grad-h, IAD, AV switches) and of
-// the momentum-energy loops, per form; larger batches hide more latency and cost registers
-#ifndef SPHX_BATCH_LIGHT_F32
-#define SPHX_BATCH_LIGHT_F32 4
-#endif
-#ifndef SPHX_BATCH_LIGHT_F64
-#define SPHX_BATCH_LIGHT_F64 8
-#endif
-#ifndef SPHX_BATCH_MOM_F32
-#define SPHX_BATCH_MOM_F32 2
-#endif
-#ifndef SPHX_BATCH_MOM_F64
-#define SPHX_BATCH_MOM_F64 2
-#endif
+//! waves per block of the light loops (XMass, grad-h, IAD, AV switches) and of momentum-energy. The FP64
+//! momentum records of a group take 90-102 KB of LDS, one block per CU: eight waves give two per SIMD.
+constexpr int kLightWaves = 4;
+template<class T>
+constexpr int kMomWaves = isMixed<T> ? 4 : 8;
 
-// waves per SIMD the register allocator must leave room for (amdgpu_waves_per_eu) in the light
-// loops and in momentum-energy, per form; 1 leaves the choice to the compiler
-#ifndef SPHX_WAVES_LIGHT_F32
-#define SPHX_WAVES_LIGHT_F32 1
-#endif
-#ifndef SPHX_WAVES_LIGHT_F64
-#define SPHX_WAVES_LIGHT_F64 1
-#endif
-#ifndef SPHX_WAVES_MOM_F32
-#define SPHX_WAVES_MOM_F32 1
-#endif
-#ifndef SPHX_WAVES_MOM_F64
-#define SPHX_WAVES_MOM_F64 1
-#endif
-template<class T>
-constexpr int kWavesLight = isMixed<T> ? SPHX_WAVES_LIGHT_F32 : SPHX_WAVES_LIGHT_F64;
-template<class T>
-constexpr int kWavesMom = isMixed<T> ? SPHX_WAVES_MOM_F32 : SPHX_WAVES_MOM_F64;
-
-//! launch attributes of the pair-loop kernels (T: the HydroType template parameter)
-#define SPHX_LIGHT_LOOP(T) __launch_bounds__(kPairWaves * kWave) __attribute__((amdgpu_waves_per_eu(kWavesLight<T>)))
-#define SPHX_MOM_LOOP(T) __launch_bounds__(kPairWaves * kWave) __attribute__((amdgpu_waves_per_eu(kWavesMom<T>)))
-template<class T>
-constexpr int kBatchLight = isMixed<T> ? SPHX_BATCH_LIGHT_F32 : SPHX_BATCH_LIGHT_F64;
-template<class T>
-constexpr int kBatchMom = isMixed<T> ? SPHX_BATCH_MOM_F32 : SPHX_BATCH_MOM_F64;
+//! waves per block of the adjoint loops, which take one group per wave
+constexpr int kVjpWaves = 4;
 
 struct Lists
 {
-    const uint32_t* nbrs;
+    NeighborLists   lists;
     const uint32_t* nc;
-    uint32_t        first, last, ngmax, ngmax4; // [first, last): the searched targets
-    Groups          groups;                     // the call's target groups, one wavefront each
+    uint32_t        first, last, ngmax; // [first, last): the searched targets
+    uint32_t        stage;              // records the launch's LDS holds
+    Groups          groups;             // the call's target groups
 };
 
+//! a lane's target
 struct Lane
 {
-    uint32_t        i;     // target index
-    bool            valid; // lane holds a target
-    unsigned        n;     // neighbours to visit
-    const uint32_t* list;  // this lane's slot 0; slot k at list[laneSlot(k)]
+    uint32_t i;     // target index (a lane without a target: the first searched particle)
+    uint32_t r;     // its place in the searched range
+    unsigned n;     // neighbours to visit (0 without a target)
+    bool     valid; // lane holds a target
 };
 
-//! the wave's group index among the call's target groups
-__device__ __forceinline__ uint32_t waveGroup()
+/*! lane l takes the l-th target of group g; its list is that of the (i - first)-th searched target,
+ * whatever the grouping. Targets outside the searched range [first, last) are not taken. */
+__device__ __forceinline__ Lane groupTarget(const Lists& L, uint32_t g)
 {
-    return __builtin_amdgcn_readfirstlane(xcdBlock(blockIdx.x, gridDim.x) * kPairWaves + threadIdx.x / kWave);
-}
-
-/*! lane l of the wave of group g takes the group's l-th target; its list sits at block (i - first) / 64,
- * lane (i - first) % 64 of the searched range, whatever the grouping. Targets outside the searched
- * range [first, last) are not taken. */
-__device__ __forceinline__ Lane laneTarget(const Lists& L)
-{
-    Lane           t;
-    const unsigned lane = threadIdx.x % kWave;
-    const uint32_t g    = waveGroup();
-    uint32_t       i0 = 0, i1 = 0;
-    bool           oversized;
+    Lane     t;
+    uint32_t i0 = 0, i1 = 0;
+    bool     oversized;
     if (g < L.groups.num) { groupRange(L.groups, g, i0, i1, oversized); }
-    t.i            = i0 + lane;
-    t.valid        = t.i < i1 && t.i >= L.first && t.i < L.last;
-    t.n            = t.valid ? min(L.nc[t.i] - 1, L.ngmax) : 0u;
-    const uint32_t r = t.valid ? t.i - L.first : 0u;
-    t.list         = L.nbrs + listOffset(r / kGroup, L.ngmax4, 0, r % kGroup);
+    t.i     = i0 + threadIdx.x % kWave;
+    t.valid = t.i < i1 && t.i >= L.first && t.i < L.last;
+    t.n     = t.valid ? min(L.nc[t.i] - 1, L.ngmax) : 0u;
+    t.i     = t.valid ? t.i : L.first;
+    t.r     = t.i - L.first;
+    if (L.lists.owner && L.lists.owner[t.r] == NeighborLists::kNoGroup) { t.n = 0; } // the search left it out
     return t;
 }
 
-inline unsigned pairBlocks(const Lists& L) { return ceilDiv(L.groups.num, kPairWaves); }
+//! group of a pair-loop block
+__device__ __forceinline__ uint32_t blockGroup() { return xcdBlock(blockIdx.x, gridDim.x); }
 
-/*! Dynamic LDS per block that caps a pair loop at `waves` waves per SIMD (0: no cap): the CU's 160 KB
- * then holds at most 4 `waves` / kPairWaves blocks. A gather-bound loop can run faster with fewer waves in
- * flight than its register use allows, since more waves evict each other's records from L1. Caps per
- * loop family of the FP32 form, from a sweep of 2-6 at 8M particles: AV switches 3 (2.98 -> 2.75 ms,
- * 4 waves by registers otherwise), XMass 6 (1.27 -> 1.22 ms, 8 otherwise); the others ran as fast or
- * faster uncapped. */
-inline size_t occupancyCap(int waves)
+//! target of a lane of the adjoint loops (one group per wave)
+__device__ __forceinline__ Lane vjpTarget(const Lists& L)
 {
-    // blocks per CU = 4 SIMDs x waves / (waves per block)
-    return waves > 0 ? size_t(160 * 1024) * kPairWaves / (4 * size_t(waves)) : 0;
+    return groupTarget(L, __builtin_amdgcn_readfirstlane(xcdBlock(blockIdx.x, gridDim.x) * kVjpWaves + threadIdx.x / kWave));
 }
-#ifndef SPHX_CAP_XMASS
-#define SPHX_CAP_XMASS 6
-#endif
-#ifndef SPHX_CAP_GRADH
-#define SPHX_CAP_GRADH 0
-#endif
-#ifndef SPHX_CAP_IAD
-#define SPHX_CAP_IAD 0
-#endif
-#ifndef SPHX_CAP_AV
-#define SPHX_CAP_AV 3
-#endif
-#ifndef SPHX_CAP_MOM
-#define SPHX_CAP_MOM 0
-#endif
+
+inline unsigned vjpBlocks(const Lists& L) { return ceilDiv(L.groups.num, kVjpWaves); }
 
 //! lt::lookup (sph/include/sph/table_lookup.hpp:10-26): linear interpolation of a 20000-point
 //! table on [0,2], zero beyond the support. The table is stored per interval (both end values
@@ -197,100 +149,218 @@ __device__ __forceinline__ T fastSqrt(T a)
     else { return sqrt(a); }
 }
 
-//! a / sqrt(d2)
+//! a / sqrt(d2). FP64: the hardware's reciprocal root (2^-24) and two Newton steps, to about an ulp
 template<class T>
 __device__ __forceinline__ T overDistance(T a, T d2)
 {
     if constexpr (isMixed<T>) { return a * __builtin_amdgcn_rsqf(d2); }
-    else { return a / sqrt(d2); }
+    else
+    {
+        double r = __builtin_amdgcn_rsq(d2);
+        r        = r + r * (0.5 - 0.5 * (d2 * r) * r);
+        r        = r + r * (0.5 - 0.5 * (d2 * r) * r);
+        return a * r;
+    }
 }
 
-/*! Batched walk over one lane's neighbour list.
- *
- * A pair loop visits its neighbours U at a time (U = 1, 2 or a multiple of 4): load(k) makes the records of
- * slots k..k+U-1 current (their list entries were requested one batch earlier with aligned vector
- * loads from the lane's quads) and requests the list entries of the following batch.
- * The loop then forms the U separations and issues the U table fetches before it consumes any of
- * them, so one batch costs two memory round trips (records, tables) instead of three per
- * neighbour. Slots beyond the lane's count take the batch's first valid entry and their pair
- * terms are zeroed (live). Slot 0 of a valid target always holds a valid particle index (the
- * search writes the target itself there when it has no neighbours), so every index used for a
- * record load names a particle. Valid targets only. */
-template<int U, class R>
-struct NeighborBatch
+//! LDS of a pair-loop block: the staged records, then the partial sums
+extern __shared__ Chunk16 pairLds[];
+
+//! bytes of a staged neighbour of `bytes` of records: an odd number of 16-byte chunks, so that the records of
+//! different neighbours start in all sixteen 16-byte bank groups
+__host__ __device__ constexpr uint32_t stagedBytes(uint32_t bytes) { return 16u * ((bytes / 16u) | 1u); }
+
+/*! copy the records of the group's table to LDS (all waves), record e at dst + e * stride. Each thread has B
+ * chunks in flight: their table entries, then their records, load together, so a block pays two memory
+ * latencies per B * blockDim chunks rather than per chunk. */
+template<class R>
+__device__ __forceinline__ void stageRecords(const uint32_t* __restrict__ table, uint32_t count, const R* __restrict__ rec,
+                                             char* dst, uint32_t stride)
 {
-    static_assert(U == 1 || U == 2 || U % 4 == 0, "batch of 1, 2 or a multiple of 4 slots");
-
-    const uint32_t* list;
-    const R*        rec;
-    unsigned        n, lastSlot;
-    uint32_t        next[U]; // list entries of the next batch
-    uint32_t        j[U];    // particle indices of the current batch
-    R               r[U];    // records of the current batch
-
-    __device__ __forceinline__ NeighborBatch(const Lane& t, const R* __restrict__ records)
-        : list(t.list), rec(records), n(t.n), lastSlot(t.n ? t.n - 1 : 0)
+    constexpr uint32_t NC = sizeof(R) / 16;
+    constexpr uint32_t B  = NC < 3 ? 4 : 8;
+    static_assert(sizeof(R) % 16 == 0, "records are whole 16-byte chunks");
+    const Chunk16* src   = reinterpret_cast<const Chunk16*>(rec);
+    const uint32_t total = count * NC;
+    for (uint32_t q0 = threadIdx.x; q0 < total; q0 += B * blockDim.x)
     {
-        slots(0, next);
+        uint32_t j[B];
+        Chunk16  v[B];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (uint32_t u = 0; u < B; ++u)
+            j[u] = table[min(q0 + u * blockDim.x, total - 1) / NC];
+#pragma unroll
+        for (uint32_t u = 0; u < B; ++u)
+            v[u] = src[size_t(j[u]) * NC + min(q0 + u * blockDim.x, total - 1) % NC];
+#pragma unroll
+        for (uint32_t u = 0; u < B; ++u)
         {
-            // an opaque definition: otherwise the compiler merges this load with the look-ahead
-            // load of the loop into one load at the top of each batch, undoing the look-ahead
-            asm volatile("" : "+v"(next[u]));
+            // past the end: the last chunk again, the same value at the same place
+            const uint32_t q = min(q0 + u * blockDim.x, total - 1);
+            *reinterpret_cast<Chunk16*>(dst + (q / NC) * stride + 16 * (q % NC)) = v[u];
         }
     }
+}
 
-    //! list entries of slots k..k+U-1 (clamped as described above)
-    __device__ __forceinline__ void slots(unsigned k, uint32_t out[U]) const
-    {
-        const unsigned  kq = min(k, lastSlot) & ~unsigned(U - 1);
-        const uint32_t* p  = list + laneSlot(kq);
-        uint32_t        v[U];
-        if constexpr (U % 4 == 0)
-        {
+template<class R>
+__device__ __forceinline__ R stagedRecord(const char* src)
+{
+    constexpr uint32_t NC = sizeof(R) / 16;
+    Chunk16            c[NC];
 #pragma unroll
-            for (int c = 0; c < U; c += 4)
+    for (uint32_t k = 0; k < NC; ++k)
+        c[k] = reinterpret_cast<const Chunk16*>(src)[k];
+    R r;
+    __builtin_memcpy(&r, c, sizeof(R));
+    return r;
+}
+
+/*! Walk over the neighbours of a block's targets, wave w taking the quads w, w + W, .. of each list:
+ * pair(live, records...) for every slot, with the neighbour's record of each of Rs. Slots past a lane's count
+ * (the rest of its last quad) hold the list's last neighbour again, with live = false. U of a quad's
+ * records are in flight at a time, and the next quad of the list. */
+template<int W, int U, class... Rs>
+struct PairWalk
+{
+    static_assert(U == 1 || U == 2 || U == 4, "whole parts of a quad");
+    static constexpr uint32_t kStride = stagedBytes(uint32_t((sizeof(Rs) + ...)));
+
+    const Lists& L;
+    const Lane&  t;
+    bool         staged;
+
+    //! stages the group's records, unless they do not fit or are not one group's
+    __device__ __forceinline__ PairWalk(const Lists& lists, const Lane& lane, const Rs*... rec)
+        : L(lists)
+        , t(lane)
+        , staged(false)
+    {
+        if (L.lists.tableCount != nullptr)
+        {
+            const bool     some  = t.n > 0;
+            const uint32_t b     = some ? L.lists.group(t.r) : 0u;
+            const uint64_t mask  = ballot(some);
+            const uint32_t b0    = mask ? __builtin_amdgcn_readlane(b, __builtin_ctzll(mask)) : 0u;
+            const uint32_t count = mask ? L.lists.tableCount[b0] : 0u;
+            if (ballot(some && b != b0) == 0 && count <= L.stage)
             {
-                const uint4 q = *reinterpret_cast<const uint4*>(list + laneSlot(kq + c));
-                v[c] = q.x, v[c + 1] = q.y, v[c + 2] = q.z, v[c + 3] = q.w;
+                staged             = true;
+                const uint32_t* tb = L.lists.table + size_t(b0) * kTableCap;
+                uint32_t        at = 0;
+                ((stageRecords(tb, count, rec, ldsBytes() + at, kStride), at += uint32_t(sizeof(Rs))), ...);
             }
         }
-        else if constexpr (U == 2)
-        {
-            const uint2 q = *reinterpret_cast<const uint2*>(p);
-            v[0] = q.x, v[1] = q.y;
-        }
-        else { v[0] = p[0]; }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            out[u] = kq + u <= lastSlot ? v[u] : v[0];
+        __syncthreads();
     }
 
-    __device__ __forceinline__ void load(unsigned k)
+    __device__ __forceinline__ static char* ldsBytes() { return reinterpret_cast<char*>(pairLds); }
+
+    template<class F>
+    __device__ __forceinline__ void operator()(F&& pair, const Rs*... rec) const
     {
-#pragma unroll
-        for (int u = 0; u < U; ++u)
+        const uint32_t g = t.r / kGroup, lane = t.r % kGroup, k0 = 4 * (threadIdx.x / kWave);
+        if (staged)
         {
-            j[u] = next[u];
-            r[u] = rec[j[u]];
+            static_assert(W % 2 == 0, "a wave's quads lie at one place of their octets");
+            constexpr size_t step = size_t(4 * W) * kGroup; // list words from a quad to the wave's next
+            const uint16_t*  list = static_cast<const uint16_t*>(L.lists.nbrs) +
+                                   localOffset(g, paddedNgmax8(L.ngmax), k0, lane);
+            uint64_t next = k0 < t.n ? *reinterpret_cast<const uint64_t*>(list) : 0;
+            for (uint32_t k = k0; k < t.n; k += 4 * W)
+            {
+                uint64_t q = next;
+                list += k + 4 * W < t.n ? step : 0;
+                next = *reinterpret_cast<const uint64_t*>(list);
+                asm volatile("" : "+v"(next)); // the load stays here, ahead of its use
+#pragma unroll 1
+                for (int u0 = 0; u0 < 4; u0 += U)
+                {
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                    {
+                        const char* from = ldsBytes() + (uint32_t(q >> (16 * u)) & 0xffffu) * kStride;
+                        uint32_t    at   = 0;
+                        auto        load = [&](auto* p)
+                        {
+                            using R    = std::remove_const_t<std::remove_pointer_t<decltype(p)>>;
+                            const R rj = stagedRecord<R>(from + at);
+                            at += uint32_t(sizeof(R));
+                            return rj;
+                        };
+                        const std::tuple<Rs...> r{load(rec)...};
+                        std::apply([&](const Rs&... rj) { pair(k + u0 + u < t.n, rj...); }, r);
+                    }
+                    q >>= 16 * (U % 4);
+                }
+            }
         }
-        slots(k + U, next);
-    }
-
-    //! whether member u of the batch starting at slot k is a real neighbour
-    __device__ __forceinline__ bool in(unsigned k, int u) const { return k + u < n; }
-
-    //! the argument z = (r/h)^2 of member u's kernel weight, moved to the edge of the support for a
-    //! clamped slot. Every pair term of the loops is proportional to a kernel weight, so a clamped slot
-    //! contributes exactly zero without a branch (a branch would let the compiler sink that member's
-    //! loads behind it).
-    template<class T>
-    __device__ __forceinline__ T live2(unsigned k, int u, T z) const
-    {
-        return in(k, u) ? z : T(4);
+        else
+        {
+            for (uint32_t k = k0; k < t.n; k += 4 * W)
+            {
+#pragma unroll 1
+                for (uint32_t u = 0; u < 4; ++u)
+                {
+                    const uint32_t j = L.lists.entry(t.r, k + u);
+                    pair(k + u < t.n, rec[j]...);
+                }
+            }
+        }
     }
 };
+
+/*! Add the waves' partial sums v[0..N) of each lane's target in wave order; the first M are combined by maximum
+ * instead. True on the first wave, which then holds the totals. */
+template<int W, int N, int M = 0>
+__device__ __forceinline__ bool waveSums(double (&v)[N])
+{
+    double*        part = reinterpret_cast<double*>(pairLds);
+    const unsigned lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+    __syncthreads(); // every wave has read its records
+    if (w > 0)
+    {
+#pragma unroll
+        for (int q = 0; q < N; ++q)
+            part[((w - 1) * N + q) * kWave + lane] = v[q];
+    }
+    __syncthreads();
+    if (w > 0) { return false; }
+#pragma unroll
+    for (int q = 0; q < N; ++q)
+    {
+#pragma unroll
+        for (int p = 0; p < W - 1; ++p)
+        {
+            const double x = part[(p * N + q) * kWave + lane];
+            if (q < M) { v[q] = x > v[q] ? x : v[q]; }
+            else { v[q] += x; }
+        }
+    }
+    return true;
+}
+
+/*! host: the records a launch stages and its dynamic LDS, for records of `recBytes` and N partial sums. The stage
+ * holds the tables of 99.5% of the blocks, or the 160 KB of a CU if they are larger; the other blocks read
+ * from global memory. */
+struct PairLaunch
+{
+    uint32_t stage;
+    size_t   lds;
+};
+inline PairLaunch pairLaunch(const sphx_workspace* ws, size_t recBytes, int waves, int sums)
+{
+    const size_t part = size_t(waves - 1) * sums * kWave * sizeof(double);
+    if (!ws->nbLocal) { return {0, part}; }
+    uint64_t blocks = 0, seen = 0;
+    for (uint32_t b = 0; b < kTableBins; ++b)
+        blocks += ws->nbTableHist[b];
+    uint32_t bins = 0;
+    while (bins < kTableBins && seen * 1000 < blocks * 995)
+        seen += ws->nbTableHist[bins++];
+    const uint32_t each  = stagedBytes(uint32_t(recBytes));
+    const uint32_t stage = std::min(bins * kTableBin, uint32_t(160 * 1024) / each);
+    return {stage, std::max(part, size_t(stage) * each)};
+}
 
 /*! The SPH kernel W(v) = sinc(pi v / 2)^n and dW/dv on [0, 2), zero from v = 2 on.
  *
@@ -303,8 +373,9 @@ struct NeighborBatch
  * integer n (the reference's sinc indices); for other n the FP32 form takes FP32 log2 / exp2 and the
  * FP64 form its tables.
  *
- * FP32 form: P and d sinc/dz of degree 6, relative error 6e-11, in FP64 arithmetic (which on this GPU
- * issues at the FP32 rate, since FP32 ops are not packed here), so W is exact to its final rounding.
+ * FP32 form: sinc and z d sinc/dz as polynomials of y = 1 - z/4 (degree 6 and 7, errors below 6e-11), in
+ * FP64 arithmetic (which on this GPU issues at the FP32 rate, since FP32 ops are not packed here), so W is exact
+ * to its final rounding. y is one fused multiply-add of the squared distance.
  *
  * FP64 form: the reference interpolates W linearly in a 20000-point table, up to 6e-9 off the function
  * for n = 6, and the FP64 results are held to that interpolant. With t = the fraction of v / dx,
@@ -318,15 +389,15 @@ constexpr double kHalfPiSq = 2.4674011002723396547; // (pi/2)^2
 
 /*! The loops are compiled per variant, chosen on the host for a launch (launchVariant):
  * kCommon: the default sinc index 6, its powers unrolled; in the FP32 form the wrapping fixed-point
- * separation as well. kWide (FP32 form): the exact separations of boxes a few smoothing lengths wide, any
- * index. kAnyIndex: any other sinc index. */
+ * separation as well, in units of the fixed point (DevBox::raw). kWide (FP32 form): the exact separations of
+ * boxes a few smoothing lengths wide, any index. kAnyIndex: any other index, or (FP32 form) periodic
+ * dimensions of different lengths. */
 enum Variant
 {
     kCommon,
     kWide,
     kAnyIndex
 };
-constexpr int kDefaultIndex = 6;
 
 //! x^k for a small integer k >= 0 (wave-uniform loop)
 __device__ __forceinline__ double sincPower(double x, int k)
@@ -340,17 +411,30 @@ __device__ __forceinline__ double sincPower(double x, int k)
     return r;
 }
 
-//! sinc(pi v / 2) at z = v^2 in [0, 4], relative error 6e-11 (FP32 form)
-__device__ __forceinline__ double sincOfZ6(double z)
+//! sinc(pi v / 2) at y = 1 - v^2 / 4 in [0, 1], relative error 6e-11 (FP32 form)
+__device__ __forceinline__ double sincOfY(double y)
 {
-    double p = 1.4453064921222513e-09;
-    p        = p * z - 1.3731223424662021e-07;
-    p        = p * z + 8.607989820798515e-06;
-    p        = p * z - 0.00037411264408295246;
-    p        = p * z + 0.010425519738884937;
-    p        = p * z - 0.161233516047257;
-    p        = p * z + 0.9999999999728735;
-    return p - 0.25 * z * p;
+    double p = 5.919975391732741e-06;
+    p        = p * y + 0.00010508787551814265;
+    p        = p * y + 0.0015894063856577154;
+    p        = p * y + 0.016416305415662014;
+    p        = p * y + 0.10688328287516924;
+    p        = p * y + 0.3749999974191315;
+    p        = p * y + 0.5000000000263431;
+    return p * y;
+}
+
+//! z d sinc(pi v / 2) / dz = v/2 d sinc/dv at y = 1 - v^2 / 4, absolute error 6e-11
+__device__ __forceinline__ double sincSlopeOfY(double y)
+{
+    double q = 4.132672691073703e-05;
+    q        = q * y + 0.0005894009530895289;
+    q        = q * y + 0.007316207227363674;
+    q        = q * y + 0.05771828331287214;
+    q        = q * y + 0.25498464086819245;
+    q        = q * y + 0.42935013419273005;
+    q        = q * y - 0.24999999328291864;
+    return q * y - 0.5000000000524906;
 }
 
 //! d sinc(pi v / 2) / dz, absolute error 6e-11
@@ -434,6 +518,26 @@ __device__ __forceinline__ InterpolationPoint interpolationPoint(double z, doubl
     return i;
 }
 
+//! length of a separation's unit (DevBox::unit)
+template<class T>
+__device__ __forceinline__ T unitOf(const DevBox& b)
+{
+    return isMixed<T> ? T(b.unit) : T(1);
+}
+
+//! what the records and targets hold of 1/h for the kernel argument of a squared distance in units of the
+//! separations: (unit / h)^2, times -1/4 in the FP32 form
+template<class T>
+__device__ __forceinline__ T kernelScale(T unitOverH)
+{
+    return isMixed<T> ? T(-0.25) * unitOverH * unitOverH : unitOverH * unitOverH;
+}
+template<class T>
+__device__ __forceinline__ T kernelScale(const DevBox& b, T hInv)
+{
+    return kernelScale(hInv * unitOf<T>(b));
+}
+
 template<class T>
 struct SincKernel;
 
@@ -444,7 +548,16 @@ struct SincKernel<double>
     const TabPair<double>* wTab;
     const TabQuad<double>* wqTab;
 
-    //! W at z = v^2
+    //! the loops' kernel argument of a pair at squared distance d2, kernelScale(1/h) = scale: z = v^2
+    __device__ __forceinline__ static double arg(double d2, double scale) { return d2 * scale; }
+    //! the argument held to [0, 4], and to the edge of the support for a slot that is not live: every pair term
+    //! is proportional to a kernel value, so such a slot contributes exactly zero without a branch
+    __device__ __forceinline__ static double clamp(double z, bool live)
+    {
+        return fmin(fmax(z, live ? 0.0 : 4.0), 4.0);
+    }
+
+    //! W at z in [0, 4]
     template<int V>
     __device__ __forceinline__ double w(double z) const
     {
@@ -452,7 +565,6 @@ struct SincKernel<double>
         else
         {
             constexpr double n         = kDefaultIndex;
-            z                          = z < 4.0 ? z : 4.0;
             const double             s = sincOfZ9(z);
             const InterpolationPoint i = interpolationPoint(z, s);
             const double             q = i.s1 * i.s1; // s1^(n-2) = q^2
@@ -463,7 +575,7 @@ struct SincKernel<double>
         }
     }
 
-    //! W and v dW/dv at z = v^2
+    //! W and v dW/dv at z in [0, 4]
     template<int V>
     __device__ __forceinline__ void wAndVdw(double z, double& w, double& vdw) const
     {
@@ -477,7 +589,6 @@ struct SincKernel<double>
         else
         {
             constexpr double n          = kDefaultIndex;
-            z                           = z < 4.0 ? z : 4.0;
             const double             s  = sincOfZ9(z);
             const InterpolationPoint i  = interpolationPoint(z, s);
             const double             q  = i.s1 * i.s1, p3 = q * i.s1, p2 = q * q; // s1^(n-3), s1^(n-2)
@@ -532,24 +643,35 @@ struct SincKernel<float>
             return s > 0.0 ? double(__builtin_amdgcn_exp2f((n - 1.0f) * __builtin_amdgcn_logf(float(s)))) : 0.0;
         }
     }
-    template<int V>
-    __device__ __forceinline__ double w(float zf) const
+    //! the loops' kernel argument of a pair at squared distance d2, kernelScale(1/h) = scale: y = 1 - v^2 / 4
+    __device__ __forceinline__ static float arg(float d2, float scale) { return d2 * scale + 1.0f; }
+    //! the argument held to [0, 1], and to the edge of the support for a slot that is not live: every pair term
+    //! is proportional to a kernel value, so such a slot contributes exactly zero without a branch
+    __device__ __forceinline__ static float clamp(float y, bool live)
     {
-        const double s = sincOfZ6(double(fminf(zf, 4.0f)));
+        return __builtin_amdgcn_fmed3f(y, 0.0f, live ? 1.0f : 0.0f);
+    }
+
+    //! W at y in [0, 1]
+    template<int V>
+    __device__ __forceinline__ double w(float y) const
+    {
+        const double s = sincOfY(double(y));
         return power<V>(s) * s;
     }
+    //! W and v dW/dv
     template<int V>
-    __device__ __forceinline__ void wAndVdw(float zf, double& w, double& vdw) const
+    __device__ __forceinline__ void wAndVdw(float yf, double& w, double& vdw) const
     {
-        const double z = double(fminf(zf, 4.0f));
-        const double s = sincOfZ6(z), p = power<V>(s);
+        const double y = double(yf);
+        const double s = sincOfY(y), p = power<V>(s);
         w              = p * s;
-        vdw            = (2.0 * index<V>()) * z * p * sincSlope6(z);
+        vdw            = (2.0 * index<V>()) * p * sincSlopeOfY(y);
     }
     __device__ __forceinline__ void wAndDw(float vf, float& w, float& dw) const
     {
         const double v = double(fminf(vf, 2.0f)), z = v * v;
-        const double s = sincOfZ6(z), p = power<kAnyIndex>(s);
+        const double s = sincOfY(1.0 - 0.25 * z), p = power<kAnyIndex>(s);
         w              = float(p * s);
         dw             = float((2.0 * double(n)) * v * p * sincSlope6(z));
     }
@@ -644,7 +766,8 @@ __device__ __forceinline__ float wideFixedSeparation(const DevBox& b, int q, dou
     return float(d) * b.fixStep[q];
 }
 
-template<bool Fold, class T, class Ri, class Rj>
+/*! separation x_i - x_j of a pair (DevBox::unit is its unit) */
+template<bool Fold, int V, class T, class Ri, class Rj>
 __device__ __forceinline__ Sep<T> pairSeparation(const DevBox& b, double r2h, const Ri& ri, const Rj& rj)
 {
     Sep<T> s;
@@ -653,6 +776,12 @@ __device__ __forceinline__ Sep<T> pairSeparation(const DevBox& b, double r2h, co
         s.x = wideFixedSeparation(b, 0, r2h, ri.x, rj.x);
         s.y = wideFixedSeparation(b, 1, r2h, ri.y, rj.y);
         s.z = wideFixedSeparation(b, 2, r2h, ri.z, rj.z);
+    }
+    else if constexpr (isMixed<T> && V == kCommon)
+    {
+        s.x = float(int32_t(ri.x - rj.x));
+        s.y = float(int32_t(ri.y - rj.y));
+        s.z = float(int32_t(ri.z - rj.z));
     }
     else if constexpr (isMixed<T>)
     {
@@ -671,19 +800,20 @@ __device__ __forceinline__ Sep<T> pairSeparation(const DevBox& b, double r2h, co
  * exact 64-bit difference. The variant is a kernel template argument, chosen on the host
  * (launchVariant), so that the common loop carries none of the registers of the others. */
 template<class T, int V, class R>
-__device__ __forceinline__ bool recordNeedsFold(const DevBox& b, const R& ri, double r2h)
+__device__ __forceinline__ bool recordNeedsFold(const DevBox& b, const Lane& t, const R& ri, double r2h)
 {
     if constexpr (isMixed<T>) { return V == kWide; }
-    else { return waveNeedsFold(b, ri.x, ri.y, ri.z, r2h); }
+    else { return waveNeedsFold(b, ri.x, ri.y, ri.z, t.valid ? r2h : -INFINITY); }
 }
 
-//! host: launch(std::integral_constant<int, V>) with the loop variant V of this search and sinc index
+//! host: launch(std::integral_constant<int, V>) with the loop variant V of this search, box and sinc index
 template<class T, class F>
-inline void launchVariant(const sphx_workspace* ws, F&& launch)
+inline void launchVariant(const sphx_workspace* ws, const DevBox& box, F&& launch)
 {
-    if (isMixed<T> && ws->nbWide) { launch(std::integral_constant<int, kWide>{}); }
-    else if (ws->sincIndex != double(kDefaultIndex)) { launch(std::integral_constant<int, kAnyIndex>{}); }
-    else { launch(std::integral_constant<int, kCommon>{}); }
+    const bool common = isMixed<T> ? box.raw : ws->sincIndex == double(kDefaultIndex);
+    if (common) { launch(std::integral_constant<int, kCommon>{}); }
+    else if (isMixed<T> && ws->nbWide) { launch(std::integral_constant<int, kWide>{}); }
+    else { launch(std::integral_constant<int, kAnyIndex>{}); }
 }
 
 //! run `loop` with the fold compiled in or out, chosen once per wave
@@ -752,18 +882,14 @@ __device__ __forceinline__ double courantDt(T maxvs, T h, T c, float Kcour)
     return double(T(Kcour * h / v));
 }
 
-//! artificial_viscosity (kernels.hpp:71-84), beta = 2
+//! artificial_viscosity (kernels.hpp:71-84), beta = 2: -vsig w for approaching particles, else 0, without a
+//! branch (a NaN of coincident particles gives 0, as the comparison would)
 template<class T>
-__device__ __forceinline__ T artificialViscosity(T alpha_i, T alpha_j, T c_i, T c_j, T w_ij)
+__device__ __forceinline__ T artificialViscosity(T alpha_i, T alpha_j, T c_sum, T w_ij)
 {
     constexpr T beta = 2.0;
-    T           visc = 0.0;
-    if (w_ij < T(0))
-    {
-        T vsig = (alpha_i + alpha_j) * T(0.25) * (c_i + c_j) - beta * w_ij;
-        visc   = -vsig * w_ij;
-    }
-    return visc;
+    const T     w    = w_ij < T(0) ? w_ij : T(0);
+    return (beta * w - (alpha_i + alpha_j) * T(0.25) * c_sum) * w;
 }
 
 //! arguments shared by all pair kernels
@@ -789,8 +915,7 @@ inline PairArgs makePairArgs(sphx_workspace* ws, const DevBox& box, const sphx_f
     SPHX_REQUIRE(f->x && f->y && f->z && f->nc, SPHX_ERR_ARG, "x, y, z and nc are required");
     PairArgs c;
     c.x = f->x, c.y = f->y, c.z = f->z, c.box = box, c.K = p->K;
-    c.L            = Lists{ws->nbrs.get(), f->nc, ws->nbFirst, ws->nbLast, p->ngmax, paddedNgmax(p->ngmax),
-                               groupsFor(ws, first, last)};
+    c.L            = Lists{neighborLists(ws), f->nc, ws->nbFirst, ws->nbLast, p->ngmax, 0, groupsFor(ws, first, last)};
     c.numParticles = uint32_t(ws->tree.numParticles);
     return c;
 }
@@ -814,16 +939,15 @@ inline SincKernel<T> sincKernel(sphx_workspace* ws)
     return k;
 }
 
-/*! wave minimum then one atomic per wave; with per-group steps (block time steps), also
+/*! block minimum (its first wave's lanes) then one atomic per block; with per-group steps (block time steps), also
  * groupDt[g] = min(groupDt[g], the group's minimum) as a float (hydro_ve/momentum_energy_gpu.cu:96-104) */
-template<class T>
 __device__ __forceinline__ void reduceMinDt(unsigned long long* dst, double dt, const Groups& G)
 {
     double m = waveMin(dt);
-    if (threadIdx.x % kWave == 0)
+    if (threadIdx.x == 0)
     {
         atomicMinPositive(dst, m);
-        const uint32_t g = waveGroup();
+        const uint32_t g = blockGroup();
         if (G.dt != nullptr && g < G.num) { G.dt[g] = fminf(G.dt[g], float(m)); }
     }
 }

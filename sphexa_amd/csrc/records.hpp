@@ -4,8 +4,8 @@
 // Read from the SoA Dataset arrays, every field is a separate 64-lane gather touching tens of
 // cache lines; the loops were bound by the vector-memory address path, not by ALU or HBM.
 // Before each pair loop a coalesced pack kernel therefore writes exactly the fields that loop
-// needs for j into one 16-byte aligned record per particle (workspace memory, SFC order), so a
-// neighbour costs a few 16-byte loads from one or two cache lines. Positions are FP64 in the plain
+// needs for j into one 16-byte aligned record per particle (workspace memory, SFC order), which the
+// loop's blocks copy to LDS chunk by chunk (stageRecords). Positions are FP64 in the plain
 // form and 32-bit fixed point in the FP32 form (Coord, pairs.hpp). Derived per-particle
 // quantities (1/h, m/rho, xm/kx, kx m/xm) are formed in the pack with the same expression the
 // pair loop would evaluate, so results are unchanged.
@@ -58,23 +58,32 @@ struct alignas(16) RecAv
     T      vol, c, divv, vx, vy, vz;
 };
 
-//! std momentum-energy: vol = m/rho, pro = p/rho
+//! std momentum-energy: scale = kernelScale(1/h), vol = m/(rho h^3), pro = p/rho, alpha the per-particle AV
+//! coefficient or 1, and the IAD matrix per unit of the separations
 template<class T>
 struct alignas(16) RecMomStd
 {
     Coord<T> x, y, z;
-    T      vx, vy, vz, hInv, m, vol, pro, c, c11, c12, c13, c22, c23, c33;
+    T      vx, vy, vz, scale, m, vol, pro, c, alpha, c11, c12, c13, c22, c23, c33;
 };
 
-//! VE momentum-energy: rho = kx m/xm, vol = m/rho (the AV-cleaning gradients stay in SoA)
+//! AV cleaning: the velocity gradients of VE momentum-energy, per unit of the separations
+template<class T>
+struct alignas(16) RecGradV
+{
+    T g[6];
+};
+
+//! VE momentum-energy: scale = kernelScale(1/h), rho = kx m/xm, vol = m/(rho h^3), prho = p/(kx m^2 gradh h^3), and
+//! the IAD matrix per unit of the separations
 template<class T>
 struct alignas(16) RecMomVe
 {
     Coord<T> x, y, z;
-    T      vx, vy, vz, hInv, m, c, rho, vol, xm, alpha, prho, c11, c12, c13, c22, c23, c33;
+    T      vx, vy, vz, scale, m, c, rho, vol, xm, alpha, prho, c11, c12, c13, c22, c23, c33;
 };
 
-// 16-byte loads per neighbour, FP32 form: 1 (mass, volume), 2 (grad-h, VE IAD), 3 (AV), 5 (momentum)
+// 16-byte chunks per record, FP32 form: 1 (mass, volume), 2 (grad-h, VE IAD), 3 (AV), 5 (momentum)
 static_assert(sizeof(RecMass<float>) == 16 && sizeof(RecVol<float>) == 16, "record layout");
 static_assert(sizeof(RecGradh<float>) == 32 && sizeof(RecIadVe<float>) == 32 && sizeof(RecAv<float>) == 48,
               "record layout");

@@ -1,0 +1,107 @@
+"""Neighbour lists as table positions and the pair loops' record sources: staged tables, tables of other groups
+than the call's, tables that do not fit, and the FP32 form's fixed point in boxes of several shapes.
+
+Lists and counts are compared entry by entry; results of one search over different target ranges and
+groupings bit for bit; fields against the oracle at the repository's bars (FP64 1e-10 of the field's
+largest magnitude; mixed density 1e-5, accelerations 1e-4)."""
+import numpy as np
+import pytest
+
+from sphexa_amd import abi, ic
+from sphexa_amd.particles import STD_FIELDS, VE_FIELDS, ParticleSet, ideal_gas_cv, std_step, ve_step
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ws():
+    from sphexa_amd.lib import Workspace
+
+    return Workspace(0)
+
+
+def std_loops(ws, ps, box, params, ranges):
+    f = ps.fields()
+    for a, b in ranges:
+        ws.pair("sphx_density_std", box, f, params, a, b)
+    ws.eos("sphx_eos_std", f, params, 0, ps.n)
+    for a, b in ranges:
+        ws.pair("sphx_iad_std", box, f, params, a, b)
+    for a, b in ranges:
+        ws.momentum_energy_std(box, f, params, a, b)
+    return {k: ps.host(k).copy() for k in ("rho", "c11", "c23", "ax", "ay", "az", "du")}
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("n", [63, 64, 65, 129, 4096, 5000])
+def test_ranges_of_one_search_bitwise(ws, mixed, n):
+    """blocks whose targets' lists lie in two tables (ranges off the search's groups) give the same bits"""
+    arr, box = ic.evrard_sphere(n, seed=n)
+    arr["vx"] = 0.1 * np.sin(6.0 * arr["x"])
+    box = abi.Box.make(box["lo"], box["hi"], abi.OPEN)
+    params = abi.Params.defaults(ws.K, hydro_type=abi.SPHX_F32 if mixed else abi.SPHX_F64)
+    ps = ParticleSet.from_host(arr, STD_FIELDS, mixed=mixed)
+    std_step(ws, ps, box, params)
+    whole = std_loops(ws, ps, box, params, [(0, n)])
+    cut = std_loops(ws, ps, box, params, [(0, n // 3), (n // 3, n - 7), (n - 7, n)])
+    for k, v in whole.items():
+        np.testing.assert_array_equal(cut[k], v, err_msg=k)
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_table_that_does_not_fit(ws, mixed):
+    """supports of 4000 neighbours, far over ngmax: the group's table overflows and the search stores global
+    lists; counts, the kept entries and the density are the oracle's"""
+    import torch
+
+    from oracle import oracle as O
+    from oracle import pipeline
+
+    arr, spec = ic.turbulence_box(20, seed=3)
+    arr["h"] = arr["h"] * 3.5
+    box = abi.Box.make(spec["lo"], spec["hi"], abi.PERIODIC)
+    params = abi.Params.defaults(ws.K, hydro_type=abi.SPHX_F32 if mixed else abi.SPHX_F64)
+    hydro = np.float32 if mixed else np.float64
+    o = pipeline.run(O.load("orc"), arr, box, abi.Params.defaults(ws.K), form="std", iterate_h=False)
+    ps = ParticleSet.from_host(arr, STD_FIELDS, mixed=mixed)
+    ws.domain_sync(box, ps.sync_fields(), params, ps.n)
+    f = ps.fields()
+    ws.find_neighbors(box, f, params, 0, ps.n, False)
+    lists = torch.zeros(ps.n, params.ngmax, dtype=torch.int32, device="cuda")
+    ws.copy_neighbors(lists, 0, ps.n)
+    assert ps.host("nc").min() > 2049
+    if not mixed:  # float h moves pairs at the very edge of the support
+        np.testing.assert_array_equal(ps.host("nc"), o["a"]["nc"])
+        np.testing.assert_array_equal(lists.cpu().numpy().view(np.uint32), np.asarray(o["nbrs"]))
+        ws.pair("sphx_density_std", box, f, params, 0, ps.n)
+        np.testing.assert_allclose(ps.host("rho"), o["a"]["rho"].astype(hydro), rtol=1e-10)
+    else:
+        ws.pair("sphx_density_std", box, f, params, 0, ps.n)
+        assert np.isfinite(ps.host("rho")).all()
+
+
+@pytest.mark.parametrize("lengths,boundary", [((1.0, 1.0, 0.5), abi.PERIODIC),
+                                              ((1.0, 1.0, 0.5), [abi.PERIODIC, abi.PERIODIC, abi.OPEN]),
+                                              ((1.0, 0.7, 0.5), abi.OPEN)])
+def test_mixed_box_shapes(ws, lengths, boundary):
+    """the fixed point with one unit for all dimensions (one periodic length, or none) and without (several)"""
+    from oracle import oracle as O
+    from oracle import pipeline
+
+    side = [int(24 * v) for v in lengths]
+    rng = np.random.default_rng(8)
+    g = np.meshgrid(*[(np.arange(s) + 0.5) / 24.0 for s in side], indexing="ij")
+    x, y, z = (c.ravel() + rng.uniform(-0.1, 0.1, c.size) / 24.0 for c in g)
+    n = x.size
+    arr = dict(x=x, y=y, z=z, h=np.full(n, 1.44 / 24.0), m=np.full(n, 1.0 / n), vx=0.1 * np.sin(6 * x),
+               vy=0.1 * np.cos(5 * y), vz=0.05 * z, alpha=np.full(n, 0.3),
+               temp=np.full(n, 1.0 / ideal_gas_cv(10.0, 5.0 / 3.0)))
+    box = abi.Box.make([0.0] * 3, list(lengths), boundary)
+    o = pipeline.run(O.load("orc"), arr, box, abi.Params.defaults(ws.K, minDt=1e-4), form="ve")
+    ps = ParticleSet.from_host(arr, VE_FIELDS, mixed=True)
+    ve_step(ws, ps, box, abi.Params.defaults(ws.K, hydro_type=abi.SPHX_F32, minDt=1e-4))
+    np.testing.assert_array_equal(ps.host("nc"), o["a"]["nc"])
+    for k, bar in (("xm", 1e-5), ("kx", 1e-5), ("ax", 1e-4), ("ay", 1e-4), ("az", 1e-4), ("du", 1e-4)):
+        ref = o["a"][k]
+        err = np.max(np.abs(ps.host(k) - ref)) / np.max(np.abs(ref))
+        assert err <= bar, (k, err)
