@@ -12,15 +12,18 @@
 // image the group sees, in LDS; the wave reads each back as a broadcast, one ballot per leaf).
 // The particles of the surviving leaves within reach of the group box are compacted into full
 // tiles of 64 in a double-buffered LDS area (coalesced loads of the next window overlap the
-// sweep), and the wave tests each tile reading every candidate with one broadcast LDS access,
-// every lane against its own target with the reference predicate
+// sweep). A tile's 64 x 64 tests are one FP32 matrix product on the matrix cores whose signs are the hits
+// (tileMask); where any of them is too close to zero to be certain, and in boxes too small for one periodic
+// image per leaf, the tile is tested with the reference predicate
 // (domain/include/cstone/findneighbors.hpp:33-60,93,116-140): d2 = dx*dx + dy*dy + dz*dz with
 // dx = x_j - x_i, periodic images folded by one box length, unfused FP64 arithmetic, keep if
 // d2 < Th(4)*h_i*h_i and j != i. The lists, counts and, past ngmax, the kept first ngmax hits
-// are therefore bit-identical to the CPU search; they are stored in the group layout of
-// common.hpp (listOffset): a lane
-// shifts its entries through a register quad and stores 16 bytes at a time, and the pair loops read
-// four slots of all 64 lanes with one coalesced load.
+// are therefore bit-identical to the CPU search; a lane shifts its entries through four registers and
+// stores 16 bytes at a time (ListWriter), in the layouts of common.hpp.
+//
+// Measured: 8M turbulence 5.2 -> 4.8 ms, 4M Evrard sphere 3.7 -> 3.2 ms against exact tests of every tile
+// (vector instructions per group 21.2k -> 16.0k). Bound by latency at four waves per SIMD (16 waves fill a CU's LDS and
+// 128 registers a wave), the vector ALU busy two thirds of the time.
 #include <cstring>
 
 #include "pairs.hpp"
@@ -79,6 +82,10 @@ struct SearchArgs
     int                  toRho;
 };
 
+/* words from one component of the matrix operand to the next: the 16 rows and 4 components that the lanes
+ * read together (tileMask) lie in 64 different banks */
+constexpr int kMatStride = 68;
+
 //! per-wave LDS: traversal stack, candidate leaves, the kept leaves' particle ranges, and the
 //! double-buffered candidate tile (with the candidates' masses for the fused XMass only)
 template<bool Mass, bool Local>
@@ -89,11 +96,12 @@ struct WaveLds
     int32_t  bufRank[kBufCap];      // ... and their visiting-order ranks
     uint32_t leafLo[kLeafCap];      // kept leaves: first particle
     uint32_t leafPre[kLeafCap + 1]; // kept leaves: exclusive prefix of particle counts, then the total
-    int32_t  leafImg[kLeafCap];     // kept leaves: periodic image code (imageShift)
+    uint8_t  leafImg[kLeafCap];     // kept leaves: periodic image code (imageShift)
     double   tx[2][kWave], ty[2][kWave], tz[2][kWave];
     uint32_t tj[2][kWave]; // particle index of each staged candidate
     double   tm[2][Mass ? kWave : 1]; // its mass (fused XMass only)
-    uint32_t self[Local ? kWave : 1]; // local lists: the target's own place in the tile
+    uint8_t  self[Local ? kWave : 4]; // local lists: the target's own place in the tile
+    float    mx[Mass ? 1 : 4 * kMatStride]; // the tile's candidates as matrix operand (tileMask)
 };
 
 // sixteen waves of the search share a CU's 160 KB of LDS (the fused search + XMass, with its masses,
@@ -216,103 +224,193 @@ __device__ __forceinline__ uint32_t waveOr(uint32_t v)
 
 enum class Fold
 {
-    none,    // all pairs of the tile use the direct image
-    shifted, // one periodic image (shift multiple of the box length) serves all pairs
+    shifted, // one periodic image (shift a multiple of the box length, or 0) serves all pairs of the tile
     perPair  // box too small for a single image: rint fold per pair, as the reference
 };
 
-//! Test the `n` staged candidates against the lane's target. Hits are recorded as bits of a
-//! per-lane mask over the tile's candidates and appended afterwards in candidate order, so the
-//! list keeps the traversal order while the test loop stays free of the divergent append.
-/* Local lists: a target's own bit is cleared (a lane finds its place through `self`), the candidates
- * that some target keeps take the next positions of the group's table, and their entries of tj become
- * those positions. */
-template<Fold mode, bool Local, class Sink>
-__device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, const double* tx, const double* ty,
-                                          const double* tz, uint32_t* tj, const double* tm, uint32_t* self,
-                                          uint32_t n, double sx, double sy, double sz, unsigned& count,
-                                          ListWriter<Local>& out, Sink& sink)
+//! exact hits of the tile's n candidates (n <= 64) against the lane's target, one bit per candidate
+template<Fold mode, class Lds>
+__device__ __forceinline__ uint64_t exactMask(const SearchArgs& a, const Target& t, const Lds& lds, int buf, uint32_t n,
+                                              const double shift[3])
 {
 #pragma clang fp contract(off)
-    const DevBox&  b     = a.box;
-    const unsigned ngmax = a.ngmax;
-    auto test32 = [&](uint32_t c0, uint32_t cn) {
-        uint32_t m = 0;
+    const DevBox& b  = a.box;
+    const double *tx = lds.tx[buf], *ty = lds.ty[buf], *tz = lds.tz[buf];
+    uint64_t      m  = 0;
+    for (uint32_t c0 = 0; c0 < n; c0 += 32)
+    {
+        uint32_t       w  = 0;
+        const uint32_t cn = uniform(min(n - c0, 32u));
 #pragma unroll 4
         for (uint32_t c = 0; c < cn; ++c)
         {
             double dx = tx[c0 + c] - t.x, dy = ty[c0 + c] - t.y, dz = tz[c0 + c] - t.z;
-            if constexpr (mode == Fold::shifted) { dx = dx - sx, dy = dy - sy, dz = dz - sz; }
-            if constexpr (mode == Fold::perPair)
+            if constexpr (mode == Fold::shifted) { dx = dx - shift[0], dy = dy - shift[1], dz = dz - shift[2]; }
+            else
             {
                 dx = dx - double(b.pbc[0]) * b.len[0] * rint(dx * b.ilen[0]);
                 dy = dy - double(b.pbc[1]) * b.len[1] * rint(dy * b.ilen[1]);
                 dz = dz - double(b.pbc[2]) * b.len[2] * rint(dz * b.ilen[2]);
             }
             double d2 = dx * dx + dy * dy + dz * dz;
-            m |= d2 < t.r2 ? (1u << c) : 0u;
+            w |= d2 < t.r2 ? (1u << c) : 0u;
         }
-        return m;
-    };
-    // a tile holds at most 64 candidates: one 64-bit hit mask per lane, drained in one pass (the
-    // drain runs as many rounds as the busiest lane has hits, and one mask over the whole tile
-    // needs fewer rounds than two over its halves)
-    for (uint32_t c0 = 0; c0 < n; c0 += 64)
+        m |= uint64_t(w) << c0;
+    }
+    return m;
+}
+
+/*! The targets of a wave as the right operand of the distance matrix (tileMask). Coordinates are relative to the
+ * group's centre and scaled by a power of two so that no separation exceeds 1. */
+struct TargetMatrix
+{
+    double origin[3]; // the group's centre
+    double scale;
+    float  b[4];      // per block of 16 targets: this lane's element, -2 t (component lane / 16) or 1
+    float  diff[4];   // per block: |t|^2 - r^2 of this lane's column
+};
+
+/*! Hits of the tile's candidates as one matrix product per 16 candidates and 16 targets: with D the matrix of
+ * |p - t|^2 - r^2 = [p, |p|^2] . [-2 t, 1] + (|t|^2 - r^2), v_mfma_f32_16x16x4_f32 forms 256 of its elements with K = 4,
+ * and a hit is a sign bit. Element (row, column) of a product lies in lane 16 (row / 4) + column, register row % 4; the
+ * rows are taken from the candidates so that a lane's 16 elements per target block are consecutive
+ * candidates, and two row swaps of the wave bring each lane its own target's four runs of 16 bits.
+ *
+ * With all coordinates at most 1 in size the product is within 21 * 2^-24 of the exact value (rounding of the
+ * coordinates 3, of |p|^2 and |t|^2 - r^2 2, of the sums 16); `close` is set when any element is within 2^-19 of zero,
+ * and the tile is then tested exactly. That leaves the reference's FP64 predicate for every pair. About 3% of
+ * the tiles on a lattice are tested twice. The vector ALU spends 1.5 instructions per candidate here and 11 in
+ * exactMask, where this loop was two fifths of the search. */
+template<class Lds>
+__device__ __forceinline__ uint64_t tileMask(Lds& lds, int buf, uint32_t n, const TargetMatrix& g, const double shift[3],
+                                             bool& close)
+{
+    using float4v       = float __attribute__((ext_vector_type(4)));
+    const unsigned lane = laneId();
+    float          p[4] = {0.0f, 0.0f, 0.0f, 4.0f}; // past the tile: far from every target
+    if (lane < n)
     {
-        const uint32_t cn = uniform(min(n - c0, 64u));
-        uint64_t       m  = test32(c0, min(cn, 32u));
-        if (cn > 32u) { m |= uint64_t(test32(c0 + 32u, cn - 32u)) << 32; }
-        if (!t.active) { m = 0; }
-        if constexpr (Local)
-        {
-            const unsigned lane = laneId();
-            const uint32_t j    = lane < cn ? tj[c0 + lane] : 0xffffffffu;
-            self[lane]          = kWave;
-            __builtin_amdgcn_wave_barrier();
-            // the wave's targets are consecutive particles from lane 0's on
-            const uint32_t rel = j - (t.i - lane);
-            if (rel < uint32_t(kWave)) { self[rel] = lane; }
-            __builtin_amdgcn_wave_barrier();
-            const uint32_t own = self[lane];
-            if (own < uint32_t(kWave)) { m &= ~(uint64_t(1) << own); }
-            const uint64_t used = uint64_t(waveOr(uint32_t(m))) | uint64_t(waveOr(uint32_t(m >> 32))) << 32;
-            const uint32_t pos  = out.inTable + laneRank(used);
-            if ((used >> lane) & 1u)
-            {
-                if (pos < kTableCap) { a.table[size_t(out.group) * kTableCap + pos] = j; }
-                tj[c0 + lane] = pos;
-            }
-            out.inTable += uint32_t(__popcll(used));
-            __builtin_amdgcn_wave_barrier();
-        }
-        while (m)
-        {
+        p[0] = float((lds.tx[buf][lane] - (g.origin[0] + shift[0])) * g.scale);
+        p[1] = float((lds.ty[buf][lane] - (g.origin[1] + shift[1])) * g.scale);
+        p[2] = float((lds.tz[buf][lane] - (g.origin[2] + shift[2])) * g.scale);
+        p[3] = float(double(p[0]) * double(p[0]) + double(p[1]) * double(p[1]) + double(p[2]) * double(p[2]));
+    }
 #pragma unroll
-            for (int u = 0; u < Sink::kBatch; ++u)
-            {
-                const bool     have  = m != 0;
-                const uint32_t c     = c0 + (have ? uint32_t(__builtin_ctzll(m)) : 0u);
-                const uint32_t j     = tj[c];
-                const bool     keep  = have && (Local || j != t.i);
-                const bool     store = keep && count < ngmax;
-                m &= m - 1;
-                if (store) { out.put(count, j); }
-                count += keep ? 1u : 0u;
-                if constexpr (Sink::kStageMass)
-                {
-                    double dx = tx[c] - t.x, dy = ty[c] - t.y, dz = tz[c] - t.z;
-                    if constexpr (mode == Fold::shifted) { dx = dx - sx, dy = dy - sy, dz = dz - sz; }
-                    if constexpr (mode == Fold::perPair)
-                    {
-                        dx = dx - double(b.pbc[0]) * b.len[0] * rint(dx * b.ilen[0]);
-                        dy = dy - double(b.pbc[1]) * b.len[1] * rint(dy * b.ilen[1]);
-                        dz = dz - double(b.pbc[2]) * b.len[2] * rint(dz * b.ilen[2]);
-                    }
-                    sink.stage(u, store, dx, dy, dz, tm[c]);
-                }
-            }
-            sink.flush();
+    for (int k = 0; k < 4; ++k)
+        lds.mx[k * kMatStride + lane] = p[k];
+    __builtin_amdgcn_wave_barrier();
+    // row 4 q + i of block a is candidate 16 q + 4 a + i
+    const float* src = lds.mx + (lane / 16) * kMatStride + 16 * ((lane % 16) / 4) + lane % 4;
+    float        m[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        m[k] = src[4 * k];
+    __builtin_amdgcn_wave_barrier();
+    uint32_t f[4];
+    float    least = 1.0f;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+    {
+        const float4v c = {g.diff[b], g.diff[b], g.diff[b], g.diff[b]};
+        uint32_t      w = 0;
+#pragma unroll
+        for (int k = 3; k >= 0; --k)
+        {
+            const float4v d = __builtin_amdgcn_mfma_f32_16x16x4f32(m[k], g.b[b], c, 0, 0, 0);
+#pragma unroll
+            for (int i = 3; i >= 0; --i)
+                w = __builtin_amdgcn_alignbit(w, __float_as_uint(d[i]), 31);
+            least = fminf(least, fminf(fabsf(d[0]), fabsf(d[1])));
+            least = fminf(least, fminf(fabsf(d[2]), fabsf(d[3])));
         }
+        f[b] = w;
+    }
+    close = ballot(!(least > 0x1p-19f)) != 0;
+    // lane row q, run b  <->  lane row b, run q
+    auto s0 = __builtin_amdgcn_permlane32_swap(f[0], f[2], false, false);
+    auto s1 = __builtin_amdgcn_permlane32_swap(f[1], f[3], false, false);
+    auto r0 = __builtin_amdgcn_permlane16_swap(s0[0], s1[0], false, false);
+    auto r1 = __builtin_amdgcn_permlane16_swap(s0[1], s1[1], false, false);
+    const uint64_t hits = uint64_t(r0[0] | r0[1] << 16) | uint64_t(r1[0] | r1[1] << 16) << 32;
+    return n < uint32_t(kWave) ? hits & ((uint64_t(1) << n) - 1) : hits;
+}
+
+/* Sweep the tile's n candidates: their hits as one bit per candidate and target (a tile holds at most 64), appended
+ * afterwards in candidate order, so that each list keeps the traversal order while the tests stay free of the
+ * divergent append. The append runs as many rounds as the busiest lane has hits.
+ * Local lists: a target's own bit is cleared (a lane finds its place through `self`), the candidates
+ * that some target keeps take the next positions of the group's table, and their entries of tj become
+ * those positions. */
+template<bool Local, class Sink, class Lds>
+__device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, Lds& lds, const TargetMatrix& g, int buf,
+                                          uint32_t n, bool perPair, const double shift[3], unsigned& count,
+                                          ListWriter<Local>& out, Sink& sink)
+{
+    const unsigned ngmax = a.ngmax;
+    uint32_t*      tj    = lds.tj[buf];
+    uint64_t       m     = 0;
+    bool           exact = true;
+    if constexpr (!Sink::kStageMass)
+    {
+        if (!perPair) { m = tileMask(lds, buf, n, g, shift, exact); }
+    }
+    if (exact)
+    {
+        m = perPair ? exactMask<Fold::perPair>(a, t, lds, buf, n, shift)
+                    : exactMask<Fold::shifted>(a, t, lds, buf, n, shift);
+    }
+    if (!t.active) { m = 0; }
+    if constexpr (Local)
+    {
+        const unsigned lane = laneId();
+        const uint32_t j    = lane < n ? tj[lane] : 0xffffffffu;
+        lds.self[lane]      = uint8_t(kWave);
+        __builtin_amdgcn_wave_barrier();
+        // the wave's targets are consecutive particles from lane 0's on
+        const uint32_t rel = j - (t.i - lane);
+        if (rel < uint32_t(kWave)) { lds.self[rel] = uint8_t(lane); }
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t own = lds.self[lane];
+        if (own < uint32_t(kWave)) { m &= ~(uint64_t(1) << own); }
+        const uint64_t used = uint64_t(waveOr(uint32_t(m))) | uint64_t(waveOr(uint32_t(m >> 32))) << 32;
+        const uint32_t pos  = out.inTable + laneRank(used);
+        if ((used >> lane) & 1u)
+        {
+            if (pos < kTableCap) { a.table[size_t(out.group) * kTableCap + pos] = j; }
+            tj[lane] = pos;
+        }
+        out.inTable += uint32_t(__popcll(used));
+        __builtin_amdgcn_wave_barrier();
+    }
+    while (m)
+    {
+#pragma unroll
+        for (int u = 0; u < Sink::kBatch; ++u)
+        {
+            const bool     have  = m != 0;
+            const uint32_t c     = have ? uint32_t(__builtin_ctzll(m)) : 0u;
+            const uint32_t j     = tj[c];
+            const bool     keep  = have && (Local || j != t.i);
+            const bool     store = keep && count < ngmax;
+            m &= m - 1;
+            if (store) { out.put(count, j); }
+            count += keep ? 1u : 0u;
+            if constexpr (Sink::kStageMass)
+            {
+#pragma clang fp contract(off)
+                const DevBox& b  = a.box;
+                double        dx = lds.tx[buf][c] - t.x, dy = lds.ty[buf][c] - t.y, dz = lds.tz[buf][c] - t.z;
+                if (perPair)
+                {
+                    dx = dx - double(b.pbc[0]) * b.len[0] * rint(dx * b.ilen[0]);
+                    dy = dy - double(b.pbc[1]) * b.len[1] * rint(dy * b.ilen[1]);
+                    dz = dz - double(b.pbc[2]) * b.len[2] * rint(dz * b.ilen[2]);
+                }
+                else { dx = dx - shift[0], dy = dy - shift[1], dz = dz - shift[2]; }
+                sink.stage(u, store, dx, dy, dz, lds.tm[buf][c]);
+            }
+        }
+        sink.flush();
     }
 }
 
@@ -365,21 +463,15 @@ __device__ __forceinline__ double imageShift(const DevBox& b, int code, int d)
 
 //! sweep the first n candidates of tile buffer `buf`, all of image `code`
 template<bool Local, class Sink, class Lds>
-__device__ __forceinline__ void sweepBuffer(const SearchArgs& a, const Target& t, Lds& lds, int buf, uint32_t n,
-                                            int code, unsigned& count, ListWriter<Local>& out, Sink& sink)
+__device__ __forceinline__ void sweepBuffer(const SearchArgs& a, const Target& t, Lds& lds, const TargetMatrix& g, int buf,
+                                            uint32_t n, int code, unsigned& count, ListWriter<Local>& out, Sink& sink)
 {
     __builtin_amdgcn_wave_barrier(); // a wave's LDS accesses complete in order
     out.swept += n;
-    const double* tx = lds.tx[buf];
-    const double* ty = lds.ty[buf];
-    const double* tz = lds.tz[buf];
-    if (code == kPerPairImage)
-        sweepTile<Fold::perPair>(a, t, tx, ty, tz, lds.tj[buf], lds.tm[buf], lds.self, n, 0, 0, 0, count, out, sink);
-    else if (code != kNoShiftImage)
-        sweepTile<Fold::shifted>(a, t, tx, ty, tz, lds.tj[buf], lds.tm[buf], lds.self, n, imageShift(a.box, code, 0),
-                                 imageShift(a.box, code, 1), imageShift(a.box, code, 2), count, out, sink);
-    else
-        sweepTile<Fold::none>(a, t, tx, ty, tz, lds.tj[buf], lds.tm[buf], lds.self, n, 0, 0, 0, count, out, sink);
+    const bool   perPair  = code == kPerPairImage;
+    const double shift[3] = {perPair ? 0.0 : imageShift(a.box, code, 0), perPair ? 0.0 : imageShift(a.box, code, 1),
+                             perPair ? 0.0 : imageShift(a.box, code, 2)};
+    sweepTile(a, t, lds, g, buf, n, perPair, shift, count, out, sink);
     __builtin_amdgcn_wave_barrier();
 }
 
@@ -396,7 +488,8 @@ __device__ __forceinline__ void sweepBuffer(const SearchArgs& a, const Target& t
  *    window's loads are in flight. The candidate order is therefore the traversal order, as in
  *    the reference. */
 template<bool Local, class Sink, class Lds>
-__device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t, Lds& lds, const int32_t* leaves, int nLeaf,
+__device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t, Lds& lds, const TargetMatrix& g,
+                            const int32_t* leaves, int nLeaf,
                             const double gc[3],
                             const double ge[3], double reach, unsigned& count, ListWriter<Local>& out,
                             Sink& sink)
@@ -475,7 +568,7 @@ __device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t
     {
         const unsigned r = laneRank(keepMask);
         lds.leafLo[r]    = lo;
-        lds.leafImg[r]   = code;
+        lds.leafImg[r]   = uint8_t(code);
         lds.leafPre[r]   = incl - cnt;
     }
     const uint32_t total = uniform(__shfl(incl, kWave - 1, kWave));
@@ -527,57 +620,57 @@ __device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t
     int      cur     = 0;             // tile buffer being filled
     uint32_t acc     = 0;             // candidates in it
     int      tileImg = runImg;        // their image
+    bool     more    = true;          // a window is loaded
     while (true)
     {
-        const int      img = runImg;  // image of the loaded window
-        const uint32_t end = E;
-        if (img != tileImg && acc > 0) // a tile holds one image
+        // take the loaded window, unless its image ends the tile (a tile holds one image)
+        if (more && (acc == 0 || runImg == tileImg))
         {
-            sweepBuffer(a, t, lds, cur, acc, tileImg, count, out, sink);
-            acc = 0, cur ^= 1;
-        }
-        tileImg = img;
-        // keep the window's particles within reach of the group box under its image
-        bool keep = valid;
-        if (keep && img != kPerPairImage)
-        {
-            const double q[3] = {px - imageShift(b, img, 0), py - imageShift(b, img, 1), pz - imageShift(b, img, 2)};
-            double       d2   = 0.0;
-            for (int d = 0; d < 3; ++d)
+            tileImg = runImg;
+            // keep the window's particles within reach of the group box under its image
+            bool keep = valid;
+            if (keep && tileImg != kPerPairImage)
             {
-                double v = fabs(q[d] - gc[d]) - ge[d];
-                v        = v > 0.0 ? v : 0.0;
-                d2 += v * v;
+                const double q[3] = {px - imageShift(b, tileImg, 0), py - imageShift(b, tileImg, 1),
+                                     pz - imageShift(b, tileImg, 2)};
+                double       d2   = 0.0;
+                for (int d = 0; d < 3; ++d)
+                {
+                    double v = fabs(q[d] - gc[d]) - ge[d];
+                    v        = v > 0.0 ? v : 0.0;
+                    d2 += v * v;
+                }
+                keep = d2 < reach2;
             }
-            keep = d2 < reach2;
+            const uint64_t kmask = ballot(keep);
+            if (keep)
+            {
+                const uint32_t slot = acc + laneRank(kmask);
+                const int      bb   = slot < uint32_t(kWave) ? cur : cur ^ 1;
+                const uint32_t sl   = slot < uint32_t(kWave) ? slot : slot - kWave;
+                lds.tx[bb][sl] = px, lds.ty[bb][sl] = py, lds.tz[bb][sl] = pz;
+                lds.tj[bb][sl] = idx;
+                if constexpr (Sink::kStageMass) { lds.tm[bb][sl] = pm; }
+            }
+            acc += uint32_t(__popcll(kmask));
+            // next window's loads go out before the sweep
+            S    = E;
+            more = S < total;
+            if (more)
+            {
+                plan(E, valid, idx);
+                load(valid, idx);
+            }
         }
-        const uint64_t kmask = ballot(keep);
-        if (keep)
+        // a full tile, or the last one of its image
+        if (acc >= uint32_t(kWave) || (acc > 0 && (!more || runImg != tileImg)))
         {
-            const uint32_t slot = acc + laneRank(kmask);
-            const int      bb   = slot < uint32_t(kWave) ? cur : cur ^ 1;
-            const uint32_t sl   = slot < uint32_t(kWave) ? slot : slot - kWave;
-            lds.tx[bb][sl] = px, lds.ty[bb][sl] = py, lds.tz[bb][sl] = pz;
-            lds.tj[bb][sl] = idx;
-            if constexpr (Sink::kStageMass) { lds.tm[bb][sl] = pm; }
+            const uint32_t n = min(acc, uint32_t(kWave));
+            sweepBuffer(a, t, lds, g, cur, n, tileImg, count, out, sink);
+            acc -= n, cur ^= 1;
         }
-        acc += uint32_t(__popcll(kmask));
-        // next window's loads go out before the sweep
-        S                = end;
-        const bool more  = S < total;
-        if (more)
-        {
-            plan(E, valid, idx);
-            load(valid, idx);
-        }
-        if (acc >= uint32_t(kWave))
-        {
-            sweepBuffer(a, t, lds, cur, kWave, tileImg, count, out, sink);
-            acc -= kWave, cur ^= 1;
-        }
-        if (!more) { break; }
+        if (!more && acc == 0) { break; }
     }
-    if (acc > 0) { sweepBuffer(a, t, lds, cur, acc, tileImg, count, out, sink); }
 }
 
 //! Sort the first n entries of the found-leaf buffer by rank (bitonic network over the next
@@ -660,6 +753,32 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
     }
     double reach  = waveMax(t.active ? radius : 0.0) + a.slack;
     double reach2 = reach * reach;
+    if (ballot(t.active) == 0) { return 0; }
+
+    TargetMatrix g;
+    if constexpr (!Sink::kStageMass)
+    {
+        // every kept candidate and every target within 1 of the centre after scaling, and every separation
+        const double size = 2.0 * sqrt(ge[0] * ge[0] + ge[1] * ge[1] + ge[2] * ge[2]) + reach;
+        g.scale           = size > 0.0 && size < 1e300 ? ldexp(1.0, -(ilogb(size) + 1)) : 1.0;
+        float q[3], diff;
+        for (int d = 0; d < 3; ++d)
+        {
+            g.origin[d] = gc[d];
+            q[d]        = t.active ? float((p[d] - gc[d]) * g.scale) : 0.0f;
+        }
+        diff = t.active ? float(double(q[0]) * double(q[0]) + double(q[1]) * double(q[1]) + double(q[2]) * double(q[2]) -
+                                t.r2 * (g.scale * g.scale))
+                        : 4.0f; // no hits
+        if (!(fabsf(q[0]) + fabsf(q[1]) + fabsf(q[2]) < 4.0f)) { q[0] = q[1] = q[2] = 0.0f, diff = 4.0f; } // NaN: none
+        for (int b4 = 0; b4 < 4; ++b4)
+        {
+            const int   col = 16 * b4 + int(lane % 16);
+            const float bx = __shfl(q[0], col, kWave), by = __shfl(q[1], col, kWave), bz = __shfl(q[2], col, kWave);
+            g.b[b4]        = lane < 16 ? -2.0f * bx : lane < 32 ? -2.0f * by : lane < 48 ? -2.0f * bz : 1.0f;
+            g.diff[b4]     = __shfl(diff, col, kWave);
+        }
+    }
 
     unsigned count = 0;
     int      top   = 1;
@@ -678,7 +797,7 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
         }
         for (int done = 0; done < final; done += kLeafCap)
         {
-            flushLeaves(a, t, lds, lds.bufNode + done, min(kLeafCap, final - done), gc, ge, reach, count, out, sink);
+            flushLeaves(a, t, lds, g, lds.bufNode + done, min(kLeafCap, final - done), gc, ge, reach, count, out, sink);
         }
         // move the rest to the front
         const int rest = nBuf - final;
@@ -692,7 +811,7 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
         nBuf = rest;
     };
 
-    while (top > 0)
+    for (bool done = false; !done;)
     {
         const bool batch = top + 7 * kWave <= kStackCap - 160 && nBuf + kWave <= kBufCap - 8;
         const int  k     = batch ? min(kWave, top) : 1;
@@ -744,24 +863,26 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
         top += 8 * __popcll(mInt);
         __builtin_amdgcn_wave_barrier();
 
-        // leaves ranked below the first pending node are final
-        if (nBuf >= kLeafCap || nBuf > kBufCap - 8 - kWave)
+        // leaves ranked below the first pending node are final; all are when none is pending
+        done         = top == 0;
+        bool  sweep  = done;
+        int32_t limit = INT32_MAX;
+        if (!done && (nBuf >= kLeafCap || nBuf > kBufCap - 8 - kWave))
         {
             // the first pending node: the first visited child of the first pushed node, whose rank
             // is its parent's, or else the node left below the popped ones
-            int32_t limit = INT32_MAX;
             if (mInt) { limit = __builtin_amdgcn_readlane(rank, __builtin_ctzll(mInt)); }
-            else if (top > 0) { limit = a.rankLo[lds.stack[top - 1]]; }
+            else { limit = a.rankLo[lds.stack[top - 1]]; }
             int           final = 0;
             for (int q = 0; q < nBuf; q += kWave)
             {
                 const int i = q + int(lane);
                 final += __popcll(ballot(i < nBuf && lds.bufRank[i] < limit));
             }
-            if (final >= kLeafCap || (nBuf > kBufCap - 8 && final > 0)) { sweepFound(limit); }
+            sweep = final >= kLeafCap || (nBuf > kBufCap - 8 && final > 0);
         }
+        if (sweep) { sweepFound(limit); }
     }
-    sweepFound(INT32_MAX);
     return count;
 }
 
@@ -860,29 +981,25 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     };
     resetSink();
 
-    bool     valid = t.active;
-    unsigned count = searchGroup(a, t, double(2) * double(hi), lds, out, sink);
-    unsigned ncSph = 1 + count;
-
-    int      updates = 0;
-    unsigned ngmin   = a.ng0 / 4;
-    if (a.iterateH)
+    const bool     valid   = t.active;
+    unsigned       ncSph   = 1;
+    int            updates = 0;
+    const unsigned ngmin   = a.ng0 / 4;
+    while (true)
     {
-        while (true)
+        const unsigned count = searchGroup(a, t, double(2) * double(hi), lds, out, sink);
+        if (t.active) { ncSph = 1 + count; }
+        if (!a.iterateH) { break; }
+        const bool repeat = valid && (ngmin > ncSph || (ncSph - 1) > a.ngmax) && updates < 10;
+        if (!ballot(repeat)) { break; }
+        if (repeat)
         {
-            bool repeat = valid && (ngmin > ncSph || (ncSph - 1) > a.ngmax) && updates < 10;
-            if (!ballot(repeat)) { break; }
-            if (repeat)
-            {
-                updates++;
-                hi = updateH(a.ng0, ncSph, hi);
-                setRadius(t, hi, a.slack);
-                resetSink();
-            }
-            t.active       = repeat;
-            unsigned again = searchGroup(a, t, double(2) * double(hi), lds, out, sink);
-            if (repeat) { ncSph = 1 + again; }
+            updates++;
+            hi = updateH(a.ng0, ncSph, hi);
+            setRadius(t, hi, a.slack);
+            resetSink();
         }
+        t.active = repeat;
     }
     if (valid)
     {
