@@ -158,7 +158,7 @@ __global__ void __launch_bounds__(256) eosStdPolytropicKernel(const T* __restric
 
 /* IADJLoopSTD (hydro_std/iad_kern.hpp:11-76): tau_ab = sum_j m_j/rho_j W_ij r_a r_b, inverted */
 template<class T, int V>
-__global__ void __launch_bounds__(kLightWaves * kWave)
+__global__ void __launch_bounds__(kLightWaves * kWave) SPHX_LIGHT_WAVES(T)
     iadStdKernel(PairArgs a, const RecVol<T>* __restrict__ rec, const T* __restrict__ h, SincKernel<T> kern,
                  T* c11, T* c12, T* c13, T* c22, T* c23, T* c33, MomStdFields nf, RecMomStd<T>* __restrict__ next)
 {
@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(kMomWaves<T> * kWave)
     T      maxvs = 0;
     T      momx = 0, momy = 0, momz = 0;
     double energy = 0.0;
-    PairWalk<kMomWaves<T>, 2, RecMomStd<T>> walk(a.L, t, rec);
+    PairWalk<kMomWaves<T>, isMixed<T> ? 2 : 1, RecMomStd<T>> walk(a.L, t, rec);
     withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
         walk([&](bool live, const RecMomStd<T>& rj) {
             const Sep<T> r = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj);

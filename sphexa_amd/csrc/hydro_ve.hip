@@ -25,7 +25,7 @@ __global__ void __launch_bounds__(kPackThreads) packGradh(PairArgs a, const T* _
 
 /* veDefGradhJLoop (hydro_ve/ve_def_gradh_kern.hpp:44-90): kx and the grad-h term */
 template<class T, int V>
-__global__ void __launch_bounds__(kLightWaves * kWave)
+__global__ void __launch_bounds__(kLightWaves * kWave) SPHX_LIGHT_WAVES(T)
     veDefGradhKernel(PairArgs a, const RecGradh<T>* __restrict__ rec, const T* __restrict__ h,
                      SincKernel<T> kern, T* __restrict__ kx, T* __restrict__ gradh, RecIadVe<T>* __restrict__ next,
                      const T* __restrict__ vx, const T* __restrict__ vy, const T* __restrict__ vz)
@@ -190,7 +190,7 @@ __global__ void __launch_bounds__(kPackThreads) packIadVe(PairArgs a, IadVeField
  *   M[a][c] = sum_j (v_ja - v_ia) xm_j W_ij r_ij,c,
  * so the 9 moments M are accumulated alongside tau and combined with C_i after the inversion. */
 template<class T, int V>
-__global__ void __launch_bounds__(kLightWaves * kWave)
+__global__ void __launch_bounds__(kLightWaves * kWave) SPHX_LIGHT_WAVES(T)
     iadDivvCurlvKernel(PairArgs a, IadVeFields f, const RecIadVe<T>* __restrict__ rec, SincKernel<T> kern,
                        RecAv<T>* __restrict__ next, const T* __restrict__ cNext)
 {
@@ -285,7 +285,7 @@ __global__ void __launch_bounds__(kPackThreads) packAv(PairArgs a, AvFields f, R
 /* AVswitchesJLoop (hydro_ve/av_switches_kern.hpp:44-137). grad(div v) is linear in C_i:
  * gd_b = -K/h_i^3 sum_c C_i[b][c] sum_j f_j W_ij r_ij,c with f_j = xm_j/kx_j (divv_i - divv_j). */
 template<class T, int V>
-__global__ void __launch_bounds__(kLightWaves * kWave)
+__global__ void __launch_bounds__(kLightWaves * kWave) SPHX_LIGHT_WAVES(T)
     avSwitchesKernel(PairArgs a, AvFields f, const RecAv<T>* __restrict__ rec, SincKernel<T> kern, double dt,
                      T alphamin, T alphamax, T decay, RecMomVe<T>* __restrict__ next)
 {
@@ -303,7 +303,10 @@ __global__ void __launch_bounds__(kLightWaves * kWave)
             const Sep<T> r = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj);
             T rx = r.x, ry = r.y, rz = r.z;
             T rv = rx * (ri.vx - rj.vx) + ry * (ri.vy - rj.vy) + rz * (ri.vz - rj.vz);
-            T vs = live && rv < T(0) ? ri.c + rj.c - T(3) * overDistance(rv, r.d2) : T(0);
+            // (a slot that is not live repeats a neighbour: the maximum stays)
+            T vs = ri.c + rj.c - T(3) * overDistance(rv, r.d2);
+            asm volatile("" : "+v"(vs)); // a select, not a branch around the record's loads
+            vs   = rv < T(0) ? vs : T(0);
             vsig = vsig < vs ? vs : vsig;
             T fw = rj.vol * (ri.divv - rj.divv) * T(kern.template w<V>(kern.clamp(kern.arg(r.d2, scale), live)));
             S0 += fw * rx, S1 += fw * ry, S2 += fw * rz;
@@ -419,7 +422,7 @@ __device__ __forceinline__ T ramExp2(T v)
 
 /* momentumAndEnergyJLoop<avClean> (hydro_ve/momentum_energy_kern.hpp:66-222) + tsKCourant */
 template<class T, bool avClean, int V>
-__global__ void __launch_bounds__(kMomWaves<T> * kWave)
+__global__ void __launch_bounds__((kMomWaves<T, avClean> * kWave))
     momentumVeKernel(PairArgs a, MomVeFields f, const RecMomVe<T>* __restrict__ rec,
                      const RecGradV<T>* __restrict__ gradV, SincKernel<T> kern, T Atmin,
                      T Atmax, T ramp, float Kcour, unsigned long long* minDt)
@@ -493,7 +496,7 @@ __global__ void __launch_bounds__(kMomWaves<T> * kWave)
     const bool needFold = recordNeedsFold<T, V>(a.box, t, ri, r2h);
     if constexpr (avClean)
     {
-        PairWalk<kMomWaves<T>, 2, RecMomVe<T>, RecGradV<T>> walk(a.L, t, rec, gradV);
+        PairWalk<kMomWaves<T, avClean>, isMixed<T> ? 2 : 1, RecMomVe<T>, RecGradV<T>> walk(a.L, t, rec, gradV);
         withFold(needFold, [&](auto fold) {
             walk([&](bool live, const RecMomVe<T>& rj, const RecGradV<T>& gj) { pairTerms(fold, live, rj, &gj); }, rec,
                  gradV);
@@ -501,13 +504,13 @@ __global__ void __launch_bounds__(kMomWaves<T> * kWave)
     }
     else
     {
-        PairWalk<kMomWaves<T>, 2, RecMomVe<T>> walk(a.L, t, rec);
+        PairWalk<kMomWaves<T, avClean>, isMixed<T> ? 2 : 1, RecMomVe<T>> walk(a.L, t, rec);
         withFold(needFold, [&](auto fold) {
             walk([&](bool live, const RecMomVe<T>& rj) { pairTerms(fold, live, rj, nullptr); }, rec);
         });
     }
     double sum[6] = {maxvs, momx, momy, momz, energy, avEnergy};
-    if (!waveSums<kMomWaves<T>, 6, 1>(sum)) { return; }
+    if (!waveSums<kMomWaves<T, avClean>, 6, 1>(sum)) { return; }
     double dtLane = INFINITY;
     if (t.valid)
     {
@@ -651,13 +654,14 @@ void launchMomVe(sphx_workspace* ws, PairArgs a, const MomVeFields& mf, const sp
         packGradV<T><<<ceilDiv(a.numParticles, kPackThreads), kPackThreads, 0, ws->stream>>>(a.box, mf, gradV, a.numParticles);
         SPHX_CHECK_LAUNCH();
     }
-    const PairLaunch run = pairLaunch(ws, sizeof(RecMomVe<T>) + (avClean ? sizeof(RecGradV<T>) : 0), kMomWaves<T>, 6);
+    const PairLaunch run = pairLaunch(ws, sizeof(RecMomVe<T>) + (avClean ? sizeof(RecGradV<T>) : 0),
+                                      avClean ? kMomWaves<T, true> : kMomWaves<T>, 6);
     a.L.stage            = run.stage;
     KernelScope timer(ws, "momentum_ve");
     launchVariant<T>(ws, a.box, [&](auto variant) {
         constexpr int V = decltype(variant)::value;
         if (avClean)
-            momentumVeKernel<T, true, V><<<blocks, kMomWaves<T> * kWave, run.lds, ws->stream>>>(
+            momentumVeKernel<T, true, V><<<blocks, kMomWaves<T, true> * kWave, run.lds, ws->stream>>>(
                 a, mf, rec, gradV, sincKernel<T>(ws), T(p->Atmin), T(p->Atmax), T(p->ramp), float(p->Kcour), dt);
         else
             momentumVeKernel<T, false, V><<<blocks, kMomWaves<T> * kWave, run.lds, ws->stream>>>(

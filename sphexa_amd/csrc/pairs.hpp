@@ -1,7 +1,7 @@
 // Helpers shared by the SPH pair-loop kernels (std and VE).
 //
-// Launch shape: one block of W waves (4, or 8 where the records fill a CU's LDS) per group of 64 consecutive targets (the neighbour-search
-// group), blocks renumbered per XCD (xcdBlock) so that neighbouring groups share an L2. Lane l of
+// Launch shape: one block of W waves (4, or 8 to 12 where the records fill a CU's LDS) per group of 64 consecutive
+// targets (the neighbour-search group), blocks renumbered per XCD (xcdBlock) so that neighbouring groups share an L2. Lane l of
 // every wave owns target first + 64 g + l; wave w takes the quads w, w + W, .. of its list, and the
 // waves' partial sums are added at the end in a fixed order (waveSums), so a target's result does
 // not depend on the grouping of the call.
@@ -13,10 +13,10 @@
 // table to LDS, chunk c of all records side by side, and every neighbour is read from there
 // (PairWalk). Groups whose table does not fit the launch's LDS, and global lists,
 // read the records from global memory in the same order. Measured (ms; gathers from global memory, then this):
-// mixed VE at 8M particles, XMass 1.27 -> 0.81, grad-h 2.13 -> 1.36, IAD 2.17 -> 1.57, AV switches 2.84 -> 1.78,
-// momentum-energy 4.92 -> 3.24; FP64 VE at 4.1M, 2.35 -> 1.05, 2.90 -> 2.06, 3.26 -> 2.07, 4.06 -> 2.30, 6.76 ->
-// 5.26 (with the kernel evaluated instead of gathered from its table). What bounds them now: the FP32 form
-// the vector ALU (62-86% of its issue slots), the FP64 form the latency of a block's phases at 2-3 waves per SIMD.
+// mixed VE at 8M particles, XMass 1.27 -> 0.78, grad-h 2.13 -> 1.33, IAD 2.17 -> 1.55, AV switches 2.84 -> 1.47,
+// momentum-energy 4.92 -> 3.24; FP64 VE at 4.1M, 2.35 -> 1.03, 2.90 -> 1.73, 3.26 -> 2.10, 4.06 -> 2.05, 6.76 ->
+// 5.11 (with the kernel evaluated instead of gathered from its table). What bounds them now: the FP32 form
+// the vector ALU (67-90% of its issue slots), the FP64 form the latency of a block's phases at 2-3 waves per SIMD.
 //
 // Two arithmetic forms share each kernel template:
 //  * T = double ("plain" FP64): the reference JLoop formulas in FP64.
@@ -37,21 +37,30 @@ namespace sphx
 template<class T>
 constexpr bool isMixed = std::is_same_v<T, float>;
 
-//! waves per block of the light loops (XMass, grad-h, IAD, AV switches) and of momentum-energy. The FP64
-//! momentum records of a group take 90-102 KB of LDS, one block per CU: eight waves give two per SIMD.
+/*! Waves per block. The light loops (XMass, grad-h, IAD, AV switches) take four. The FP64 momentum records of a
+ * group take 92-112 KB of LDS, one block per CU, so the block has to bring the CU's waves: twelve (three per SIMD,
+ * 168 registers each), or eight with AV cleaning, whose FP64 loop needs more registers. FP64 VE momentum at 4.1M
+ * particles: four waves 8.85 ms, eight 5.25, twelve 5.11. */
 constexpr int kLightWaves = 4;
-template<class T>
-constexpr int kMomWaves = isMixed<T> ? 4 : 8;
+template<class T, bool avClean = false>
+constexpr int kMomWaves = isMixed<T> ? 4 : avClean ? 8 : 12;
+
+//! waves per SIMD that a light loop's registers must leave room for: five in the FP32 form, three in the FP64 form
+//! (its LDS holds three blocks or more); without the bound some take a few registers too many for that
+#define SPHX_LIGHT_WAVES(T) __attribute__((amdgpu_waves_per_eu(isMixed<T> ? 5 : 3, isMixed<T> ? 8 : 3)))
 
 //! waves per block of the adjoint loops, which take one group per wave
 constexpr int kVjpWaves = 4;
 
 struct Lists
 {
+    static constexpr uint32_t kNoBlock = 0xffffffffu;
+
     NeighborLists   lists;
     const uint32_t* nc;
     uint32_t        first, last, ngmax; // [first, last): the searched targets
     uint32_t        stage;              // records the launch's LDS holds
+    uint32_t        block0;             // list block of the call's first group, whose targets are whole blocks; or kNoBlock
     Groups          groups;             // the call's target groups
 };
 
@@ -228,23 +237,38 @@ struct PairWalk
     const Lists& L;
     const Lane&  t;
     bool         staged;
+    uint64_t     next; // local lists: the wave's first quad
 
-    //! stages the group's records, unless they do not fit or are not one group's
+    //! stages the group's records, unless they do not fit or are not one group's. Where the call's groups are the
+    //! search's, the table and the first quad of the lists load without waiting for the targets' counts.
     __device__ __forceinline__ PairWalk(const Lists& lists, const Lane& lane, const Rs*... rec)
         : L(lists)
         , t(lane)
         , staged(false)
+        , next(0)
     {
         if (L.lists.tableCount != nullptr)
         {
-            const bool     some  = t.n > 0;
-            const uint32_t b     = some ? L.lists.group(t.r) : 0u;
-            const uint64_t mask  = ballot(some);
-            const uint32_t b0    = mask ? __builtin_amdgcn_readlane(b, __builtin_ctzll(mask)) : 0u;
-            const uint32_t count = mask ? L.lists.tableCount[b0] : 0u;
-            if (ballot(some && b != b0) == 0 && count <= L.stage)
+            bool     one;
+            uint32_t b0;
+            if (L.block0 != Lists::kNoBlock)
             {
-                staged             = true;
+                b0  = L.block0 + blockGroup();
+                one = true;
+            }
+            else
+            {
+                const bool     some = t.n > 0;
+                const uint32_t b    = some ? L.lists.group(t.r) : 0u;
+                const uint64_t mask = ballot(some);
+                b0                  = mask ? __builtin_amdgcn_readlane(b, __builtin_ctzll(mask)) : 0u;
+                one                 = ballot(some && b != b0) == 0 && mask != 0;
+            }
+            const uint32_t count = L.lists.tableCount[b0];
+            if (one && count <= L.stage)
+            {
+                staged = true;
+                if (firstSlot() < paddedNgmax8(L.ngmax)) { next = *reinterpret_cast<const uint64_t*>(listStart()); }
                 const uint32_t* tb = L.lists.table + size_t(b0) * kTableCap;
                 uint32_t        at = 0;
                 ((stageRecords(tb, count, rec, ldsBytes() + at, kStride), at += uint32_t(sizeof(Rs))), ...);
@@ -253,19 +277,23 @@ struct PairWalk
         __syncthreads();
     }
 
+    __device__ __forceinline__ static uint32_t firstSlot() { return 4 * (threadIdx.x / kWave); }
+    __device__ __forceinline__ const uint16_t* listStart() const
+    {
+        return static_cast<const uint16_t*>(L.lists.nbrs) +
+               localOffset(t.r / kGroup, paddedNgmax8(L.ngmax), firstSlot(), t.r % kGroup);
+    }
     __device__ __forceinline__ static char* ldsBytes() { return reinterpret_cast<char*>(pairLds); }
 
     template<class F>
-    __device__ __forceinline__ void operator()(F&& pair, const Rs*... rec) const
+    __device__ __forceinline__ void operator()(F&& pair, const Rs*... rec)
     {
-        const uint32_t g = t.r / kGroup, lane = t.r % kGroup, k0 = 4 * (threadIdx.x / kWave);
+        const uint32_t k0 = firstSlot();
         if (staged)
         {
             static_assert(W % 2 == 0, "a wave's quads lie at one place of their octets");
             constexpr size_t step = size_t(4 * W) * kGroup; // list words from a quad to the wave's next
-            const uint16_t*  list = static_cast<const uint16_t*>(L.lists.nbrs) +
-                                   localOffset(g, paddedNgmax8(L.ngmax), k0, lane);
-            uint64_t next = k0 < t.n ? *reinterpret_cast<const uint64_t*>(list) : 0;
+            const uint16_t*  list = listStart();
             for (uint32_t k = k0; k < t.n; k += 4 * W)
             {
                 uint64_t q = next;
@@ -915,7 +943,10 @@ inline PairArgs makePairArgs(sphx_workspace* ws, const DevBox& box, const sphx_f
     SPHX_REQUIRE(f->x && f->y && f->z && f->nc, SPHX_ERR_ARG, "x, y, z and nc are required");
     PairArgs c;
     c.x = f->x, c.y = f->y, c.z = f->z, c.box = box, c.K = p->K;
-    c.L            = Lists{neighborLists(ws), f->nc, ws->nbFirst, ws->nbLast, p->ngmax, 0, groupsFor(ws, first, last)};
+    const Groups G = groupsFor(ws, first, last);
+    const bool   whole = !ws->nbOwned && G.start == nullptr && (first - ws->nbFirst) % kGroup == 0;
+    c.L = Lists{neighborLists(ws), f->nc,    ws->nbFirst, ws->nbLast, p->ngmax, 0,
+                whole ? (first - ws->nbFirst) / kGroup : Lists::kNoBlock, G};
     c.numParticles = uint32_t(ws->tree.numParticles);
     return c;
 }
