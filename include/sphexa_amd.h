@@ -294,7 +294,7 @@ int sphx_sort_keys_noalloc(int device, void* stream, uint64_t* keys, uint32_t* o
 int sphx_gather(sphx_workspace_t* ws, const uint32_t* order, const void* in, void* out, size_t n, int elemBytes);
 
 /* Cornerstone leaves (bucket size `bucketSize`), linked octree, leaf layout and geometric node
- * centres from sorted keys, kept in the workspace. Replaces computeOctree / buildOctreeGpu /
+ * centres from sorted keys, kept in the workspace; SPHX_ERR_ARG if the keys are not sorted. Replaces computeOctree / buildOctreeGpu /
  * computeNodeLayout / nodeFpCenters as combined by Domain::sync + octreeProperties on one rank
  * (domain/include/cstone/tree/csarray.hpp:430-440, tree/octree_gpu.cu:137-157,
  * focus/source_center.hpp:130-141, domain/include/cstone/domain/domain.hpp:416-428). */

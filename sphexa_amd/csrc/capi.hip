@@ -284,6 +284,7 @@ int sphx_build_tree(sphx_workspace_t* ws, const uint64_t* sortedKeys, size_t n, 
         ws->nbValid  = false;
         ws->syncTree = false;
         buildTree(ws, sortedKeys, n, bucketSize, makeDevBox(box));
+        SPHX_HIP(hipStreamSynchronize(ws->stream));
         return SPHX_OK;
     });
 }

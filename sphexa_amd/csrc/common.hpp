@@ -159,24 +159,21 @@ struct DevBuf
     }
 };
 
-//! per-build temporaries of the top-down tree construction, kept for reuse
+//! per-build temporaries of the tree construction, kept for reuse
 struct TreeBuildScratch
 {
-    DevBuf<Key>      nodeKey, leafKey, leafKeySorted;
-    DevBuf<uint32_t> lo, hi, flag, rank, leafFlag, leafRank, leafNode, leafNodeSorted;
-    DevBuf<uint8_t>  level;
-    DevBuf<int32_t>  levelStart;
+    DevBuf<uint32_t> planCounts, intLo, intPlace, dfRank, intPush; // the internal nodes by rank and in depth-first order
+    DevBuf<Key>      intKey, dfKey;
     // the one-step update of a later sync: node counts, node and leaf ops, the new leaves
-    DevBuf<uint32_t> nodeCnt, changed;
+    DevBuf<uint32_t> nodeCnt;
     DevBuf<int32_t>  nodeOp, leafOp;
     DevBuf<Key>      nextLeaves;
 
     void releaseAll()
     {
-        nodeKey.release(), leafKey.release(), leafKeySorted.release(), lo.release(), hi.release();
-        flag.release(), rank.release(), leafFlag.release(), leafRank.release(), leafNode.release();
-        leafNodeSorted.release(), level.release(), levelStart.release();
-        nodeCnt.release(), changed.release(), nodeOp.release(), leafOp.release(), nextLeaves.release();
+        planCounts.release(), intLo.release(), intPlace.release(), dfRank.release(), intPush.release();
+        intKey.release(), dfKey.release();
+        nodeCnt.release(), nodeOp.release(), leafOp.release(), nextLeaves.release();
     }
 };
 
@@ -211,8 +208,8 @@ struct Tree
     // the neighbour search's visiting order (singleTraversal, traversal/traversal.hpp:52-93):
     // leaf children in octant order, then internal children in reverse octant order, depth first.
     // rankLo: position of a node's first leaf in that order; childPush: an internal node's
-    // children from last to first visited, 3 bits per octant; subtreeLeaves: scratch
-    DevBuf<int32_t>      rankLo, subtreeLeaves;
+    // children from last to first visited, 3 bits per octant; offset: scratch
+    DevBuf<int32_t>      rankLo, offset;
     DevBuf<uint32_t>     childPush;
     bool                 valid = false;
     TreeBuildScratch     build;
@@ -221,7 +218,7 @@ struct Tree
     {
         prefixes.release(), leaves.release(), childOffsets.release(), parents.release();
         internalToLeaf.release(), levelRange.release(), counts.release(), layout.release();
-        centers.release(), sizes.release(), rankLo.release(), subtreeLeaves.release(), childPush.release();
+        centers.release(), sizes.release(), rankLo.release(), offset.release(), childPush.release();
         build.releaseAll();
         valid = false;
     }

@@ -1,13 +1,23 @@
-// Cornerstone leaf array + linked octree + layout + geometric node centres, built top-down.
+// Cornerstone leaf array + linked octree + layout + geometric node centres, built from the sorted keys at once.
 //
 // The reference converges a leaf array by repeated count/split/merge sweeps (computeOctree,
 // domain/include/cstone/tree/csarray.hpp:409-440) and then derives the internal tree by sorting
 // placeholder-bit prefixes (buildOctreeGpu, tree/octree_gpu.cu:137-157). Its fixed point is
 // unique: a node is internal iff it holds more than `bucket` particles and lies above the
-// deepest level. Descending level by level from the root and splitting exactly those nodes
-// produces that same tree, and because children are appended in key order behind their
-// level-ordered parents, the node array comes out directly in the reference's sorted
-// prefix order (level-major, SFC-minor). One host read-back per level sizes the next one.
+// deepest level. That can be read off the sorted keys without descending level by level: the node of level l whose
+// first particle is i is internal iff key i - 1 lies outside it and key i + bucket inside. So
+//  1. every key counts the levels at which it opens an internal node (planCountKernel), per block and level;
+//  2. a scan gives each internal node its rank in the reference's node order, which is level by level and
+//     along the curve within a level, and its place in depth-first order (planScanKernel, planEmitKernel);
+//  3. eight threads per internal node link its children (childKernel): the r-th internal node's children are nodes
+//     1 + 8 r .. 8 + 8 r; a leaf's place in the leaf array and the leaves below a node follow from
+//     depth-first places, each split adding seven leaves;
+//  4. every node adds up its place in the search's visiting order along its ancestors (visitKernel).
+// Five launches and one host read of the internal nodes per level, where a level-by-level descent took about forty
+// launches and a read per level. What bounds it: launch latency up to about a million particles, then reading the
+// keys twice and the chains of searches in childKernel (33 us at 1M particles). Measured, a whole std step with
+// the former descent and with this: 0.65 -> 0.51 ms at 1728 particles (FP64), 1.98 -> 1.77 ms at 1M (mixed); a mixed VE
+// step at 8M 15.2 -> 14.8 ms.
 #include <cstring> // rocprim uses memset without including it
 #include <rocprim/rocprim.hpp>
 
@@ -30,79 +40,197 @@ __device__ __forceinline__ uint32_t lowerBound(const Key* keys, uint32_t lo, uin
     return lo;
 }
 
-__global__ void initRoot(Key* nodeKey, uint32_t* lo, uint32_t* hi, uint8_t* level, uint32_t n)
+/*! first index in [lo, n) whose key is at least v, by doubling steps from lo: the searches of a node's children
+ * end within the node */
+__device__ __forceinline__ uint32_t lowerBoundFrom(const Key* keys, uint32_t lo, uint32_t n, Key v)
 {
-    nodeKey[0] = 0;
-    lo[0]      = 0;
-    hi[0]      = n;
-    level[0]   = 0;
+    uint32_t step = 1, a = lo;
+    while (a < n && keys[a] < v)
+    {
+        lo = a + 1;
+        a  = n - a > step ? a + step : n;
+        step *= 2;
+    }
+    return lowerBound(keys, lo, min(a, n), v);
 }
 
-__global__ void classifyKernel(const uint32_t* lo, const uint32_t* hi, uint32_t* flag, uint32_t begin, uint32_t end,
-                               unsigned bucket, unsigned level)
+constexpr unsigned kPlanWaves = 4;
+constexpr unsigned kPlanTiles = 8; // tiles of 64 keys per wave
+constexpr unsigned kPlanKeys  = kPlanWaves * kPlanTiles * kWave;
+constexpr unsigned kPlanRows  = kMaxLevel + 1; // internal nodes per level, then keys out of order
+
+//! keys past the curve (removed particles) count as its last one
+__device__ __forceinline__ Key onCurve(Key k)
 {
-    uint32_t i = begin + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= end) { return; }
-    flag[i] = (hi[i] - lo[i] > bucket) && (level < kMaxLevel);
+    constexpr Key last = (Key(1) << 63) - 1;
+    return k < last ? k : last;
 }
 
-//! each internal node of the level writes its 8 children behind the level; 8 consecutive threads
-//! per node, thread c finding the first particle of child c (the searches run side by side
-//! instead of as one chain of dependent loads)
-__global__ void expandKernel(const Key* __restrict__ keys, Key* nodeKey, uint32_t* lo, uint32_t* hi, uint8_t* nodeLevel,
-                             const uint32_t* flag, const uint32_t* inclRank, uint32_t internalBefore,
-                             uint32_t begin, uint32_t end, unsigned level)
+//! deepest level whose node holds both keys
+__device__ __forceinline__ int commonLevel(Key a, Key b)
 {
-    const size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const size_t i = begin + t / 8;
-    const int    c = int(t % 8);
-    if (i >= end || !flag[i]) { return; } // uniform over the node's 8 threads
-    uint32_t r     = inclRank[i] - 1 - internalBefore; // rank among this level's internal nodes
-    uint32_t slot  = end + 8 * r + uint32_t(c);
-    Key      k     = nodeKey[i];
-    Key      range = nodeRange(level + 1);
-    uint32_t a = lo[i], b = hi[i];
-    uint32_t first = (c == 0) ? a : lowerBound(keys, a, b, k + Key(c) * range);
-    uint32_t next  = __shfl_down(first, 1, 8); // first particle of child c + 1
-    nodeKey[slot]   = k + Key(c) * range;
-    lo[slot]        = first;
-    hi[slot]        = (c == 7) ? b : next;
-    nodeLevel[slot] = uint8_t(level + 1);
+    a = onCurve(a), b = onCurve(b);
+    return a == b ? int(kMaxLevel) : (__builtin_clzll(a ^ b) - 1) / 3;
 }
 
-//! prefixes, child links, parents, centres; leaves are collected for the key sort
-__global__ void linkKernel(const Key* nodeKey, const uint8_t* nodeLevel, const uint32_t* flag, const uint32_t* inclRank,
-                           const int32_t* levelStart, uint32_t numNodes, DevBox box, Key* prefixes,
-                           TreeNodeIndex* childOffsets, TreeNodeIndex* parents, TreeNodeIndex* internalToLeaf,
-                           double* centers, double* sizes, Key* leafKey, uint32_t* leafNode, const uint32_t* leafRank)
+//! key i is the first of the internal nodes of levels (p, l] (none when l <= p)
+__device__ __forceinline__ void openedLevels(const Key* __restrict__ keys, uint32_t n, unsigned bucket, uint32_t i, int& p,
+                                             int& l)
+{
+    p = 0, l = -1;
+    if (i >= n) { return; }
+    const Key      k = keys[i];
+    const uint64_t j = uint64_t(i) + bucket;
+    if (j < n) { l = min(commonLevel(k, keys[j]), int(kMaxLevel) - 1); }
+    p = i == 0 ? -1 : commonLevel(keys[i - 1], k);
+}
+
+//! internal nodes per level (row) that the keys of each block open: counts[level * gridDim.x + block]; the last row
+//! counts the keys below their predecessor, from which no tree can be linked
+__global__ void __launch_bounds__(kPlanWaves* kWave)
+    planCountKernel(const Key* __restrict__ keys, uint32_t n, unsigned bucket, uint32_t* __restrict__ counts)
+{
+    __shared__ uint32_t cnt[kPlanRows];
+    if (threadIdx.x < kPlanRows) { cnt[threadIdx.x] = 0; }
+    __syncthreads();
+    for (unsigned t = 0; t < kPlanTiles; ++t)
+    {
+        const uint32_t i = blockIdx.x * kPlanKeys + t * kPlanWaves * kWave + threadIdx.x;
+        int            p, l;
+        openedLevels(keys, n, bucket, i, p, l);
+        for (int v = p + 1; v <= l; ++v)
+            atomicAdd(&cnt[v], 1u);
+        if (i > 0 && i < n && keys[i] < keys[i - 1]) { atomicAdd(&cnt[kMaxLevel], 1u); }
+    }
+    __syncthreads();
+    if (threadIdx.x < kPlanRows) { counts[size_t(threadIdx.x) * gridDim.x + blockIdx.x] = cnt[threadIdx.x]; }
+}
+
+//! block l: exclusive scan of row l of `counts` in place, and its total
+__global__ void __launch_bounds__(256) planScanKernel(uint32_t* __restrict__ counts, uint32_t blocks,
+                                                      uint32_t* __restrict__ totals)
+{
+    __shared__ uint32_t part[256 / kWave];
+    uint32_t*           row  = counts + size_t(blockIdx.x) * blocks;
+    const unsigned      lane = laneId(), w = threadIdx.x / kWave;
+    uint32_t            run  = 0;
+    for (uint32_t b0 = 0; b0 < blocks; b0 += 256)
+    {
+        const uint32_t b    = b0 + threadIdx.x;
+        const uint32_t v    = b < blocks ? row[b] : 0u;
+        uint32_t       incl = v;
+        for (int o = 1; o < kWave; o <<= 1)
+        {
+            const uint32_t x = __shfl_up(incl, o, kWave);
+            incl += lane >= unsigned(o) ? x : 0u;
+        }
+        if (lane == kWave - 1) { part[w] = incl; }
+        __syncthreads();
+        uint32_t before = run, all = 0;
+        for (unsigned q = 0; q < 256 / kWave; ++q)
+        {
+            before += q < w ? part[q] : 0u;
+            all += part[q];
+        }
+        if (b < blocks) { row[b] = before + incl - v; }
+        run += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) { totals[blockIdx.x] = run; }
+}
+
+//! internal nodes of the shallower levels, per level (kernel argument; [kMaxLevel]: all of them)
+struct LevelBase
+{
+    uint32_t base[kMaxLevel + 1];
+};
+
+//! the internal nodes by rank (level by level) and in depth-first order
+struct InternalNodes
+{
+    Key*      key;   // by rank: first key of the node ...
+    uint32_t* lo;    // ... first particle ...
+    uint32_t* place; // ... and its place in depth-first order
+    Key*      dfKey; // by place: first key ...
+    uint32_t* rank;  // ... and rank
+    uint32_t* push;  // by rank: children from last to first visited (childPush)
+};
+
+//! writes the internal nodes; the waves of a block take consecutive runs of its keys
+__global__ void __launch_bounds__(kPlanWaves* kWave)
+    planEmitKernel(const Key* __restrict__ keys, uint32_t n, unsigned bucket, const uint32_t* __restrict__ counts,
+                   LevelBase levels, InternalNodes out)
+{
+    __shared__ uint32_t next[kPlanWaves][kMaxLevel]; // count, then rank of the wave's first node, per level
+    __shared__ uint32_t place[kPlanWaves];           // depth-first place of its first node
+    const unsigned      w = threadIdx.x / kWave, lane = laneId();
+    const uint32_t      first = blockIdx.x * kPlanKeys + w * kPlanTiles * kWave;
+    if (lane < kMaxLevel) { next[w][lane] = 0; }
+    __syncthreads();
+    int p[kPlanTiles], l[kPlanTiles];
+#pragma unroll
+    for (unsigned t = 0; t < kPlanTiles; ++t)
+    {
+        openedLevels(keys, n, bucket, first + t * kWave + lane, p[t], l[t]);
+        for (int v = p[t] + 1; v <= l[t]; ++v)
+            atomicAdd(&next[w][v], 1u);
+    }
+    __syncthreads();
+    if (w == 0)
+    {
+        uint32_t before = lane < kMaxLevel ? counts[size_t(lane) * gridDim.x + blockIdx.x] : 0u;
+        for (unsigned q = 0; q < kPlanWaves; ++q)
+        {
+            const uint32_t all = waveSum(before);
+            if (lane == 0) { place[q] = all; }
+            if (lane < kMaxLevel)
+            {
+                const uint32_t c = next[q][lane];
+                next[q][lane]    = levels.base[lane] + before;
+                before += c;
+            }
+        }
+    }
+    __syncthreads();
+    uint32_t at = place[w], r = lane < kMaxLevel ? next[w][lane] : 0u; // lane v holds the next rank of level v
+#pragma unroll
+    for (unsigned t = 0; t < kPlanTiles; ++t)
+    {
+        uint64_t open = ballot(l[t] > p[t]);
+        while (open)
+        {
+            const int s = __builtin_ctzll(open);
+            open &= open - 1;
+            const int      from = __builtin_amdgcn_readlane(p[t], s) + 1, to = __builtin_amdgcn_readlane(l[t], s);
+            const uint32_t i    = first + t * kWave + uint32_t(s);
+            if (int(lane) >= from && int(lane) <= to)
+            {
+                const Key      k = onCurve(keys[i]) & ~(nodeRange(lane) - 1);
+                const uint32_t q = at + lane - uint32_t(from); // outermost first
+                out.key[r] = k, out.lo[r] = i, out.place[r] = q;
+                out.dfKey[q] = k, out.rank[q] = r;
+                ++r;
+            }
+            at += uint32_t(to - from + 1);
+        }
+    }
+}
+
+//! arrays of the linked tree (Tree) as kernel arguments
+struct TreeArrays
+{
+    Key *          prefixes, *leaves;
+    TreeNodeIndex *childOffsets, *parents, *internalToLeaf, *levelRange;
+    uint32_t *     counts, *layout, *childPush;
+    int32_t *      rankLo, *offset; // offset: leaves visited between a node's parent's first leaf and its own
+    double *       centers, *sizes;
+};
+
+//! geometric centre and half size of the node of key k and level l: hilbertIBox + centerAndSize
+//! (sfc/hilbert.hpp:259-274, sfc/box.hpp:318-334)
+__device__ __forceinline__ void nodeBox(const DevBox& box, Key k, unsigned l, size_t i, double* centers, double* sizes)
 {
 #pragma clang fp contract(off)
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= numNodes) { return; }
-    Key      k = nodeKey[i];
-    unsigned l = nodeLevel[i];
-    prefixes[i] = encodePlaceholder(k, 3 * l);
-
-    if (flag[i])
-    {
-        // ranks of internal nodes are global (inclusive scan over all nodes); the level's
-        // first internal rank is the count of internal nodes on shallower levels
-        uint32_t rankInLevel = inclRank[i] - 1 - (levelStart[l] == 0 ? 0 : inclRank[levelStart[l] - 1]);
-        TreeNodeIndex child  = levelStart[l + 1] + 8 * TreeNodeIndex(rankInLevel);
-        childOffsets[i]      = child;
-        parents[(child - 1) / 8] = TreeNodeIndex(i);
-        internalToLeaf[i]    = -1;
-    }
-    else
-    {
-        childOffsets[i]   = 0;
-        uint32_t s        = leafRank[i];
-        leafKey[s]        = k;
-        leafNode[s]       = i;
-    }
-
-    // geometric centre / half size: hilbertIBox + centerAndSize (sfc/hilbert.hpp:259-274,
-    // sfc/box.hpp:318-334)
     unsigned ix, iy, iz;
     hilbertDecode(k, ix, iy, iz);
     unsigned     cube = (1u << kMaxLevel) >> l;
@@ -113,110 +241,114 @@ __global__ void linkKernel(const Key* nodeKey, const uint8_t* nodeLevel, const u
     {
         int    imin = int(ic[d]), imax = int(ic[d] + cube);
         double half = 0.5 * uL * box.len[d];
-        centers[3 * size_t(i) + d] = box.lo[d] + double(imax + imin) * half;
-        sizes[3 * size_t(i) + d]   = double(imax - imin) * half;
+        centers[3 * i + d] = box.lo[d] + double(imax + imin) * half;
+        sizes[3 * i + d]   = double(imax - imin) * half;
     }
 }
 
-__global__ void leafFlagKernel(const uint32_t* flag, uint32_t* leafFlag, uint32_t numNodes)
+/*! Eight threads per internal node, thread c its c-th child: the child's particles, links, box, its place in the leaf
+ * array or its rank, and the visiting order among its siblings. singleTraversal (traversal/traversal.hpp:52-93) handles
+ * a node's leaf children in octant order as it meets them, pushes its internal children in octant order and pops
+ * the last pushed first. */
+__global__ void __launch_bounds__(256) childKernel(const Key* __restrict__ keys, uint32_t n, unsigned bucket,
+                                                   LevelBase levels, InternalNodes in, DevBox box, TreeArrays t)
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < numNodes) { leafFlag[i] = 1u - flag[i]; }
-}
+    const uint32_t id = blockIdx.x * blockDim.x + threadIdx.x, total = levels.base[kMaxLevel];
+    const uint32_t r = id / 8;
+    const int      c = int(id % 8);
+    if (r >= total) { return; } // uniform over the node's 8 threads
+    unsigned l = 0;
+    while (levels.base[l + 1] <= r) { ++l; }
+    const Key      range = nodeRange(l + 1), k = in.key[r] + Key(c) * range;
+    const uint32_t place = in.place[r];
+    const bool     atEnd = in.key[r] + 8 * range == nodeRange(0);
 
-__global__ void exclusiveFromInclusive(const uint32_t* incl, const uint32_t* v, uint32_t* excl, uint32_t n)
-{
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) { excl[i] = incl[i] - v[i]; }
-}
-
-__global__ void leafFinalize(const Key* sortedLeafKey, const uint32_t* sortedLeafNode, const uint32_t* lo,
-                             const uint32_t* hi, Key* leaves, uint32_t* counts, uint32_t* layout,
-                             TreeNodeIndex* internalToLeaf, uint32_t L, uint32_t n)
-{
-    uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s > L) { return; }
-    if (s == L)
+    // particles and depth-first places of the child: its own first, and the next child's
+    const uint32_t first = c == 0 ? in.lo[r] : lowerBoundFrom(keys, in.lo[r], n, k);
+    const uint32_t q0    = c == 0 ? place + 1 : lowerBoundFrom(in.dfKey, place + 1, total, k);
+    uint32_t       last  = __shfl_down(first, 1, 8), q1 = __shfl_down(q0, 1, 8);
+    if (c == 7)
     {
-        leaves[L] = nodeRange(0);
-        layout[L] = n;
-        return;
+        last = atEnd ? n : lowerBoundFrom(keys, first, n, k + range);
+        q1   = atEnd ? total : lowerBoundFrom(in.dfKey, q0, total, k + range);
     }
-    uint32_t node        = sortedLeafNode[s];
-    leaves[s]            = sortedLeafKey[s];
-    counts[s]            = hi[node] - lo[node];
-    layout[s]            = lo[node];
-    internalToLeaf[node] = TreeNodeIndex(s);
-}
-
-//! leaves in the subtree of each node of one level (the deeper levels are done)
-__global__ void subtreeLeavesKernel(const TreeNodeIndex* childOffsets, int32_t* leaves, int32_t first, int32_t last)
-{
-    const int32_t i = first + int32_t(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= last) { return; }
-    const TreeNodeIndex c = childOffsets[i];
-    int32_t             s = 1;
-    if (c != 0)
+    const uint32_t node   = 1 + id;
+    const bool     leaf   = last - first <= bucket || l + 1 >= kMaxLevel;
+    const int32_t  leaves = leaf ? 1 : 1 + 7 * int32_t(q1 - q0);
+    t.prefixes[node]      = encodePlaceholder(k, 3 * (l + 1));
+    nodeBox(box, k, l + 1, node, t.centers, t.sizes);
+    if (leaf)
     {
-        s = 0;
-        for (int o = 0; o < 8; ++o)
-            s += leaves[c + o];
+        // leaves before it: its preceding siblings on the way down as one each, and seven per internal
+        // node that ended before (those before it in depth-first order without its l + 1 ancestors)
+        uint32_t digits = 0;
+        for (unsigned v = 1; v <= l + 1; ++v)
+            digits += unsigned(k >> (3 * (kMaxLevel - v))) & 7u;
+        const uint32_t at      = digits + 7 * (q0 - (l + 1));
+        t.childOffsets[node]   = 0;
+        t.internalToLeaf[node] = TreeNodeIndex(at);
+        t.leaves[at] = k, t.counts[at] = last - first, t.layout[at] = first;
     }
-    leaves[i] = s;
-}
-
-/*! Visiting order of the search for the children of each internal node of one level (the
- *  shallower levels are done): singleTraversal (traversal/traversal.hpp:52-93) handles a node's
- *  leaf children in octant order as it meets them, pushes its internal children in octant order
- *  and pops the last pushed first. rankLo of a child = rankLo of the parent plus the leaves visited
- *  before it; childPush lists the children from last to first visited. */
-__global__ void visitOrderKernel(const TreeNodeIndex* childOffsets, const int32_t* leaves, int32_t* rankLo,
-                                 uint32_t* childPush, int32_t first, int32_t last)
-{
-    const int32_t i = first + int32_t(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= last) { return; }
-    const TreeNodeIndex c = childOffsets[i];
-    if (c == 0) { return; }
-    int32_t  base = rankLo[i];
-    bool     isLeaf[8];
-    for (int o = 0; o < 8; ++o)
-        isLeaf[o] = childOffsets[c + o] == 0;
-    uint32_t push = 0;
-    int      slot = 7; // childPush slot 7 = the first visited
-    for (int o = 0; o < 8; ++o)
+    else
     {
-        if (!isLeaf[o]) { continue; }
-        rankLo[c + o] = base++;
-        push |= uint32_t(o) << (3 * slot--);
+        const uint32_t rank    = in.rank[q0];
+        t.childOffsets[node]   = TreeNodeIndex(1 + 8 * rank);
+        t.parents[rank]        = TreeNodeIndex(node);
+        t.internalToLeaf[node] = -1;
     }
-    for (int o = 7; o >= 0; --o)
+    // visiting order among the siblings
+    const unsigned mask   = unsigned(ballot(leaf) >> (laneId() & ~7u)) & 0xffu;
+    const int      nLeaf  = __popc(mask);
+    int32_t        offset = leaf ? __popc(mask & ((1u << c) - 1u)) : nLeaf;
+    int            pos    = leaf ? offset : nLeaf;
+    for (int o = 1; o < 8; ++o)
     {
-        if (isLeaf[o]) { continue; }
-        rankLo[c + o] = base;
-        base += leaves[c + o];
-        push |= uint32_t(o) << (3 * slot--);
+        const int32_t other = __shfl(leaves, o, 8);
+        if (!leaf && o > c && !((mask >> o) & 1u)) { offset += other, ++pos; }
     }
-    childPush[i] = push;
+    uint32_t push = uint32_t(c) << (3 * (7 - pos));
+    push |= __shfl_xor(push, 1, 8), push |= __shfl_xor(push, 2, 8), push |= __shfl_xor(push, 4, 8);
+    t.offset[node] = offset;
+    if (c == 0) { in.push[r] = push; }
+    if (id == 0)
+    {
+        t.prefixes[0] = encodePlaceholder(0, 0), t.childOffsets[0] = 1, t.parents[0] = 0, t.internalToLeaf[0] = -1;
+        t.offset[0] = 0;
+        nodeBox(box, 0, 0, 0, t.centers, t.sizes);
+        const uint32_t L = 1 + 7 * total;
+        t.leaves[L] = nodeRange(0), t.layout[L] = n;
+    }
 }
 
-__global__ void zeroRankKernel(int32_t* rankLo) { rankLo[0] = 0; }
-
-template<class T>
-void growCopy(sphx_workspace* ws, DevBuf<T>& buf, size_t used, size_t need)
+//! a node's place in the visiting order, along its ancestors; children's order of internal nodes; level ranges
+__global__ void __launch_bounds__(256) visitKernel(LevelBase levels, InternalNodes in, TreeArrays t)
 {
-    if (need <= buf.cap) { return; }
-    DevBuf<T> nb;
-    nb.reserve(std::max(need, 2 * buf.cap));
-    if (used) SPHX_HIP(hipMemcpyAsync(nb.ptr, buf.ptr, used * sizeof(T), hipMemcpyDeviceToDevice, ws->stream));
-    SPHX_HIP(hipStreamSynchronize(ws->stream));
-    buf.release();
-    buf = nb;
+    const uint32_t node = blockIdx.x * blockDim.x + threadIdx.x, numNodes = 1 + 8 * levels.base[kMaxLevel];
+    if (node <= kMaxLevel + 1)
+    {
+        // level l + 1 holds the children of level l; the levels below the deepest start at the end
+        t.levelRange[node] = node == 0 ? 0 : TreeNodeIndex(node <= kMaxLevel ? 1 + 8 * levels.base[node - 1] : numNodes);
+    }
+    if (node >= numNodes) { return; }
+    int32_t rank = 0;
+    for (TreeNodeIndex a = TreeNodeIndex(node); a > 0; a = t.parents[(a - 1) / 8])
+        rank += t.offset[a];
+    t.rankLo[node]            = rank;
+    const TreeNodeIndex child = t.childOffsets[node];
+    t.childPush[node]         = child ? in.push[(child - 1) / 8] : 0u;
 }
 
-} // namespace
-
-namespace
+//! the tree of at most `bucket` keys: the root as its only leaf
+__global__ void rootLeafKernel(uint32_t n, DevBox box, TreeArrays t)
 {
+    if (threadIdx.x <= kMaxLevel + 1) { t.levelRange[threadIdx.x] = threadIdx.x == 0 ? 0 : 1; }
+    if (threadIdx.x > 0) { return; }
+    t.prefixes[0] = encodePlaceholder(0, 0), t.childOffsets[0] = 0, t.internalToLeaf[0] = 0;
+    t.leaves[0] = 0, t.leaves[1] = nodeRange(0);
+    t.counts[0] = n, t.layout[0] = 0, t.layout[1] = n;
+    t.parents[0] = 0, t.rankLo[0] = 0, t.childPush[0] = 0;
+    nodeBox(box, 0, 0, 0, t.centers, t.sizes);
+}
 
 /* The linked tree whose nodes are exactly the octree nodes holding more than `bucket` of the sorted
  * keys `keys` (and their children): the converged cornerstone tree of particle keys with the bucket
@@ -225,134 +357,54 @@ namespace
  * in units of keys. */
 void buildLinked(sphx_workspace* ws, const Key* keys, size_t nParticles, unsigned bucket, const DevBox& box)
 {
-    hipStream_t  st = ws->stream;
-    uint32_t     n  = uint32_t(nParticles);
-    auto&        s   = ws->tree.build;
-    size_t       cap = std::max<size_t>(4096, 16 * (nParticles / (bucket + 1) + 1));
-    s.nodeKey.reserve(cap), s.lo.reserve(cap), s.hi.reserve(cap), s.flag.reserve(cap), s.rank.reserve(cap);
-    s.level.reserve(cap);
-
-    initRoot<<<1, 1, 0, st>>>(s.nodeKey.get(), s.lo.get(), s.hi.get(), s.level.get(), n);
+    hipStream_t    st     = ws->stream;
+    const uint32_t n      = uint32_t(nParticles);
+    auto&          s      = ws->tree.build;
+    const uint32_t blocks = std::max(1u, ceilDiv(n, kPlanKeys));
+    s.planCounts.reserve(size_t(blocks) * kPlanRows + kPlanRows);
+    uint32_t* counts = s.planCounts.get();
+    uint32_t* totals = counts + size_t(blocks) * kPlanRows;
+    planCountKernel<<<blocks, kPlanWaves * kWave, 0, st>>>(keys, n, bucket, counts);
     SPHX_CHECK_LAUNCH();
-
-    std::vector<int32_t> levelStart(kMaxLevel + 3, 0);
-    uint32_t             begin = 0, end = 1;
-    unsigned             level = 0;
-    uint32_t             internalBefore = 0;
-    size_t               scanBytes      = 0;
-    while (true)
-    {
-        levelStart[level] = int32_t(begin);
-        uint32_t cnt      = end - begin;
-        classifyKernel<<<ceilDiv(cnt, 256), 256, 0, st>>>(s.lo.get(), s.hi.get(), s.flag.get(), begin, end, bucket,
-                                                           level);
-        SPHX_CHECK_LAUNCH();
-        // global inclusive scan of flags up to `end` (so ranks are tree-global)
-        SPHX_HIP(rocprim::inclusive_scan(nullptr, scanBytes, s.flag.get(), s.rank.get(), end, rocprim::plus<uint32_t>(),
-                                         st));
-        void* tmp = scratchBytes(ws, scanBytes);
-        SPHX_HIP(rocprim::inclusive_scan(tmp, scanBytes, s.flag.get(), s.rank.get(), end, rocprim::plus<uint32_t>(),
-                                         st));
-        uint32_t totalInternal = 0;
-        SPHX_HIP(hipMemcpyAsync(&totalInternal, s.rank.get() + end - 1, 4, hipMemcpyDeviceToHost, st));
-        SPHX_HIP(hipStreamSynchronize(st));
-        uint32_t numInternalHere = totalInternal - internalBefore;
-        if (numInternalHere == 0) { break; }
-
-        size_t need = size_t(end) + 8 * size_t(numInternalHere);
-        growCopy(ws, s.nodeKey, end, need), growCopy(ws, s.lo, end, need), growCopy(ws, s.hi, end, need);
-        growCopy(ws, s.flag, end, need), growCopy(ws, s.rank, end, need), growCopy(ws, s.level, end, need);
-
-        expandKernel<<<ceilDiv(size_t(cnt) * 8, 256), 256, 0, st>>>(keys, s.nodeKey.get(), s.lo.get(), s.hi.get(),
-                                                                   s.level.get(), s.flag.get(), s.rank.get(),
-                                                                   internalBefore, begin, end, level);
-        SPHX_CHECK_LAUNCH();
-        internalBefore = totalInternal;
-        begin          = end;
-        end            = uint32_t(need);
-        level++;
-    }
-    for (unsigned l = level + 1; l <= kMaxLevel + 2; ++l)
-        levelStart[l] = int32_t(end);
-
-    uint32_t numNodes    = end;
-    uint32_t numInternal = internalBefore;
-    uint32_t L           = numNodes - numInternal;
+    planScanKernel<<<kPlanRows, 256, 0, st>>>(counts, blocks, totals);
+    SPHX_CHECK_LAUNCH();
+    uint32_t perLevel[kPlanRows];
+    SPHX_HIP(hipMemcpyAsync(perLevel, totals, sizeof(perLevel), hipMemcpyDeviceToHost, st));
+    SPHX_HIP(hipStreamSynchronize(st));
+    SPHX_REQUIRE(perLevel[kMaxLevel] == 0, SPHX_ERR_ARG, "the keys of a tree must be sorted");
+    LevelBase levels;
+    levels.base[0] = 0;
+    for (unsigned l = 0; l < kMaxLevel; ++l)
+        levels.base[l + 1] = levels.base[l] + perLevel[l];
+    const uint32_t numInternal = levels.base[kMaxLevel], numNodes = 1 + 8 * numInternal, L = 1 + 7 * numInternal;
 
     Tree& t = ws->tree;
     t.prefixes.reserve(numNodes), t.childOffsets.reserve(numNodes + 1), t.internalToLeaf.reserve(numNodes);
-    t.parents.reserve(std::max<uint32_t>(1, (numNodes - 1) / 8)), t.levelRange.reserve(kMaxLevel + 2);
+    t.parents.reserve(std::max(1u, numInternal)), t.levelRange.reserve(kMaxLevel + 2);
     t.centers.reserve(3 * size_t(numNodes)), t.sizes.reserve(3 * size_t(numNodes));
     t.leaves.reserve(L + 1), t.counts.reserve(L), t.layout.reserve(L + 1);
-
-    DevBuf<int32_t>& dLevelStart = s.levelStart;
-    dLevelStart.reserve(kMaxLevel + 3);
-    SPHX_HIP(hipMemcpyAsync(dLevelStart.get(), levelStart.data(), (kMaxLevel + 3) * 4, hipMemcpyHostToDevice, st));
-
-    // leaf ranks in level order, then sort leaves by key
-    s.leafFlag.reserve(numNodes), s.leafRank.reserve(numNodes);
-    s.leafKey.reserve(L), s.leafNode.reserve(L), s.leafKeySorted.reserve(L), s.leafNodeSorted.reserve(L);
-    leafFlagKernel<<<ceilDiv(numNodes, 256), 256, 0, st>>>(s.flag.get(), s.leafFlag.get(), numNodes);
-    SPHX_CHECK_LAUNCH();
-    SPHX_HIP(rocprim::inclusive_scan(nullptr, scanBytes, s.leafFlag.get(), s.leafRank.get(), numNodes,
-                                     rocprim::plus<uint32_t>(), st));
-    SPHX_HIP(rocprim::inclusive_scan(scratchBytes(ws, scanBytes), scanBytes, s.leafFlag.get(), s.leafRank.get(),
-                                     numNodes, rocprim::plus<uint32_t>(), st));
-    exclusiveFromInclusive<<<ceilDiv(numNodes, 256), 256, 0, st>>>(s.leafRank.get(), s.leafFlag.get(),
-                                                                    s.leafRank.get(), numNodes);
-    SPHX_CHECK_LAUNCH();
-
-    linkKernel<<<ceilDiv(numNodes, 256), 256, 0, st>>>(
-        s.nodeKey.get(), s.level.get(), s.flag.get(), s.rank.get(), dLevelStart.get(), numNodes, box, t.prefixes.get(),
-        t.childOffsets.get(), t.parents.get(), t.internalToLeaf.get(), t.centers.get(), t.sizes.get(), s.leafKey.get(),
-        s.leafNode.get(), s.leafRank.get());
-    SPHX_CHECK_LAUNCH();
-
-    // leaf keys lie below 2^63 and are multiples of nodeRange(deepest level): only the bits
-    // between decide their order
-    const unsigned lowBit    = 3u * (kMaxLevel - std::min(level, kMaxLevel));
-    size_t         sortBytes = 0;
-    SPHX_HIP(rocprim::radix_sort_pairs(nullptr, sortBytes, s.leafKey.get(), s.leafKeySorted.get(), s.leafNode.get(),
-                                       s.leafNodeSorted.get(), L, lowBit, 63, st));
-    SPHX_HIP(rocprim::radix_sort_pairs(scratchBytes(ws, sortBytes), sortBytes, s.leafKey.get(), s.leafKeySorted.get(),
-                                       s.leafNode.get(), s.leafNodeSorted.get(), L, lowBit, 63, st));
-    leafFinalize<<<ceilDiv(L + 1, 256), 256, 0, st>>>(s.leafKeySorted.get(), s.leafNodeSorted.get(), s.lo.get(),
-                                                      s.hi.get(), t.leaves.get(), t.counts.get(), t.layout.get(),
-                                                      t.internalToLeaf.get(), L, n);
-    SPHX_CHECK_LAUNCH();
-
-    std::vector<int32_t> levelRange(kMaxLevel + 2);
-    for (unsigned l = 0; l <= kMaxLevel; ++l)
-        levelRange[l] = levelStart[l];
-    levelRange[kMaxLevel + 1] = int32_t(numNodes);
-    SPHX_HIP(hipMemcpyAsync(t.levelRange.get(), levelRange.data(), (kMaxLevel + 2) * 4, hipMemcpyHostToDevice, st));
-
-    // the search's visiting order: subtree leaf counts bottom-up, then ranks top-down
-    t.rankLo.reserve(numNodes), t.subtreeLeaves.reserve(numNodes), t.childPush.reserve(numNodes);
-    for (int l = int(level); l >= 0; --l)
+    t.rankLo.reserve(numNodes), t.offset.reserve(numNodes), t.childPush.reserve(numNodes);
+    const TreeArrays arrays{t.prefixes.get(), t.leaves.get(),  t.childOffsets.get(), t.parents.get(), t.internalToLeaf.get(),
+                            t.levelRange.get(), t.counts.get(), t.layout.get(),      t.childPush.get(), t.rankLo.get(),
+                            t.offset.get(),   t.centers.get(), t.sizes.get()};
+    if (numInternal == 0)
     {
-        const int32_t a = levelRange[l], b = levelRange[l + 1];
-        if (b > a)
-        {
-            subtreeLeavesKernel<<<ceilDiv(size_t(b - a), 256), 256, 0, st>>>(t.childOffsets.get(),
-                                                                          t.subtreeLeaves.get(), a, b);
-            SPHX_CHECK_LAUNCH();
-        }
+        rootLeafKernel<<<1, kWave, 0, st>>>(n, box, arrays);
+        SPHX_CHECK_LAUNCH();
     }
-    zeroRankKernel<<<1, 1, 0, st>>>(t.rankLo.get());
-    SPHX_CHECK_LAUNCH();
-    for (int l = 0; l < int(level); ++l)
+    else
     {
-        const int32_t a = levelRange[l], b = levelRange[l + 1];
-        if (b > a)
-        {
-            visitOrderKernel<<<ceilDiv(size_t(b - a), 256), 256, 0, st>>>(
-                t.childOffsets.get(), t.subtreeLeaves.get(), t.rankLo.get(), t.childPush.get(), a, b);
-            SPHX_CHECK_LAUNCH();
-        }
+        s.intKey.reserve(numInternal), s.intLo.reserve(numInternal), s.intPlace.reserve(numInternal);
+        s.dfKey.reserve(numInternal), s.dfRank.reserve(numInternal), s.intPush.reserve(numInternal);
+        const InternalNodes in{s.intKey.get(), s.intLo.get(),  s.intPlace.get(),
+                               s.dfKey.get(),  s.dfRank.get(), s.intPush.get()};
+        planEmitKernel<<<blocks, kPlanWaves * kWave, 0, st>>>(keys, n, bucket, counts, levels, in);
+        SPHX_CHECK_LAUNCH();
+        childKernel<<<ceilDiv(8 * size_t(numInternal), 256), 256, 0, st>>>(keys, n, bucket, levels, in, box, arrays);
+        SPHX_CHECK_LAUNCH();
+        visitKernel<<<ceilDiv(numNodes, 256), 256, 0, st>>>(levels, in, arrays);
+        SPHX_CHECK_LAUNCH();
     }
-    SPHX_HIP(hipStreamSynchronize(st));
-
     t.numLeafNodes     = int32_t(L);
     t.numInternalNodes = int32_t(numInternal);
     t.numNodes         = int32_t(numNodes);
@@ -365,10 +417,11 @@ void buildLinked(sphx_workspace* ws, const Key* keys, size_t nParticles, unsigne
 __global__ void nodeCountKernel(const Key* __restrict__ prefixes, const TreeNodeIndex* __restrict__ childOffsets,
                                 const TreeNodeIndex* __restrict__ internalToLeaf, const Key* __restrict__ leaves,
                                 const uint32_t* __restrict__ layout, const uint32_t* __restrict__ counts, uint32_t L,
-                                uint32_t N, uint32_t* __restrict__ nodeCnt)
+                                uint32_t N, uint32_t* __restrict__ nodeCnt, int32_t* __restrict__ leafOp)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) { return; }
+    if (i == 0) { leafOp[L] = 0, leafOp[L + 1] = 0; } // the scan's end, and no change so far
     if (childOffsets[i] == 0)
     {
         nodeCnt[i] = counts[internalToLeaf[i]];
@@ -407,7 +460,7 @@ __global__ void nodeOpKernel(const Key* __restrict__ prefixes, const TreeNodeInd
  * reference's in-place loop. Leaves store their final op by leaf index; any node left != 1 marks a change. */
 __global__ void protectKernel(const Key* __restrict__ prefixes, const TreeNodeIndex* __restrict__ parents,
                               const TreeNodeIndex* __restrict__ internalToLeaf, const int32_t* __restrict__ op,
-                              uint32_t N, int32_t* __restrict__ leafOp, uint32_t* __restrict__ changed)
+                              uint32_t N, int32_t* __restrict__ leafOp, int32_t* __restrict__ changed)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) { return; }
@@ -418,7 +471,7 @@ __global__ void protectKernel(const Key* __restrict__ prefixes, const TreeNodeIn
         while (op[a] == 0) { a = parents[(a - 1) / 8]; }
         o = decodePlaceholder(prefixes[i]) == decodePlaceholder(prefixes[a]) ? op[a] : 0;
     }
-    if (o != 1) { *changed = 1u; }
+    if (o != 1) { *changed = 1; }
     const TreeNodeIndex leaf = internalToLeaf[i];
     if (leaf >= 0) { leafOp[leaf] = o; }
 }
@@ -456,12 +509,6 @@ __global__ void leafLayoutKernel(const Key* __restrict__ leaves, uint32_t L, con
     if (s < L) { counts[s] = (s + 1 == L ? n : lowerBound(keys, lo, n, leaves[s + 1])) - lo; }
 }
 
-__global__ void setLeafOpEnd(int32_t* leafOp, uint32_t L, uint32_t* changed)
-{
-    leafOp[L] = 0;
-    *changed  = 0u;
-}
-
 } // namespace
 
 void buildTree(sphx_workspace* ws, const Key* keys, size_t nParticles, unsigned bucket, const DevBox& box)
@@ -480,29 +527,28 @@ bool updateTree(sphx_workspace* ws, const Key* keys, size_t nParticles, unsigned
     hipStream_t    st = ws->stream;
     auto&          s  = t.build;
     const uint32_t N = uint32_t(t.numNodes), L = uint32_t(t.numLeafNodes);
-    s.nodeCnt.reserve(N), s.nodeOp.reserve(N), s.leafOp.reserve(size_t(L) + 1), s.changed.reserve(1);
-    setLeafOpEnd<<<1, 1, 0, st>>>(s.leafOp.get(), L, s.changed.get());
-    SPHX_CHECK_LAUNCH();
+    s.nodeCnt.reserve(N), s.nodeOp.reserve(N), s.leafOp.reserve(size_t(L) + 2);
+    int32_t* changed = s.leafOp.get() + L + 1; // behind the leaves' ops and their end, so one read takes both
     nodeCountKernel<<<ceilDiv(N, 256), 256, 0, st>>>(t.prefixes.get(), t.childOffsets.get(), t.internalToLeaf.get(),
                                                       t.leaves.get(), t.layout.get(), t.counts.get(), L, N,
-                                                      s.nodeCnt.get());
+                                                      s.nodeCnt.get(), s.leafOp.get());
     SPHX_CHECK_LAUNCH();
     nodeOpKernel<<<ceilDiv(N, 256), 256, 0, st>>>(t.prefixes.get(), t.childOffsets.get(), t.parents.get(),
                                                    s.nodeCnt.get(), N, bucket, s.nodeOp.get());
     SPHX_CHECK_LAUNCH();
     protectKernel<<<ceilDiv(N, 256), 256, 0, st>>>(t.prefixes.get(), t.parents.get(), t.internalToLeaf.get(),
-                                                    s.nodeOp.get(), N, s.leafOp.get(), s.changed.get());
+                                                    s.nodeOp.get(), N, s.leafOp.get(), changed);
     SPHX_CHECK_LAUNCH();
     size_t bytes = 0;
     SPHX_HIP(rocprim::exclusive_scan(nullptr, bytes, s.leafOp.get(), s.leafOp.get(), 0, size_t(L) + 1,
                                      rocprim::plus<int32_t>(), st));
     SPHX_HIP(rocprim::exclusive_scan(scratchBytes(ws, bytes), bytes, s.leafOp.get(), s.leafOp.get(), 0,
                                      size_t(L) + 1, rocprim::plus<int32_t>(), st));
-    int32_t  newL    = 0;
-    uint32_t changed = 0;
-    SPHX_HIP(hipMemcpyAsync(&newL, s.leafOp.get() + L, 4, hipMemcpyDeviceToHost, st));
-    SPHX_HIP(hipMemcpyAsync(&changed, s.changed.get(), 4, hipMemcpyDeviceToHost, st));
+    int32_t read[2]; // leaves of the new array, whether any node changed
+    SPHX_HIP(hipMemcpyAsync(read, s.leafOp.get() + L, sizeof(read), hipMemcpyDeviceToHost, st));
     SPHX_HIP(hipStreamSynchronize(st));
+    const int32_t newL      = read[0];
+    const bool    unchanged = read[1] == 0;
     SPHX_REQUIRE(newL >= 1, SPHX_ERR_STATE, "tree update left no leaf");
     s.nextLeaves.reserve(size_t(newL) + 1);
     rebalanceKernel<<<ceilDiv(size_t(L) + 1, 256), 256, 0, st>>>(t.leaves.get(), s.leafOp.get(), L,
@@ -516,9 +562,8 @@ bool updateTree(sphx_workspace* ws, const Key* keys, size_t nParticles, unsigned
     leafLayoutKernel<<<ceilDiv(size_t(newL) + 1, 256), 256, 0, st>>>(t.leaves.get(), uint32_t(newL), keys, n,
                                                                      t.layout.get(), t.counts.get());
     SPHX_CHECK_LAUNCH();
-    SPHX_HIP(hipStreamSynchronize(st));
     t.numParticles = nParticles;
-    return changed == 0;
+    return unchanged;
 }
 
 } // namespace sphx
