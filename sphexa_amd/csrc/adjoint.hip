@@ -1,14 +1,21 @@
 // Adjoint (vector-Jacobian product) kernels of the std density, IAD and momentum-energy passes.
 //
-// No counterpart in the reference. Each kernel re-walks the neighbour lists of the last search
+// No counterpart in the reference. Each kernel walks the neighbour lists of the last search
 // (held fixed: they are the checkpoint of the forward), recomputes the pair terms of its forward
 // loop and accumulates the reverse-mode derivatives. A pair term of target i and neighbour j has
-// derivatives for both: the target's are summed in registers and added to its gradient once; the
-// neighbour's are written to the pair's record in a per-pair buffer (no atomics), and a second
-// kernel sums, for every particle j, the records of the pairs that have j as neighbour, in the
-// order of their pair index (AdjointPairs: target i's pairs are p = pairStart[i] + k, and a sort of
-// (j, p) keys gives each j its pairs in increasing p). Results are therefore the same bit for bit
-// from run to run. Kernel derivatives use the tabulated dW/dv interpolated like W (FP64) or are
+// derivatives for both. The target's are summed over its list (the ...VjpKernel of a pass). The
+// neighbour's are summed by the neighbour: the pair index (AdjointPairs) lists for every particle j the
+// targets that have j as neighbour, in increasing order, and the ...VjpSourceKernel walks them and
+// forms each pair again from the target's side. No pair is written to memory and no atomics are
+// used; results are the same bit for bit from run to run.
+//
+// Both walks read the other particle as one record (16-byte chunks, packed by the call for every
+// particle; positions in FP64, which form the separations of both forms). What bounds them: the
+// gathers of the records, one tag lookup of the vector cache per lane and chunk (about 0.23 ms per
+// chunk at 2M particles), and the FP64 kernel evaluations. Measured at 2M particles, mixed form, with
+// each pair's neighbour side written to memory and summed afterwards, and with this (ms):
+// density 6.2 -> 1.8, IAD 6.3 -> 2.4, momentum-energy 13.7 -> 4.4.
+// Kernel derivatives use the tabulated dW/dv interpolated like W (FP64) or are
 // evaluated like W (FP32). Launch shape and list layout as the forward loops (pairs.hpp).
 // Derivations, with r = x_i - x_j after the fold, d = |r|, v = d / h_i:
 //
@@ -33,6 +40,8 @@ namespace sphx
 namespace
 {
 
+constexpr unsigned kPackThreads = 256;
+
 //! the target's own gradient: one lane per target, so a plain read-modify-write
 template<class T>
 __device__ __forceinline__ void addOwn(void* p, uint32_t i, T v)
@@ -40,42 +49,74 @@ __device__ __forceinline__ void addOwn(void* p, uint32_t i, T v)
     static_cast<T*>(p)[i] += v;
 }
 
-/*! values per pair record: NQ rounded up to whole 16-byte words (FP32) or 32-byte sectors (FP64); records
- * move as 16-byte vector loads and stores. Measured at 2M particles: whole sectors help the FP64 records
- * (momentum 17.7 -> 16.5 ms), while the FP32 ones run faster at their 16-byte size (density 4.9 against
- * 6.0 ms padded). */
-template<class T, int NQ>
-constexpr int kPaddedNq = int((NQ * sizeof(T) + (sizeof(T) == 8 ? 31 : 15)) / (sizeof(T) == 8 ? 32 : 16) *
-                              (sizeof(T) == 8 ? 32 : 16) / sizeof(T));
-
-/*! where the pair records of a call go: the record of pair p (NQP values of T, 16-byte aligned) at
- * buf + recordOf[p] * NQP, its place among the pairs sorted by neighbour, so that the records a
- * neighbour sums are one contiguous row */
-template<class T>
-struct PairOut
+//! the targets of every particle (AdjointPairs) and the call's range of them
+struct SourceRows
 {
-    T*              buf;
-    const uint32_t* pairStart; // per searched target, from the searched range's first
-    const uint32_t* recordOf;
-    uint32_t        nbFirst;
+    const uint32_t *rowStart, *targets;
+    uint32_t        first, last, n;
+};
 
-    //! the first pair index of target i
-    __device__ __forceinline__ uint32_t firstPair(uint32_t i) const { return pairStart[i - nbFirst]; }
+//! the particle of this lane, one wave per 64 consecutive particles
+__device__ __forceinline__ uint32_t sourceParticle()
+{
+    const uint32_t g = __builtin_amdgcn_readfirstlane(xcdBlock(blockIdx.x, gridDim.x) * kVjpWaves + threadIdx.x / kWave);
+    return g * kWave + laneId();
+}
 
-    template<int NQP>
-    __device__ __forceinline__ void store(uint32_t e, const T (&v)[NQP]) const
+/*! pair(rec[i]) for every target i of the call that has j as neighbour, in increasing order: U targets and their
+ * records in flight. A slot past the row reads the next row's target (the index is padded by a quad). */
+template<int U, class Rec, class F>
+__device__ __forceinline__ void overTargets(const SourceRows& R, uint32_t j, const Rec* __restrict__ rec, F&& pair)
+{
+    constexpr int   NC    = int(sizeof(Rec) / 16);
+    const uint32_t  count = R.rowStart[j + 1] - R.rowStart[j];
+    const uint32_t* row   = R.targets + R.rowStart[j];
+    uint32_t        next[U];
+    __builtin_memcpy(next, row, sizeof(next));
+    for (uint32_t k = 0; k < count; k += U)
     {
-        static_assert(NQP * sizeof(T) % 16 == 0, "whole 16-byte words");
-        uint4* dst = reinterpret_cast<uint4*>(buf + size_t(e) * NQP);
+        uint32_t i[U];
+        uint4    w[U][NC];
 #pragma unroll
-        for (int c = 0; c < int(NQP * sizeof(T) / 16); ++c)
+        for (int u = 0; u < U; ++u)
         {
-            uint4 w;
-            __builtin_memcpy(&w, reinterpret_cast<const char*>(v) + 16 * c, 16);
-            dst[c] = w;
+            i[u]             = next[u];
+            const uint4* src = reinterpret_cast<const uint4*>(rec + i[u]);
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                w[u][c] = src[c];
+        }
+        __builtin_memcpy(next, row + min(k + U, count), sizeof(next));
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                asm volatile("" : "+v"(w[u][c].x)); // the batch's loads stay above the branches
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+            if (k + u < count && i[u] >= R.first && i[u] < R.last)
+            {
+                Rec r;
+                __builtin_memcpy(&r, w[u], sizeof(r));
+                pair(r);
+            }
         }
     }
-};
+}
+
+//! separation x_i - x_j for a neighbour j that does not know whether its targets' separations wrap: the fold, with
+//! the target's cut-off r, only where some lane's does
+template<class T>
+__device__ __forceinline__ void sourceSeparation(const DevBox& b, double r, double xi, double yi, double zi, double xj,
+                                                 double yj, double zj, T& rx, T& ry, T& rz)
+{
+    const bool wraps = (b.pbc[0] && fabs(xi - xj) > r) || (b.pbc[1] && fabs(yi - yj) > r) || (b.pbc[2] && fabs(zi - zj) > r);
+    if (ballot(wraps)) { separation<true>(b, r, xi, yi, zi, xj, yj, zj, rx, ry, rz); }
+    else { separation<false>(b, r, xi, yi, zi, xj, yj, zj, rx, ry, rz); }
+}
 
 template<class T>
 __device__ __forceinline__ T pow4Inv(T hInv)
@@ -90,11 +131,43 @@ struct DensityVjpArgs
     void *      gx, *gy, *gz, *gh;
 };
 
-constexpr int kDensityNq = 3; // neighbour-side record: gx, gy, gz
+//! a neighbour for the target's sums, and a target for the neighbour's
+template<class T>
+struct alignas(16) RecDensityVjpJ
+{
+    double x, y, z;
+    T      m;
+};
+template<class T>
+struct alignas(16) RecDensityVjpI
+{
+    double x, y, z;
+    T      h, coef; // coef: K h^-4 times the cotangent of rho
+};
+
+template<class T>
+__device__ __forceinline__ T densityVjpCoef(const PairArgs& a, const DensityVjpArgs& f, uint32_t i, T hInv)
+{
+    return ld<T>(f.gRho, i) * T(a.K) * pow4Inv(hInv);
+}
+
+template<class T>
+__global__ void __launch_bounds__(kPackThreads)
+    packDensityVjp(PairArgs a, DensityVjpArgs f, uint32_t first, uint32_t last, RecDensityVjpJ<T>* __restrict__ recJ,
+                   RecDensityVjpI<T>* __restrict__ recI, uint32_t n)
+{
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) { return; }
+    const double x = a.x[k], y = a.y[k], z = a.z[k];
+    recJ[k] = {x, y, z, ld<T>(f.m, k)};
+    if (k < first || k >= last) { return; }
+    const T h = ld<T>(f.h, k);
+    recI[k]   = {x, y, z, h, densityVjpCoef<T>(a, f, k, T(1) / h)};
+}
 
 template<class T>
 __global__ void __launch_bounds__(kVjpWaves * kWave)
-    densityStdVjpKernel(PairArgs a, DensityVjpArgs f, SincKernel<T> kern, PairOut<T> out)
+    densityStdVjpKernel(PairArgs a, DensityVjpArgs f, SincKernel<T> kern, const RecDensityVjpJ<T>* __restrict__ rec)
 {
     const Lane t = vjpTarget(a.L);
     if (!t.valid) { return; }
@@ -103,46 +176,60 @@ __global__ void __launch_bounds__(kVjpWaves * kWave)
     const T        hInv = T(1) / hi;
     const double   r2h  = 2.0 * double(hi);
     const double   xi = a.x[i], yi = a.y[i], zi = a.z[i];
-    const T        coef = ld<T>(f.gRho, i) * T(a.K) * pow4Inv(hInv);
+    const T        coef = densityVjpCoef<T>(a, f, i, hInv);
     T              rho0 = ld<T>(f.m, i), sumVdW = 0, gxi = 0, gyi = 0, gzi = 0;
-    const uint32_t ps = out.firstPair(i);
     withFold(waveNeedsFold(a.box, xi, yi, zi, r2h), [&](auto fold) {
-        // U neighbours at a time: their list entries, record places and fields load before any is used
+        // a quad of neighbours at a time: their list entries and records load before any is used
         constexpr int U = 4;
         for (unsigned k0 = 0; k0 < t.n; k0 += U)
         {
-            uint32_t j[U], e[U];
+            uint32_t j[U];
             a.L.lists.quad(t.r, k0, j);
+            RecDensityVjpJ<T> rj[U];
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                e[u] = out.recordOf[ps + min(k0 + u, t.n - 1)];
-            double xj[U], yj[U], zj[U];
-            T      mj[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                xj[u] = a.x[j[u]], yj[u] = a.y[j[u]], zj[u] = a.z[j[u]], mj[u] = ld<T>(f.m, j[u]);
+                rj[u] = rec[j[u]];
 #pragma unroll
             for (int u = 0; u < U; ++u)
             {
                 if (k0 + u >= t.n) { break; }
                 T rx, ry, rz;
-                separation<decltype(fold)::value>(a.box, r2h, xi, yi, zi, xj[u], yj[u], zj[u], rx, ry, rz);
+                separation<decltype(fold)::value>(a.box, r2h, xi, yi, zi, rj[u].x, rj[u].y, rj[u].z, rx, ry, rz);
                 T d = sqrt(rx * rx + ry * ry + rz * rz);
                 T v = d * hInv;
                 T w, dw;
                 kern.wAndDw(v, w, dw);
-                rho0 += mj[u] * w;
-                sumVdW += mj[u] * v * dw;
-                T c = d > T(0) ? coef * mj[u] * dw / d : T(0);
+                rho0 += rj[u].m * w;
+                sumVdW += rj[u].m * v * dw;
+                T c = d > T(0) ? coef * rj[u].m * dw / d : T(0);
                 gxi += c * rx, gyi += c * ry, gzi += c * rz;
-                T rec[kPaddedNq<T, kDensityNq>] = {};
-                rec[0] = -c * rx, rec[1] = -c * ry, rec[2] = -c * rz;
-                out.store(e[u], rec);
             }
         }
     });
     addOwn<T>(f.gx, i, gxi), addOwn<T>(f.gy, i, gyi), addOwn<T>(f.gz, i, gzi);
     addOwn<T>(f.gh, i, -coef * (T(3) * rho0 + sumVdW));
+}
+
+template<class T>
+__global__ void __launch_bounds__(kVjpWaves * kWave)
+    densityStdVjpSourceKernel(PairArgs a, DensityVjpArgs f, SincKernel<T> kern, SourceRows rows,
+                              const RecDensityVjpI<T>* __restrict__ rec)
+{
+    const uint32_t j = sourceParticle();
+    if (j >= rows.n) { return; }
+    const double xj = a.x[j], yj = a.y[j], zj = a.z[j];
+    const T      mj = ld<T>(f.m, j);
+    T            gx = 0, gy = 0, gz = 0;
+    overTargets<4>(rows, j, rec, [&](const RecDensityVjpI<T>& ri) {
+        T rx, ry, rz;
+        sourceSeparation(a.box, 2.0 * double(ri.h), ri.x, ri.y, ri.z, xj, yj, zj, rx, ry, rz);
+        T d = sqrt(rx * rx + ry * ry + rz * rz);
+        T w, dw;
+        kern.wAndDw(d * (T(1) / ri.h), w, dw);
+        T c = d > T(0) ? ri.coef * mj * dw / d : T(0);
+        gx -= c * rx, gy -= c * ry, gz -= c * rz;
+    });
+    addOwn<T>(f.gx, j, gx), addOwn<T>(f.gy, j, gy), addOwn<T>(f.gz, j, gz);
 }
 
 struct IadVjpArgs
@@ -151,11 +238,59 @@ struct IadVjpArgs
     void *      gx, *gy, *gz, *gh, *grho;
 };
 
-constexpr int kIadNq = 4; // neighbour-side record: gx, gy, gz, grho
+//! a neighbour for the target's sums, and a target for the neighbour's
+template<class T>
+struct alignas(16) RecIadVjpJ
+{
+    double x, y, z;
+    T      m, rho;
+};
+template<class T>
+struct alignas(16) RecIadVjpI
+{
+    double x, y, z;
+    T      h, B[9]; // B: tauBar
+};
+
+//! tauBar = -(K/h^3) C G C of target i; returns 3/h tr(G C)
+template<class T>
+__device__ __forceinline__ T iadVjpTarget(const PairArgs& a, const IadVjpArgs& f, uint32_t i, T hInv, T (&B)[9])
+{
+    T C6[6], G6[6];
+    for (int q = 0; q < 6; ++q)
+        C6[q] = ld<T>(f.c[q], i), G6[q] = ld<T>(f.g[q], i);
+    const T C[3][3] = {{C6[0], C6[1], C6[2]}, {C6[1], C6[3], C6[4]}, {C6[2], C6[4], C6[5]}};
+    const T G[3][3] = {{G6[0], G6[1] / 2, G6[2] / 2}, {G6[1] / 2, G6[3], G6[4] / 2}, {G6[2] / 2, G6[4] / 2, G6[5]}};
+    T       CG[3][3];
+    for (int p = 0; p < 3; ++p)
+        for (int q = 0; q < 3; ++q)
+            CG[p][q] = C[p][0] * G[0][q] + C[p][1] * G[1][q] + C[p][2] * G[2][q];
+    const T s = -T(a.K) * hInv * hInv * hInv;
+    for (int p = 0; p < 3; ++p)
+        for (int q = 0; q < 3; ++q)
+            B[3 * p + q] = s * (CG[p][0] * C[0][q] + CG[p][1] * C[1][q] + CG[p][2] * C[2][q]);
+    return T(3) * hInv *
+           (G6[0] * C6[0] + G6[1] * C6[1] + G6[2] * C6[2] + G6[3] * C6[3] + G6[4] * C6[4] + G6[5] * C6[5]);
+}
+
+template<class T>
+__global__ void __launch_bounds__(kPackThreads)
+    packIadVjp(PairArgs a, IadVjpArgs f, uint32_t first, uint32_t last, RecIadVjpJ<T>* __restrict__ recJ,
+               RecIadVjpI<T>* __restrict__ recI, uint32_t n)
+{
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) { return; }
+    const double x = a.x[k], y = a.y[k], z = a.z[k];
+    recJ[k] = {x, y, z, ld<T>(f.m, k), ld<T>(f.rho, k)};
+    if (k < first || k >= last) { return; }
+    RecIadVjpI<T> r{x, y, z, ld<T>(f.h, k), {}};
+    iadVjpTarget<T>(a, f, k, T(1) / r.h, r.B);
+    recI[k] = r;
+}
 
 template<class T>
 __global__ void __launch_bounds__(kVjpWaves * kWave)
-    iadStdVjpKernel(PairArgs a, IadVjpArgs f, SincKernel<T> kern, PairOut<T> out)
+    iadStdVjpKernel(PairArgs a, IadVjpArgs f, SincKernel<T> kern, const RecIadVjpJ<T>* __restrict__ rec)
 {
     const Lane t = vjpTarget(a.L);
     if (!t.valid) { return; }
@@ -165,73 +300,76 @@ __global__ void __launch_bounds__(kVjpWaves * kWave)
     const double   r2h  = 2.0 * double(hi);
     const double   xi = a.x[i], yi = a.y[i], zi = a.z[i];
 
-    T C6[6], G6[6];
-    for (int q = 0; q < 6; ++q)
-        C6[q] = ld<T>(f.c[q], i), G6[q] = ld<T>(f.g[q], i);
-    const T C[3][3] = {{C6[0], C6[1], C6[2]}, {C6[1], C6[3], C6[4]}, {C6[2], C6[4], C6[5]}};
-    const T G[3][3] = {{G6[0], G6[1] / 2, G6[2] / 2}, {G6[1] / 2, G6[3], G6[4] / 2}, {G6[2] / 2, G6[4] / 2, G6[5]}};
-    T       CG[3][3], B[3][3];
-    for (int p = 0; p < 3; ++p)
-        for (int q = 0; q < 3; ++q)
-            CG[p][q] = C[p][0] * G[0][q] + C[p][1] * G[1][q] + C[p][2] * G[2][q];
-    const T s = -T(a.K) * hInv * hInv * hInv;
-    for (int p = 0; p < 3; ++p)
-        for (int q = 0; q < 3; ++q)
-            B[p][q] = s * (CG[p][0] * C[0][q] + CG[p][1] * C[1][q] + CG[p][2] * C[2][q]);
-    T ghi = T(3) * hInv *
-            (G6[0] * C6[0] + G6[1] * C6[1] + G6[2] * C6[2] + G6[3] * C6[3] + G6[4] * C6[4] + G6[5] * C6[5]);
+    T B[9];
+    T ghi = iadVjpTarget<T>(a, f, i, hInv, B);
     T gxi = 0, gyi = 0, gzi = 0;
-
-    const uint32_t ps = out.firstPair(i);
     withFold(waveNeedsFold(a.box, xi, yi, zi, r2h), [&](auto fold) {
-        // U neighbours at a time: their list entries, record places and fields load before any is used
+        // a quad of neighbours at a time: their list entries and records load before any is used
         constexpr int U = 4;
         for (unsigned k0 = 0; k0 < t.n; k0 += U)
         {
-            uint32_t j[U], e[U];
+            uint32_t j[U];
             a.L.lists.quad(t.r, k0, j);
+            RecIadVjpJ<T> rj[U];
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                e[u] = out.recordOf[ps + min(k0 + u, t.n - 1)];
-            double xj[U], yj[U], zj[U];
-            T      mjs[U], rhojs[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                xj[u] = a.x[j[u]], yj[u] = a.y[j[u]], zj[u] = a.z[j[u]];
-                mjs[u] = ld<T>(f.m, j[u]), rhojs[u] = ld<T>(f.rho, j[u]);
-            }
+                rj[u] = rec[j[u]];
 #pragma unroll
             for (int u = 0; u < U; ++u)
             {
                 if (k0 + u >= t.n) { break; }
                 T r[3];
-                separation<decltype(fold)::value>(a.box, r2h, xi, yi, zi, xj[u], yj[u], zj[u], r[0], r[1], r[2]);
+                separation<decltype(fold)::value>(a.box, r2h, xi, yi, zi, rj[u].x, rj[u].y, rj[u].z, r[0], r[1], r[2]);
                 T d = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
                 T v = d * hInv;
                 T w, dw;
                 kern.wAndDw(v, w, dw);
-                T mj   = mjs[u];
-                T rhoj = rhojs[u];
-                T Vj   = mj / rhoj;
+                T Vj = rj[u].m / rj[u].rho;
                 T Br[3];
                 for (int p = 0; p < 3; ++p)
-                    Br[p] = B[p][0] * r[0] + B[p][1] * r[1] + B[p][2] * r[2];
+                    Br[p] = B[3 * p] * r[0] + B[3 * p + 1] * r[1] + B[3 * p + 2] * r[2];
                 T q      = r[0] * Br[0] + r[1] * Br[1] + r[2] * Br[2];
                 T radial = d > T(0) ? Vj * dw * q * hInv / d : T(0);
-                T dr[3];
-                for (int p = 0; p < 3; ++p)
-                    dr[p] = radial * r[p] + T(2) * Vj * w * Br[p];
-                gxi += dr[0], gyi += dr[1], gzi += dr[2];
+                gxi += radial * r[0] + T(2) * Vj * w * Br[0];
+                gyi += radial * r[1] + T(2) * Vj * w * Br[1];
+                gzi += radial * r[2] + T(2) * Vj * w * Br[2];
                 ghi += -Vj * dw * q * d * hInv * hInv;
-                T rec[kPaddedNq<T, kIadNq>] = {};
-                rec[0] = -dr[0], rec[1] = -dr[1], rec[2] = -dr[2], rec[3] = -mj / (rhoj * rhoj) * w * q;
-                out.store(e[u], rec);
             }
         }
     });
     addOwn<T>(f.gx, i, gxi), addOwn<T>(f.gy, i, gyi), addOwn<T>(f.gz, i, gzi);
     addOwn<T>(f.gh, i, ghi);
+}
+
+template<class T>
+__global__ void __launch_bounds__(kVjpWaves * kWave)
+    iadStdVjpSourceKernel(PairArgs a, IadVjpArgs f, SincKernel<T> kern, SourceRows rows,
+                          const RecIadVjpI<T>* __restrict__ rec)
+{
+    const uint32_t j = sourceParticle();
+    if (j >= rows.n) { return; }
+    const double xj = a.x[j], yj = a.y[j], zj = a.z[j];
+    const T      mj = ld<T>(f.m, j), rhoj = ld<T>(f.rho, j), Vj = mj / rhoj;
+    T            gx = 0, gy = 0, gz = 0, wq = 0;
+    overTargets<isMixed<T> ? 4 : 2>(rows, j, rec, [&](const RecIadVjpI<T>& ri) {
+        T r[3];
+        sourceSeparation(a.box, 2.0 * double(ri.h), ri.x, ri.y, ri.z, xj, yj, zj, r[0], r[1], r[2]);
+        const T hInv = T(1) / ri.h;
+        T       d    = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
+        T       w, dw;
+        kern.wAndDw(d * hInv, w, dw);
+        T Br[3];
+        for (int p = 0; p < 3; ++p)
+            Br[p] = ri.B[3 * p] * r[0] + ri.B[3 * p + 1] * r[1] + ri.B[3 * p + 2] * r[2];
+        T q      = r[0] * Br[0] + r[1] * Br[1] + r[2] * Br[2];
+        T radial = d > T(0) ? Vj * dw * q * hInv / d : T(0);
+        gx -= radial * r[0] + T(2) * Vj * w * Br[0];
+        gy -= radial * r[1] + T(2) * Vj * w * Br[1];
+        gz -= radial * r[2] + T(2) * Vj * w * Br[2];
+        wq += w * q;
+    });
+    addOwn<T>(f.gx, j, gx), addOwn<T>(f.gy, j, gy), addOwn<T>(f.gz, j, gz);
+    addOwn<T>(f.grho, j, -mj / (rhoj * rhoj) * wq);
 }
 
 struct MomVjpArgs
@@ -240,16 +378,6 @@ struct MomVjpArgs
     const void *gax, *gay, *gaz, *gdu;
     void *      gx, *gy, *gz, *gh, *grho, *gp, *galpha, *gC[6];
 };
-
-template<class T>
-__device__ __forceinline__ void loadC(const MomVjpArgs& f, uint32_t k, T M[3][3])
-{
-    T c11 = ld<T>(f.C[0], k), c12 = ld<T>(f.C[1], k), c13 = ld<T>(f.C[2], k);
-    T c22 = ld<T>(f.C[3], k), c23 = ld<T>(f.C[4], k), c33 = ld<T>(f.C[5], k);
-    M[0][0] = c11, M[0][1] = c12, M[0][2] = c13;
-    M[1][0] = c12, M[1][1] = c22, M[1][2] = c23;
-    M[2][0] = c13, M[2][1] = c23, M[2][2] = c33;
-}
 
 //! stored-entry cotangent of a symmetric matrix used as M r, from the matrix cotangent u r^T
 template<class T>
@@ -263,142 +391,246 @@ __device__ __forceinline__ void symOuter(const T u[3], const T r[3], T out[6])
     out[5] = u[2] * r[2];
 }
 
-// neighbour-side record: gx, gy, gz, gh, grho, gp, galpha, gC[6]
-constexpr int kMomNq = 13;
+//! what both sides of a pair need of a particle
+template<class T>
+struct MomVjpParticle
+{
+    double x, y, z;
+    T      vx, vy, vz, h, c, alpha, C[6];
+};
+//! a neighbour for the target's sums, and a target for the neighbour's
+template<class T>
+struct alignas(16) RecMomVjpJ
+{
+    MomVjpParticle<T> p;
+    T                 vol, m, prj; // vol: m / rho, prj: p / rho
+};
+template<class T>
+struct alignas(16) RecMomVjpI
+{
+    MomVjpParticle<T> p;
+    T                 vol, pro, ge, Ga[3]; // pro: p / rho^2; Ga, ge: K times the cotangents of a, -K/2 times that of du
+};
+
+template<class T>
+__device__ __forceinline__ MomVjpParticle<T> loadMomVjp(const PairArgs& a, const MomVjpArgs& f, uint32_t k)
+{
+    MomVjpParticle<T> r{a.x[k],
+                        a.y[k],
+                        a.z[k],
+                        ld<T>(f.vx, k),
+                        ld<T>(f.vy, k),
+                        ld<T>(f.vz, k),
+                        ld<T>(f.h, k),
+                        ld<T>(f.c, k),
+                        f.alpha ? ld<T>(f.alpha, k) : T(1),
+                        {}};
+    for (int q = 0; q < 6; ++q)
+        r.C[q] = ld<T>(f.C[q], k);
+    return r;
+}
+
+template<class T>
+__device__ __forceinline__ RecMomVjpJ<T> loadMomVjpJ(const PairArgs& a, const MomVjpArgs& f, uint32_t k)
+{
+    const T rho = ld<T>(f.rho, k), m = ld<T>(f.m, k);
+    return {loadMomVjp<T>(a, f, k), m / rho, m, ld<T>(f.p, k) / rho};
+}
+
+template<class T>
+__device__ __forceinline__ RecMomVjpI<T> loadMomVjpI(const PairArgs& a, const MomVjpArgs& f, uint32_t k)
+{
+    const T rho = ld<T>(f.rho, k);
+    return {loadMomVjp<T>(a, f, k),
+            ld<T>(f.m, k) / rho,
+            ld<T>(f.p, k) / (rho * rho),
+            f.gdu ? -T(a.K) * T(0.5) * ld<T>(f.gdu, k) : T(0),
+            {T(a.K) * ld<T>(f.gax, k), T(a.K) * ld<T>(f.gay, k), T(a.K) * ld<T>(f.gaz, k)}};
+}
+
+template<class T>
+__global__ void __launch_bounds__(kPackThreads)
+    packMomVjp(PairArgs a, MomVjpArgs f, uint32_t first, uint32_t last, RecMomVjpJ<T>* __restrict__ recJ,
+               RecMomVjpI<T>* __restrict__ recI, uint32_t n)
+{
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) { return; }
+    recJ[k] = loadMomVjpJ<T>(a, f, k);
+    if (k >= first && k < last) { recI[k] = loadMomVjpI<T>(a, f, k); }
+}
+
+//! C r of a symmetric matrix by its stored entries
+template<class T>
+__device__ __forceinline__ void symTimes(const T (&C)[6], const T (&r)[3], T (&out)[3])
+{
+    out[0] = C[0] * r[0] + C[1] * r[1] + C[2] * r[2];
+    out[1] = C[1] * r[0] + C[3] * r[1] + C[4] * r[2];
+    out[2] = C[2] * r[0] + C[4] * r[1] + C[5] * r[2];
+}
+
+//! reverse-mode derivatives of one pair term of target i and neighbour j; each side uses its own
+template<class T>
+struct MomPairBar
+{
+    T r[3];                // by x_i (and, negated, by x_j)
+    T hi, hj, alpha;       // by h_i, h_j, and by either alpha
+    T tAi[3], tAj[3];      // by C_i r and C_j r
+    T pro, volI, volJ, prj; // by p_i / rho_i^2, the volumes, and p_j / rho_j
+};
+
+template<class T>
+__device__ __forceinline__ MomPairBar<T> momPairBar(const SincKernel<T>& kern, const RecMomVjpI<T>& I,
+                                                    const RecMomVjpJ<T>& J, const T (&r)[3], T hiInv, T hjInv)
+{
+    const MomVjpParticle<T>&i = I.p, &j = J.p;
+    T d      = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
+    T dInv   = d > T(0) ? T(1) / d : T(0);
+    T vij[3] = {i.vx - j.vx, i.vy - j.vy, i.vz - j.vz};
+    T hiInv3 = hiInv * hiInv * hiInv, hjInv3 = hjInv * hjInv * hjInv;
+    T v1 = d * hiInv, v2 = d * hjInv;
+    T W1, dW1, W2, dW2;
+    kern.wAndDw(v1, W1, dW1);
+    kern.wAndDw(v2, W2, dW2);
+    T Wi = hiInv3 * W1, Wj = hjInv3 * W2;
+    T tAi[3], tAj[3];
+    symTimes(i.C, r, tAi);
+    symTimes(j.C, r, tAj);
+    T w    = (r[0] * vij[0] + r[1] * vij[1] + r[2] * vij[2]) * dInv;
+    T visc = 0, dvisc_dw = 0, dvisc_dalpha = 0;
+    if (w < T(0))
+    {
+        T a4         = (i.alpha + j.alpha) / T(4) * (i.c + j.c);
+        visc         = T(0.5) * (-(a4 - T(2) * w) * w);
+        dvisc_dw     = T(0.5) * (-a4 + T(4) * w);
+        dvisc_dalpha = T(0.5) * (-(i.c + j.c) / T(4) * w);
+    }
+    T aa = Wi * (J.m * I.pro + visc * I.vol);
+    T bb = J.vol * Wj * (J.prj + visc);
+    T ae = Wi * (T(2) * J.m * I.pro + visc * I.vol);
+    T be = visc * J.vol * Wj;
+
+    T aaBar = I.Ga[0] * tAi[0] + I.Ga[1] * tAi[1] + I.Ga[2] * tAi[2];
+    T bbBar = I.Ga[0] * tAj[0] + I.Ga[1] * tAj[1] + I.Ga[2] * tAj[2];
+    T aeBar = I.ge * (vij[0] * tAi[0] + vij[1] * tAi[1] + vij[2] * tAi[2]);
+    T beBar = I.ge * (vij[0] * tAj[0] + vij[1] * tAj[1] + vij[2] * tAj[2]);
+
+    MomPairBar<T> o;
+    for (int p = 0; p < 3; ++p)
+    {
+        o.tAi[p] = aa * I.Ga[p] + I.ge * ae * vij[p];
+        o.tAj[p] = bb * I.Ga[p] + I.ge * be * vij[p];
+    }
+    T fromI[3], fromJ[3];
+    symTimes(i.C, o.tAi, fromI);
+    symTimes(j.C, o.tAj, fromJ);
+
+    T WiBar = aaBar * (J.m * I.pro + visc * I.vol) + aeBar * (T(2) * J.m * I.pro + visc * I.vol);
+    T WjBar = bbBar * J.vol * (J.prj + visc) + beBar * visc * J.vol;
+    o.pro   = (aaBar + T(2) * aeBar) * Wi * J.m;
+    o.volI  = (aaBar + aeBar) * Wi * visc;
+    o.volJ  = bbBar * Wj * (J.prj + visc) + beBar * visc * Wj;
+    o.prj   = bbBar * J.vol * Wj;
+    T viscBar = (aaBar + aeBar) * Wi * I.vol + (bbBar + beBar) * J.vol * Wj;
+    T wBar    = viscBar * dvisc_dw;
+    o.alpha   = viscBar * dvisc_dalpha;
+    T dBar    = WiBar * hiInv3 * hiInv * dW1 + WjBar * hjInv3 * hjInv * dW2;
+    T radial  = (dBar - wBar * w * dInv) * dInv, along = wBar * dInv;
+    for (int p = 0; p < 3; ++p)
+        o.r[p] = fromI[p] + fromJ[p] + (radial * r[p] + along * vij[p]);
+    o.hi = -WiBar * hiInv3 * hiInv * (T(3) * W1 + v1 * dW1);
+    o.hj = -WjBar * hjInv3 * hjInv * (T(3) * W2 + v2 * dW2);
+    return o;
+}
 
 template<class T>
 __global__ void __launch_bounds__(kVjpWaves * kWave)
-    momentumStdVjpKernel(PairArgs a, MomVjpArgs f, SincKernel<T> kern, PairOut<T> out)
+    momentumStdVjpKernel(PairArgs a, MomVjpArgs f, SincKernel<T> kern, const RecMomVjpJ<T>* __restrict__ rec)
 {
     const Lane t = vjpTarget(a.L);
     if (!t.valid) { return; }
-    const uint32_t i      = t.i;
-    const T        hi     = ld<T>(f.h, i);
-    const T        hiInv  = T(1) / hi;
-    const T        hiInv3 = hiInv * hiInv * hiInv;
-    const double   r2h    = 2.0 * double(hi);
-    const double   xi = a.x[i], yi = a.y[i], zi = a.z[i];
-    const T        vxi = ld<T>(f.vx, i), vyi = ld<T>(f.vy, i), vzi = ld<T>(f.vz, i);
-    const T        roi = ld<T>(f.rho, i), pri = ld<T>(f.p, i), ci = ld<T>(f.c, i), mi = ld<T>(f.m, i);
-    const T        vol_i = mi / roi, pro_i = pri / (roi * roi);
-    const T        alpha_i = f.alpha ? ld<T>(f.alpha, i) : T(1);
-    T              Ci[3][3];
-    loadC<T>(f, i, Ci);
-    const T Ga[3] = {T(a.K) * ld<T>(f.gax, i), T(a.K) * ld<T>(f.gay, i), T(a.K) * ld<T>(f.gaz, i)};
-    const T ge    = f.gdu ? -T(a.K) * T(0.5) * ld<T>(f.gdu, i) : T(0);
+    const uint32_t      i     = t.i;
+    const RecMomVjpI<T> I     = loadMomVjpI<T>(a, f, i);
+    const T             hiInv = T(1) / I.p.h;
+    const double        r2h   = 2.0 * double(I.p.h);
 
-    T gx_i = 0, gy_i = 0, gz_i = 0, gh_i = 0, grho_i = 0, gp_i = 0, galpha_i = 0;
-    T gC_i[6] = {0, 0, 0, 0, 0, 0};
-
-    const uint32_t ps = out.firstPair(i);
-    withFold(waveNeedsFold(a.box, xi, yi, zi, r2h), [&](auto fold) {
-        uint32_t jq[4];
-        for (unsigned k = 0; k < t.n; ++k)
+    T gr[3] = {0, 0, 0}, gh = 0, galpha = 0, pro = 0, vol = 0;
+    T gC[6] = {0, 0, 0, 0, 0, 0};
+    withFold(waveNeedsFold(a.box, I.p.x, I.p.y, I.p.z, r2h), [&](auto fold) {
+        constexpr unsigned U = isMixed<T> ? 2 : 1; // records in flight
+        for (unsigned k0 = 0; k0 < t.n; k0 += 4)
         {
-            if ((k & 3u) == 0) { a.L.lists.quad(t.r, k, jq); }
-            const uint32_t j = jq[0];
-            jq[0] = jq[1], jq[1] = jq[2], jq[2] = jq[3];
-            const uint32_t e = out.recordOf[ps + k];
-            T              r[3];
-            separation<decltype(fold)::value>(a.box, r2h, xi, yi, zi, a.x[j], a.y[j], a.z[j], r[0], r[1], r[2]);
-            T d      = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
-            T vij[3] = {vxi - ld<T>(f.vx, j), vyi - ld<T>(f.vy, j), vzi - ld<T>(f.vz, j)};
-            T hjInv  = T(1) / ld<T>(f.h, j);
-            T hjInv3 = hjInv * hjInv * hjInv;
-            T v1 = d * hiInv, v2 = d * hjInv;
-            T W1, dW1, W2, dW2;
-            kern.wAndDw(v1, W1, dW1);
-            kern.wAndDw(v2, W2, dW2);
-            T Wi = hiInv3 * W1, Wj = hjInv3 * W2;
-            T Cj[3][3];
-            loadC<T>(f, j, Cj);
-            T tAi[3], tAj[3];
-            for (int p = 0; p < 3; ++p)
+            uint32_t j[4];
+            a.L.lists.quad(t.r, k0, j);
+#pragma unroll
+            for (unsigned s = 0; s < 4; s += U)
             {
-                tAi[p] = Ci[p][0] * r[0] + Ci[p][1] * r[1] + Ci[p][2] * r[2];
-                tAj[p] = Cj[p][0] * r[0] + Cj[p][1] * r[1] + Cj[p][2] * r[2];
+                if (k0 + s >= t.n) { break; }
+                RecMomVjpJ<T> rj[U];
+#pragma unroll
+                for (unsigned u = 0; u < U; ++u)
+                    rj[u] = rec[j[s + u]];
+#pragma unroll
+                for (unsigned u = 0; u < U; ++u)
+                {
+                    if (k0 + s + u >= t.n) { break; }
+                    T r[3];
+                    separation<decltype(fold)::value>(a.box, r2h, I.p.x, I.p.y, I.p.z, rj[u].p.x, rj[u].p.y, rj[u].p.z,
+                                                      r[0], r[1], r[2]);
+                    const MomPairBar<T> b = momPairBar(kern, I, rj[u], r, hiInv, T(1) / rj[u].p.h);
+                    for (int p = 0; p < 3; ++p)
+                        gr[p] += b.r[p];
+                    T c6[6];
+                    symOuter(b.tAi, r, c6);
+                    for (int q = 0; q < 6; ++q)
+                        gC[q] += c6[q];
+                    gh += b.hi, galpha += b.alpha, pro += b.pro, vol += b.volI;
+                }
             }
-            T rv      = r[0] * vij[0] + r[1] * vij[1] + r[2] * vij[2];
-            T w       = d > T(0) ? rv / d : T(0);
-            T alpha_j = f.alpha ? ld<T>(f.alpha, j) : T(1);
-            T cj      = ld<T>(f.c, j);
-            T visc = 0, dvisc_dw = 0, dvisc_dalpha = 0;
-            if (w < T(0))
-            {
-                T a4         = (alpha_i + alpha_j) / T(4) * (ci + cj);
-                visc         = T(0.5) * (-(a4 - T(2) * w) * w);
-                dvisc_dw     = T(0.5) * (-a4 + T(4) * w);
-                dvisc_dalpha = T(0.5) * (-(ci + cj) / T(4) * w);
-            }
-            T mj = ld<T>(f.m, j), roj = ld<T>(f.rho, j), pj = ld<T>(f.p, j);
-            T vol_j = mj / roj, prj = pj / roj;
-
-            T aa = Wi * (mj * pro_i + visc * vol_i);
-            T bb = vol_j * Wj * (prj + visc);
-            T ae = Wi * (T(2) * mj * pro_i + visc * vol_i);
-            T be = visc * vol_j * Wj;
-
-            T aaBar = Ga[0] * tAi[0] + Ga[1] * tAi[1] + Ga[2] * tAi[2];
-            T bbBar = Ga[0] * tAj[0] + Ga[1] * tAj[1] + Ga[2] * tAj[2];
-            T aeBar = ge * (vij[0] * tAi[0] + vij[1] * tAi[1] + vij[2] * tAi[2]);
-            T beBar = ge * (vij[0] * tAj[0] + vij[1] * tAj[1] + vij[2] * tAj[2]);
-
-            T tAiBar[3], tAjBar[3], rBar[3];
-            for (int p = 0; p < 3; ++p)
-            {
-                tAiBar[p] = aa * Ga[p] + ge * ae * vij[p];
-                tAjBar[p] = bb * Ga[p] + ge * be * vij[p];
-            }
-            for (int p = 0; p < 3; ++p)
-                rBar[p] = Ci[0][p] * tAiBar[0] + Ci[1][p] * tAiBar[1] + Ci[2][p] * tAiBar[2] + Cj[0][p] * tAjBar[0] +
-                          Cj[1][p] * tAjBar[1] + Cj[2][p] * tAjBar[2];
-            T rec[kPaddedNq<T, kMomNq>] = {};
-            T ci6[6], cj6[6];
-            symOuter(tAiBar, r, ci6);
-            symOuter(tAjBar, r, cj6);
-            for (int q = 0; q < 6; ++q)
-            {
-                gC_i[q] += ci6[q];
-                rec[7 + q] = cj6[q];
-            }
-
-            T WiBar    = aaBar * (mj * pro_i + visc * vol_i) + aeBar * (T(2) * mj * pro_i + visc * vol_i);
-            T WjBar    = bbBar * vol_j * (prj + visc) + beBar * visc * vol_j;
-            T proBar_i = (aaBar + T(2) * aeBar) * Wi * mj;
-            T viscBar  = (aaBar + aeBar) * Wi * vol_i + (bbBar + beBar) * vol_j * Wj;
-            T volBar_i = (aaBar + aeBar) * Wi * visc;
-            T volBar_j = bbBar * Wj * (prj + visc) + beBar * visc * Wj;
-            T prjBar   = bbBar * vol_j * Wj;
-
-            T wBar = viscBar * dvisc_dw;
-            galpha_i += viscBar * dvisc_dalpha;
-            rec[6] = viscBar * dvisc_dalpha;
-            if (d > T(0))
-            {
-                T dBar = WiBar * hiInv3 * hiInv * dW1 + WjBar * hjInv3 * hjInv * dW2;
-                for (int p = 0; p < 3; ++p)
-                    rBar[p] += dBar * r[p] / d + wBar * (vij[p] / d - w * r[p] / (d * d));
-            }
-            gh_i += -WiBar * hiInv3 * hiInv * (T(3) * W1 + v1 * dW1);
-            rec[3] = -WjBar * hjInv3 * hjInv * (T(3) * W2 + v2 * dW2);
-
-            gp_i += proBar_i / (roi * roi);
-            grho_i += -T(2) * proBar_i * pri / (roi * roi * roi) - volBar_i * mi / (roi * roi);
-            rec[5] = prjBar / roj;
-            rec[4] = -volBar_j * mj / (roj * roj) - prjBar * pj / (roj * roj);
-
-            gx_i += rBar[0], gy_i += rBar[1], gz_i += rBar[2];
-            rec[0] = -rBar[0], rec[1] = -rBar[1], rec[2] = -rBar[2];
-            out.store(e, rec);
         }
     });
-    addOwn<T>(f.gx, i, gx_i), addOwn<T>(f.gy, i, gy_i), addOwn<T>(f.gz, i, gz_i), addOwn<T>(f.gh, i, gh_i);
-    addOwn<T>(f.grho, i, grho_i), addOwn<T>(f.gp, i, gp_i), addOwn<T>(f.galpha, i, galpha_i);
+    const T rho = ld<T>(f.rho, i), rho2 = rho * rho;
+    addOwn<T>(f.gx, i, gr[0]), addOwn<T>(f.gy, i, gr[1]), addOwn<T>(f.gz, i, gr[2]), addOwn<T>(f.gh, i, gh);
+    addOwn<T>(f.grho, i, -T(2) * pro * ld<T>(f.p, i) / (rho2 * rho) - vol * ld<T>(f.m, i) / rho2);
+    addOwn<T>(f.gp, i, pro / rho2), addOwn<T>(f.galpha, i, galpha);
     for (int q = 0; q < 6; ++q)
-        addOwn<T>(f.gC[q], i, gC_i[q]);
+        addOwn<T>(f.gC[q], i, gC[q]);
+}
+
+template<class T>
+__global__ void __launch_bounds__(kVjpWaves * kWave)
+    momentumStdVjpSourceKernel(PairArgs a, MomVjpArgs f, SincKernel<T> kern, SourceRows rows,
+                               const RecMomVjpI<T>* __restrict__ rec)
+{
+    const uint32_t j = sourceParticle();
+    if (j >= rows.n) { return; }
+    const RecMomVjpJ<T> J     = loadMomVjpJ<T>(a, f, j);
+    const T             hjInv = T(1) / J.p.h;
+
+    T gr[3] = {0, 0, 0}, gh = 0, galpha = 0, prj = 0, vol = 0;
+    T gC[6] = {0, 0, 0, 0, 0, 0};
+    overTargets<isMixed<T> ? 2 : 1>(rows, j, rec, [&](const RecMomVjpI<T>& I) {
+        T r[3];
+        sourceSeparation(a.box, 2.0 * double(I.p.h), I.p.x, I.p.y, I.p.z, J.p.x, J.p.y, J.p.z, r[0], r[1], r[2]);
+        const MomPairBar<T> b = momPairBar(kern, I, J, r, T(1) / I.p.h, hjInv);
+        for (int p = 0; p < 3; ++p)
+            gr[p] -= b.r[p];
+        T c6[6];
+        symOuter(b.tAj, r, c6);
+        for (int q = 0; q < 6; ++q)
+            gC[q] += c6[q];
+        gh += b.hj, galpha += b.alpha, prj += b.prj, vol += b.volJ;
+    });
+    const T rho = ld<T>(f.rho, j), rho2 = rho * rho;
+    addOwn<T>(f.gx, j, gr[0]), addOwn<T>(f.gy, j, gr[1]), addOwn<T>(f.gz, j, gr[2]), addOwn<T>(f.gh, j, gh);
+    addOwn<T>(f.grho, j, -vol * J.m / rho2 - prj * ld<T>(f.p, j) / rho2);
+    addOwn<T>(f.gp, j, prj / rho), addOwn<T>(f.galpha, j, galpha);
+    for (int q = 0; q < 6; ++q)
+        addOwn<T>(f.gC[q], j, gC[q]);
 }
 
 /* ---- the pair index of the adjoints --------------------------------------------------------------- */
+
+constexpr uint32_t kTargetPad = 4; // entries behind the last row (overTargets reads whole batches)
 
 //! stored pairs of each searched target (the last entry 0, so the exclusive scan ends with the total)
 __global__ void pairCountKernel(const uint32_t* __restrict__ nc, uint32_t nbFirst, uint32_t nt, uint32_t ngmax,
@@ -409,108 +641,32 @@ __global__ void pairCountKernel(const uint32_t* __restrict__ nc, uint32_t nbFirs
     else if (t == nt) { cnt[t] = 0; }
 }
 
-//! key (j << pbits) | p of every stored pair p = pairStart[t] + k, j the neighbour in slot k of target t
-__global__ void pairKeysKernel(NeighborLists lists, const uint32_t* __restrict__ pairStart, uint32_t nt, int pbits,
-                               uint64_t* __restrict__ keys)
+//! every stored pair p = pairStart[t] + k by its neighbour j and its target
+__global__ void pairsKernel(NeighborLists lists, const uint32_t* __restrict__ pairStart, uint32_t nbFirst, uint32_t nt,
+                            uint32_t* __restrict__ js, uint32_t* __restrict__ targets)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nt) { return; }
     const uint32_t p0 = pairStart[t], n = pairStart[t + 1] - p0;
     for (uint32_t k = 0; k < n; ++k)
-    {
-        const uint32_t j = lists.entry(t, k);
-        keys[p0 + k]     = (uint64_t(j) << pbits) | uint64_t(p0 + k);
-    }
+        js[p0 + k] = lists.entry(t, k), targets[p0 + k] = nbFirst + t;
 }
 
-//! rowStart[j] = first sorted key of neighbour j (lower bound of j << pbits), j = 0 .. n
-__global__ void rowStartKernel(const uint64_t* __restrict__ sorted, uint64_t pairs, int pbits, uint32_t n,
-                               uint32_t* __restrict__ rowStart)
+//! rowStart[j] = first pair of neighbour j in the pairs sorted by neighbour, j = 0 .. n; the targets' padding
+__global__ void rowStartKernel(const uint32_t* __restrict__ js, uint64_t pairs, uint32_t n,
+                               uint32_t* __restrict__ rowStart, uint32_t* __restrict__ targets)
 {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < kTargetPad) { targets[pairs + j] = 0; }
     if (j > n) { return; }
-    const uint64_t key = uint64_t(j) << pbits;
-    uint64_t       lo = 0, hi = pairs;
+    uint64_t lo = 0, hi = pairs;
     while (lo < hi)
     {
         const uint64_t mid = (lo + hi) / 2;
-        if (sorted[mid] < key) { lo = mid + 1; }
+        if (js[mid] < j) { lo = mid + 1; }
         else { hi = mid; }
     }
     rowStart[j] = uint32_t(lo);
-}
-
-//! recordOf[p] = e for the e-th sorted key, pair p
-__global__ void recordOfKernel(const uint64_t* __restrict__ sorted, uint64_t pairs, uint64_t pmask,
-                               uint32_t* __restrict__ recordOf)
-{
-    const uint64_t e = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (e < pairs) { recordOf[sorted[e] & pmask] = uint32_t(e); }
-}
-
-template<class T, int NQ>
-struct PullOut
-{
-    T* g[NQ];
-};
-
-/*! g_q[j] += sum of field q of the records of the pairs that have j as neighbour (the contiguous row
- * rowStart[j] .. rowStart[j + 1] of the records), in increasing pair index, counting only the pairs of
- * targets [tFirst, tLast) of the call (pair indices [pairStart[tFirst], pairStart[tLast]); with allPairs
- * every pair belongs to the call and the keys are not read) */
-template<class T, int NQ>
-__global__ void __launch_bounds__(256) pullKernel(const uint64_t* __restrict__ sorted, const uint32_t* __restrict__ rowStart,
-                                                  const uint32_t* __restrict__ pairStart, uint32_t tFirst, uint32_t tLast,
-                                                  uint64_t pmask, bool allPairs, const T* __restrict__ buf,
-                                                  PullOut<T, NQ> out, uint32_t n)
-{
-    constexpr int NQP = kPaddedNq<T, NQ>;
-    constexpr int NV  = int(NQP * sizeof(T) / 16); // 16-byte words per record
-    constexpr int U   = 4;                         // records in flight per thread
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) { return; }
-    const uint64_t pLo = pairStart[tFirst], pHi = pairStart[tLast];
-    T              acc[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-        acc[q] = T(0);
-    const uint32_t e0 = rowStart[j], e1 = rowStart[j + 1];
-    for (uint32_t e = e0; e < e1; e += U)
-    {
-        bool use[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-        {
-            use[u] = e + u < e1;
-            if (!allPairs && use[u])
-            {
-                const uint64_t p = sorted[e + u] & pmask;
-                use[u]           = p >= pLo && p < pHi;
-            }
-        }
-        uint4 w[U][NV];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-        {
-            const uint4* rec = reinterpret_cast<const uint4*>(buf + size_t(use[u] ? e + u : e0) * NQP);
-#pragma unroll
-            for (int c = 0; c < NV; ++c)
-                w[u][c] = rec[c];
-        }
-        // summed in pair order; a slot past the row or outside the call's targets adds nothing
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-        {
-            T v[NQP];
-            __builtin_memcpy(v, w[u], sizeof(v));
-#pragma unroll
-            for (int q = 0; q < NQ; ++q)
-                acc[q] = use[u] ? acc[q] + v[q] : acc[q];
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-        out.g[q][j] += acc[q];
 }
 
 int bitsFor(uint64_t v)
@@ -544,62 +700,49 @@ void buildAdjointPairs(sphx_workspace* ws)
     uint32_t pairs = 0;
     SPHX_HIP(hipMemcpyAsync(&pairs, A.pairStart.get() + nt, sizeof(pairs), hipMemcpyDeviceToHost, ws->stream));
     SPHX_HIP(hipStreamSynchronize(ws->stream));
-    const int pbits = bitsFor(pairs), jbits = bitsFor(n);
-    A.keys.reserve(std::max<uint64_t>(pairs, 1));
-    A.sorted.reserve(std::max<uint64_t>(pairs, 1));
+    A.js.reserve(std::max<uint64_t>(pairs, 1)), A.jsSorted.reserve(std::max<uint64_t>(pairs, 1));
+    A.targetsByPair.reserve(std::max<uint64_t>(pairs, 1)), A.targets.reserve(uint64_t(pairs) + kTargetPad);
     A.rowStart.reserve(size_t(n) + 1);
     if (pairs > 0)
     {
-        pairKeysKernel<<<ceilDiv(nt, 256), 256, 0, ws->stream>>>(neighborLists(ws), A.pairStart.get(), nt, pbits,
-                                                                 A.keys.get());
+        pairsKernel<<<ceilDiv(nt, 256), 256, 0, ws->stream>>>(neighborLists(ws), A.pairStart.get(), ws->nbFirst, nt,
+                                                              A.js.get(), A.targetsByPair.get());
         SPHX_CHECK_LAUNCH();
-        size_t sortBytes = 0;
-        SPHX_HIP(rocprim::radix_sort_keys(nullptr, sortBytes, A.keys.get(), A.sorted.get(), size_t(pairs), 0,
-                                          pbits + jbits, ws->stream));
+        // stable: each neighbour's targets stay in increasing order
+        const unsigned bits      = unsigned(bitsFor(n));
+        size_t         sortBytes = 0;
+        SPHX_HIP(rocprim::radix_sort_pairs(nullptr, sortBytes, A.js.get(), A.jsSorted.get(), A.targetsByPair.get(),
+                                           A.targets.get(), size_t(pairs), 0, bits, ws->stream));
         void* tmp = scratchBytes(ws, sortBytes);
-        SPHX_HIP(rocprim::radix_sort_keys(tmp, sortBytes, A.keys.get(), A.sorted.get(), size_t(pairs), 0,
-                                          pbits + jbits, ws->stream));
+        SPHX_HIP(rocprim::radix_sort_pairs(tmp, sortBytes, A.js.get(), A.jsSorted.get(), A.targetsByPair.get(),
+                                           A.targets.get(), size_t(pairs), 0, bits, ws->stream));
     }
-    rowStartKernel<<<ceilDiv(size_t(n) + 1, 256), 256, 0, ws->stream>>>(A.sorted.get(), pairs, pbits, n,
-                                                                        A.rowStart.get());
+    rowStartKernel<<<ceilDiv(size_t(n) + kTargetPad, 256), 256, 0, ws->stream>>>(A.jsSorted.get(), pairs, n,
+                                                                                 A.rowStart.get(), A.targets.get());
     SPHX_CHECK_LAUNCH();
-    A.recordOf.reserve(std::max<uint64_t>(pairs, 1));
-    if (pairs > 0)
-    {
-        recordOfKernel<<<ceilDiv(pairs, 256), 256, 0, ws->stream>>>(A.sorted.get(), pairs,
-                                                                    (uint64_t(1) << pbits) - 1, A.recordOf.get());
-        SPHX_CHECK_LAUNCH();
-    }
-    A.pairs  = pairs;
-    A.pbits  = pbits;
     A.serial = ws->searchSerial;
 }
 
-//! the pair records of a call with nq values of T per pair
-template<class T>
-PairOut<T> pairOut(sphx_workspace* ws, int nq)
+//! the records of a call: one of each kind per particle
+template<class J, class I>
+std::pair<J*, I*> vjpRecords(sphx_workspace* ws)
 {
-    auto& A = ws->adj;
-    A.pairBuf.reserve(std::max<uint64_t>(A.pairs, 1) * nq * sizeof(T) + 16);
-    return PairOut<T>{reinterpret_cast<T*>(A.pairBuf.get()), A.pairStart.get(), A.recordOf.get(), ws->nbFirst};
+    static_assert(sizeof(J) % 16 == 0 && sizeof(I) % 16 == 0, "whole 16-byte chunks");
+    const size_t n = ws->tree.numParticles;
+    ws->adj.records.reserve((n + 1) * (sizeof(J) + sizeof(I)));
+    J* j = reinterpret_cast<J*>(ws->adj.records.get());
+    return {j, reinterpret_cast<I*>(j + n + 1)};
 }
 
-//! add every particle's neighbour-side sums of the call over targets [first, last) to g[0..NQ)
-template<class T, int NQ>
-void pull(sphx_workspace* ws, const PairOut<T>& po, uint32_t first, uint32_t last, void* const (&g)[NQ])
+SourceRows sourceRows(const sphx_workspace* ws, uint32_t first, uint32_t last)
 {
-    const auto&    A = ws->adj;
-    const uint32_t n = uint32_t(ws->tree.numParticles);
-    PullOut<T, NQ> out;
-    for (int q = 0; q < NQ; ++q)
-        out.g[q] = static_cast<T*>(g[q]);
-    const uint64_t pmask = (A.pbits >= 64) ? ~uint64_t(0) : ((uint64_t(1) << A.pbits) - 1);
-    if (n == 0) { return; }
-    const bool allPairs = first == ws->nbFirst && last == ws->nbLast;
-    pullKernel<T, NQ><<<ceilDiv(n, 256), 256, 0, ws->stream>>>(A.sorted.get(), A.rowStart.get(), A.pairStart.get(),
-                                                                first - ws->nbFirst, last - ws->nbFirst, pmask,
-                                                                allPairs, po.buf, out, n);
-    SPHX_CHECK_LAUNCH();
+    return {ws->adj.rowStart.get(), ws->adj.targets.get(), first, last, uint32_t(ws->tree.numParticles)};
+}
+
+//! blocks of a walk over every particle
+unsigned sourceBlocks(const sphx_workspace* ws)
+{
+    return unsigned(ceilDiv(ceilDiv(size_t(ws->tree.numParticles), kWave), kVjpWaves));
 }
 
 //! the adjoints take consecutive groups of 64 (no group view), the layout of their pair index
@@ -628,13 +771,17 @@ void densityStdVjp(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f
     unsigned       blocks = vjpBlocks(a.L);
     if (blocks == 0) { return; }
     buildAdjointPairs(ws);
-    void* const g[kDensityNq] = {out->x, out->y, out->z};
-    auto        run           = [&](auto zero) {
-        using T      = decltype(zero);
-        PairOut<T> o = pairOut<T>(ws, kPaddedNq<T, kDensityNq>);
-        densityStdVjpKernel<T><<<blocks, kVjpWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), o);
+    const uint32_t n   = uint32_t(ws->tree.numParticles);
+    auto           run = [&](auto zero) {
+        using T           = decltype(zero);
+        auto [recJ, recI] = vjpRecords<RecDensityVjpJ<T>, RecDensityVjpI<T>>(ws);
+        packDensityVjp<T><<<ceilDiv(n, kPackThreads), kPackThreads, 0, ws->stream>>>(a, d, first, last, recJ, recI, n);
         SPHX_CHECK_LAUNCH();
-        pull<T, kDensityNq>(ws, o, first, last, g);
+        densityStdVjpKernel<T><<<blocks, kVjpWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), recJ);
+        SPHX_CHECK_LAUNCH();
+        densityStdVjpSourceKernel<T><<<sourceBlocks(ws), kVjpWaves * kWave, 0, ws->stream>>>(
+            a, d, sincKernel<T>(ws), sourceRows(ws, first, last), recI);
+        SPHX_CHECK_LAUNCH();
     };
     if (p->hydro_type == SPHX_F32) { run(0.0f); }
     else { run(0.0); }
@@ -662,13 +809,17 @@ void iadStdVjp(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f, co
     unsigned blocks = vjpBlocks(a.L);
     if (blocks == 0) { return; }
     buildAdjointPairs(ws);
-    void* const g[kIadNq] = {out->x, out->y, out->z, out->rho};
-    auto        run       = [&](auto zero) {
-        using T      = decltype(zero);
-        PairOut<T> o = pairOut<T>(ws, kPaddedNq<T, kIadNq>);
-        iadStdVjpKernel<T><<<blocks, kVjpWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), o);
+    const uint32_t n   = uint32_t(ws->tree.numParticles);
+    auto           run = [&](auto zero) {
+        using T           = decltype(zero);
+        auto [recJ, recI] = vjpRecords<RecIadVjpJ<T>, RecIadVjpI<T>>(ws);
+        packIadVjp<T><<<ceilDiv(n, kPackThreads), kPackThreads, 0, ws->stream>>>(a, d, first, last, recJ, recI, n);
         SPHX_CHECK_LAUNCH();
-        pull<T, kIadNq>(ws, o, first, last, g);
+        iadStdVjpKernel<T><<<blocks, kVjpWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), recJ);
+        SPHX_CHECK_LAUNCH();
+        iadStdVjpSourceKernel<T><<<sourceBlocks(ws), kVjpWaves * kWave, 0, ws->stream>>>(
+            a, d, sincKernel<T>(ws), sourceRows(ws, first, last), recI);
+        SPHX_CHECK_LAUNCH();
     };
     if (p->hydro_type == SPHX_F32) { run(0.0f); }
     else { run(0.0); }
@@ -712,14 +863,17 @@ void momentumEnergyStdVjp(sphx_workspace* ws, const DevBox& box, const sphx_fiel
     unsigned blocks = vjpBlocks(a.L);
     if (blocks == 0) { return; }
     buildAdjointPairs(ws);
-    void* const g[kMomNq] = {out->x,   out->y,   out->z,   out->h,   out->rho, out->p,  out->alpha,
-                             out->c11, out->c12, out->c13, out->c22, out->c23, out->c33};
-    auto        run       = [&](auto zero) {
-        using T      = decltype(zero);
-        PairOut<T> o = pairOut<T>(ws, kPaddedNq<T, kMomNq>);
-        momentumStdVjpKernel<T><<<blocks, kVjpWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), o);
+    const uint32_t n   = uint32_t(ws->tree.numParticles);
+    auto           run = [&](auto zero) {
+        using T           = decltype(zero);
+        auto [recJ, recI] = vjpRecords<RecMomVjpJ<T>, RecMomVjpI<T>>(ws);
+        packMomVjp<T><<<ceilDiv(n, kPackThreads), kPackThreads, 0, ws->stream>>>(a, d, first, last, recJ, recI, n);
         SPHX_CHECK_LAUNCH();
-        pull<T, kMomNq>(ws, o, first, last, g);
+        momentumStdVjpKernel<T><<<blocks, kVjpWaves * kWave, 0, ws->stream>>>(a, d, sincKernel<T>(ws), recJ);
+        SPHX_CHECK_LAUNCH();
+        momentumStdVjpSourceKernel<T><<<sourceBlocks(ws), kVjpWaves * kWave, 0, ws->stream>>>(
+            a, d, sincKernel<T>(ws), sourceRows(ws, first, last), recI);
+        SPHX_CHECK_LAUNCH();
     };
     if (p->hydro_type == SPHX_F32) { run(0.0f); }
     else { run(0.0); }
