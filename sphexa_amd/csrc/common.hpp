@@ -254,6 +254,7 @@ struct sphx_workspace
 
     // neighbour lists of the last search, and their groups' tables when they are local lists
     sphx::DevBuf<uint32_t> nbrs, nbTable, nbTableCount, nbOwner;
+    sphx::DevBuf<char>     nbGroupStats; // the search's statistics per group
     bool                   nbLocal = false, nbOwned = false;
     uint32_t               nbTableHist[sphx::kTableBins + 1] = {}; // groups by table size; the last bin: over kTableCap
     uint32_t               nbFirst = 0, nbLast = 0, nbNgmax = 0;

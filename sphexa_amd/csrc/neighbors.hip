@@ -21,9 +21,11 @@
 // are therefore bit-identical to the CPU search; a lane shifts its entries through four registers and
 // stores 16 bytes at a time (ListWriter), in the layouts of common.hpp.
 //
-// Measured: 8M turbulence 5.2 -> 4.8 ms, 4M Evrard sphere 3.7 -> 3.2 ms against exact tests of every tile
-// (vector instructions per group 21.2k -> 16.0k). Bound by latency at four waves per SIMD (16 waves fill a CU's LDS and
-// 128 registers a wave), the vector ALU busy two thirds of the time.
+// Measured (ms; with exact tests of every tile, hits appended tile by tile and statistics by atomics of every group, then
+// this): 8M turbulence, mixed 5.2 -> 3.8, 4.1M FP64 3.1 -> 2.3, 1M 0.79 -> 0.54, 4M Evrard sphere 3.7 -> 2.8; vector
+// instructions per group 21.2k -> 13.9k. Bound by the vector ALU (three quarters of its issue slots at 8M) and, at four waves
+// per SIMD (16 waves fill a CU's LDS and 128 registers a wave), by latency: the chains of a window's plan, loads and
+// filter, and of the appends.
 #include <cstring>
 
 #include "pairs.hpp"
@@ -44,8 +46,18 @@ constexpr int kWavesPerBlock = SPHX_SEARCH_WAVES_PER_BLOCK;
 constexpr int kStackCap      = 952;  // LDS node stack per wave (bound argued at searchGroupInto)
 constexpr int kLeafCap       = 64;   // leaves per sweep of candidate leaves (one per lane)
 constexpr int kBufCap        = 128;  // LDS buffer of found leaves awaiting their turn in visiting order
-constexpr int kPerPairImage  = 64;   // image code of a leaf swept with the per-pair fold
+constexpr int kEachImage     = 64;   // image code of a leaf whose particles each have one image for the whole group
+constexpr int kPerPairImage  = 65;   // image code of a leaf swept with the per-pair fold
 constexpr int kNoShiftImage  = 13;   // image code of shift (0, 0, 0)
+
+/*! Statistics of one group's search. The groups write them side by side and groupStatsKernel reduces them: with four
+ * to six atomics per group on one cache line, which took about 10 ns each, a search could not get below 41 ns
+ * per group in any form (8M particles, mixed: 5.16 ms with them, 3.79 without; 1M: 0.75 and 0.54). */
+struct alignas(16) GroupStat
+{
+    double   hMax;
+    uint32_t stored, maxCount, fails, wide, swept, bad;
+};
 
 struct SearchArgs
 {
@@ -69,8 +81,7 @@ struct SearchArgs
     uint32_t*            table;      // local lists: the groups' tables ...
     uint32_t*            tableCount; // ... and their sizes (over kTableCap: the table did not fit)
     uint32_t*            nc;
-    unsigned long long*  stats; // [0] stored pairs, [1] max count, [2] non-converged particles, [kStatWide] wide
-                                // support, [kStatTests] candidate distance tests (swept candidates x 64 lanes)
+    GroupStat*           groupStats; // per group, reduced by groupStatsKernel
     double               minLen; // shortest box length
     // fused XMass: masses, kernel table (TabPair of h's type), normalisation, output (xm or rho)
     const void*          m;
@@ -86,21 +97,21 @@ struct SearchArgs
  * read together (tileMask) lie in 64 different banks */
 constexpr int kMatStride = 68;
 
-//! per-wave LDS: traversal stack, candidate leaves, the kept leaves' particle ranges, and the
-//! double-buffered candidate tile (with the candidates' masses for the fused XMass only)
+constexpr int kPendingTiles = 4; // swept tiles whose hits are appended together (Pending)
+
+//! per-wave LDS: traversal stack, candidate leaves, and the double-buffered candidate tile (with the
+//! candidates' masses for the fused XMass only)
 template<bool Mass, bool Local>
 struct WaveLds
 {
     int32_t  stack[kStackCap];      // pending nodes, the first in visiting order on top
     int32_t  bufNode[kBufCap];      // found leaves ...
     int32_t  bufRank[kBufCap];      // ... and their visiting-order ranks
-    uint32_t leafLo[kLeafCap];      // kept leaves: first particle
-    uint32_t leafPre[kLeafCap + 1]; // kept leaves: exclusive prefix of particle counts, then the total
-    uint8_t  leafImg[kLeafCap];     // kept leaves: periodic image code (imageShift)
     double   tx[2][kWave], ty[2][kWave], tz[2][kWave];
     uint32_t tj[2][kWave]; // particle index of each staged candidate
     double   tm[2][Mass ? kWave : 1]; // its mass (fused XMass only)
     uint8_t  self[Local ? kWave : 4]; // local lists: the target's own place in the tile
+    uint16_t pos[Local ? kPendingTiles * kWave : 2]; // table positions of the pending tiles' candidates (Pending)
     float    mx[Mass ? 1 : 4 * kMatStride]; // the tile's candidates as matrix operand (tileMask)
 };
 
@@ -203,11 +214,25 @@ struct XMassSum
 
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
-__device__ __forceinline__ double uniformD(double v)
+//! maximum over the wave (uniform result; NaN where no lane has a number): as waveOr
+__device__ __forceinline__ double waveMaxD(double v)
 {
-    uint64_t b = __double_as_longlong(v);
-    uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(b)), hi = __builtin_amdgcn_readfirstlane(uint32_t(b >> 32));
-    return __longlong_as_double((long long)((uint64_t(hi) << 32) | lo));
+    auto step = [&](auto ctrl, auto rows) {
+        const uint64_t b  = __double_as_longlong(v);
+        const uint32_t lo = uint32_t(b), hi = uint32_t(b >> 32);
+        const uint32_t l2 = __builtin_amdgcn_update_dpp(lo, lo, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+        const uint32_t h2 = __builtin_amdgcn_update_dpp(hi, hi, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+        v                 = fmax(v, __longlong_as_double((long long)((uint64_t(h2) << 32) | l2)));
+    };
+    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+    const uint64_t b = __double_as_longlong(v);
+    return __longlong_as_double((long long)((uint64_t(uint32_t(__builtin_amdgcn_readlane(uint32_t(b >> 32), 63))) << 32) |
+                                            uint32_t(__builtin_amdgcn_readlane(uint32_t(b), 63))));
 }
 
 //! bitwise or over the wave (uniform result): row steps, then the two row broadcasts, total in lane 63
@@ -260,12 +285,19 @@ __device__ __forceinline__ uint64_t exactMask(const SearchArgs& a, const Target&
     return m;
 }
 
+//! separation v from the group's centre under the nearest image (kEachImage)
+__device__ __forceinline__ double groupImage(const DevBox& b, int d, double v)
+{
+    return b.pbc[d] ? v - b.len[d] * rint(v * b.ilen[d]) : v;
+}
+
 /*! The targets of a wave as the right operand of the distance matrix (tileMask). Coordinates are relative to the
  * group's centre and scaled by a power of two so that no separation exceeds 1. */
 struct TargetMatrix
 {
     double origin[3]; // the group's centre
     double scale;
+    bool   each;      // every candidate within reach has one image for all targets (kEachImage)
     float  b[4];      // per block of 16 targets: this lane's element, -2 t (component lane / 16) or 1
     float  diff[4];   // per block: |t|^2 - r^2 of this lane's column
 };
@@ -282,17 +314,22 @@ struct TargetMatrix
  * the tiles on a lattice are tested twice. The vector ALU spends 1.5 instructions per candidate here and 11 in
  * exactMask, where this loop was two fifths of the search. */
 template<class Lds>
-__device__ __forceinline__ uint64_t tileMask(Lds& lds, int buf, uint32_t n, const TargetMatrix& g, const double shift[3],
-                                             bool& close)
+__device__ __forceinline__ uint64_t tileMask(const DevBox& box, Lds& lds, int buf, uint32_t n, const TargetMatrix& g,
+                                             const double shift[3], bool fold, bool& close)
 {
     using float4v       = float __attribute__((ext_vector_type(4)));
     const unsigned lane = laneId();
     float          p[4] = {0.0f, 0.0f, 0.0f, 4.0f}; // past the tile: far from every target
     if (lane < n)
     {
-        p[0] = float((lds.tx[buf][lane] - (g.origin[0] + shift[0])) * g.scale);
-        p[1] = float((lds.ty[buf][lane] - (g.origin[1] + shift[1])) * g.scale);
-        p[2] = float((lds.tz[buf][lane] - (g.origin[2] + shift[2])) * g.scale);
+        double q[3] = {lds.tx[buf][lane] - (g.origin[0] + shift[0]), lds.ty[buf][lane] - (g.origin[1] + shift[1]),
+                       lds.tz[buf][lane] - (g.origin[2] + shift[2])};
+        if (fold)
+        {
+            for (int d = 0; d < 3; ++d)
+                q[d] = groupImage(box, d, q[d]);
+        }
+        p[0] = float(q[0] * g.scale), p[1] = float(q[1] * g.scale), p[2] = float(q[2] * g.scale);
         p[3] = float(double(p[0]) * double(p[0]) + double(p[1]) * double(p[1]) + double(p[2]) * double(p[2]));
     }
 #pragma unroll
@@ -335,24 +372,83 @@ __device__ __forceinline__ uint64_t tileMask(Lds& lds, int buf, uint32_t n, cons
     return n < uint32_t(kWave) ? hits & ((uint64_t(1) << n) - 1) : hits;
 }
 
+/*! Hits of up to kPendingTiles swept tiles of a group with local lists, one bit per candidate, waiting to be
+ * appended together: the append runs as many rounds as the busiest lane has hits, and over four tiles that is
+ * much closer to a lane's share than tile by tile (about 130 rounds for the 91 neighbours of a lattice, against 250). The
+ * next entry's table position is read from LDS while the previous one is appended. A round spends about 25
+ * instructions of the vector ALU and, alone on its SIMD, a few hundred cycles. */
+struct Pending
+{
+    uint32_t w[2 * kPendingTiles] = {}; // word i: candidates 32 i .. of lds.pos
+    int      tiles                = 0;  // (uniform)
+
+    __device__ __forceinline__ void push(uint64_t m)
+    {
+#pragma unroll
+        for (int k = 0; k < kPendingTiles; ++k)
+        {
+            if (tiles == k) { w[2 * k] = uint32_t(m), w[2 * k + 1] = uint32_t(m >> 32); }
+        }
+        ++tiles;
+    }
+
+    template<class Writer>
+    __device__ __forceinline__ void drain(const uint16_t* pos, unsigned ngmax, unsigned& count, Writer& out)
+    {
+        uint32_t left = 0;
+#pragma unroll
+        for (int i = 0; i < 2 * kPendingTiles; ++i)
+            left += __popc(w[i]);
+        bool     have = false; // an entry is on its way from LDS
+        uint32_t e    = 0;
+        auto     put  = [&]() {
+            if (have)
+            {
+                if (count < ngmax) { out.put(count, e); }
+                ++count;
+            }
+        };
+        while (left)
+        {
+            if (w[0] == 0)
+            {
+#pragma unroll
+                for (int i = 0; i + 1 < 2 * kPendingTiles; ++i)
+                    w[i] = w[i + 1];
+                w[2 * kPendingTiles - 1] = 0;
+                pos += 32;
+            }
+            const bool     more = w[0] != 0;
+            const uint32_t c    = more ? uint32_t(__builtin_ctz(w[0])) : 0u;
+            const uint32_t next = pos[c];
+            put();
+            w[0] &= w[0] - 1;
+            left -= more ? 1u : 0u;
+            have = more, e = next;
+        }
+        put();
+        tiles = 0;
+    }
+};
+
 /* Sweep the tile's n candidates: their hits as one bit per candidate and target (a tile holds at most 64), appended
  * afterwards in candidate order, so that each list keeps the traversal order while the tests stay free of the
- * divergent append. The append runs as many rounds as the busiest lane has hits.
+ * divergent append.
  * Local lists: a target's own bit is cleared (a lane finds its place through `self`), the candidates
- * that some target keeps take the next positions of the group's table, and their entries of tj become
- * those positions. */
+ * that some target keeps take the next positions of the group's table, and the hits wait in `pending`. */
 template<bool Local, class Sink, class Lds>
 __device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, Lds& lds, const TargetMatrix& g, int buf,
-                                          uint32_t n, bool perPair, const double shift[3], unsigned& count,
-                                          ListWriter<Local>& out, Sink& sink)
+                                          uint32_t n, int code, const double shift[3], unsigned& count,
+                                          ListWriter<Local>& out, Pending& pending, double (&next)[3], Sink& sink)
 {
-    const unsigned ngmax = a.ngmax;
-    uint32_t*      tj    = lds.tj[buf];
-    uint64_t       m     = 0;
-    bool           exact = true;
+    const unsigned ngmax   = a.ngmax;
+    const bool     perPair = code >= kEachImage; // the exact tests fold each pair as the reference
+    uint32_t*      tj      = lds.tj[buf];
+    uint64_t       m       = 0;
+    bool           exact   = true;
     if constexpr (!Sink::kStageMass)
     {
-        if (!perPair) { m = tileMask(lds, buf, n, g, shift, exact); }
+        if (code != kPerPairImage) { m = tileMask(a.box, lds, buf, n, g, shift, code == kEachImage, exact); }
     }
     if (exact)
     {
@@ -360,28 +456,40 @@ __device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, 
                     : exactMask<Fold::shifted>(a, t, lds, buf, n, shift);
     }
     if (!t.active) { m = 0; }
+    // the next window's particles arrive before the stores below go out: loads and stores return in order, and
+    // waiting for them later would wait for the stores too
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        asm volatile("" : "+v"(next[d]));
     if constexpr (Local)
     {
         const unsigned lane = laneId();
         const uint32_t j    = lane < n ? tj[lane] : 0xffffffffu;
-        lds.self[lane]      = uint8_t(kWave);
-        __builtin_amdgcn_wave_barrier();
         // the wave's targets are consecutive particles from lane 0's on
         const uint32_t rel = j - (t.i - lane);
-        if (rel < uint32_t(kWave)) { lds.self[rel] = uint8_t(lane); }
-        __builtin_amdgcn_wave_barrier();
-        const uint32_t own = lds.self[lane];
-        if (own < uint32_t(kWave)) { m &= ~(uint64_t(1) << own); }
+        if (ballot(rel < uint32_t(kWave)))
+        {
+            lds.self[lane] = uint8_t(kWave);
+            __builtin_amdgcn_wave_barrier();
+            if (rel < uint32_t(kWave)) { lds.self[rel] = uint8_t(lane); }
+            __builtin_amdgcn_wave_barrier();
+            const uint32_t own = lds.self[lane];
+            if (own < uint32_t(kWave)) { m &= ~(uint64_t(1) << own); }
+        }
         const uint64_t used = uint64_t(waveOr(uint32_t(m))) | uint64_t(waveOr(uint32_t(m >> 32))) << 32;
         const uint32_t pos  = out.inTable + laneRank(used);
         if ((used >> lane) & 1u)
         {
             if (pos < kTableCap) { a.table[size_t(out.group) * kTableCap + pos] = j; }
-            tj[lane] = pos;
+            lds.pos[pending.tiles * kWave + lane] = uint16_t(pos);
         }
         out.inTable += uint32_t(__popcll(used));
+        pending.push(m);
         __builtin_amdgcn_wave_barrier();
+        if (pending.tiles == kPendingTiles) { pending.drain(lds.pos, ngmax, count, out); }
+        return;
     }
+    // (global lists: as many rounds per tile as the busiest lane has hits)
     while (m)
     {
 #pragma unroll
@@ -390,7 +498,7 @@ __device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, 
             const bool     have  = m != 0;
             const uint32_t c     = have ? uint32_t(__builtin_ctzll(m)) : 0u;
             const uint32_t j     = tj[c];
-            const bool     keep  = have && (Local || j != t.i);
+            const bool     keep  = have && j != t.i;
             const bool     store = keep && count < ngmax;
             m &= m - 1;
             if (store) { out.put(count, j); }
@@ -414,31 +522,29 @@ __device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, 
     }
 }
 
-__device__ __forceinline__ double readlaneD(double v, int q)
-{
-    uint64_t b  = __double_as_longlong(v);
-    uint32_t lo = __builtin_amdgcn_readlane(uint32_t(b), q), hi = __builtin_amdgcn_readlane(uint32_t(b >> 32), q);
-    return __longlong_as_double((long long)((uint64_t(hi) << 32) | lo));
-}
-
-//! inclusive prefix sum over the wave
+//! inclusive prefix sum over the wave: sums within rows of 16, then the rows before
 __device__ __forceinline__ uint32_t waveInclusiveSum(uint32_t v)
 {
-    const unsigned lane = laneId();
-    for (int o = 1; o < kWave; o <<= 1)
-    {
-        uint32_t w = __shfl_up(v, o, kWave);
-        v += lane >= unsigned(o) ? w : 0u;
-    }
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true); // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true); // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true); // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true); // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false); // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false); // row_bcast:31
     return v;
 }
 
 /* Periodic image of a candidate leaf relative to the group centre: the shift by whole box lengths
  * k_d = rint((c_d - g_d) / L_d), k_d in {-1, 0, 1}, coded (k_x+1) + 3 (k_y+1) + 9 (k_z+1), which
- * serves all pairs of the leaf; kPerPairImage when the group, the leaf and the reach together
- * exceed a quarter box in a periodic dimension (then the per-pair fold of the reference). */
+ * serves all pairs of the leaf, unless the group, the leaf and the reach together exceed a quarter box in a
+ * periodic dimension. Then, while the group and the reach stay within half a box (`each`), every candidate
+ * within reach of the group still has one image that serves all targets, the one nearest to the group's centre
+ * (kEachImage): a pair closer than the reach under any other would put the candidate within half a box of the centre
+ * twice. Else each pair folds by itself as in the reference (kPerPairImage), without the filter by the group's box
+ * and without the matrix tests: boxes a few smoothing lengths wide. With one image per candidate where it is
+ * possible, the search of a periodic box of 18^3 particles with 100 neighbours takes 181 us instead of 280. */
 __device__ __forceinline__ int imageCode(const DevBox& b, const double c[3], const double s[3], const double gc[3],
-                                         const double ge[3], double reach)
+                                         const double ge[3], double reach, bool each)
 {
     int  code    = 0;
     bool perPair = false;
@@ -452,7 +558,7 @@ __device__ __forceinline__ int imageCode(const DevBox& b, const double c[3], con
         }
         code = 3 * code + (k + 1);
     }
-    return perPair ? kPerPairImage : code;
+    return !perPair ? code : each ? kEachImage : kPerPairImage;
 }
 
 __device__ __forceinline__ double imageShift(const DevBox& b, int code, int d)
@@ -464,14 +570,15 @@ __device__ __forceinline__ double imageShift(const DevBox& b, int code, int d)
 //! sweep the first n candidates of tile buffer `buf`, all of image `code`
 template<bool Local, class Sink, class Lds>
 __device__ __forceinline__ void sweepBuffer(const SearchArgs& a, const Target& t, Lds& lds, const TargetMatrix& g, int buf,
-                                            uint32_t n, int code, unsigned& count, ListWriter<Local>& out, Sink& sink)
+                                            uint32_t n, int code, unsigned& count, ListWriter<Local>& out,
+                                            Pending& pending, double (&next)[3], Sink& sink)
 {
     __builtin_amdgcn_wave_barrier(); // a wave's LDS accesses complete in order
     out.swept += n;
-    const bool   perPair  = code == kPerPairImage;
+    const bool   perPair  = code >= kEachImage;
     const double shift[3] = {perPair ? 0.0 : imageShift(a.box, code, 0), perPair ? 0.0 : imageShift(a.box, code, 1),
                              perPair ? 0.0 : imageShift(a.box, code, 2)};
-    sweepTile(a, t, lds, g, buf, n, perPair, shift, count, out, sink);
+    sweepTile(a, t, lds, g, buf, n, code, shift, count, out, pending, next, sink);
     __builtin_amdgcn_wave_barrier();
 }
 
@@ -479,8 +586,8 @@ __device__ __forceinline__ void sweepBuffer(const SearchArgs& a, const Target& t
  *
  * 1. Lane q takes leaf q: its box, particle range and periodic image load in parallel. The leaf
  *    is kept if some active target's sphere reaches its box (the box is broadcast to the wave
- *    lane by lane). Kept leaves get their first particle, image and the exclusive prefix of
- *    their particle counts in LDS, in traversal order.
+ *    lane by lane). Lane r then holds the r-th kept leaf in traversal order: its first particle, image
+ *    and the exclusive prefix of the particle counts.
  * 2. Their particles are read as one stream, 64 per window (a window never spans two images).
  *    Each lane loads one particle and keeps it if it lies within reach of the group box under
  *    its leaf's image. Kept particles are appended, in stream order, to the tile being filled.
@@ -492,7 +599,7 @@ __device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t
                             const int32_t* leaves, int nLeaf,
                             const double gc[3],
                             const double ge[3], double reach, unsigned& count, ListWriter<Local>& out,
-                            Sink& sink)
+                            Pending& pending, Sink& sink)
 {
 #pragma clang fp contract(off)
     const DevBox&  b    = a.box;
@@ -513,22 +620,22 @@ __device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t
         const uint32_t leaf = uint32_t(a.internalToLeaf[node]);
         lo                  = a.layout[leaf];
         cnt                 = a.layout[leaf + 1] - lo;
-        code                = imageCode(b, c, sz, gc, ge, reach);
+        code                = imageCode(b, c, sz, gc, ge, reach, g.each);
     }
     uint64_t keepMask = 0;
     {
+        // each leaf's box, its centre moved to its image if it has one for the whole group, goes to the idle
+        // tile buffers and is read back as an LDS broadcast
         const double p[3] = {t.x, t.y, t.z};
-        if (!ballot(code == kPerPairImage))
+        if (int(lane) < nLeaf)
         {
-            // every leaf has one image for the whole group: its box, centre moved to that image,
-            // goes to the idle tile buffers and is read back as an LDS broadcast per leaf
-            if (int(lane) < nLeaf)
-            {
-                lds.tx[0][lane] = c[0] - imageShift(b, code, 0), lds.tx[1][lane] = sz[0];
-                lds.ty[0][lane] = c[1] - imageShift(b, code, 1), lds.ty[1][lane] = sz[1];
-                lds.tz[0][lane] = c[2] - imageShift(b, code, 2), lds.tz[1][lane] = sz[2];
-            }
-            __builtin_amdgcn_wave_barrier();
+            const int one      = code < kEachImage ? code : kNoShiftImage;
+            lds.tx[0][lane] = c[0] - imageShift(b, one, 0), lds.tx[1][lane] = sz[0];
+            lds.ty[0][lane] = c[1] - imageShift(b, one, 1), lds.ty[1][lane] = sz[1];
+            lds.tz[0][lane] = c[2] - imageShift(b, one, 2), lds.tz[1][lane] = sz[2];
+        }
+        __builtin_amdgcn_wave_barrier();
+        auto test = [&](auto fold) {
             for (int q = 0; q < nLeaf; ++q)
             {
                 const double cq[3] = {lds.tx[0][q], lds.ty[0][q], lds.tz[0][q]};
@@ -536,78 +643,65 @@ __device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t
                 double       d2    = 0.0;
                 for (int d = 0; d < 3; ++d)
                 {
-                    double v = fabs(cq[d] - p[d]) - sq[d];
-                    v        = v > 0.0 ? v : 0.0;
-                    d2 += v * v;
-                }
-                keepMask |= ballot(t.active && d2 < t.reach2) ? (uint64_t(1) << q) : uint64_t(0);
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-        else
-        {
-            for (int q = 0; q < nLeaf; ++q)
-            {
-                double d2 = 0.0;
-                for (int d = 0; d < 3; ++d)
-                {
-                    double v = readlaneD(c[d], q) - p[d];
-                    if (b.pbc[d]) { v = v - b.len[d] * rint(v * b.ilen[d]); }
-                    v = fabs(v) - readlaneD(sz[d], q);
+                    double v = cq[d] - p[d];
+                    if constexpr (decltype(fold)::value) { v = groupImage(b, d, v); }
+                    v = fabs(v) - sq[d];
                     v = v > 0.0 ? v : 0.0;
                     d2 += v * v;
                 }
                 keepMask |= ballot(t.active && d2 < t.reach2) ? (uint64_t(1) << q) : uint64_t(0);
             }
-        }
+        };
+        if (ballot(code >= kEachImage)) { test(std::true_type{}); }
+        else { test(std::false_type{}); }
+        __builtin_amdgcn_wave_barrier();
     }
-    const bool     kept   = (keepMask >> lane) & 1u;
-    const int      nKept  = __popcll(keepMask);
-    const uint32_t incl   = waveInclusiveSum(kept ? cnt : 0u);
-    if (kept)
-    {
-        const unsigned r = laneRank(keepMask);
-        lds.leafLo[r]    = lo;
-        lds.leafImg[r]   = uint8_t(code);
-        lds.leafPre[r]   = incl - cnt;
-    }
-    const uint32_t total = uniform(__shfl(incl, kWave - 1, kWave));
-    if (lane == 0) { lds.leafPre[nKept] = total; }
-    __builtin_amdgcn_wave_barrier();
+    if (keepMask == 0) { return; }
+    // lane r takes the r-th kept leaf (the others' lanes follow, empty)
+    const uint64_t kept  = uint64_t(1) << lane & keepMask;
+    const int      nKept = __popcll(keepMask);
+    const unsigned r     = laneRank(keepMask);
+    const int      to    = 4 * int(kept ? r : unsigned(nKept) + lane - r);
+    lo                   = __builtin_amdgcn_ds_permute(to, int(lo));
+    code                 = __builtin_amdgcn_ds_permute(to, code);
+    cnt                  = __builtin_amdgcn_ds_permute(to, int(kept ? cnt : 0u));
+    const uint32_t incl  = waveInclusiveSum(cnt);
+    const uint32_t pre   = incl - cnt; // stream position of the leaf's first particle
+    const uint32_t off   = lo - pre;
+    const bool     leaf  = int(lane) < nKept;
+    const uint32_t total = __builtin_amdgcn_readlane(incl, kWave - 1);
     if (total == 0) { return; }
 
     // 2. the kept leaves' particles as one stream of windows, compacted into full tiles
     const double reach2 = reach * reach;
     uint32_t     S      = 0;  // stream position of the current window
-    int          qs     = 0;  // kept leaf holding S
     uint32_t     runEnd = 0;  // stream end of the run of leaves with the current window's image
     int          runImg = kNoShiftImage;
     // plan the window at S: its end, and this lane's particle (valid, index)
     auto plan = [&](uint32_t& E, bool& valid, uint32_t& idx) {
-        while (qs + 1 < nKept && lds.leafPre[qs + 1] <= S) { qs++; }
+        int q = __popcll(ballot(leaf && pre <= S)) - 1; // kept leaf holding S
         if (S >= runEnd)
         {
-            runImg = lds.leafImg[qs];
-            int q  = qs + 1;
-            while (q < nKept && lds.leafImg[q] == runImg) { q++; }
-            runEnd = lds.leafPre[q];
+            runImg              = __builtin_amdgcn_readlane(code, q);
+            const uint64_t past = ballot(leaf && int(lane) > q && code != runImg);
+            runEnd              = past ? uint32_t(__builtin_amdgcn_readlane(pre, __builtin_ctzll(past))) : total;
         }
         E                = min(S + uint32_t(kWave), runEnd);
         const uint32_t p = S + lane;
         valid            = p < E;
-        idx              = 0;
-        if (valid)
+        idx              = p + uint32_t(__builtin_amdgcn_readlane(off, q));
+        while (++q < nKept)
         {
-            int q = qs;
-            while (q + 1 < nKept && lds.leafPre[q + 1] <= p) { q++; }
-            idx = lds.leafLo[q] + (p - lds.leafPre[q]);
+            const uint32_t start = __builtin_amdgcn_readlane(pre, q), o = __builtin_amdgcn_readlane(off, q);
+            if (start >= E) { break; }
+            idx = p >= start ? p + o : idx;
         }
     };
-    double   px = 0, py = 0, pz = 0, pm = 0;
+    double   pn[3] = {0, 0, 0}, pm = 0;
     auto     load = [&](bool valid, uint32_t idx) {
         if (valid)
         {
-            px = a.x[idx], py = a.y[idx], pz = a.z[idx];
+            pn[0] = a.x[idx], pn[1] = a.y[idx], pn[2] = a.z[idx];
             if constexpr (Sink::kStageMass) { pm = double(static_cast<const decltype(sink.hInv)*>(a.m)[idx]); }
         }
     };
@@ -631,12 +725,18 @@ __device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t
             bool keep = valid;
             if (keep && tileImg != kPerPairImage)
             {
-                const double q[3] = {px - imageShift(b, tileImg, 0), py - imageShift(b, tileImg, 1),
-                                     pz - imageShift(b, tileImg, 2)};
-                double       d2   = 0.0;
+                const int one  = tileImg < kEachImage ? tileImg : kNoShiftImage;
+                double    q[3] = {pn[0] - imageShift(b, one, 0) - gc[0], pn[1] - imageShift(b, one, 1) - gc[1],
+                                  pn[2] - imageShift(b, one, 2) - gc[2]};
+                double    d2   = 0.0;
+                if (tileImg == kEachImage)
+                {
+                    for (int d = 0; d < 3; ++d)
+                        q[d] = groupImage(b, d, q[d]);
+                }
                 for (int d = 0; d < 3; ++d)
                 {
-                    double v = fabs(q[d] - gc[d]) - ge[d];
+                    double v = fabs(q[d]) - ge[d];
                     v        = v > 0.0 ? v : 0.0;
                     d2 += v * v;
                 }
@@ -648,7 +748,7 @@ __device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t
                 const uint32_t slot = acc + laneRank(kmask);
                 const int      bb   = slot < uint32_t(kWave) ? cur : cur ^ 1;
                 const uint32_t sl   = slot < uint32_t(kWave) ? slot : slot - kWave;
-                lds.tx[bb][sl] = px, lds.ty[bb][sl] = py, lds.tz[bb][sl] = pz;
+                lds.tx[bb][sl] = pn[0], lds.ty[bb][sl] = pn[1], lds.tz[bb][sl] = pn[2];
                 lds.tj[bb][sl] = idx;
                 if constexpr (Sink::kStageMass) { lds.tm[bb][sl] = pm; }
             }
@@ -666,52 +766,42 @@ __device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t
         if (acc >= uint32_t(kWave) || (acc > 0 && (!more || runImg != tileImg)))
         {
             const uint32_t n = min(acc, uint32_t(kWave));
-            sweepBuffer(a, t, lds, g, cur, n, tileImg, count, out, sink);
+            sweepBuffer(a, t, lds, g, cur, n, tileImg, count, out, pending, pn, sink);
             acc -= n, cur ^= 1;
         }
         if (!more && acc == 0) { break; }
     }
 }
 
-//! Sort the first n entries of the found-leaf buffer by rank (bitonic network over the next
-//! power of two, the padding ranked last; ranks of distinct leaves are distinct)
+//! Sort the first n <= 128 entries of the found-leaf buffer by rank: an entry's place is the number of smaller
+//! ranks (the ranks of distinct leaves are distinct)
 template<class Lds>
 __device__ __forceinline__ void sortFoundLeaves(Lds& lds, int n)
 {
-    const unsigned lane = laneId();
+    static_assert(kBufCap == 2 * kWave, "two entries per lane");
+    const int  lane = int(laneId());
+    const bool on0 = lane < n, on1 = lane + kWave < n;
+    const int  r0 = on0 ? lds.bufRank[lane] : INT32_MAX, r1 = on1 ? lds.bufRank[lane + kWave] : INT32_MAX;
     // leaves found in one pop arrive in order: often there is nothing to sort
-    bool inversion = false;
-    for (int q = int(lane); q + 1 < n; q += kWave)
-        inversion = inversion || lds.bufRank[q] > lds.bufRank[q + 1];
+    const bool inversion = (lane + 1 < n && r0 > lds.bufRank[lane + 1]) ||
+                           (lane + kWave + 1 < n && r1 > lds.bufRank[lane + kWave + 1]);
     if (!ballot(inversion)) { return; }
-    int size = 2;
-    while (size < n) { size <<= 1; }
-    for (int q = n + int(lane); q < size; q += kWave)
+    const int node0 = on0 ? lds.bufNode[lane] : 0, node1 = on1 ? lds.bufNode[lane + kWave] : 0;
+    int       at0 = 0, at1 = 0;
+    for (int q = 0; q < min(n, kWave); ++q)
     {
-        lds.bufRank[q] = INT32_MAX;
-        lds.bufNode[q] = -1;
+        const int r = __builtin_amdgcn_readlane(r0, q);
+        at0 += r < r0 ? 1 : 0, at1 += r < r1 ? 1 : 0;
+    }
+    for (int q = kWave; q < n; ++q)
+    {
+        const int r = __builtin_amdgcn_readlane(r1, q - kWave);
+        at0 += r < r0 ? 1 : 0, at1 += r < r1 ? 1 : 0;
     }
     __builtin_amdgcn_wave_barrier();
-    for (int k = 2; k <= size; k <<= 1)
-    {
-        for (int j = k >> 1; j > 0; j >>= 1)
-        {
-            for (int p = int(lane); p < (size >> 1); p += kWave)
-            {
-                const int  i  = 2 * j * (p / j) + (p % j);
-                const int  l  = i + j;
-                const bool up = (i & k) == 0;
-                const int  ri = lds.bufRank[i], rl = lds.bufRank[l];
-                if ((ri > rl) == up)
-                {
-                    const int ni = lds.bufNode[i], nl = lds.bufNode[l];
-                    lds.bufRank[i] = rl, lds.bufRank[l] = ri;
-                    lds.bufNode[i] = nl, lds.bufNode[l] = ni;
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
+    if (on0) { lds.bufRank[at0] = r0, lds.bufNode[at0] = node0; }
+    if (on1) { lds.bufRank[at1] = r1, lds.bufNode[at1] = node1; }
+    __builtin_amdgcn_wave_barrier();
 }
 
 /* Collect all leaves whose (periodic) distance to the active targets' bounding box is below the
@@ -742,20 +832,26 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
     const unsigned lane = laneId();
     const DevBox&  b    = a.box;
 
-    double gmin[3], gmax[3], gc[3], ge[3];
+    double gc[3], ge[3];
     double p[3] = {t.x, t.y, t.z};
     for (int d = 0; d < 3; ++d)
     {
-        gmin[d] = waveMin(t.active ? p[d] : INFINITY);
-        gmax[d] = waveMax(t.active ? p[d] : -INFINITY);
-        gc[d]   = 0.5 * (gmin[d] + gmax[d]);
-        ge[d]   = 0.5 * (gmax[d] - gmin[d]);
+        const double gmin = -waveMaxD(t.active ? -p[d] : -INFINITY), gmax = waveMaxD(t.active ? p[d] : -INFINITY);
+        gc[d]             = 0.5 * (gmin + gmax);
+        ge[d]             = 0.5 * (gmax - gmin);
     }
-    double reach  = waveMax(t.active ? radius : 0.0) + a.slack;
+    double reach  = waveMaxD(t.active ? radius : 0.0) + a.slack;
     double reach2 = reach * reach;
     if (ballot(t.active) == 0) { return 0; }
 
     TargetMatrix g;
+    g.each = true;
+    for (int d = 0; d < 3; ++d)
+    {
+        // (below 2^-20 of the box the rounding of a coordinate would count in the matrix tests)
+        const double w = ge[d] + reach;
+        if (b.pbc[d]) { g.each = g.each && w * (1.0 + 1e-6) <= 0.5 * b.len[d] && w >= 0x1p-20 * b.len[d]; }
+    }
     if constexpr (!Sink::kStageMass)
     {
         // every kept candidate and every target within 1 of the centre after scaling, and every separation
@@ -781,6 +877,7 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
     }
 
     unsigned count = 0;
+    Pending  pending;
     int      top   = 1;
     int      nBuf  = 0;
     if (lane == 0) { lds.stack[0] = 0; }
@@ -797,7 +894,8 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
         }
         for (int done = 0; done < final; done += kLeafCap)
         {
-            flushLeaves(a, t, lds, g, lds.bufNode + done, min(kLeafCap, final - done), gc, ge, reach, count, out, sink);
+            flushLeaves(a, t, lds, g, lds.bufNode + done, min(kLeafCap, final - done), gc, ge, reach, count, out,
+                        pending, sink);
         }
         // move the rest to the front
         const int rest = nBuf - final;
@@ -883,6 +981,10 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
         }
         if (sweep) { sweepFound(limit); }
     }
+    if constexpr (Local)
+    {
+        if (pending.tiles) { pending.drain(lds.pos, a.ngmax, count, out); }
+    }
     return count;
 }
 
@@ -944,7 +1046,6 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     bool     oversized;
     groupRange(a.groups, g, base, end, oversized);
     base = uniform(base), end = uniform(end);
-    if (oversized && lane == 0) { atomicAdd(&a.stats[kStatBadGroups], 1ull); }
     WaveLds<XMass, Local>& lds = ldsMem[wid];
 
     Target t;
@@ -1016,40 +1117,74 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
         }
     }
 
-    unsigned stored = valid ? min(ncSph - 1, a.ngmax) : 0;
-    unsigned sum    = waveSum(stored);
-    unsigned mx     = waveMax(valid ? ncSph : 0u);
-    unsigned fails  = __popcll(ballot(valid && updates >= 10));
+    const unsigned stored = waveSum(valid ? min(ncSph - 1, a.ngmax) : 0u);
+    const unsigned mx     = waveMax(valid ? ncSph : 0u);
+    const unsigned fails  = __popcll(ballot(valid && updates >= 10));
     // support 2h reaching half a box length: the FP32 pair loops then take exact separations
-    unsigned wide = __popcll(ballot(valid && 4.0 * double(hi) * (1.0 + 1e-6) >= a.minLen));
-    // largest h: sets the fixed-point period of the FP32 pair loops (positive doubles order as
-    // their bit patterns)
-    double hMax = waveMax(valid ? double(hi) : 0.0);
+    const unsigned wide = __popcll(ballot(valid && 4.0 * double(hi) * (1.0 + 1e-6) >= a.minLen));
+    // largest h: sets the fixed-point period of the FP32 pair loops
+    const double hMax = waveMaxD(valid ? double(hi) : 0.0);
     if (lane == 0)
     {
-        atomicMax(&a.stats[kStatHMax], (unsigned long long)__double_as_longlong(hMax));
-        atomicAdd(&a.stats[0], (unsigned long long)sum);
-        atomicMax(&a.stats[1], (unsigned long long)mx);
-        if (fails) { atomicAdd(&a.stats[2], (unsigned long long)fails); }
-        if (wide) { atomicAdd(&a.stats[kStatWide], (unsigned long long)wide); }
-        atomicAdd(&a.stats[kStatTests], (unsigned long long)out.swept * kWave);
+        a.groupStats[g] = {hMax, stored, mx, fails, wide, out.swept, oversized ? 1u : 0u};
         if constexpr (Local) { a.tableCount[g] = out.inTable; }
     }
 }
 
-//! histogram of the groups' table sizes: bin s / kTableBin, the last one for tables that did not fit
-__global__ void __launch_bounds__(256) tableHistKernel(const uint32_t* __restrict__ tableCount, uint32_t blocks,
-                                                       uint32_t* hist)
+/*! Statistics of the search from its groups': stats[0] stored pairs, [1] max count, [2] non-converged particles,
+ * [kStatWide] wide support, [kStatTests] candidate distance tests (swept candidates x 64 lanes),
+ * [kStatBadGroups], [kStatHMax]; with tableCount also the histogram of the groups' table sizes: bin s / kTableBin, the
+ * last one for tables that did not fit. One block's atomics per slot. */
+__global__ void __launch_bounds__(256)
+    groupStatsKernel(const GroupStat* __restrict__ groupStats, const uint32_t* __restrict__ tableCount, uint32_t groups,
+                     unsigned long long* __restrict__ stats)
 {
-    __shared__ uint32_t part[kTableBins + 1];
+    __shared__ uint32_t           part[kTableBins + 1];
+    __shared__ unsigned long long sum[6], hBits;
+    __shared__ uint32_t           most;
     if (threadIdx.x <= kTableBins) { part[threadIdx.x] = 0; }
+    if (threadIdx.x < 6) { sum[threadIdx.x] = 0; }
+    if (threadIdx.x == 0) { hBits = 0, most = 0; }
     __syncthreads();
-    for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < blocks; g += gridDim.x * blockDim.x)
+    unsigned long long v[5] = {};
+    double             hMax = 0.0;
+    uint32_t           mx   = 0;
+    for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < groups; g += gridDim.x * blockDim.x)
     {
-        const uint32_t s = tableCount[g];
-        atomicAdd(&part[s > kTableCap ? kTableBins : (s == 0 ? 0 : (s - 1) / kTableBin)], 1u);
+        const GroupStat q = groupStats[g];
+        v[0] += q.stored, v[1] += q.fails, v[2] += q.wide, v[3] += q.swept, v[4] += q.bad;
+        mx   = max(mx, q.maxCount);
+        hMax = fmax(hMax, q.hMax);
+        if (tableCount != nullptr)
+        {
+            const uint32_t s = tableCount[g];
+            atomicAdd(&part[s > kTableCap ? kTableBins : (s == 0 ? 0 : (s - 1) / kTableBin)], 1u);
+        }
+    }
+    for (int k = 0; k < 5; ++k)
+        v[k] = waveSum(v[k]);
+    mx   = waveMax(mx);
+    hMax = waveMaxD(hMax);
+    if (laneId() == 0)
+    {
+        for (int k = 0; k < 5; ++k)
+            atomicAdd(&sum[k], v[k]);
+        atomicMax(&most, mx);
+        // positive doubles order as their bit patterns
+        atomicMax(&hBits, (unsigned long long)__double_as_longlong(hMax));
     }
     __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        atomicMax(&stats[kStatHMax], hBits);
+        atomicAdd(&stats[0], sum[0]);
+        atomicMax(&stats[1], (unsigned long long)most);
+        if (sum[1]) { atomicAdd(&stats[2], sum[1]); }
+        if (sum[2]) { atomicAdd(&stats[kStatWide], sum[2]); }
+        atomicAdd(&stats[kStatTests], sum[3] * kWave);
+        if (sum[4]) { atomicAdd(&stats[kStatBadGroups], sum[4]); }
+    }
+    uint32_t* hist = reinterpret_cast<uint32_t*>(stats + kStatHist);
     if (threadIdx.x <= kTableBins && part[threadIdx.x]) { atomicAdd(&hist[threadIdx.x], part[threadIdx.x]); }
 }
 
@@ -1123,7 +1258,8 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     a.table      = ws->nbTable.get();
     a.tableCount = ws->nbTableCount.get();
     a.nc         = f->nc;
-    a.stats    = reinterpret_cast<unsigned long long*>(ws->counters.get());
+    ws->nbGroupStats.reserve(std::max<size_t>(1, groups) * sizeof(GroupStat));
+    a.groupStats = reinterpret_cast<GroupStat*>(ws->nbGroupStats.get());
     a.minLen   = std::min(box.len[0], std::min(box.len[1], box.len[2]));
     a.m = nullptr, a.wh = nullptr, a.sincN = 0, a.sincInt = -1, a.K = 0, a.xmOut = nullptr, a.toRho = 0;
     const bool f32 = p->hydro_type == SPHX_F32;
@@ -1168,13 +1304,10 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
                 else searchKernel<double, true, false><<<grid, block, 0, ws->stream>>>(a, static_cast<double*>(f->h));
             }
             SPHX_CHECK_LAUNCH();
-            if (local)
-            {
-                tableHistKernel<<<std::min(ceilDiv(groups, 256), 64u), 256, 0, ws->stream>>>(
-                    ws->nbTableCount.get(), groups,
-                    reinterpret_cast<uint32_t*>(ws->counters.get()) + 2 * kStatHist);
-                SPHX_CHECK_LAUNCH();
-            }
+            groupStatsKernel<<<std::min(ceilDiv(groups, 256), 64u), 256, 0, ws->stream>>>(
+                a.groupStats, local ? ws->nbTableCount.get() : nullptr, groups,
+                reinterpret_cast<unsigned long long*>(ws->counters.get()));
+            SPHX_CHECK_LAUNCH();
         }
         SPHX_HIP(hipMemcpyAsync(stats, ws->counters.get(), sizeof(stats), hipMemcpyDeviceToHost, ws->stream));
         SPHX_HIP(hipStreamSynchronize(ws->stream));
