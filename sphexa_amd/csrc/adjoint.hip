@@ -633,11 +633,11 @@ __global__ void __launch_bounds__(kVjpWaves * kWave)
 constexpr uint32_t kTargetPad = 4; // entries behind the last row (overTargets reads whole batches)
 
 //! stored pairs of each searched target (the last entry 0, so the exclusive scan ends with the total)
-__global__ void pairCountKernel(const uint32_t* __restrict__ nc, uint32_t nbFirst, uint32_t nt, uint32_t ngmax,
+__global__ void pairCountKernel(NeighborLists lists, const uint32_t* __restrict__ nc, uint32_t nbFirst, uint32_t nt,
                                 uint32_t* __restrict__ cnt)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < nt) { cnt[t] = min(nc[nbFirst + t] - 1u, ngmax); }
+    if (t < nt) { cnt[t] = lists.searched(t) ? min(nc[nbFirst + t] - 1u, lists.ngmax) : 0u; }
     else if (t == nt) { cnt[t] = 0; }
 }
 
@@ -693,7 +693,8 @@ void buildAdjointPairs(sphx_workspace* ws)
     const size_t cntBytes = ((size_t(nt) + 1) * sizeof(uint32_t) + 255) & ~size_t(255);
     char*        base     = static_cast<char*>(scratchBytes(ws, cntBytes + tmpBytes));
     uint32_t*    cnt      = reinterpret_cast<uint32_t*>(base);
-    pairCountKernel<<<ceilDiv(size_t(nt) + 1, 256), 256, 0, ws->stream>>>(ws->nbNc, ws->nbFirst, nt, ws->nbNgmax, cnt);
+    pairCountKernel<<<ceilDiv(size_t(nt) + 1, 256), 256, 0, ws->stream>>>(neighborLists(ws), ws->nbNc, ws->nbFirst, nt,
+                                                                          cnt);
     SPHX_CHECK_LAUNCH();
     SPHX_HIP(rocprim::exclusive_scan(base + cntBytes, tmpBytes, cnt, A.pairStart.get(), 0u, size_t(nt) + 1,
                                      rocprim::plus<uint32_t>(), ws->stream));

@@ -73,6 +73,9 @@ struct NeighborLists
     //! group whose table the r-th target's list refers to
     __device__ __forceinline__ uint32_t group(uint32_t r) const { return owner ? owner[r] : r / kGroup; }
 
+    //! the search took the r-th target (a group view may leave targets out: they have no list)
+    __device__ __forceinline__ bool searched(uint32_t r) const { return owner == nullptr || owner[r] != kNoGroup; }
+
     //! particles in slots k..k+3 (k a multiple of 4) of the r-th searched target; slots past its count hold its
     //! last neighbour again
     __device__ __forceinline__ void quad(uint32_t r, uint32_t k, uint32_t (&j)[4]) const

@@ -1188,15 +1188,49 @@ __global__ void __launch_bounds__(256)
     if (threadIdx.x <= kTableBins && part[threadIdx.x]) { atomicAdd(&hist[threadIdx.x], part[threadIdx.x]); }
 }
 
-//! row i - first of `out` = stored list of target i
-__global__ void copyListsKernel(NeighborLists lists, const uint32_t* __restrict__ nc, uint32_t* __restrict__ out,
-                                uint32_t searchFirst, uint32_t first, uint32_t last)
+constexpr unsigned kCopyWaves = 4;
+constexpr unsigned kCopyRun   = 32; // entries of each row per round
+
+/*! row i - first of `out` = stored list of target i. A wave takes the 64 targets of one list block: it reads kCopyRun
+ * entries of each (16-byte runs of the 64 lists lie side by side), turns the tile in LDS and writes 128 bytes per row and
+ * half wave. One thread per row, each writing its own 4 bytes, took 349 us for 250k particles and 25M
+ * entries; this takes 64. Bound by the table lookups and the writes (105 MB). */
+__global__ void __launch_bounds__(kCopyWaves* kWave)
+    copyListsKernel(NeighborLists lists, const uint32_t* __restrict__ nc, uint32_t* __restrict__ out,
+                    uint32_t searchFirst, uint32_t first, uint32_t last)
 {
-    uint32_t i = first + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= last) { return; }
-    uint32_t n = min(nc[i] - 1, lists.ngmax);
-    for (uint32_t k = 0; k < n; ++k)
-        out[size_t(i - first) * lists.ngmax + k] = lists.entry(i - searchFirst, k);
+    __shared__ uint32_t tile[kCopyWaves][kWave][kCopyRun + 1];
+    const unsigned      w = threadIdx.x / kWave, lane = laneId();
+    const uint32_t      block = (first - searchFirst) / kGroup + blockIdx.x * kCopyWaves + w;
+    const uint64_t      i     = uint64_t(searchFirst) + uint64_t(block) * kGroup + lane;
+    const bool          on    = i >= first && i < last && lists.searched(uint32_t(i - searchFirst));
+    const uint32_t      n     = on ? min(nc[i] - 1, lists.ngmax) : 0u;
+    const uint32_t      r     = on ? uint32_t(i - searchFirst) : 0u;
+    const uint32_t      most  = waveMax(n);
+    for (uint32_t k0 = 0; k0 < most; k0 += kCopyRun)
+    {
+#pragma unroll
+        for (uint32_t k = 0; k < kCopyRun; k += 4)
+        {
+            uint32_t j[4];
+            if (k0 + k < n)
+            {
+                lists.quad(r, k0 + k, j);
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    tile[w][lane][k + u] = j[u];
+            }
+        }
+        __builtin_amdgcn_wave_barrier(); // a wave's LDS accesses complete in order
+        const uint32_t k = lane % kCopyRun;
+        for (uint32_t row = lane / kCopyRun; row < kWave; row += kWave / kCopyRun)
+        {
+            const uint32_t rowN = __shfl(n, int(row), kWave);
+            const uint64_t to   = uint64_t(searchFirst) + uint64_t(block) * kGroup + row - first;
+            if (k0 + k < rowN) { out[to * lists.ngmax + k0 + k] = tile[w][row][k]; }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
 }
 
 } // namespace
@@ -1366,8 +1400,10 @@ void copyNeighbors(sphx_workspace* ws, uint32_t* out, uint32_t first, uint32_t l
         staging.reserve(len);
         dst = staging.get();
     }
-    copyListsKernel<<<ceilDiv(last - first, 256), 256, 0, ws->stream>>>(neighborLists(ws), ws->nbNc, dst, ws->nbFirst,
-                                                                        first, last);
+    // the list blocks that hold [first, last)
+    const uint32_t blocks = (last - 1 - ws->nbFirst) / kGroup - (first - ws->nbFirst) / kGroup + 1;
+    copyListsKernel<<<ceilDiv(blocks, kCopyWaves), kCopyWaves * kWave, 0, ws->stream>>>(
+        neighborLists(ws), ws->nbNc, dst, ws->nbFirst, first, last);
     SPHX_CHECK_LAUNCH();
     if (!onDevice)
     {

@@ -86,7 +86,7 @@ __device__ __forceinline__ Lane groupTarget(const Lists& L, uint32_t g)
     t.n     = t.valid ? min(L.nc[t.i] - 1, L.ngmax) : 0u;
     t.i     = t.valid ? t.i : L.first;
     t.r     = t.i - L.first;
-    if (L.lists.owner && L.lists.owner[t.r] == NeighborLists::kNoGroup) { t.n = 0; } // the search left it out
+    if (!L.lists.searched(t.r)) { t.n = 0; }
     return t;
 }
 
