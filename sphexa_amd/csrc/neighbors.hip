@@ -22,7 +22,7 @@
 // stores 16 bytes at a time (ListWriter), in the layouts of common.hpp.
 //
 // Measured (ms; with exact tests of every tile, hits appended tile by tile and statistics by atomics of every group, then
-// this): 8M turbulence, mixed 5.2 -> 3.8, 4.1M FP64 3.1 -> 2.3, 1M 0.79 -> 0.54, 4M Evrard sphere 3.7 -> 2.8; vector
+// this): 8M turbulence, mixed 5.2 -> 3.6, 4.1M FP64 3.1 -> 2.2, 1M 0.79 -> 0.51, 4M Evrard sphere 3.7 -> 2.8; vector
 // instructions per group 21.2k -> 13.9k. Bound by the vector ALU (three quarters of its issue slots at 8M) and, at four waves
 // per SIMD (16 waves fill a CU's LDS and 128 registers a wave), by latency: the chains of a window's plan, loads and
 // filter, and of the appends.
@@ -375,8 +375,9 @@ __device__ __forceinline__ uint64_t tileMask(const DevBox& box, Lds& lds, int bu
 /*! Hits of up to kPendingTiles swept tiles of a group with local lists, one bit per candidate, waiting to be
  * appended together: the append runs as many rounds as the busiest lane has hits, and over four tiles that is
  * much closer to a lane's share than tile by tile (about 130 rounds for the 91 neighbours of a lattice, against 250). The
- * next entry's table position is read from LDS while the previous one is appended. A round spends about 25
- * instructions of the vector ALU and, alone on its SIMD, a few hundred cycles. */
+ * next entry's table position is read from LDS while the previous one is appended. A round spends about 33
+ * instructions of the vector ALU (45 when each asked whether its entry still fits: search of 8M particles
+ * 3.79 -> 3.60 ms) and, alone on its SIMD, a few hundred cycles. */
 struct Pending
 {
     uint32_t w[2 * kPendingTiles] = {}; // word i: candidates 32 i .. of lds.pos
@@ -395,38 +396,47 @@ struct Pending
     template<class Writer>
     __device__ __forceinline__ void drain(const uint16_t* pos, unsigned ngmax, unsigned& count, Writer& out)
     {
-        uint32_t left = 0;
+        uint32_t hits = 0;
 #pragma unroll
         for (int i = 0; i < 2 * kPendingTiles; ++i)
-            left += __popc(w[i]);
-        bool     have = false; // an entry is on its way from LDS
-        uint32_t e    = 0;
-        auto     put  = [&]() {
-            if (have)
-            {
-                if (count < ngmax) { out.put(count, e); }
-                ++count;
-            }
-        };
-        while (left)
-        {
-            if (w[0] == 0)
-            {
+            hits += __popc(w[i]);
+        // the entries that still fit, after the first one
+        uint32_t slot = count, left = min(hits, ngmax - min(count, ngmax));
+        auto     next = [&]() {
 #pragma unroll
-                for (int i = 0; i + 1 < 2 * kPendingTiles; ++i)
-                    w[i] = w[i + 1];
-                w[2 * kPendingTiles - 1] = 0;
-                pos += 32;
-            }
-            const bool     more = w[0] != 0;
-            const uint32_t c    = more ? uint32_t(__builtin_ctz(w[0])) : 0u;
-            const uint32_t next = pos[c];
-            put();
+            for (int i = 0; i + 1 < 2 * kPendingTiles; ++i)
+                w[i] = w[i + 1];
+            w[2 * kPendingTiles - 1] = 0;
+            pos += 32;
+        };
+        auto take = [&]() {
+            const uint32_t e = pos[__builtin_ctz(w[0])];
             w[0] &= w[0] - 1;
-            left -= more ? 1u : 0u;
-            have = more, e = next;
+            return e;
+        };
+        if (left)
+        {
+            while (w[0] == 0) { next(); }
+            uint32_t e = take(); // on its way from LDS while the one before it is put
+            while (--left)
+            {
+                asm volatile("" : "+v"(w[0])); // (one word per round: the lanes with hits don't wait for the others)
+                if (w[0] == 0) { next(); }
+                if (w[0] == 0)
+                {
+                    ++left; // an empty word: the lane sits this round out
+                    continue;
+                }
+                const uint32_t after = take();
+                out.put(slot++, e);
+                e = after;
+            }
+            out.put(slot, e);
         }
-        put();
+        count += hits;
+#pragma unroll
+        for (int i = 0; i < 2 * kPendingTiles; ++i)
+            w[i] = 0;
         tiles = 0;
     }
 };
