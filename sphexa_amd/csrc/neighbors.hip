@@ -1198,6 +1198,13 @@ __global__ void __launch_bounds__(256)
     if (threadIdx.x <= kTableBins && part[threadIdx.x]) { atomicAdd(&hist[threadIdx.x], part[threadIdx.x]); }
 }
 
+//! clears the search's slots of the counters (those between are the time step's)
+__global__ void __launch_bounds__(kWave) clearStatsKernel(unsigned long long* stats)
+{
+    static_assert(kCounterSlots <= kWave, "one slot per lane");
+    if (threadIdx.x < 3 || (threadIdx.x >= kStatWide && threadIdx.x < kCounterSlots)) { stats[threadIdx.x] = 0; }
+}
+
 constexpr unsigned kCopyWaves = 4;
 constexpr unsigned kCopyRun   = 32; // entries of each row per round
 
@@ -1325,8 +1332,8 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     uint32_t           hist[kTableBins + 1];
     auto               run = [&](bool local)
     {
-        fill64(ws, reinterpret_cast<uint64_t*>(ws->counters.get()), 0, 3);
-        fill64(ws, reinterpret_cast<uint64_t*>(ws->counters.get()) + kStatWide, 0, kCounterSlots - kStatWide);
+        clearStatsKernel<<<1, kWave, 0, ws->stream>>>(reinterpret_cast<unsigned long long*>(ws->counters.get()));
+        SPHX_CHECK_LAUNCH();
         if (groups > 0)
         {
             unsigned    blocks = ceilDiv(groups, kWavesPerBlock);

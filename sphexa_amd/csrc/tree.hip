@@ -15,7 +15,8 @@
 //  4. every node adds up its place in the search's visiting order along its ancestors (visitKernel).
 // Five launches and one host read of the internal nodes per level, where a level-by-level descent took about forty
 // launches and a read per level. What bounds it: launch latency up to about a million particles, then reading the
-// keys twice and the chains of searches in childKernel (33 us at 1M particles). Measured, a whole std step with
+// keys twice and the chains of searches in childKernel (33 us at 1M particles by halves, 19 with seven probes
+// at a time). Measured, a whole std step with
 // the former descent and with this: 0.65 -> 0.51 ms at 1728 particles (FP64), 1.98 -> 1.77 ms at 1M (mixed); a mixed VE
 // step at 8M 15.2 -> 14.8 ms.
 #include <cstring> // rocprim uses memset without including it
@@ -29,29 +30,52 @@ namespace sphx
 namespace
 {
 
-__device__ __forceinline__ uint32_t lowerBound(const Key* keys, uint32_t lo, uint32_t hi, Key v)
+/*! first index in [lo, hi) whose key is at least v, else hi. Seven probes at a time: what a search costs is its chain of
+ * dependent loads, a third as long as by halves. */
+__device__ __forceinline__ uint32_t lowerBound(const Key* __restrict__ keys, uint32_t lo, uint32_t hi, Key v)
 {
-    while (lo < hi)
+    while (hi - lo >= 8)
     {
-        uint32_t mid = lo + (hi - lo) / 2;
-        if (keys[mid] < v) lo = mid + 1;
-        else hi = mid;
+        const uint32_t step  = (hi - lo) / 8;
+        uint32_t       below = 0;
+#pragma unroll
+        for (uint32_t i = 1; i < 8; ++i)
+            below += keys[lo + i * step] < v ? 1u : 0u;
+        hi = below < 7 ? lo + (below + 1) * step : hi;
+        lo = below > 0 ? lo + below * step + 1 : lo;
     }
-    return lo;
+    if (lo == hi) { return lo; }
+    uint32_t below = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 7; ++i)
+    {
+        const Key k = keys[min(lo + i, hi - 1)]; // (all loads go out together)
+        below += lo + i < hi && k < v ? 1u : 0u;
+    }
+    return lo + below;
 }
 
-/*! first index in [lo, n) whose key is at least v, by doubling steps from lo: the searches of a node's children
- * end within the node */
-__device__ __forceinline__ uint32_t lowerBoundFrom(const Key* keys, uint32_t lo, uint32_t n, Key v)
+//! the same in [lo, n), for searches that end soon: eight probes at doubling distances bracket the end
+__device__ __forceinline__ uint32_t lowerBoundFrom(const Key* __restrict__ keys, uint32_t lo, uint32_t n, Key v)
 {
-    uint32_t step = 1, a = lo;
-    while (a < n && keys[a] < v)
+    if (lo >= n) { return n; }
+    uint32_t a = lo;
+    for (uint64_t step = 16;; step <<= 8)
     {
-        lo = a + 1;
-        a  = n - a > step ? a + step : n;
-        step *= 2;
+        uint32_t below = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+        {
+            const uint64_t q = lo + (step << k);
+            below += keys[q < n ? q : n - 1] < v && q < n ? 1u : 0u;
+        }
+        if (below > 0) { a = uint32_t(lo + (step << (below - 1))) + 1; }
+        if (below < 8)
+        {
+            const uint64_t end = lo + (step << below);
+            return lowerBound(keys, a, uint32_t(end < n ? end : n), v);
+        }
     }
-    return lowerBound(keys, lo, min(a, n), v);
 }
 
 constexpr unsigned kPlanWaves = 4;
@@ -263,15 +287,15 @@ __global__ void __launch_bounds__(256) childKernel(const Key* __restrict__ keys,
     const uint32_t place = in.place[r];
     const bool     atEnd = in.key[r] + 8 * range == nodeRange(0);
 
-    // particles and depth-first places of the child: its own first, and the next child's
-    const uint32_t first = c == 0 ? in.lo[r] : lowerBoundFrom(keys, in.lo[r], n, k);
-    const uint32_t q0    = c == 0 ? place + 1 : lowerBoundFrom(in.dfKey, place + 1, total, k);
-    uint32_t       last  = __shfl_down(first, 1, 8), q1 = __shfl_down(q0, 1, 8);
-    if (c == 7)
-    {
-        last = atEnd ? n : lowerBoundFrom(keys, first, n, k + range);
-        q1   = atEnd ? total : lowerBoundFrom(in.dfKey, q0, total, k + range);
-    }
+    // particles and depth-first places of the child: its own first (the first child's are the node's), and the next
+    // child's; thread 0 finds the node's end
+    const uint32_t lo0 = in.lo[r];
+    const Key      sought = c == 0 ? k + 8 * range : k;
+    uint32_t       first = lowerBoundFrom(keys, lo0, n, sought), q0 = lowerBoundFrom(in.dfKey, place + 1, total, sought);
+    const uint32_t end = atEnd ? n : __shfl(first, 0, 8), qEnd = atEnd ? total : __shfl(q0, 0, 8);
+    if (c == 0) { first = lo0, q0 = place + 1; }
+    uint32_t last = __shfl_down(first, 1, 8), q1 = __shfl_down(q0, 1, 8);
+    if (c == 7) { last = end, q1 = qEnd; }
     const uint32_t node   = 1 + id;
     const bool     leaf   = last - first <= bucket || l + 1 >= kMaxLevel;
     const int32_t  leaves = leaf ? 1 : 1 + 7 * int32_t(q1 - q0);
@@ -498,15 +522,17 @@ __global__ void rebalanceKernel(const Key* __restrict__ leaves, const int32_t* _
     }
 }
 
-//! first particle and count of every leaf of the linked leaf array (computeNodeCounts: binary searches)
+//! first particle and count of every leaf of the linked leaf array (computeNodeCounts)
 __global__ void leafLayoutKernel(const Key* __restrict__ leaves, uint32_t L, const Key* __restrict__ keys, uint32_t n,
                                  uint32_t* __restrict__ layout, uint32_t* __restrict__ counts)
 {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s > L) { return; }
-    const uint32_t lo = s == L ? n : lowerBound(keys, 0, n, leaves[s]);
-    layout[s]         = lo;
-    if (s < L) { counts[s] = (s + 1 == L ? n : lowerBound(keys, lo, n, leaves[s + 1])) - lo; }
+    const uint32_t lo   = s == L ? n : lowerBound(keys, 0, n, leaves[s]);
+    uint32_t       next = __shfl_down(lo, 1, kWave); // the next leaf's, by the lane beside
+    if (s < L && laneId() == kWave - 1) { next = s + 1 == L ? n : lowerBoundFrom(keys, lo, n, leaves[s + 1]); }
+    layout[s] = lo;
+    if (s < L) { counts[s] = next - lo; }
 }
 
 } // namespace
