@@ -56,7 +56,7 @@ __host__ __device__ inline size_t localOffset(uint32_t g, uint32_t ngmax8, uint3
  * 350-900 on the Evrard sphere; a search that meets a larger table stores global lists instead. */
 constexpr uint32_t kTableCap = 2048;
 //! bins of the table sizes' histogram, kTableBin entries each
-constexpr uint32_t kTableBin  = 64;
+constexpr uint32_t kTableBin  = 32;
 constexpr uint32_t kTableBins = kTableCap / kTableBin;
 
 /*! the stored lists of the last search (see the layouts above) */

@@ -279,7 +279,7 @@ void launchDensity(sphx_workspace* ws, PairArgs a, const sphx_fields_t* f, const
     RecGradh<T>* next = !toRho && chainable(a, p) ? recordBuffer<RecGradh<T>>(ws, a.numParticles, 1) : nullptr;
     RecVol<T>*   nextVol = toRho && chainable(a, p) ? recordBuffer<RecVol<T>>(ws, a.numParticles, 1) : nullptr;
     {
-        const PairLaunch run = pairLaunch(ws, sizeof(RecMass<T>), kLightWaves, 1);
+        const PairLaunch run = pairLaunch(ws, sizeof(RecMass<T>), kLightWaves, 1, kLightPerSimd<T>);
         a.L.stage            = run.stage;
         KernelScope timer(ws, toRho ? "density_std" : "xmass");
         launchVariant<T>(ws, a.box, [&](auto variant) {
@@ -318,7 +318,7 @@ void launchIadStd(sphx_workspace* ws, PairArgs a, const sphx_fields_t* f, const 
                              ? recordBuffer<RecMomStd<T>>(ws, a.numParticles, 1 - in)
                              : nullptr;
     {
-        const PairLaunch run = pairLaunch(ws, sizeof(RecVol<T>), kLightWaves, 6);
+        const PairLaunch run = pairLaunch(ws, sizeof(RecVol<T>), kLightWaves, 6, kLightPerSimd<T>);
         a.L.stage            = run.stage;
         KernelScope timer(ws, "iad_std");
         launchVariant<T>(ws, a.box, [&](auto variant) {
@@ -344,7 +344,7 @@ void launchMomentumStd(sphx_workspace* ws, PairArgs a, const MomStdFields& mf, c
         packMomStd<T><<<ceilDiv(a.numParticles, kPackThreads), kPackThreads, 0, ws->stream>>>(a, mf, rec);
         SPHX_CHECK_LAUNCH();
     }
-    const PairLaunch run = pairLaunch(ws, sizeof(RecMomStd<T>), kMomWaves<T>, 5);
+    const PairLaunch run = pairLaunch(ws, sizeof(RecMomStd<T>), kMomWaves<T>, 5, kMomPerSimd<T>);
     a.L.stage            = run.stage;
     KernelScope timer(ws, "momentum_std");
     launchVariant<T>(ws, a.box, [&](auto variant) {

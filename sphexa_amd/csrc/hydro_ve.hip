@@ -563,7 +563,7 @@ void launchGradh(sphx_workspace* ws, PairArgs a, const sphx_fields_t* f, const s
                             ? recordBuffer<RecIadVe<T>>(ws, a.numParticles, out)
                             : nullptr;
     {
-        const PairLaunch run = pairLaunch(ws, sizeof(RecGradh<T>), kLightWaves, 3);
+        const PairLaunch run = pairLaunch(ws, sizeof(RecGradh<T>), kLightWaves, 3, kLightPerSimd<T>);
         a.L.stage            = run.stage;
         KernelScope timer(ws, "ve_def_gradh");
         launchVariant<T>(ws, a.box, [&](auto variant) {
@@ -592,7 +592,7 @@ void launchIadVe(sphx_workspace* ws, PairArgs a, const IadVeFields& vf, const sp
     }
     RecAv<T>* next = chainable(a, p) && f->c ? recordBuffer<RecAv<T>>(ws, a.numParticles, 1 - in) : nullptr;
     {
-        const PairLaunch run = pairLaunch(ws, sizeof(RecIadVe<T>), kLightWaves, 15);
+        const PairLaunch run = pairLaunch(ws, sizeof(RecIadVe<T>), kLightWaves, 15, kLightPerSimd<T>);
         a.L.stage            = run.stage;
         KernelScope timer(ws, "iad_divv_curlv");
         launchVariant<T>(ws, a.box, [&](auto variant) {
@@ -621,7 +621,7 @@ void launchAv(sphx_workspace* ws, PairArgs a, const AvFields& af, const sphx_fie
     RecMomVe<T>* next =
         chainable(a, p) && f->m && f->prho ? recordBuffer<RecMomVe<T>>(ws, a.numParticles, 1 - in) : nullptr;
     {
-        const PairLaunch run = pairLaunch(ws, sizeof(RecAv<T>), kLightWaves, 4);
+        const PairLaunch run = pairLaunch(ws, sizeof(RecAv<T>), kLightWaves, 4, kLightPerSimd<T>);
         a.L.stage            = run.stage;
         KernelScope timer(ws, "av_switches");
         launchVariant<T>(ws, a.box, [&](auto variant) {
@@ -655,7 +655,8 @@ void launchMomVe(sphx_workspace* ws, PairArgs a, const MomVeFields& mf, const sp
         SPHX_CHECK_LAUNCH();
     }
     const PairLaunch run = pairLaunch(ws, sizeof(RecMomVe<T>) + (avClean ? sizeof(RecGradV<T>) : 0),
-                                      avClean ? kMomWaves<T, true> : kMomWaves<T>, 6);
+                                      avClean ? kMomWaves<T, true> : kMomWaves<T>, 6,
+                                      avClean ? kMomPerSimd<T, true> : kMomPerSimd<T>);
     a.L.stage            = run.stage;
     KernelScope timer(ws, "momentum_ve");
     launchVariant<T>(ws, a.box, [&](auto variant) {

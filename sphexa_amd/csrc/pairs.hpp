@@ -13,9 +13,10 @@
 // table to LDS, chunk c of all records side by side, and every neighbour is read from there
 // (PairWalk). Groups whose table does not fit the launch's LDS, and global lists,
 // read the records from global memory in the same order. Measured (ms; gathers from global memory, then this):
-// mixed VE at 8M particles, XMass 1.27 -> 0.78, grad-h 2.13 -> 1.33, IAD 2.17 -> 1.55, AV switches 2.84 -> 1.47,
-// momentum-energy 4.92 -> 3.24; FP64 VE at 4.1M, 2.35 -> 1.03, 2.90 -> 1.73, 3.26 -> 2.10, 4.06 -> 2.05, 6.76 ->
-// 5.11 (with the kernel evaluated instead of gathered from its table). What bounds them now: the FP32 form
+// mixed VE at 8M particles, XMass 1.27 -> 0.79, grad-h 2.13 -> 1.30, IAD 2.17 -> 1.49, AV switches 2.84 -> 1.42,
+// momentum-energy 4.92 -> 3.24; FP64 VE at 4.1M, 2.35 -> 1.02, 2.90 -> 1.70, 3.26 -> 1.74, 4.06 -> 1.77, 6.76 ->
+// 5.1-5.4 (with the kernel evaluated instead of gathered from its table; a card at its power limit runs
+// momentum slower when the loops before it are faster). What bounds them now: the FP32 form
 // the vector ALU (67-90% of its issue slots), the FP64 form the latency of a block's phases at 2-3 waves per SIMD.
 //
 // Two arithmetic forms share each kernel template:
@@ -26,6 +27,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <tuple>
 #include <type_traits>
 
@@ -47,7 +49,13 @@ constexpr int kMomWaves = isMixed<T> ? 4 : avClean ? 8 : 12;
 
 //! waves per SIMD that a light loop's registers must leave room for: five in the FP32 form, three in the FP64 form
 //! (its LDS holds three blocks or more); without the bound some take a few registers too many for that
-#define SPHX_LIGHT_WAVES(T) __attribute__((amdgpu_waves_per_eu(isMixed<T> ? 5 : 3, isMixed<T> ? 8 : 3)))
+template<class T>
+constexpr int kLightPerSimd = isMixed<T> ? 5 : 3;
+#define SPHX_LIGHT_WAVES(T) __attribute__((amdgpu_waves_per_eu(kLightPerSimd<T>, isMixed<T> ? 8 : 3)))
+
+//! waves per SIMD that the momentum loop's registers leave room for
+template<class T, bool avClean = false>
+constexpr int kMomPerSimd = isMixed<T> ? 4 : kMomWaves<T, avClean> / 4;
 
 //! waves per block of the adjoint loops, which take one group per wave
 constexpr int kVjpWaves = 4;
@@ -326,11 +334,13 @@ struct PairWalk
         {
             for (uint32_t k = k0; k < t.n; k += 4 * W)
             {
+                uint32_t j[4];
+                L.lists.quad(t.r, k, j);
 #pragma unroll 1
                 for (uint32_t u = 0; u < 4; ++u)
                 {
-                    const uint32_t j = L.lists.entry(t.r, k + u);
-                    pair(k + u < t.n, rec[j]...);
+                    pair(k + u < t.n, rec[j[0]]...);
+                    j[0] = j[1], j[1] = j[2], j[2] = j[3];
                 }
             }
         }
@@ -367,27 +377,47 @@ __device__ __forceinline__ bool waveSums(double (&v)[N])
     return true;
 }
 
-/*! host: the records a launch stages and its dynamic LDS, for records of `recBytes` and N partial sums. The stage
- * holds the tables of 99.5% of the blocks, or the 160 KB of a CU if they are larger; the other blocks read
- * from global memory. */
+/*! host: the records a launch stages and its dynamic LDS, for records of `recBytes`, N partial sums and a kernel whose
+ * registers leave room for `perSimd` waves on a SIMD. A block whose table does not fit the stage reads its
+ * neighbours from global memory, about three times as long; a smaller stage leaves room for more blocks on a CU, and the
+ * loops' time goes with about the power -0.4 of the waves per SIMD. The number of blocks per CU is the one with the
+ * least product of both, the stage what its share of the 160 KB holds. Measured against a stage for 99.5% of the
+ * tables (ms): mixed std momentum of the 4M Evrard sphere 2.15 -> 1.69 (three blocks instead of two, 8% of the
+ * blocks gathering), FP64 AV switches and IAD at 4.1M 2.04 -> 1.77 and 2.07 -> 1.74, mixed IAD at 2M 0.42 -> 0.38. */
 struct PairLaunch
 {
     uint32_t stage;
     size_t   lds;
 };
-inline PairLaunch pairLaunch(const sphx_workspace* ws, size_t recBytes, int waves, int sums)
+inline PairLaunch pairLaunch(const sphx_workspace* ws, size_t recBytes, int waves, int sums, int perSimd)
 {
-    const size_t part = size_t(waves - 1) * sums * kWave * sizeof(double);
-    if (!ws->nbLocal) { return {0, part}; }
-    uint64_t blocks = 0, seen = 0;
+    constexpr double kGathered = 3.0;
+    constexpr size_t kLds = 160 * 1024, kLdsUnit = 1280; // of a CU, and what it is given out in
+    const size_t     part      = size_t(waves - 1) * sums * kWave * sizeof(double);
+    uint64_t         blocks    = 0;
     for (uint32_t b = 0; b < kTableBins; ++b)
         blocks += ws->nbTableHist[b];
-    uint32_t bins = 0;
-    while (bins < kTableBins && seen * 1000 < blocks * 995)
-        seen += ws->nbTableHist[bins++];
-    const uint32_t each  = stagedBytes(uint32_t(recBytes));
-    const uint32_t stage = std::min(bins * kTableBin, uint32_t(160 * 1024) / each);
-    return {stage, std::max(part, size_t(stage) * each)};
+    if (!ws->nbLocal || blocks == 0) { return {0, part}; }
+    const uint32_t each = stagedBytes(uint32_t(recBytes));
+    PairLaunch     best{0, part};
+    double         least = INFINITY;
+    for (int perCu = 1; perCu == 1 || perCu * waves <= 4 * perSimd; ++perCu)
+    {
+        const size_t room = kLds / kLdsUnit / perCu * kLdsUnit;
+        if (part > room) { break; }
+        const uint32_t fit    = std::min(uint32_t(room / each), kTableCap);
+        uint64_t       staged = 0;
+        uint32_t       stage  = 0; // the largest table among those that fit
+        for (uint32_t b = 0; (b + 1) * kTableBin <= fit; ++b)
+        {
+            staged += ws->nbTableHist[b];
+            if (ws->nbTableHist[b]) { stage = (b + 1) * kTableBin; }
+        }
+        const double share = double(staged) / double(blocks);
+        const double time  = (share + (1.0 - share) * kGathered) / std::pow(double(perCu), 0.4);
+        if (time < least) { least = time, best = {stage, std::max(part, size_t(stage) * each)}; }
+    }
+    return best;
 }
 
 /*! The SPH kernel W(v) = sinc(pi v / 2)^n and dW/dv on [0, 2), zero from v = 2 on.
