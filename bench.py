@@ -32,13 +32,15 @@ METRIC = "SPH particle-updates/s (nbr search+density+IAD+force), mixed vs FP64, 
 # MI355X published peaks
 PEAK_FP64_VECTOR_TFLOPS = 78.6
 PEAK_FP32_VECTOR_TFLOPS = 157.3
+PEAK_FP32_MATRIX_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
 
 # Algorithmic flops per unit of each kernel of the VE pass, counting + - * as 1, division and
 # square root as 1, each table lookup as 7 (index, two loads' difference, slope, offset, fma),
 # whichever way the kernel obtains W:
-#  search        per candidate distance test: 3 differences, 3 squares, 2 adds (FP64 in both forms,
-#                the reference's exact predicate), plus the h iteration's re-searches
+#  search        per candidate distance test: 4 multiply-adds of an FP32 matrix product (both forms; tiles with
+#                a distance too close to the radius are tested again in FP64, not counted), plus the h
+#                iteration's re-searches
 #  xmass         per pair 19 (xmassJLoop, sph/include/sph/hydro_ve/xmass_kern.hpp:51-79)
 #  ve_def_gradh  per pair 33 (veDefGradhJLoop, hydro_ve/ve_def_gradh_kern.hpp:44-90)
 #  iad_divv_curlv per pair 37 + 59 (IADJLoop, hydro_ve/iad_kern.hpp:44-109; divV_curlVJLoop,
@@ -59,12 +61,12 @@ FLOPS_PER_PAIR_MOM_VE = FLOPS_PER_PAIR["momentum_ve"]
 # counter runs scaled by a plain copy kernel of known size (read x 2.0, write x 1.0); see the
 # counter summaries under profiles/. Counters cannot be read from inside the timed run, so the
 # measured figures are carried here for the default workload only.
-MEASURED_TRAFFIC = {("search", 200, "mixed"): 6.034e9, ("search", 200, "fp64"): 7.291e9,
-                    ("momentum_ve", 200, "mixed"): 4.987e9, ("momentum_ve", 200, "fp64"): 6.926e9,
-                    ("av_switches", 200, "mixed"): 4.815e9, ("av_switches", 200, "fp64"): 6.398e9,
-                    ("iad_divv_curlv", 200, "mixed"): 4.297e9, ("iad_divv_curlv", 200, "fp64"): 5.343e9,
-                    ("ve_def_gradh", 200, "mixed"): 4.054e9, ("ve_def_gradh", 200, "fp64"): 4.727e9,
-                    ("xmass", 200, "mixed"): 3.638e9, ("xmass", 200, "fp64"): 4.143e9}
+MEASURED_TRAFFIC = {("search", 200, "mixed"): 3.786e9, ("search", 200, "fp64"): 5.074e9,
+                    ("momentum_ve", 200, "mixed"): 3.113e9, ("momentum_ve", 200, "fp64"): 4.372e9,
+                    ("av_switches", 200, "mixed"): 3.558e9, ("av_switches", 200, "fp64"): 5.089e9,
+                    ("iad_divv_curlv", 200, "mixed"): 3.014e9, ("iad_divv_curlv", 200, "fp64"): 4.164e9,
+                    ("ve_def_gradh", 200, "mixed"): 2.718e9, ("ve_def_gradh", 200, "fp64"): 3.391e9,
+                    ("xmass", 200, "mixed"): 2.386e9, ("xmass", 200, "fp64"): 2.783e9}
 
 
 def parse():
@@ -485,9 +487,9 @@ def run_adjoint(side, mixed, steps, warmup):
 def kernel_rooflines(r, mixed):
     """Roofline entry of every kernel of the VE pass: algorithmic flops per launch (per unit above
     times the units of the launch) over the kernel's mean duration from HIP events on its stream,
-    against the FP64 vector peak for FP64 work (the search's distance tests in both forms) and the
-    FP32 peaks for the FP32 pair loops: 157.3 TFLOP/s with packed FP32 issue, 78.6 TFLOP/s without
-    (the library is compiled with packed FP32 off)."""
+    against the FP32 matrix peak for the search's distance tests, the FP64 vector peak for FP64 pair
+    loops and the FP32 peaks for the FP32 ones: 157.3 TFLOP/s with packed FP32 issue, 78.6 TFLOP/s
+    without (the library is compiled with packed FP32 off)."""
     out = {}
     side = round(r["n"] ** (1.0 / 3.0))
     form = "mixed" if mixed else "fp64"
@@ -495,7 +497,7 @@ def kernel_rooflines(r, mixed):
         ms = r["kernel_ms"][k]
         if k == "search":
             flops = FLOPS_PER_TEST_SEARCH * r["search_tests"]
-            fp64 = True
+            fp64 = False
             units = dict(candidate_tests=r["search_tests"], tests_per_stored_pair=round(r["search_tests"] / r["pairs"], 2))
         else:
             flops = FLOPS_PER_PAIR[k] * r["pairs"] + FLOPS_PER_TARGET.get(k, 0) * r["n"]
@@ -503,8 +505,11 @@ def kernel_rooflines(r, mixed):
             units = dict(pairs=r["pairs"])
         ach = flops / (ms * 1e-3) / 1e12
         e = dict(bound="valu", achieved=round(ach, 3), unit="TFLOP/s", avg_launch_ms=round(ms, 4),
-                 flops_per_launch=int(flops), precision="fp64" if fp64 else "fp32", **units)
-        if fp64:
+                 flops_per_launch=int(flops),
+                 precision="fp32 matrix" if k == "search" else "fp64" if fp64 else "fp32", **units)
+        if k == "search":
+            e.update(peak=PEAK_FP32_MATRIX_TFLOPS, frac=round(ach / PEAK_FP32_MATRIX_TFLOPS, 4))
+        elif fp64:
             e.update(peak=PEAK_FP64_VECTOR_TFLOPS, frac=round(ach / PEAK_FP64_VECTOR_TFLOPS, 4))
         else:
             e.update(peak=PEAK_FP32_VECTOR_TFLOPS, frac=round(ach / PEAK_FP32_VECTOR_TFLOPS, 4),

@@ -4,7 +4,8 @@
 
 Each .hip file is compiled to an object in parallel with hipcc, then linked into
 sphexa_amd/libsphexa_amd.so. Packed FP32 instructions are disabled for all device code
-(-packed-fp32-ops); FP64 neighbour predicates use explicit per-function contraction pragmas.
+(-packed-fp32-ops); products and sums contract within a statement only (-ffp-contract=on), so that two
+instantiations of a loop give the same bits, and FP64 neighbour predicates not at all (per-function pragmas).
 """
 import concurrent.futures as cf
 import os

@@ -23,7 +23,7 @@
 //
 // Measured (ms; with exact tests of every tile, hits appended tile by tile and statistics by atomics of every group, then
 // this): 8M turbulence, mixed 5.2 -> 3.6, 4.1M FP64 3.1 -> 2.2, 1M 0.79 -> 0.51, 4M Evrard sphere 3.7 -> 2.8; vector
-// instructions per group 21.2k -> 13.9k. Bound by the vector ALU (three quarters of its issue slots at 8M) and, at four waves
+// instructions per group 21.2k -> 13.9k. Bound by the vector ALU (four fifths of its issue slots at 8M) and, at four waves
 // per SIMD (16 waves fill a CU's LDS and 128 registers a wave), by latency: the chains of a window's plan, loads and
 // filter, and of the appends.
 #include <cstring>
@@ -179,7 +179,7 @@ struct ListOnly
 
 //! ... or the XMass sum of xmassJLoop (hydro_ve/xmass_kern.hpp:51-79): m_i + sum_j m_j W(r_ij / h_i)
 //! over the stored neighbours in list order, r_ij from the same separation as the pair loop
-//! (minimum image, then rounded to h's type), compensated for the FP32 form. Hits are staged
+//! (minimum image, then rounded to h's type), in FP64. Hits are staged
 //! kBatch at a time: their kernel values are fetched together, then accumulated in list order,
 //! slots without a stored hit leaving the sum untouched (bitwise the one-at-a-time sum).
 template<class Th>
