@@ -346,11 +346,14 @@ int sphx_compute_groups(sphx_workspace_t* ws, const sphx_box_t* box, const sphx_
  * neighbour search, every pair loop, sphx_compute_positions and sphx_update_smoothing_length, when
  * called with [first, last) = [groups->firstBody, groups->lastBody), run one wavefront per group
  * instead of consecutive groups of 64 from first. The view is copied (its device arrays must stay
- * valid while in use); NULL restores consecutive groups. Groups of the search must partition
- * [firstBody, lastBody) and hold at most 64 particles each (the search returns SPHX_ERR_ARG for a
- * larger one); the pair loops accept any subset of the searched targets (the block time-step
- * propagators' active groups), whose neighbour lists stay indexed by particle. Record chaining is
- * not applied while a view is set. */
+ * valid while in use); NULL restores consecutive groups. Groups of the search hold at most 64
+ * particles each (the search returns SPHX_ERR_ARG for a larger one). A target of
+ * [firstBody, lastBody) in no group has no list: until the next search, sphx_copy_neighbors leaves its
+ * row, and the pair loops and adjoints its results, as they were (as a neighbour it takes part like
+ * any particle). A target in several groups is searched once. The pair loops accept any
+ * groups of searched targets (the block time-step propagators' active groups), whose neighbour lists
+ * stay indexed by particle. Record chaining is not applied while a view is set, nor after a search
+ * that left targets out. */
 int sphx_set_groups(sphx_workspace_t* ws, const sphx_groups_t* groups);
 
 /* ---- neighbour search ---------------------------------------------------------------------- */
@@ -379,7 +382,8 @@ int sphx_find_neighbors_xmass(sphx_workspace_t* ws, const sphx_box_t* box, const
 
 /* Copy the stored neighbour list of targets [first,last), a sub-range of the last search's range,
  * into `out` (device or host memory, row-major [last-first][ngmax], row k for target first + k,
- * entries beyond min(nc-1, ngmax) unspecified). Test/inspection
+ * entries beyond min(nc-1, ngmax) unspecified; rows of targets that the search's group view left out
+ * are not written). Test/inspection
  * helper matching the CPU Dataset's d.neighbors layout (particles_data.hpp:250-251). */
 int sphx_copy_neighbors(sphx_workspace_t* ws, uint32_t* out, uint32_t first, uint32_t last);
 

@@ -65,7 +65,7 @@ struct NeighborLists
     const void*     nbrs;
     const uint32_t* table;      // local lists: kTableCap particles per group ...
     const uint32_t* tableCount; // ... and how many of them are used; null for global lists
-    const uint32_t* owner;      // the searched targets' groups (kNoGroup: not searched), null: consecutive groups
+    const uint32_t* owner;      // the targets' groups (kNoGroup: not searched); null: consecutive groups, or none is needed
     uint32_t        ngmax;
 
     static constexpr uint32_t kNoGroup = 0xffffffffu;
@@ -73,7 +73,7 @@ struct NeighborLists
     //! group whose table the r-th target's list refers to
     __device__ __forceinline__ uint32_t group(uint32_t r) const { return owner ? owner[r] : r / kGroup; }
 
-    //! the search took the r-th target (a group view may leave targets out: they have no list)
+    //! the search took the r-th target (a group view may leave targets out: they have no list, in either layout)
     __device__ __forceinline__ bool searched(uint32_t r) const { return owner == nullptr || owner[r] != kNoGroup; }
 
     //! particles in slots k..k+3 (k a multiple of 4) of the r-th searched target; slots past its count hold its
@@ -92,18 +92,6 @@ struct NeighborLists
                                                         localOffset(g, paddedNgmax8(ngmax), k, lane));
         const uint32_t* t = table + size_t(group(r)) * kTableCap;
         j[0] = t[q.x & 0xffffu], j[1] = t[q.x >> 16], j[2] = t[q.y & 0xffffu], j[3] = t[q.y >> 16];
-    }
-
-    //! particle in slot k of the r-th searched target
-    __device__ __forceinline__ uint32_t entry(uint32_t r, uint32_t k) const
-    {
-        const uint32_t g = r / kGroup, lane = r % kGroup;
-        if (tableCount == nullptr)
-        {
-            return static_cast<const uint32_t*>(nbrs)[listOffset(g, paddedNgmax(ngmax), k, lane)];
-        }
-        return table[size_t(group(r)) * kTableCap +
-                     static_cast<const uint16_t*>(nbrs)[localOffset(g, paddedNgmax8(ngmax), k, lane)]];
     }
 };
 
@@ -258,7 +246,8 @@ struct sphx_workspace
     // neighbour lists of the last search, and their groups' tables when they are local lists
     sphx::DevBuf<uint32_t> nbrs, nbTable, nbTableCount, nbOwner;
     sphx::DevBuf<char>     nbGroupStats; // the search's statistics per group
-    bool                   nbLocal = false, nbOwned = false;
+    bool                   nbLocal = false, nbOwned = false; // nbOwned: nbOwner holds the search's groups
+    bool                   nbPartial = false;                // the search's view left targets of its range out
     uint32_t               nbTableHist[sphx::kTableBins + 1] = {}; // groups by table size; the last bin: over kTableCap
     uint32_t               nbFirst = 0, nbLast = 0, nbNgmax = 0;
     const uint32_t*        nbNc = nullptr; // nc array the lists were built with
@@ -437,13 +426,15 @@ __device__ __forceinline__ void groupRange(const Groups& G, uint32_t g, uint32_t
 /* 64-bit slots of the workspace counters: the search's statistics (stored pairs, maximum count,
  * non-converged targets) in 0-2, the Courant dt of the momentum loops in 3, the device maxima of the
  * time step in 4, the search's wide-support count, candidate tests and oversized groups in 5-7, the
- * largest h of the searched targets (FP64 bits) in 8, the histogram of the table sizes from 9 on */
-constexpr int kCounterSlots  = 9 + (int(kTableBins) + 2) / 2;
+ * largest h of the searched targets (FP64 bits) in 8, the number of targets searched in 9, the histogram of the
+ * table sizes from 10 on */
+constexpr int kCounterSlots  = 10 + (int(kTableBins) + 2) / 2;
 constexpr int kStatWide      = 5;
 constexpr int kStatTests     = 6;
 constexpr int kStatBadGroups = 7;
 constexpr int kStatHMax      = 8;
-constexpr int kStatHist      = 9; // first slot of the 32-bit bins of the table sizes
+constexpr int kStatTargets   = 9;
+constexpr int kStatHist      = 10; // first slot of the 32-bit bins of the table sizes
 
 constexpr unsigned kNumXcd = 8; // MI355X: 8 accelerator complex dies, one L2 each
 
@@ -644,7 +635,7 @@ inline DevBox pairBox(const sphx_workspace* ws, const sphx_box_t* b)
 inline NeighborLists neighborLists(const sphx_workspace* ws)
 {
     return NeighborLists{ws->nbrs.get(), ws->nbTable.get(), ws->nbLocal ? ws->nbTableCount.get() : nullptr,
-                         ws->nbOwned ? ws->nbOwner.get() : nullptr, ws->nbNgmax};
+                         ws->nbOwned && (ws->nbLocal || ws->nbPartial) ? ws->nbOwner.get() : nullptr, ws->nbNgmax};
 }
 
 /* ---------------------------------------------------------------------------------------------

@@ -56,8 +56,10 @@ constexpr int kNoShiftImage  = 13;   // image code of shift (0, 0, 0)
 struct alignas(16) GroupStat
 {
     double   hMax;
-    uint32_t stored, maxCount, fails, wide, swept, bad;
+    uint32_t stored, maxCount, swept;
+    uint16_t fails, wide, bad, targets;
 };
+static_assert(sizeof(GroupStat) == 32, "two 16-byte chunks per group");
 
 struct SearchArgs
 {
@@ -77,7 +79,7 @@ struct SearchArgs
     Groups               groups; // target groups, one wavefront each
     int                  iterateH;
     void*                nbrs;
-    uint32_t*            owner;      // local lists: the targets' groups (null: consecutive groups)
+    uint32_t*            owner;      // the targets' groups (null: consecutive groups), kNoGroup before the search
     uint32_t*            table;      // local lists: the groups' tables ...
     uint32_t*            tableCount; // ... and their sizes (over kTableCap: the table did not fit)
     uint32_t*            nc;
@@ -1061,6 +1063,8 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     Target t;
     t.i      = base + lane;
     t.active = t.i < end;
+    // a target of two groups is the first one's alone: its list refers to one table
+    if (a.owner && t.active) { t.active = atomicCAS(&a.owner[t.i - a.first], NeighborLists::kNoGroup, g) == NeighborLists::kNoGroup; }
     Th hi    = t.active ? h[t.i] : Th(0);
     t.x      = t.active ? a.x[t.i] : 0.0;
     t.y      = t.active ? a.y[t.i] : 0.0;
@@ -1073,7 +1077,6 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     {
         out.base  = static_cast<char*>(a.nbrs) + 2 * localOffset(r / kGroup, paddedNgmax8(a.ngmax), 0, r % kGroup);
         out.group = g;
-        if (a.owner && t.active) { a.owner[r] = g; }
     }
     else { out.base = static_cast<char*>(a.nbrs) + 4 * listOffset(r / kGroup, paddedNgmax(a.ngmax), 0, r % kGroup); }
 
@@ -1131,19 +1134,21 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     const unsigned mx     = waveMax(valid ? ncSph : 0u);
     const unsigned fails  = __popcll(ballot(valid && updates >= 10));
     // support 2h reaching half a box length: the FP32 pair loops then take exact separations
-    const unsigned wide = __popcll(ballot(valid && 4.0 * double(hi) * (1.0 + 1e-6) >= a.minLen));
+    const unsigned wide  = __popcll(ballot(valid && 4.0 * double(hi) * (1.0 + 1e-6) >= a.minLen));
+    const unsigned taken = __popcll(ballot(valid));
     // largest h: sets the fixed-point period of the FP32 pair loops
     const double hMax = waveMaxD(valid ? double(hi) : 0.0);
     if (lane == 0)
     {
-        a.groupStats[g] = {hMax, stored, mx, fails, wide, out.swept, oversized ? 1u : 0u};
+        a.groupStats[g] = {hMax, stored, mx, out.swept, uint16_t(fails), uint16_t(wide), uint16_t(oversized ? 1 : 0),
+                           uint16_t(taken)};
         if constexpr (Local) { a.tableCount[g] = out.inTable; }
     }
 }
 
 /*! Statistics of the search from its groups': stats[0] stored pairs, [1] max count, [2] non-converged particles,
  * [kStatWide] wide support, [kStatTests] candidate distance tests (swept candidates x 64 lanes),
- * [kStatBadGroups], [kStatHMax]; with tableCount also the histogram of the groups' table sizes: bin s / kTableBin, the
+ * [kStatBadGroups], [kStatHMax], [kStatTargets]; with tableCount also the histogram of the groups' table sizes: bin s / kTableBin, the
  * last one for tables that did not fit. One block's atomics per slot. */
 __global__ void __launch_bounds__(256)
     groupStatsKernel(const GroupStat* __restrict__ groupStats, const uint32_t* __restrict__ tableCount, uint32_t groups,
@@ -1156,13 +1161,13 @@ __global__ void __launch_bounds__(256)
     if (threadIdx.x < 6) { sum[threadIdx.x] = 0; }
     if (threadIdx.x == 0) { hBits = 0, most = 0; }
     __syncthreads();
-    unsigned long long v[5] = {};
+    unsigned long long v[6] = {};
     double             hMax = 0.0;
     uint32_t           mx   = 0;
     for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < groups; g += gridDim.x * blockDim.x)
     {
         const GroupStat q = groupStats[g];
-        v[0] += q.stored, v[1] += q.fails, v[2] += q.wide, v[3] += q.swept, v[4] += q.bad;
+        v[0] += q.stored, v[1] += q.fails, v[2] += q.wide, v[3] += q.swept, v[4] += q.bad, v[5] += q.targets;
         mx   = max(mx, q.maxCount);
         hMax = fmax(hMax, q.hMax);
         if (tableCount != nullptr)
@@ -1171,13 +1176,13 @@ __global__ void __launch_bounds__(256)
             atomicAdd(&part[s > kTableCap ? kTableBins : (s == 0 ? 0 : (s - 1) / kTableBin)], 1u);
         }
     }
-    for (int k = 0; k < 5; ++k)
+    for (int k = 0; k < 6; ++k)
         v[k] = waveSum(v[k]);
     mx   = waveMax(mx);
     hMax = waveMaxD(hMax);
     if (laneId() == 0)
     {
-        for (int k = 0; k < 5; ++k)
+        for (int k = 0; k < 6; ++k)
             atomicAdd(&sum[k], v[k]);
         atomicMax(&most, mx);
         // positive doubles order as their bit patterns
@@ -1193,6 +1198,7 @@ __global__ void __launch_bounds__(256)
         if (sum[2]) { atomicAdd(&stats[kStatWide], sum[2]); }
         atomicAdd(&stats[kStatTests], sum[3] * kWave);
         if (sum[4]) { atomicAdd(&stats[kStatBadGroups], sum[4]); }
+        atomicAdd(&stats[kStatTargets], sum[5]);
     }
     uint32_t* hist = reinterpret_cast<uint32_t*>(stats + kStatHist);
     if (threadIdx.x <= kTableBins && part[threadIdx.x]) { atomicAdd(&hist[threadIdx.x], part[threadIdx.x]); }
@@ -1269,7 +1275,7 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     // would outgrow the lists, and the search stores global lists (4 bytes a slot)
     const size_t blocks64    = std::max<size_t>(1, ceilDiv(last - first, kGroup));
     const bool   tryLocal    = xmassOut == kSearchOnly && groups <= 2 * blocks64 + 64;
-    const bool   owned       = tryLocal && grp.start != nullptr;
+    const bool   owned       = grp.start != nullptr;
     const size_t localWords  = blocks64 * paddedNgmax8(p->ngmax) * kGroup / 2;
     const size_t globalWords = blocks64 * paddedNgmax(p->ngmax) * kGroup;
     ws->nbrs.reserve(tryLocal ? localWords : globalWords);
@@ -1278,12 +1284,8 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
         ws->nbTable.reserve(std::max<size_t>(1, groups) * kTableCap);
         ws->nbTableCount.reserve(std::max<size_t>(1, groups));
     }
-    if (owned)
-    {
-        const size_t pairs = (size_t(last - first) + 1) / 2; // two owners per 64-bit word
-        ws->nbOwner.reserve(2 * std::max<size_t>(1, pairs));
-        fill64(ws, reinterpret_cast<uint64_t*>(ws->nbOwner.get()), ~uint64_t(0), pairs);
-    }
+    const size_t ownerPairs = owned ? (size_t(last - first) + 1) / 2 : 0; // two owners per 64-bit word
+    if (owned) { ws->nbOwner.reserve(2 * std::max<size_t>(1, ownerPairs)); }
     ws->counters.reserve(2 * kCounterSlots);
 
     double scale = 0;
@@ -1334,6 +1336,8 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     {
         clearStatsKernel<<<1, kWave, 0, ws->stream>>>(reinterpret_cast<unsigned long long*>(ws->counters.get()));
         SPHX_CHECK_LAUNCH();
+        static_assert(NeighborLists::kNoGroup == 0xffffffffu, "the fill value");
+        if (ownerPairs) { fill64(ws, reinterpret_cast<uint64_t*>(ws->nbOwner.get()), ~uint64_t(0), ownerPairs); }
         if (groups > 0)
         {
             unsigned    blocks = ceilDiv(groups, kWavesPerBlock);
@@ -1383,7 +1387,8 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     ws->nbNc         = f->nc;
     ws->nbValid      = true;
     ws->nbLocal      = local;
-    ws->nbOwned      = local && owned;
+    ws->nbOwned      = owned;
+    ws->nbPartial    = owned && stats[kStatTargets] < uint64_t(last - first);
     std::memcpy(ws->nbTableHist, hist, sizeof(hist));
     ++ws->searchSerial;
     ws->statSumPairs = stats[0];
@@ -1416,6 +1421,8 @@ void copyNeighbors(sphx_workspace* ws, uint32_t* out, uint32_t first, uint32_t l
     {
         staging.reserve(len);
         dst = staging.get();
+        // the rows of targets without a list stay as they are
+        if (ws->nbPartial) { SPHX_HIP(hipMemcpyAsync(dst, out, len * sizeof(uint32_t), hipMemcpyHostToDevice, ws->stream)); }
     }
     // the list blocks that hold [first, last)
     const uint32_t blocks = (last - 1 - ws->nbFirst) / kGroup - (first - ws->nbFirst) / kGroup + 1;

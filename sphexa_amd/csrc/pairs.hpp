@@ -69,6 +69,7 @@ struct Lists
     uint32_t        first, last, ngmax; // [first, last): the searched targets
     uint32_t        stage;              // records the launch's LDS holds
     uint32_t        block0;             // list block of the call's first group, whose targets are whole blocks; or kNoBlock
+    bool            partial;            // the search left targets of its range out
     Groups          groups;             // the call's target groups
 };
 
@@ -82,7 +83,8 @@ struct Lane
 };
 
 /*! lane l takes the l-th target of group g; its list is that of the (i - first)-th searched target,
- * whatever the grouping. Targets outside the searched range [first, last) are not taken. */
+ * whatever the grouping. Targets outside the searched range [first, last), and those that the search's view
+ * left out, are not taken: a call leaves their results as they were. */
 __device__ __forceinline__ Lane groupTarget(const Lists& L, uint32_t g)
 {
     Lane     t;
@@ -91,10 +93,10 @@ __device__ __forceinline__ Lane groupTarget(const Lists& L, uint32_t g)
     if (g < L.groups.num) { groupRange(L.groups, g, i0, i1, oversized); }
     t.i     = i0 + threadIdx.x % kWave;
     t.valid = t.i < i1 && t.i >= L.first && t.i < L.last;
+    t.valid = t.valid && L.lists.searched(t.i - L.first);
     t.n     = t.valid ? min(L.nc[t.i] - 1, L.ngmax) : 0u;
     t.i     = t.valid ? t.i : L.first;
     t.r     = t.i - L.first;
-    if (!L.lists.searched(t.r)) { t.n = 0; }
     return t;
 }
 
@@ -976,7 +978,7 @@ inline PairArgs makePairArgs(sphx_workspace* ws, const DevBox& box, const sphx_f
     const Groups G = groupsFor(ws, first, last);
     const bool   whole = !ws->nbOwned && G.start == nullptr && (first - ws->nbFirst) % kGroup == 0;
     c.L = Lists{neighborLists(ws), f->nc,    ws->nbFirst, ws->nbLast, p->ngmax, 0,
-                whole ? (first - ws->nbFirst) / kGroup : Lists::kNoBlock, G};
+                whole ? (first - ws->nbFirst) / kGroup : Lists::kNoBlock, ws->nbPartial, G};
     c.numParticles = uint32_t(ws->tree.numParticles);
     return c;
 }

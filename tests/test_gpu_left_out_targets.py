@@ -1,6 +1,9 @@
-"""Targets that a search's group view left out have no list: a copy of the lists over the whole range leaves their rows
-alone, and the adjoints take them with no neighbour. Ranges off the list blocks of 64, and counts off the rounds of the
-copy (ragged n, ngmax not a multiple of its rounds)."""
+"""Targets that a search's group view left out have no list, in either list layout: a copy of the lists over the whole
+range leaves their rows alone, the adjoints take them with no neighbour and the pair loops leave their results as they
+were. Searches that store table positions, and those that store particle indices after an earlier search of
+table positions (many small groups, tables that do not fit, the fused search). Ranges off the list blocks of
+64, and counts off the rounds of the copy (ragged n, ngmax not a multiple of its rounds). A target in two groups of
+the view has the list that it has in one."""
 import numpy as np
 import pytest
 
@@ -10,54 +13,123 @@ from sphexa_amd.particles import STD_FIELDS, ParticleSet
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("ngmax", [90, 150])
-def test_left_out_targets_have_no_list(ngmax):
-    import torch
+class Case:
+    def __init__(self, ngmax, side=11, h_factor=1.0):
+        from sphexa_amd.lib import Workspace
 
-    from sph_autograd import adjoint
-    from sphexa_amd.lib import Workspace
+        arr, spec = ic.sedov_lattice(side, seed=2)
+        arr["h"] = arr["h"] * h_factor
+        self.ws = Workspace(0)
+        self.params = abi.Params.defaults(self.ws.K, ngmax=ngmax, ng0=60)
+        self.box = abi.Box.make(spec["lo"], spec["hi"], abi.PERIODIC)
+        self.ps = ParticleSet.from_host(arr, STD_FIELDS)
+        self.n, self.ngmax = self.ps.n, ngmax
+        self.ws.domain_sync(self.box, self.ps.sync_fields(), self.params, self.n)
 
-    arr, spec = ic.sedov_lattice(11, seed=2)
-    ws = Workspace(0)
-    params = abi.Params.defaults(ws.K, ngmax=ngmax, ng0=60)
-    box = abi.Box.make(spec["lo"], spec["hi"], abi.PERIODIC)
-    ps = ParticleSet.from_host(arr, STD_FIELDS)
-    n = ps.n
-    ws.domain_sync(box, ps.sync_fields(), params, n)
+    def search(self, fused=False):
+        find = self.ws.find_neighbors_xmass if fused else self.ws.find_neighbors
+        find(self.box, self.ps.fields(), self.params, 0, self.n, False, **({"rho": True} if fused else {}))
 
-    def lists(first, last):
-        out = torch.full((last - first, ngmax), -1, dtype=torch.int32, device="cuda")
-        ws.copy_neighbors(out, first, last)
+    def lists(self, first, last, host=False):
+        import torch
+
+        out = torch.full((last - first, self.ngmax), -1, dtype=torch.int32, device="cpu" if host else "cuda")
+        self.ws.copy_neighbors(out, first, last)
         return out.cpu().numpy()
 
-    def density_vjp(cot):
-        out = {k: torch.zeros(n, dtype=torch.float64, device="cuda") for k in ("x", "y", "z", "h")}
-        ws.vjp("sphx_density_std_vjp", box, ps.fields(), params, 0, n, adjoint({"rho": cot}), adjoint(out))
+    def density_vjp(self, cot):
+        import torch
+
+        from sph_autograd import adjoint
+
+        out = {k: torch.zeros(self.n, dtype=torch.float64, device="cuda") for k in ("x", "y", "z", "h")}
+        self.ws.vjp("sphx_density_std_vjp", self.box, self.ps.fields(), self.params, 0, self.n, adjoint({"rho": cot}),
+                    adjoint(out))
         return {k: v.cpu().numpy() for k, v in out.items()}
 
-    ws.find_neighbors(box, ps.fields(), params, 0, n, False)
-    whole, stored = lists(0, n), np.minimum(ps.host("nc").astype(np.int64) - 1, ngmax)
+    def loops(self, chain):
+        """std pair loops over the whole range, every result a sentinel before"""
+        keys = ("rho", "c11", "c23", "ax", "du")
+        for k in keys:
+            self.ps.t[k].fill_(-7.0)
+        p, f = abi.chained(self.params) if chain else self.params, self.ps.fields()
+        self.ps.t["rho"].fill_(1.0)  # a density that the left-out targets keep
+        self.ws.pair("sphx_density_std", self.box, f, p, 0, self.n)
+        self.ws.eos("sphx_eos_std", f, self.params, 0, self.n)
+        self.ws.pair("sphx_iad_std", self.box, f, p, 0, self.n)
+        return {k: self.ps.host(k).copy() for k in ("rho", "c11", "c23")}
+
+    def view(self, width, every):
+        """groups of `width` consecutive particles, one in `every`; the mask of their targets"""
+        import torch
+
+        self.start = torch.arange(0, self.n, width * every, dtype=torch.int32, device="cuda")
+        self.end = torch.clamp(self.start + width, max=self.n)
+        chosen = np.zeros(self.n, bool)
+        for a, b in zip(self.start.cpu().numpy(), self.end.cpu().numpy()):
+            chosen[a:b] = True
+        return chosen
+
+    def set_view(self):
+        view = abi.Groups(firstBody=0, lastBody=self.n, numGroups=self.start.numel())
+        view.groupStart, view.groupEnd = self.start.data_ptr(), self.end.data_ptr()
+        self.ws.set_groups(view)
+
+
+@pytest.mark.parametrize("ngmax", [90, 150])
+@pytest.mark.parametrize("layout", ["tables", "many_groups", "overflow", "fused"])
+def test_left_out_targets_have_no_list(layout, ngmax):
+    import torch
+
+    # groups of 4, every second: 8 per block of 64, more than whose tables are kept; 3.5 times the smoothing
+    # length: tables of thousands of particles
+    c = Case(ngmax, side=20, h_factor=3.5) if layout == "overflow" else Case(ngmax)
+    c.search()
+    whole, stored = c.lists(0, c.n), np.minimum(c.ps.host("nc").astype(np.int64) - 1, ngmax)
     assert np.array_equal((whole >= 0).sum(1), stored) and np.all(whole[:, 0] >= 0)
-    part = lists(70, n - 3)
-    np.testing.assert_array_equal(part, whole[70:n - 3])
+    np.testing.assert_array_equal(c.lists(70, c.n - 3), whole[70:c.n - 3])
+    every = c.loops(chain=False)
 
-    start = torch.arange(0, n, 64, dtype=torch.int32, device="cuda")[::2].contiguous()
-    end = torch.clamp(start + 64, max=n)
-    chosen = np.zeros(n, bool)
-    for a, b in zip(start.cpu().numpy(), end.cpu().numpy()):
-        chosen[a:b] = True
+    chosen = c.view(4 if layout == "many_groups" else 64, 2)
     rng = np.random.default_rng(1)
-    cot = torch.from_numpy(np.where(chosen, rng.standard_normal(n), 0.0)).cuda()
-    want = density_vjp(cot)
+    cot = torch.from_numpy(np.where(chosen, rng.standard_normal(c.n), 0.0)).cuda()
+    want = c.density_vjp(cot)
 
-    view = abi.Groups(firstBody=0, lastBody=n, numGroups=start.numel())
-    view.groupStart, view.groupEnd = start.data_ptr(), end.data_ptr()
-    ws.set_groups(view)
-    ws.find_neighbors(box, ps.fields(), params, 0, n, False)
-    ws.set_groups(None)
-    some = lists(0, n)
-    np.testing.assert_array_equal(some[chosen], whole[chosen])
-    assert np.all(some[~chosen] == -1)
-    got = density_vjp(cot)
+    c.set_view()
+    c.search(fused=layout == "fused")
+    c.ws.set_groups(None)
+    for host in (False, True):
+        some = c.lists(0, c.n, host)
+        np.testing.assert_array_equal(some[chosen], whole[chosen])
+        assert np.all(some[~chosen] == -1)
+    got = c.density_vjp(cot)
     for k in want:
         np.testing.assert_array_equal(got[k], want[k], err_msg=k)
+    plain, chained = c.loops(chain=False), c.loops(chain=True)
+    np.testing.assert_array_equal(plain["rho"][chosen], every["rho"][chosen])
+    assert np.all(plain["rho"][~chosen] == 1.0)
+    for k in ("c11", "c23"):
+        assert np.all(plain[k][~chosen] == -7.0) and not np.any(plain[k][chosen] == -7.0)
+    for k in plain:
+        np.testing.assert_array_equal(chained[k], plain[k], err_msg=k)
+
+
+@pytest.mark.parametrize("width,step", [(64, 40), (30, 15)])  # 34 and 89 groups: tables, and particle indices below
+@pytest.mark.parametrize("tiny", [False, True])
+def test_targets_in_two_groups(width, step, tiny):
+    """a view whose groups overlap: every target is searched, and its list is that of one group"""
+    import torch
+
+    c = Case(150)
+    if tiny:
+        width, step = 8, 5
+    c.search()
+    whole, nc, rho = c.lists(0, c.n), c.ps.host("nc").copy(), c.loops(chain=False)["rho"]
+    c.start = torch.arange(0, c.n, step, dtype=torch.int32, device="cuda")
+    c.end = torch.clamp(c.start + width, max=c.n)
+    c.set_view()
+    c.search()
+    c.ws.set_groups(None)
+    np.testing.assert_array_equal(c.ps.host("nc"), nc)
+    np.testing.assert_array_equal(c.lists(0, c.n), whole)
+    np.testing.assert_array_equal(c.loops(chain=False)["rho"], rho)
