@@ -286,6 +286,7 @@ struct sphx_workspace
     {
         int           kind   = 0; // record type written (0: none)
         uint64_t      serial = 0; // callSerial of the producing call
+        int           alpha  = 0; // its SPHX_FLAG_STD_ALPHA
         uint32_t      n      = 0;
         int           form   = -1;
         int           buf    = 0; // record buffer holding them

@@ -136,7 +136,7 @@ enum ChainKind
     kChainAv    = 1, // sphx_iad_divv_curlv -> sphx_av_switches
     kChainMomVe = 2, // sphx_av_switches -> sphx_momentum_energy_ve
     kChainGradh = 3, // sphx_xmass -> sphx_ve_def_gradh
-    kChainMomStd = 4, // sphx_iad_std -> sphx_momentum_energy_std
+    kChainMomStd = 4, // sphx_iad_std -> sphx_momentum_energy_std (the AV coefficients of one SPHX_FLAG_STD_ALPHA)
     kChainIadVe  = 5, // sphx_ve_def_gradh -> (sphx_eos_ve) -> sphx_iad_divv_curlv
     kChainVol    = 6  // sphx_density_std -> (sphx_eos_std) -> sphx_iad_std
 };
@@ -161,6 +161,7 @@ inline int takeChain(sphx_workspace* ws, int kind, const PairArgs& a, const sphx
                    std::memcmp(&ws->eosFields, f, sizeof(*f)) == 0;
     bool ok = chainable(a, p) && c.kind == kind && (next || overEos) && c.n == a.numParticles &&
               c.form == p->hydro_type && std::memcmp(&c.fields, f, sizeof(*f)) == 0;
+    if (kind == kChainMomStd) { ok = ok && c.alpha == (p->flags & SPHX_FLAG_STD_ALPHA); }
     for (int k = 0; k < 3; ++k)
     {
         ok = ok && c.lo[k] == a.box.lo[k] && c.hi[k] == a.box.hi[k] && c.pbc[k] == a.box.pbc[k];
@@ -178,6 +179,7 @@ inline void leaveChain(sphx_workspace* ws, int kind, int buf, const PairArgs& a,
     c.n      = a.numParticles;
     c.form   = p->hydro_type;
     c.buf    = buf;
+    c.alpha  = p->flags & SPHX_FLAG_STD_ALPHA;
     c.fields = *f;
     for (int k = 0; k < 3; ++k)
     {
