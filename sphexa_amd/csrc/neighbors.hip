@@ -300,6 +300,7 @@ struct TargetMatrix
     double origin[3]; // the group's centre
     double scale;
     bool   each;      // every candidate within reach has one image for all targets (kEachImage)
+    bool   usable;    // the group's size allows the scaling
     float  b[4];      // per block of 16 targets: this lane's element, -2 t (component lane / 16) or 1
     float  diff[4];   // per block: |t|^2 - r^2 of this lane's column
 };
@@ -312,7 +313,9 @@ struct TargetMatrix
  *
  * With all coordinates at most 1 in size the product is within 21 * 2^-24 of the exact value (rounding of the
  * coordinates 3, of |p|^2 and |t|^2 - r^2 2, of the sums 16); `close` is set when any element is within 2^-19 of zero,
- * and the tile is then tested exactly. That leaves the reference's FP64 predicate for every pair. About 3% of
+ * and the tile is then tested exactly. That leaves the reference's FP64 predicate for every pair: a candidate with a
+ * coordinate that is not finite, and a target whose coordinates or radius are not numbers, have no hits there and none
+ * here, and groups out of the range of the scale are tested exactly throughout (TargetMatrix::usable). About 3% of
  * the tiles on a lattice are tested twice. The vector ALU spends 1.5 instructions per candidate here and 11 in
  * exactMask, where this loop was two fifths of the search. */
 template<class Lds>
@@ -333,6 +336,7 @@ __device__ __forceinline__ uint64_t tileMask(const DevBox& box, Lds& lds, int bu
         }
         p[0] = float(q[0] * g.scale), p[1] = float(q[1] * g.scale), p[2] = float(q[2] * g.scale);
         p[3] = float(double(p[0]) * double(p[0]) + double(p[1]) * double(p[1]) + double(p[2]) * double(p[2]));
+        if (!(p[3] < INFINITY)) { p[0] = p[1] = p[2] = 0.0f, p[3] = 4.0f; } // (the sign of a NaN would pass for a hit)
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -460,7 +464,7 @@ __device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, 
     bool           exact   = true;
     if constexpr (!Sink::kStageMass)
     {
-        if (code != kPerPairImage) { m = tileMask(a.box, lds, buf, n, g, shift, code == kEachImage, exact); }
+        if (code != kPerPairImage && g.usable) { m = tileMask(a.box, lds, buf, n, g, shift, code == kEachImage, exact); }
     }
     if (exact)
     {
@@ -868,7 +872,8 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
     {
         // every kept candidate and every target within 1 of the centre after scaling, and every separation
         const double size = 2.0 * sqrt(ge[0] * ge[0] + ge[1] * ge[1] + ge[2] * ge[2]) + reach;
-        g.scale           = size > 0.0 && size < 1e300 ? ldexp(1.0, -(ilogb(size) + 1)) : 1.0;
+        g.usable          = size > 1e-150 && size < 1e150; // (the squares of the scale and the size stay in range)
+        g.scale           = g.usable ? ldexp(1.0, -(ilogb(size) + 1)) : 1.0;
         float q[3], diff;
         for (int d = 0; d < 3; ++d)
         {
@@ -878,7 +883,7 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
         diff = t.active ? float(double(q[0]) * double(q[0]) + double(q[1]) * double(q[1]) + double(q[2]) * double(q[2]) -
                                 t.r2 * (g.scale * g.scale))
                         : 4.0f; // no hits
-        if (!(fabsf(q[0]) + fabsf(q[1]) + fabsf(q[2]) < 4.0f)) { q[0] = q[1] = q[2] = 0.0f, diff = 4.0f; } // NaN: none
+        if (!(fabsf(q[0]) + fabsf(q[1]) + fabsf(q[2]) < 4.0f) || diff != diff) { q[0] = q[1] = q[2] = 0.0f, diff = 4.0f; } // NaN: none
         for (int b4 = 0; b4 < 4; ++b4)
         {
             const int   col = 16 * b4 + int(lane % 16);

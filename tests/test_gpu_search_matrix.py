@@ -54,3 +54,47 @@ def test_lists_equal_the_oracles(case):
     used = np.arange(params.ngmax)[None, :] < stored[:, None]
     assert used.any()
     np.testing.assert_array_equal(got[used], ref[used])
+
+
+@pytest.mark.parametrize("boundary", [abi.PERIODIC, abi.OPEN])
+@pytest.mark.parametrize("value", [np.nan, -np.nan, np.inf])
+@pytest.mark.parametrize("what", ["x", "z", "h"])
+def test_particle_that_is_not_finite(what, value, boundary):
+    """a particle with a coordinate or smoothing length that is not a number is nobody's neighbour, and has none; the
+    others' lists are those of the same search without it. An infinite coordinate is likewise out of every reach."""
+    import torch
+
+    from sphexa_amd.lib import Workspace
+
+    if what == "h" and np.isinf(value):
+        pytest.skip("an infinite support holds every particle")
+    side = 20
+    rng = np.random.default_rng(9)
+    g = (np.arange(side) + 0.5) / side
+    x, y, z = (c.ravel() + rng.uniform(-0.3, 0.3, side**3) / side for c in np.meshgrid(g, g, g, indexing="ij"))
+    n = x.size
+    arr = dict(x=x, y=y, z=z, h=np.full(n, 1.25 / side), m=np.full(n, 1.0 / n), u=np.ones(n), vx=0 * x, vy=0 * x, vz=0 * x)
+    box = abi.Box.make(0.0, 1.0, boundary)
+    ws = Workspace(0)
+    params = abi.Params.defaults(ws.K)
+    ps = ParticleSet.from_host(arr, STD_FIELDS)
+    ws.domain_sync(box, ps.sync_fields(), params, n)
+
+    def lists():
+        out = torch.full((n, params.ngmax), -1, dtype=torch.int32, device="cuda")
+        ws.find_neighbors(box, ps.fields(), params, 0, n, False)
+        ws.copy_neighbors(out, 0, n)
+        return out.cpu().numpy(), ps.host("nc").astype(np.int64) - 1
+
+    # the particles go bad after the sync, as in a run that diverges between two syncs: each in another group
+    bad = np.array([5, 700, 3001, n - 1])
+    before, count = lists()
+    ps.t[what][torch.from_numpy(bad).cuda()] = value
+    after, countAfter = lists()
+    np.testing.assert_array_equal(countAfter[bad], 0)
+    is_bad = np.isin(np.arange(n), bad)
+    for i in np.flatnonzero(~is_bad):
+        want = before[i, : count[i]]
+        if what != "h":
+            want = want[~np.isin(want, bad)]
+        np.testing.assert_array_equal(after[i, : countAfter[i]], want, err_msg=str(i))
