@@ -385,6 +385,7 @@ void buildLinked(sphx_workspace* ws, const Key* keys, size_t nParticles, unsigne
     const uint32_t n      = uint32_t(nParticles);
     auto&          s      = ws->tree.build;
     const uint32_t blocks = std::max(1u, ceilDiv(n, kPlanKeys));
+    ws->tree.valid        = false; // until it is linked: no search over the former tree, or half of this one, after an error
     s.planCounts.reserve(size_t(blocks) * kPlanRows + kPlanRows);
     uint32_t* counts = s.planCounts.get();
     uint32_t* totals = counts + size_t(blocks) * kPlanRows;
