@@ -1272,6 +1272,13 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     SPHX_REQUIRE(p->ng0 <= p->ngmax, SPHX_ERR_ARG, "ng0 should be smaller than ngmax");
     SPHX_REQUIRE(p->ngmax > 0, SPHX_ERR_ARG, "ngmax must be positive");
 
+    SPHX_REQUIRE(xmassOut == kSearchOnly || ws->tablesValid, SPHX_ERR_STATE,
+                 "kernel tables not set (sphx_workspace_set_kernel)");
+    SPHX_REQUIRE(xmassOut == kSearchOnly || (f->m && (xmassOut == kSearchRho ? f->rho : f->xm)), SPHX_ERR_ARG,
+                 "the fused XMass needs m and its output field (xm or rho)");
+    // from here on the former lists are overwritten: they are gone unless this search completes
+    ws->nbValid = false;
+
     const Tree&  t      = ws->tree;
     const Groups grp    = groupsFor(ws, first, last);
     const uint32_t groups = grp.num;
@@ -1323,15 +1330,12 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     const bool f32 = p->hydro_type == SPHX_F32;
     if (xmassOut != kSearchOnly)
     {
-        SPHX_REQUIRE(ws->tablesValid, SPHX_ERR_STATE, "kernel tables not set (sphx_workspace_set_kernel)");
-        void* outField = xmassOut == kSearchRho ? f->rho : f->xm;
-        SPHX_REQUIRE(f->m && outField, SPHX_ERR_ARG, "the fused XMass needs m and its output field (xm or rho)");
         a.m     = f->m;
         a.wh    = ws->wh64.get();
         a.sincN   = sincKernel<float>(ws).n;
         a.sincInt = sincKernel<float>(ws).ni;
         a.K     = p->K;
-        a.xmOut = outField;
+        a.xmOut = xmassOut == kSearchRho ? f->rho : f->xm;
         a.toRho = xmassOut == kSearchRho;
     }
 
@@ -1390,7 +1394,6 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     ws->nbLast       = last;
     ws->nbNgmax      = p->ngmax;
     ws->nbNc         = f->nc;
-    ws->nbValid      = true;
     ws->nbLocal      = local;
     ws->nbOwned      = owned;
     ws->nbPartial    = owned && stats[kStatTargets] < uint64_t(last - first);
@@ -1403,9 +1406,9 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     std::memcpy(&ws->nbHMax, &stats[kStatHMax], sizeof(double));
     if (stats[kStatBadGroups] > 0)
     {
-        ws->nbValid = false;
         throw Error{SPHX_ERR_ARG, std::to_string(stats[kStatBadGroups]) + " target groups hold more than 64 particles"};
     }
+    ws->nbValid = true;
     return fails > 0 ? SPHX_ERR_NOT_CONVERGED : SPHX_OK;
 }
 

@@ -45,3 +45,35 @@ def test_keys_out_of_order(case):
     ws.build_tree(keys, box)
     search()
     np.testing.assert_array_equal(ps.host("nc"), nc)
+
+
+@pytest.mark.parametrize("fused", [False, True])
+def test_search_without_room_for_its_lists(case, fused):
+    """lists of 2^30 entries a target (TiB) cannot be allocated: the search reports it and the pair loops and copies say
+    that there are no lists, rather than reading the former ones' memory; a later search works"""
+    ws, box, ps, params = case
+    nc, rho = ps.host("nc").copy(), ps.host("rho").copy()
+    large = abi.Params.from_buffer_copy(params)
+    large.ngmax = 1 << 30
+    find, out = (ws.find_neighbors_xmass, dict(rho=True)) if fused else (ws.find_neighbors, {})
+    assert code_of(lambda: find(box, ps.fields(), large, 0, ps.n, False, **out)) == abi.SPHX_ERR_ALLOC
+    out = ps.t["nc"].new_zeros(ps.n * params.ngmax)
+    assert code_of(lambda: ws.copy_neighbors(out, 0, ps.n)) == abi.SPHX_ERR_STATE
+    assert code_of(lambda: ws.pair("sphx_density_std", box, ps.fields(), params, 0, ps.n)) == abi.SPHX_ERR_STATE
+    ws.find_neighbors(box, ps.fields(), params, 0, ps.n, False)
+    ws.pair("sphx_density_std", box, ps.fields(), params, 0, ps.n)
+    np.testing.assert_array_equal(ps.host("nc"), nc)
+    np.testing.assert_array_equal(ps.host("rho"), rho)
+
+
+def test_refused_search_keeps_the_lists(case):
+    """a search refused for its arguments has touched nothing: the former lists serve on"""
+    ws, box, ps, params = case
+    rho = ps.host("rho").copy()
+    wrong = abi.Params.from_buffer_copy(params)
+    wrong.ng0 = wrong.ngmax + 1
+    assert code_of(lambda: ws.find_neighbors(box, ps.fields(), wrong, 0, ps.n, False)) == abi.SPHX_ERR_ARG
+    # (the std fields hold no xm)
+    assert code_of(lambda: ws.find_neighbors_xmass(box, ps.fields(), params, 0, ps.n, False)) == abi.SPHX_ERR_ARG
+    ws.pair("sphx_density_std", box, ps.fields(), params, 0, ps.n)
+    np.testing.assert_array_equal(ps.host("rho"), rho)
