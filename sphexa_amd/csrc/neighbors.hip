@@ -1068,12 +1068,12 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     Target t;
     t.i      = base + lane;
     t.active = t.i < end;
-    // a target of two groups is the first one's alone: its list refers to one table
-    if (a.owner && t.active) { t.active = atomicCAS(&a.owner[t.i - a.first], NeighborLists::kNoGroup, g) == NeighborLists::kNoGroup; }
     Th hi    = t.active ? h[t.i] : Th(0);
     t.x      = t.active ? a.x[t.i] : 0.0;
     t.y      = t.active ? a.y[t.i] : 0.0;
     t.z      = t.active ? a.z[t.i] : 0.0;
+    // a target of two groups is the first one's alone: its list refers to one table
+    if (a.owner && t.active) { t.active = atomicCAS(&a.owner[t.i - a.first], NeighborLists::kNoGroup, g) == NeighborLists::kNoGroup; }
     setRadius(t, hi, a.slack);
     // lists are indexed by particle: target i at group (i - first) / 64, lane (i - first) % 64
     const uint32_t    r = t.active ? t.i - a.first : 0u;

@@ -93,10 +93,13 @@ __device__ __forceinline__ Lane groupTarget(const Lists& L, uint32_t g)
     if (g < L.groups.num) { groupRange(L.groups, g, i0, i1, oversized); }
     t.i     = i0 + threadIdx.x % kWave;
     t.valid = t.i < i1 && t.i >= L.first && t.i < L.last;
-    t.valid = t.valid && L.lists.searched(t.i - L.first);
-    t.n     = t.valid ? min(L.nc[t.i] - 1, L.ngmax) : 0u;
     t.i     = t.valid ? t.i : L.first;
     t.r     = t.i - L.first;
+    // (both loads go out together)
+    const bool     searched = L.lists.searched(t.r);
+    const uint32_t nc       = L.nc[t.i];
+    t.valid                 = t.valid && searched;
+    t.n                     = t.valid ? min(nc - 1, L.ngmax) : 0u;
     return t;
 }
 
