@@ -94,7 +94,7 @@ __global__ void __launch_bounds__(kLightWaves * kWave)
     const T          scale = kernelScale(a.box, hInv);
     double           r2h   = 2.0 * double(hi);
     double           sum[1] = {0.0};
-    PairWalk<kLightWaves, isMixed<T> ? 4 : 2, RecMass<T>> walk(a.L, t, rec);
+    PairWalk<kLightWaves, kLightBatch<T>, kLightGather<T, V>, RecMass<T>> walk(a.L, t, rec);
     withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
         walk([&](bool live, const RecMass<T>& rj) {
             const T d2 = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj).d2;
@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(kLightWaves * kWave) SPHX_LIGHT_WAVES(T)
     T               hiInv = T(1) / hi, scale = kernelScale(a.box, hiInv);
     double          r2h   = 2.0 * double(hi);
     T               t11 = 0, t12 = 0, t13 = 0, t22 = 0, t23 = 0, t33 = 0;
-    PairWalk<kLightWaves, isMixed<T> ? 4 : 2, RecVol<T>> walk(a.L, t, rec);
+    PairWalk<kLightWaves, kLightBatch<T>, kLightGather<T, V>, RecVol<T>> walk(a.L, t, rec);
     withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
         walk([&](bool live, const RecVol<T>& rj) {
             const Sep<T> r = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj);
@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(kMomWaves<T> * kWave)
     T      maxvs = 0;
     T      momx = 0, momy = 0, momz = 0;
     double energy = 0.0;
-    PairWalk<kMomWaves<T>, isMixed<T> ? 2 : 1, RecMomStd<T>> walk(a.L, t, rec);
+    PairWalk<kMomWaves<T>, kMomBatch<T>, kMomGather<T, V>, RecMomStd<T>> walk(a.L, t, rec);
     withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
         walk([&](bool live, const RecMomStd<T>& rj) {
             const Sep<T> r = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj);

@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(kLightWaves * kWave) SPHX_LIGHT_WAVES(T)
     double            r2h  = 2.0 * double(hi);
     const T           scale = kernelScale(a.box, hInv);
     double            sum[3] = {0.0, 0.0, 0.0}; // of W xm_j, dterh xm_j, dterh m_j
-    PairWalk<kLightWaves, isMixed<T> ? 4 : 2, RecGradh<T>> walk(a.L, t, rec);
+    PairWalk<kLightWaves, kLightBatch<T>, kLightGather<T, V>, RecGradh<T>> walk(a.L, t, rec);
     withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
         walk([&](bool live, const RecGradh<T>& rj) {
             const T d2 = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj).d2;
@@ -202,7 +202,7 @@ __global__ void __launch_bounds__(kLightWaves * kWave) SPHX_LIGHT_WAVES(T)
     double            r2h   = 2.0 * double(hi);
     T                 t11 = 0, t12 = 0, t13 = 0, t22 = 0, t23 = 0, t33 = 0;
     T                 m11 = 0, m12 = 0, m13 = 0, m21 = 0, m22 = 0, m23 = 0, m31 = 0, m32 = 0, m33 = 0;
-    PairWalk<kLightWaves, isMixed<T> ? 4 : 2, RecIadVe<T>> walk(a.L, t, rec);
+    PairWalk<kLightWaves, kLightBatch<T>, kLightGather<T, V>, RecIadVe<T>> walk(a.L, t, rec);
     withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
         walk([&](bool live, const RecIadVe<T>& rj) {
             const Sep<T> r = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj);
@@ -297,7 +297,7 @@ __global__ void __launch_bounds__(kLightWaves * kWave) SPHX_LIGHT_WAVES(T)
     double         r2h   = 2.0 * double(hi);
     T              vsig  = T(1.e-40) * ri.c;
     T              S0 = 0, S1 = 0, S2 = 0;
-    PairWalk<kLightWaves, isMixed<T> ? 4 : 2, RecAv<T>> walk(a.L, t, rec);
+    PairWalk<kLightWaves, kLightBatch<T>, kLightGather<T, V>, RecAv<T>> walk(a.L, t, rec);
     withFold(recordNeedsFold<T, V>(a.box, t, ri, r2h), [&](auto fold) {
         walk([&](bool live, const RecAv<T>& rj) {
             const Sep<T> r = pairSeparation<decltype(fold)::value, V, T>(a.box, r2h, ri, rj);
@@ -496,7 +496,7 @@ __global__ void __launch_bounds__((kMomWaves<T, avClean> * kWave))
     const bool needFold = recordNeedsFold<T, V>(a.box, t, ri, r2h);
     if constexpr (avClean)
     {
-        PairWalk<kMomWaves<T, avClean>, isMixed<T> ? 2 : 1, RecMomVe<T>, RecGradV<T>> walk(a.L, t, rec, gradV);
+        PairWalk<kMomWaves<T, avClean>, kMomBatch<T>, kMomGather<T, V, avClean>, RecMomVe<T>, RecGradV<T>> walk(a.L, t, rec, gradV);
         withFold(needFold, [&](auto fold) {
             walk([&](bool live, const RecMomVe<T>& rj, const RecGradV<T>& gj) { pairTerms(fold, live, rj, &gj); }, rec,
                  gradV);
@@ -504,7 +504,7 @@ __global__ void __launch_bounds__((kMomWaves<T, avClean> * kWave))
     }
     else
     {
-        PairWalk<kMomWaves<T, avClean>, isMixed<T> ? 2 : 1, RecMomVe<T>> walk(a.L, t, rec);
+        PairWalk<kMomWaves<T, avClean>, kMomBatch<T>, kMomGather<T, V>, RecMomVe<T>> walk(a.L, t, rec);
         withFold(needFold, [&](auto fold) {
             walk([&](bool live, const RecMomVe<T>& rj) { pairTerms(fold, live, rj, nullptr); }, rec);
         });

@@ -12,7 +12,10 @@
 // bound the loops. With local lists (common.hpp) the block first copies the records of the group's
 // table to LDS, chunk c of all records side by side, and every neighbour is read from there
 // (PairWalk). Groups whose table does not fit the launch's LDS, and global lists,
-// read the records from global memory in the same order. Measured (ms; gathers from global memory, then this):
+// read the records from global memory in the same order, two or four neighbours at a time with the next list entries
+// on their way (one at a time, the loops took up to 1.7 times as long there; 1M particles after a
+// fused search, ms, with that and with this: mixed AV switches 0.61 -> 0.35, momentum-energy 0.97 -> 0.56, FP64
+// 0.88 -> 0.63 and 1.64 -> 1.43). Measured (ms; gathers from global memory, then this):
 // mixed VE at 8M particles, XMass 1.27 -> 0.79, grad-h 2.13 -> 1.30, IAD 2.17 -> 1.49, AV switches 2.84 -> 1.42,
 // momentum-energy 4.92 -> 3.24; FP64 VE at 4.1M, 2.35 -> 1.02, 2.90 -> 1.70, 3.26 -> 1.74, 4.06 -> 1.77, 6.76 ->
 // 5.1-5.4 (with the kernel evaluated instead of gathered from its table; a card at its power limit runs
@@ -240,12 +243,13 @@ __device__ __forceinline__ R stagedRecord(const char* src)
 /*! Walk over the neighbours of a block's targets, wave w taking the quads w, w + W, .. of each list:
  * pair(live, records...) for every slot, with the neighbour's record of each of Rs. Slots past a lane's count
  * (the rest of its last quad) hold the list's last neighbour again, with live = false. U of a quad's
- * records are in flight at a time, and the next quad of the list. */
-template<int W, int U, class... Rs>
+ * staged records are in flight at a time, or G gathered ones, and the next quad of the list. */
+template<int W, int U, int G, class... Rs>
 struct PairWalk
 {
-    static_assert(U == 1 || U == 2 || U == 4, "whole parts of a quad");
-    static constexpr uint32_t kStride = stagedBytes(uint32_t((sizeof(Rs) + ...)));
+    static_assert((U == 1 || U == 2 || U == 4) && (G <= 2 || G == 4), "whole parts of a quad");
+    static constexpr uint32_t kChunks = uint32_t((sizeof(Rs) + ...)) / 16;
+    static constexpr uint32_t kStride = stagedBytes(16 * kChunks);
 
     const Lists& L;
     const Lane&  t;
@@ -337,15 +341,56 @@ struct PairWalk
         }
         else
         {
+            constexpr int B = G ? G : 1;
+            uint32_t      ahead[4] = {};
+            if (G && k0 < t.n) { L.lists.quad(t.r, k0, ahead); }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                asm volatile("" : "+v"(ahead[u])); // (else this load and the loop's become one at the top of each round)
             for (uint32_t k = k0; k < t.n; k += 4 * W)
             {
-                uint32_t j[4];
-                L.lists.quad(t.r, k, j);
-#pragma unroll 1
-                for (uint32_t u = 0; u < 4; ++u)
+                uint32_t j[4] = {ahead[0], ahead[1], ahead[2], ahead[3]};
+                if constexpr (G)
                 {
-                    pair(k + u < t.n, rec[j[0]]...);
-                    j[0] = j[1], j[1] = j[2], j[2] = j[3];
+                    // the next quad's entries (the last one's again) load while this one's records do
+                    L.lists.quad(t.r, k + 4 * W < t.n ? k + 4 * W : k, ahead);
+                }
+                else { L.lists.quad(t.r, k, j); }
+#pragma unroll 1
+                for (int u0 = 0; u0 < 4; u0 += B)
+                {
+                    Chunk16 w[B][kChunks];
+#pragma unroll
+                    for (int u = 0; u < B; ++u)
+                    {
+                        uint32_t at   = 0;
+                        auto     load = [&](auto* p)
+                        {
+                            const Chunk16* src = reinterpret_cast<const Chunk16*>(p + j[u]);
+#pragma unroll
+                            for (uint32_t c = 0; c < sizeof(*p) / 16; ++c)
+                                w[u][at + c] = src[c];
+                            at += sizeof(*p) / 16;
+                        };
+                        (load(rec), ...);
+                    }
+#pragma unroll
+                    for (int u = 0; u < B; ++u)
+                    {
+                        uint32_t at    = 0;
+                        auto     taken = [&](auto* p)
+                        {
+                            std::remove_const_t<std::remove_pointer_t<decltype(p)>> rj;
+                            __builtin_memcpy(&rj, &w[u][at], sizeof(rj));
+                            at += sizeof(rj) / 16;
+                            return rj;
+                        };
+                        const std::tuple<Rs...> r{taken(rec)...};
+                        std::apply([&](const Rs&... rj) { pair(k + u0 + u < t.n, rj...); }, r);
+                    }
+#pragma unroll
+                    for (int u = 0; u + B < 4; ++u)
+                        j[u] = j[u + B];
                 }
             }
         }
@@ -384,7 +429,7 @@ __device__ __forceinline__ bool waveSums(double (&v)[N])
 
 /*! host: the records a launch stages and its dynamic LDS, for records of `recBytes`, N partial sums and a kernel whose
  * registers leave room for `perSimd` waves on a SIMD. A block whose table does not fit the stage reads its
- * neighbours from global memory, about three times as long; a smaller stage leaves room for more blocks on a CU, and the
+ * neighbours from global memory, 1.2 (FP64) to 1.7 times as long; a smaller stage leaves room for more blocks on a CU, and the
  * loops' time goes with about the power -0.4 of the waves per SIMD. The number of blocks per CU is the one with the
  * least product of both, the stage what its share of the 160 KB holds. Measured against a stage for 99.5% of the
  * tables (ms): mixed std momentum of the 4M Evrard sphere 2.15 -> 1.69 (three blocks instead of two, 8% of the
@@ -396,7 +441,7 @@ struct PairLaunch
 };
 inline PairLaunch pairLaunch(const sphx_workspace* ws, size_t recBytes, int waves, int sums, int perSimd)
 {
-    constexpr double kGathered = 3.0;
+    constexpr double kGathered = 1.6;
     constexpr size_t kLds = 160 * 1024, kLdsUnit = 1280; // of a CU, and what it is given out in
     const size_t     part      = size_t(waves - 1) * sums * kWave * sizeof(double);
     uint64_t         blocks    = 0;
@@ -878,6 +923,18 @@ inline void launchVariant(const sphx_workspace* ws, const DevBox& box, F&& launc
     else if (isMixed<T> && ws->nbWide) { launch(std::integral_constant<int, kWide>{}); }
     else { launch(std::integral_constant<int, kAnyIndex>{}); }
 }
+
+/*! Neighbours in flight where a walk reads staged records, and where it gathers them (0: one, and its quad of list entries
+ * not ahead of time). The loops other than the common ones gather one at a time: more spill registers, in their staged
+ * blocks as well. */
+template<class T>
+constexpr int kLightBatch = isMixed<T> ? 4 : 2;
+template<class T, int V>
+constexpr int kLightGather = V == kCommon ? kLightBatch<T> : 1;
+template<class T>
+constexpr int kMomBatch = isMixed<T> ? 2 : 1;
+template<class T, int V, bool avClean = false>
+constexpr int kMomGather = V == kCommon && !avClean ? kMomBatch<T> : 0;
 
 //! run `loop` with the fold compiled in or out, chosen once per wave
 template<class F>

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from sphexa_amd import abi, ic
-from sphexa_amd.particles import STD_FIELDS, VE_FIELDS, ParticleSet, ideal_gas_cv, std_step, ve_step
+from sphexa_amd.particles import GRADV_FIELDS, STD_FIELDS, VE_FIELDS, ParticleSet, ideal_gas_cv, std_step, ve_step
 
 pytestmark = pytest.mark.gpu
 
@@ -105,3 +105,38 @@ def test_mixed_box_shapes(ws, lengths, boundary):
         ref = o["a"][k]
         err = np.max(np.abs(ps.host(k) - ref)) / np.max(np.abs(ref))
         assert err <= bar, (k, err)
+
+
+@pytest.mark.parametrize("index", [6.0, 5.0])
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("side", [4, 5, 10, 17])  # 64, 125, 1000 and 4913 targets: supports wider than half the box first
+def test_gathered_records_bitwise(index, mixed, side):
+    """the VE loops over particle indices (left by the fused search), whose records come from global memory, give the bits
+    of those over table positions, whose records are staged; with the AV cleaning, and without"""
+    from sphexa_amd.lib import Workspace
+
+    arr, spec = ic.turbulence_box(side, seed=6)
+    arr["temp"] = arr.pop("u") / ideal_gas_cv(10.0, 5.0 / 3.0)
+    box = abi.Box.make(spec["lo"], spec["hi"], abi.PERIODIC)
+    ws = Workspace(0, sinc_index=index)
+    ps = ParticleSet.from_host(arr, VE_FIELDS + GRADV_FIELDS, mixed=mixed)
+    params = abi.Params.defaults(ws.K, hydro_type=ps.hydro_type, minDt=1e-4)
+    n, f = ps.n, ps.fields()
+    alpha = ps.t["alpha"].clone()
+    ws.domain_sync(box, ps.sync_fields(), params, n)
+    result = {}
+    for fused in (False, True):
+        (ws.find_neighbors_xmass if fused else ws.find_neighbors)(box, f, params, 0, n, False)
+        ps.t["alpha"].copy_(alpha)
+        for loop in ("sphx_xmass", "sphx_ve_def_gradh"):
+            ws.pair(loop, box, f, params, 0, n)
+        ws.eos("sphx_eos_ve", f, params, 0, n)
+        for loop in ("sphx_iad_divv_curlv", "sphx_av_switches"):
+            ws.pair(loop, box, f, params, 0, n)
+        out = {}
+        for clean in (False, True):
+            ws.momentum_energy_ve(box, f, params, 0, n, clean)
+            out.update({k + str(clean): ps.host(k).copy() for k in ("ax", "ay", "az", "du")})
+        result[fused] = dict(out, **{k: ps.host(k).copy() for k in ("xm", "kx", "gradh", "c11", "divv", "curlv", "alpha")})
+    for k, v in result[False].items():
+        np.testing.assert_array_equal(result[True][k], v, err_msg=k)
