@@ -181,10 +181,11 @@ __global__ void __launch_bounds__(kVjpWaves * kWave)
     withFold(waveNeedsFold(a.box, xi, yi, zi, r2h), [&](auto fold) {
         // a quad of neighbours at a time: their list entries and records load before any is used
         constexpr int U = 4;
+        const TargetList list = a.L.lists.list(t.r);
         for (unsigned k0 = 0; k0 < t.n; k0 += U)
         {
             uint32_t j[U];
-            a.L.lists.quad(t.r, k0, j);
+            list.quad(k0, j);
             RecDensityVjpJ<T> rj[U];
 #pragma unroll
             for (int u = 0; u < U; ++u)
@@ -306,10 +307,11 @@ __global__ void __launch_bounds__(kVjpWaves * kWave)
     withFold(waveNeedsFold(a.box, xi, yi, zi, r2h), [&](auto fold) {
         // a quad of neighbours at a time: their list entries and records load before any is used
         constexpr int U = 4;
+        const TargetList list = a.L.lists.list(t.r);
         for (unsigned k0 = 0; k0 < t.n; k0 += U)
         {
             uint32_t j[U];
-            a.L.lists.quad(t.r, k0, j);
+            list.quad(k0, j);
             RecIadVjpJ<T> rj[U];
 #pragma unroll
             for (int u = 0; u < U; ++u)
@@ -557,10 +559,11 @@ __global__ void __launch_bounds__(kVjpWaves * kWave)
     T gC[6] = {0, 0, 0, 0, 0, 0};
     withFold(waveNeedsFold(a.box, I.p.x, I.p.y, I.p.z, r2h), [&](auto fold) {
         constexpr unsigned U = isMixed<T> ? 2 : 1; // records in flight
+        const TargetList list = a.L.lists.list(t.r);
         for (unsigned k0 = 0; k0 < t.n; k0 += 4)
         {
             uint32_t j[4];
-            a.L.lists.quad(t.r, k0, j);
+            list.quad(k0, j);
 #pragma unroll
             for (unsigned s = 0; s < 4; s += U)
             {
@@ -655,6 +658,7 @@ __global__ void __launch_bounds__(kVjpWaves* kWave)
     const unsigned      w = threadIdx.x / kWave, lane = laneId();
     const uint32_t      t0 = (blockIdx.x * kVjpWaves + w) * kWave, t = t0 + lane;
     const bool          on = t < nt;
+    const TargetList    list = lists.list(on ? t : 0u);
     const uint32_t      p0 = on ? pairStart[t] : 0u, n = on ? pairStart[t + 1] - p0 : 0u;
     const uint32_t      most = waveMax(n);
     for (uint32_t k0 = 0; k0 < most; k0 += kPairsRun)
@@ -665,7 +669,7 @@ __global__ void __launch_bounds__(kVjpWaves* kWave)
             uint32_t j[4];
             if (k0 + k < n)
             {
-                lists.quad(t, k0 + k, j);
+                list.quad(k0 + k, j);
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
                     tile[w][lane][k + u] = j[u];

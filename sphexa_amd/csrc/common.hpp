@@ -52,21 +52,62 @@ __host__ __device__ inline size_t localOffset(uint32_t g, uint32_t ngmax8, uint3
     return (size_t(g) * ngmax8 + (k & ~7u)) * kGroup + 8u * lane + (k & 7u);
 }
 
-/*! particles a group's table holds at most. 64 targets of 90 neighbours fill 450-640 entries on a lattice and
- * 350-900 on the Evrard sphere; a search that meets a larger table stores global lists instead. */
-constexpr uint32_t kTableCap = 2048;
-//! bins of the table sizes' histogram, kTableBin entries each
+/*! particles that each group's table has room for. 64 targets of N neighbours on a lattice fill the points within r =
+ * (3 N / 4 pi)^(1/3) spacings of a cube of 4 points an edge, 27 + 54 r + 9 pi r^2 + N (489 for N = 91; measured 450-640, and
+ * 350-900 on the Evrard sphere); this is twice that for N = ngmax, and 2048 for all but large ngmax. A group that
+ * needs more (particles far apart under long supports, or an h iteration, whose rounds add up) moves to one of a few regions
+ * for tables of tableRegion() entries. With 2048 entries whatever ngmax, hits past ngmax among them, and no regions, one
+ * such group made the search run twice and leave particle indices (ms, then and now, 250k particles, mixed): std
+ * pass at ngmax = 1200 4.53 and 2.84; search with h 1.3 times too large 1.08 and 0.84; search of 1M clustered
+ * particles from an estimate of h 69 and 53. */
+inline uint32_t tableCapacity(uint32_t ngmax)
+{
+    const double n = ngmax, r = std::cbrt(3.0 * n / (4.0 * M_PI)), lattice = 27.0 + 54.0 * r + 9.0 * M_PI * r * r + n;
+    return std::max(2048u, uint32_t(std::min(2.0 * lattice, 32768.0)) / 64 * 64);
+}
+//! the largest table: 64 targets without a common neighbour (a tile's hits beyond ngmax included), as 16-bit positions
+inline uint32_t tableRegion(uint32_t ngmax) { return uint32_t(std::min<uint64_t>(64 * (uint64_t(ngmax) + 64), 65536)); }
+//! bins of the table sizes' histogram, kTableBin entries each, then one for larger tables and one for those that did not fit
 constexpr uint32_t kTableBin  = 32;
-constexpr uint32_t kTableBins = kTableCap / kTableBin;
+constexpr uint32_t kTableBins = 128;
+constexpr uint32_t kLargeTable = kTableBins, kFailedTable = kTableBins + 1;
+
+//! a group's table: its size (kFailed: it did not fit), and its place in NeighborLists::table in units of 64 entries
+struct TableInfo
+{
+    uint32_t count, at;
+
+    static constexpr uint32_t kFailed = 0xffffffffu;
+};
+
+//! one target's stored list
+struct TargetList
+{
+    const char*     slots; // its first 16 bytes
+    const uint32_t* table; // its group's table; null for global lists
+
+    //! particles in slots k..k+3 (k a multiple of 4); slots past its count hold its last neighbour again
+    __device__ __forceinline__ void quad(uint32_t k, uint32_t (&j)[4]) const
+    {
+        if (table == nullptr)
+        {
+            const uint4 q = *reinterpret_cast<const uint4*>(slots + size_t(k / 4) * (kGroup * 16));
+            j[0] = q.x, j[1] = q.y, j[2] = q.z, j[3] = q.w;
+            return;
+        }
+        const uint2 q = *reinterpret_cast<const uint2*>(slots + size_t(k / 8) * (kGroup * 16) + 2 * (k & 4u));
+        j[0] = table[q.x & 0xffffu], j[1] = table[q.x >> 16], j[2] = table[q.y & 0xffffu], j[3] = table[q.y >> 16];
+    }
+};
 
 /*! the stored lists of the last search (see the layouts above) */
 struct NeighborLists
 {
-    const void*     nbrs;
-    const uint32_t* table;      // local lists: kTableCap particles per group ...
-    const uint32_t* tableCount; // ... and how many of them are used; null for global lists
-    const uint32_t* owner;      // the targets' groups (kNoGroup: not searched); null: consecutive groups, or none is needed
-    uint32_t        ngmax;
+    const void*      nbrs;
+    const uint32_t*  table; // local lists: the groups' tables ...
+    const TableInfo* info;  // ... and where each lies; null for global lists
+    const uint32_t*  owner; // the targets' groups (kNoGroup: not searched); null: consecutive groups, or none is needed
+    uint32_t         ngmax;
 
     static constexpr uint32_t kNoGroup = 0xffffffffu;
 
@@ -76,22 +117,17 @@ struct NeighborLists
     //! the search took the r-th target (a group view may leave targets out: they have no list, in either layout)
     __device__ __forceinline__ bool searched(uint32_t r) const { return owner == nullptr || owner[r] != kNoGroup; }
 
-    //! particles in slots k..k+3 (k a multiple of 4) of the r-th searched target; slots past its count hold its
-    //! last neighbour again
-    __device__ __forceinline__ void quad(uint32_t r, uint32_t k, uint32_t (&j)[4]) const
+    //! a group's table
+    __device__ __forceinline__ const uint32_t* tableAt(const TableInfo& t) const { return table + size_t(t.at) * 64; }
+
+    //! list of the r-th target of the searched range (of one that was not searched: not to be read)
+    __device__ __forceinline__ TargetList list(uint32_t r) const
     {
-        const uint32_t g = r / kGroup, lane = r % kGroup;
-        if (tableCount == nullptr)
-        {
-            const uint4 q = *reinterpret_cast<const uint4*>(static_cast<const uint32_t*>(nbrs) +
-                                                            listOffset(g, paddedNgmax(ngmax), k, lane));
-            j[0] = q.x, j[1] = q.y, j[2] = q.z, j[3] = q.w;
-            return;
-        }
-        const uint2     q = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(nbrs) +
-                                                        localOffset(g, paddedNgmax8(ngmax), k, lane));
-        const uint32_t* t = table + size_t(group(r)) * kTableCap;
-        j[0] = t[q.x & 0xffffu], j[1] = t[q.x >> 16], j[2] = t[q.y & 0xffffu], j[3] = t[q.y >> 16];
+        const char* base = static_cast<const char*>(nbrs);
+        if (info == nullptr) { return {base + 4 * listOffset(r / kGroup, paddedNgmax(ngmax), 0, r % kGroup), nullptr}; }
+        const uint32_t g = group(r);
+        return {base + 2 * localOffset(r / kGroup, paddedNgmax8(ngmax), 0, r % kGroup),
+                tableAt(info[g == kNoGroup ? 0 : g])};
     }
 };
 
@@ -244,11 +280,15 @@ struct sphx_workspace
     sphx::Tree tree;
 
     // neighbour lists of the last search, and their groups' tables when they are local lists
-    sphx::DevBuf<uint32_t> nbrs, nbTable, nbTableCount, nbOwner;
+    sphx::DevBuf<uint32_t> nbrs, nbTable, nbOwner;
+    sphx::DevBuf<sphx::TableInfo> nbTableInfo;
     sphx::DevBuf<char>     nbGroupStats; // the search's statistics per group
     bool                   nbLocal = false, nbOwned = false; // nbOwned: nbOwner holds the search's groups
     bool                   nbPartial = false;                // the search's view left targets of its range out
-    uint32_t               nbTableHist[sphx::kTableBins + 1] = {}; // groups by table size; the last bin: over kTableCap
+    uint32_t               nbTableHist[sphx::kTableBins + 2] = {}; // groups by table size
+    uint32_t               nbRegions = 0;    // regions for larger tables that a search has needed
+    uint32_t               nbGlobalNext = 0; // searches to come that store global lists at once, the tables of the last
+    uint32_t               nbGlobalNgmax = 0; // one with this ngmax having been too large
     uint32_t               nbFirst = 0, nbLast = 0, nbNgmax = 0;
     const uint32_t*        nbNc = nullptr; // nc array the lists were built with
     bool                   nbValid = false;
@@ -427,15 +467,16 @@ __device__ __forceinline__ void groupRange(const Groups& G, uint32_t g, uint32_t
 /* 64-bit slots of the workspace counters: the search's statistics (stored pairs, maximum count,
  * non-converged targets) in 0-2, the Courant dt of the momentum loops in 3, the device maxima of the
  * time step in 4, the search's wide-support count, candidate tests and oversized groups in 5-7, the
- * largest h of the searched targets (FP64 bits) in 8, the number of targets searched in 9, the histogram of the
- * table sizes from 10 on */
-constexpr int kCounterSlots  = 10 + (int(kTableBins) + 2) / 2;
+ * largest h of the searched targets (FP64 bits) in 8, the number of targets searched in 9, of the regions asked for
+ * in 10, the histogram of the table sizes from 11 on */
+constexpr int kCounterSlots  = 11 + (int(kTableBins) + 3) / 2;
 constexpr int kStatWide      = 5;
 constexpr int kStatTests     = 6;
 constexpr int kStatBadGroups = 7;
 constexpr int kStatHMax      = 8;
 constexpr int kStatTargets   = 9;
-constexpr int kStatHist      = 10; // first slot of the 32-bit bins of the table sizes
+constexpr int kStatRegions   = 10;
+constexpr int kStatHist      = 11; // first slot of the 32-bit bins of the table sizes
 
 constexpr unsigned kNumXcd = 8; // MI355X: 8 accelerator complex dies, one L2 each
 
@@ -635,7 +676,7 @@ inline DevBox pairBox(const sphx_workspace* ws, const sphx_box_t* b)
 //! host: the stored lists of the last search
 inline NeighborLists neighborLists(const sphx_workspace* ws)
 {
-    return NeighborLists{ws->nbrs.get(), ws->nbTable.get(), ws->nbLocal ? ws->nbTableCount.get() : nullptr,
+    return NeighborLists{ws->nbrs.get(), ws->nbTable.get(), ws->nbLocal ? ws->nbTableInfo.get() : nullptr,
                          ws->nbOwned && (ws->nbLocal || ws->nbPartial) ? ws->nbOwner.get() : nullptr, ws->nbNgmax};
 }
 

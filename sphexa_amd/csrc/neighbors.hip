@@ -80,8 +80,10 @@ struct SearchArgs
     int                  iterateH;
     void*                nbrs;
     uint32_t*            owner;      // the targets' groups (null: consecutive groups), kNoGroup before the search
-    uint32_t*            table;      // local lists: the groups' tables ...
-    uint32_t*            tableCount; // ... and their sizes (over kTableCap: the table did not fit)
+    uint32_t*            table;      // local lists: the groups' tables, tableCap entries each, then `regions` of regionCap ...
+    TableInfo*           info;       // ... and where each group's lies
+    uint32_t             tableCap, regionCap, region0, regions; // region0: the first region in units of 64 entries
+    uint32_t*            regionsTaken;
     uint32_t*            nc;
     GroupStat*           groupStats; // per group, reduced by groupStatsKernel
     double               minLen; // shortest box length
@@ -144,8 +146,12 @@ struct ListWriter
     char*    base; // the lane's slot 0
     uint32_t q0 = 0, q1 = 0, q2 = 0, q3 = 0; // the last entries, oldest first
     uint32_t swept = 0;    // candidates swept by the wave (each tested by all 64 lanes)
-    uint32_t inTable = 0;  // local lists: particles in the group's table (wave-uniform)
-    uint32_t group   = 0;  // the group
+    // local lists (the table's members are wave-uniform)
+    uint32_t slot    = 0;  // entries put
+    uint32_t inTable = 0;  // particles in the group's table
+    uint32_t cap     = 0;  // room in it
+    uint32_t at      = 0;  // its place (TableInfo)
+    bool     asked   = false; // for a region
 
     //! entry k = e: shifted in behind the previous ones, stored when it completes 16 bytes
     __device__ __forceinline__ void put(unsigned k, uint32_t e)
@@ -399,15 +405,11 @@ struct Pending
         ++tiles;
     }
 
+    //! `count`: the lane's hits so far, of which out.slot are in its list
     template<class Writer>
-    __device__ __forceinline__ void drain(const uint16_t* pos, unsigned ngmax, unsigned& count, Writer& out)
+    __device__ __forceinline__ void drain(const uint16_t* pos, unsigned ngmax, unsigned count, Writer& out)
     {
-        uint32_t hits = 0;
-#pragma unroll
-        for (int i = 0; i < 2 * kPendingTiles; ++i)
-            hits += __popc(w[i]);
-        // the entries that still fit, after the first one
-        uint32_t slot = count, left = min(hits, ngmax - min(count, ngmax));
+        uint32_t slot = out.slot, left = min(count, ngmax) - slot;
         auto     next = [&]() {
 #pragma unroll
             for (int i = 0; i + 1 < 2 * kPendingTiles; ++i)
@@ -437,9 +439,9 @@ struct Pending
                 out.put(slot++, e);
                 e = after;
             }
-            out.put(slot, e);
+            out.put(slot++, e);
         }
-        count += hits;
+        out.slot = slot;
 #pragma unroll
         for (int i = 0; i < 2 * kPendingTiles; ++i)
             w[i] = 0;
@@ -447,11 +449,30 @@ struct Pending
     }
 };
 
+//! a group's table outgrows its place: it moves to a region, if one is left (else the search stores global lists)
+template<class Writer>
+__device__ __forceinline__ void moveTable(const SearchArgs& a, Writer& out)
+{
+    uint32_t r = 0;
+    if (laneId() == 0) { r = atomicAdd(a.regionsTaken, 1u); }
+    r         = uniform(r);
+    out.asked = true;
+    if (r >= a.regions) { return; }
+    const uint32_t  at  = a.region0 + r * (a.regionCap / 64);
+    const uint32_t* src = a.table + size_t(out.at) * 64;
+    uint32_t*       dst = a.table + size_t(at) * 64;
+    __threadfence_block(); // the entries other lanes stored
+    for (uint32_t q = laneId(); q < out.inTable; q += kWave)
+        dst[q] = src[q];
+    out.at = at, out.cap = a.regionCap;
+}
+
 /* Sweep the tile's n candidates: their hits as one bit per candidate and target (a tile holds at most 64), appended
  * afterwards in candidate order, so that each list keeps the traversal order while the tests stay free of the
  * divergent append.
  * Local lists: a target's own bit is cleared (a lane finds its place through `self`), the candidates
- * that some target keeps take the next positions of the group's table, and the hits wait in `pending`. */
+ * that some target keeps take the next positions of the group's table, and the hits wait in `pending`. A target whose list
+ * is full only counts. */
 template<bool Local, class Sink, class Lds>
 __device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, Lds& lds, const TargetMatrix& g, int buf,
                                           uint32_t n, int code, const double shift[3], unsigned& count,
@@ -492,14 +513,19 @@ __device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, 
             const uint32_t own = lds.self[lane];
             if (own < uint32_t(kWave)) { m &= ~(uint64_t(1) << own); }
         }
+        const bool full = count >= ngmax;
+        count += uint32_t(__popcll(m));
+        if (full) { m = 0; }
         const uint64_t used = uint64_t(waveOr(uint32_t(m))) | uint64_t(waveOr(uint32_t(m >> 32))) << 32;
         const uint32_t pos  = out.inTable + laneRank(used);
+        const uint32_t size = out.inTable + uint32_t(__popcll(used));
+        if (size > out.cap && !out.asked) { moveTable(a, out); }
         if ((used >> lane) & 1u)
         {
-            if (pos < kTableCap) { a.table[size_t(out.group) * kTableCap + pos] = j; }
+            if (pos < out.cap) { a.table[size_t(out.at) * 64 + pos] = j; }
             lds.pos[pending.tiles * kWave + lane] = uint16_t(pos);
         }
-        out.inTable += uint32_t(__popcll(used));
+        out.inTable = size;
         pending.push(m);
         __builtin_amdgcn_wave_barrier();
         if (pending.tiles == kPendingTiles) { pending.drain(lds.pos, ngmax, count, out); }
@@ -894,6 +920,7 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
     }
 
     unsigned count = 0;
+    out.slot       = 0;
     Pending  pending;
     int      top   = 1;
     int      nBuf  = 0;
@@ -1081,7 +1108,7 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     if constexpr (Local)
     {
         out.base  = static_cast<char*>(a.nbrs) + 2 * localOffset(r / kGroup, paddedNgmax8(a.ngmax), 0, r % kGroup);
-        out.group = g;
+        out.cap = a.tableCap, out.at = g * (a.tableCap / 64);
     }
     else { out.base = static_cast<char*>(a.nbrs) + 4 * listOffset(r / kGroup, paddedNgmax(a.ngmax), 0, r % kGroup); }
 
@@ -1111,6 +1138,8 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
         if (!a.iterateH) { break; }
         const bool repeat = valid && (ngmin > ncSph || (ncSph - 1) > a.ngmax) && updates < 10;
         if (!ballot(repeat)) { break; }
+        // no list refers to the table yet when every target is searched again
+        if (Local && !ballot(valid && !repeat)) { out.inTable = 0; }
         if (repeat)
         {
             updates++;
@@ -1147,22 +1176,22 @@ searchKernel(SearchArgs a, Th* __restrict__ h)
     {
         a.groupStats[g] = {hMax, stored, mx, out.swept, uint16_t(fails), uint16_t(wide), uint16_t(oversized ? 1 : 0),
                            uint16_t(taken)};
-        if constexpr (Local) { a.tableCount[g] = out.inTable; }
+        if constexpr (Local) { a.info[g] = {out.inTable <= out.cap ? out.inTable : TableInfo::kFailed, out.at}; }
     }
 }
 
 /*! Statistics of the search from its groups': stats[0] stored pairs, [1] max count, [2] non-converged particles,
  * [kStatWide] wide support, [kStatTests] candidate distance tests (swept candidates x 64 lanes),
- * [kStatBadGroups], [kStatHMax], [kStatTargets]; with tableCount also the histogram of the groups' table sizes: bin s / kTableBin, the
- * last one for tables that did not fit. One block's atomics per slot. */
+ * [kStatBadGroups], [kStatHMax], [kStatTargets]; with `info` also the histogram of the groups' table sizes. One
+ * block's atomics per slot. */
 __global__ void __launch_bounds__(256)
-    groupStatsKernel(const GroupStat* __restrict__ groupStats, const uint32_t* __restrict__ tableCount, uint32_t groups,
+    groupStatsKernel(const GroupStat* __restrict__ groupStats, const TableInfo* __restrict__ info, uint32_t groups,
                      unsigned long long* __restrict__ stats)
 {
-    __shared__ uint32_t           part[kTableBins + 1];
+    __shared__ uint32_t           part[kTableBins + 2];
     __shared__ unsigned long long sum[6], hBits;
     __shared__ uint32_t           most;
-    if (threadIdx.x <= kTableBins) { part[threadIdx.x] = 0; }
+    if (threadIdx.x < kTableBins + 2) { part[threadIdx.x] = 0; }
     if (threadIdx.x < 6) { sum[threadIdx.x] = 0; }
     if (threadIdx.x == 0) { hBits = 0, most = 0; }
     __syncthreads();
@@ -1175,10 +1204,10 @@ __global__ void __launch_bounds__(256)
         v[0] += q.stored, v[1] += q.fails, v[2] += q.wide, v[3] += q.swept, v[4] += q.bad, v[5] += q.targets;
         mx   = max(mx, q.maxCount);
         hMax = fmax(hMax, q.hMax);
-        if (tableCount != nullptr)
+        if (info != nullptr)
         {
-            const uint32_t s = tableCount[g];
-            atomicAdd(&part[s > kTableCap ? kTableBins : (s == 0 ? 0 : (s - 1) / kTableBin)], 1u);
+            const uint32_t s = info[g].count;
+            atomicAdd(&part[s == TableInfo::kFailed ? kFailedTable : min(s == 0 ? 0u : (s - 1) / kTableBin, kLargeTable)], 1u);
         }
     }
     for (int k = 0; k < 6; ++k)
@@ -1206,13 +1235,14 @@ __global__ void __launch_bounds__(256)
         atomicAdd(&stats[kStatTargets], sum[5]);
     }
     uint32_t* hist = reinterpret_cast<uint32_t*>(stats + kStatHist);
-    if (threadIdx.x <= kTableBins && part[threadIdx.x]) { atomicAdd(&hist[threadIdx.x], part[threadIdx.x]); }
+    if (threadIdx.x < kTableBins + 2 && part[threadIdx.x]) { atomicAdd(&hist[threadIdx.x], part[threadIdx.x]); }
 }
 
 //! clears the search's slots of the counters (those between are the time step's)
-__global__ void __launch_bounds__(kWave) clearStatsKernel(unsigned long long* stats)
+constexpr unsigned kClearThreads = 128;
+__global__ void __launch_bounds__(kClearThreads) clearStatsKernel(unsigned long long* stats)
 {
-    static_assert(kCounterSlots <= kWave, "one slot per lane");
+    static_assert(kCounterSlots <= kClearThreads, "one slot per thread");
     if (threadIdx.x < 3 || (threadIdx.x >= kStatWide && threadIdx.x < kCounterSlots)) { stats[threadIdx.x] = 0; }
 }
 
@@ -1233,7 +1263,7 @@ __global__ void __launch_bounds__(kCopyWaves* kWave)
     const uint64_t      i     = uint64_t(searchFirst) + uint64_t(block) * kGroup + lane;
     const bool          on    = i >= first && i < last && lists.searched(uint32_t(i - searchFirst));
     const uint32_t      n     = on ? min(nc[i] - 1, lists.ngmax) : 0u;
-    const uint32_t      r     = on ? uint32_t(i - searchFirst) : 0u;
+    const TargetList    list  = lists.list(on ? uint32_t(i - searchFirst) : 0u);
     const uint32_t      most  = waveMax(n);
     for (uint32_t k0 = 0; k0 < most; k0 += kCopyRun)
     {
@@ -1243,7 +1273,7 @@ __global__ void __launch_bounds__(kCopyWaves* kWave)
             uint32_t j[4];
             if (k0 + k < n)
             {
-                lists.quad(r, k0 + k, j);
+                list.quad(k0 + k, j);
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
                     tile[w][lane][k + u] = j[u];
@@ -1283,19 +1313,21 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     const Groups grp    = groupsFor(ws, first, last);
     const uint32_t groups = grp.num;
     // list blocks of 64 consecutive particles from first, whatever the target groups. Local lists take 2 bytes
-    // a slot and 8 KB of table per group; with more than twice as many groups as blocks the tables
-    // would outgrow the lists, and the search stores global lists (4 bytes a slot)
+    // a slot and 8 KB of table per group (more for large ngmax); with more than twice as many groups as blocks the
+    // tables would outgrow the lists, and the search stores global lists (4 bytes a slot)
     const size_t blocks64    = std::max<size_t>(1, ceilDiv(last - first, kGroup));
-    const bool   tryLocal    = xmassOut == kSearchOnly && groups <= 2 * blocks64 + 64;
+    bool         tryLocal    = xmassOut == kSearchOnly && groups <= 2 * blocks64 + 64;
+    if (tryLocal && ws->nbGlobalNext > 0 && ws->nbGlobalNgmax == p->ngmax) { tryLocal = false, --ws->nbGlobalNext; }
+    // regions for the few groups whose table outgrows its place: one in 64 groups at first (a tenth of the tables' memory at
+    // ngmax = 150), as many as a former search asked for, at most as much memory as the tables themselves
+    const uint32_t tableCap = tableCapacity(p->ngmax), regionCap = tableRegion(p->ngmax);
+    const size_t   tables      = std::max<size_t>(1, groups) * tableCap;
+    const uint32_t mostRegions = std::max<uint32_t>(groups / 64 + 4, uint32_t(tables / regionCap));
     const bool   owned       = grp.start != nullptr;
     const size_t localWords  = blocks64 * paddedNgmax8(p->ngmax) * kGroup / 2;
     const size_t globalWords = blocks64 * paddedNgmax(p->ngmax) * kGroup;
     ws->nbrs.reserve(tryLocal ? localWords : globalWords);
-    if (tryLocal)
-    {
-        ws->nbTable.reserve(std::max<size_t>(1, groups) * kTableCap);
-        ws->nbTableCount.reserve(std::max<size_t>(1, groups));
-    }
+    if (tryLocal) { ws->nbTableInfo.reserve(std::max<size_t>(1, groups)); }
     const size_t ownerPairs = owned ? (size_t(last - first) + 1) / 2 : 0; // two owners per 64-bit word
     if (owned) { ws->nbOwner.reserve(2 * std::max<size_t>(1, ownerPairs)); }
     ws->counters.reserve(2 * kCounterSlots);
@@ -1320,8 +1352,18 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     a.iterateH = iterateH ? 1 : 0;
     a.nbrs       = ws->nbrs.get();
     a.owner      = owned ? ws->nbOwner.get() : nullptr;
-    a.table      = ws->nbTable.get();
-    a.tableCount = ws->nbTableCount.get();
+    a.info       = ws->nbTableInfo.get();
+    a.tableCap = tableCap, a.regionCap = regionCap, a.region0 = uint32_t(tables / 64);
+    a.regionsTaken = reinterpret_cast<uint32_t*>(ws->counters.get()) + 2 * kStatRegions;
+    a.regions      = 0;
+    a.table        = nullptr;
+    auto reserveTables = [&](uint32_t wanted)
+    {
+        a.regions = std::min(std::max(groups / 64 + 4, wanted), mostRegions);
+        ws->nbTable.reserve(tables + size_t(a.regions) * regionCap);
+        a.table = ws->nbTable.get();
+    };
+    if (tryLocal) { reserveTables(ws->nbRegions); }
     a.nc         = f->nc;
     ws->nbGroupStats.reserve(std::max<size_t>(1, groups) * sizeof(GroupStat));
     a.groupStats = reinterpret_cast<GroupStat*>(ws->nbGroupStats.get());
@@ -1340,10 +1382,10 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     }
 
     unsigned long long stats[kCounterSlots];
-    uint32_t           hist[kTableBins + 1];
+    uint32_t           hist[kTableBins + 2];
     auto               run = [&](bool local)
     {
-        clearStatsKernel<<<1, kWave, 0, ws->stream>>>(reinterpret_cast<unsigned long long*>(ws->counters.get()));
+        clearStatsKernel<<<1, kClearThreads, 0, ws->stream>>>(reinterpret_cast<unsigned long long*>(ws->counters.get()));
         SPHX_CHECK_LAUNCH();
         static_assert(NeighborLists::kNoGroup == 0xffffffffu, "the fill value");
         if (ownerPairs) { fill64(ws, reinterpret_cast<uint64_t*>(ws->nbOwner.get()), ~uint64_t(0), ownerPairs); }
@@ -1369,7 +1411,7 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
             }
             SPHX_CHECK_LAUNCH();
             groupStatsKernel<<<std::min(ceilDiv(groups, 256), 64u), 256, 0, ws->stream>>>(
-                a.groupStats, local ? ws->nbTableCount.get() : nullptr, groups,
+                a.groupStats, local ? a.info : nullptr, groups,
                 reinterpret_cast<unsigned long long*>(ws->counters.get()));
             SPHX_CHECK_LAUNCH();
         }
@@ -1380,14 +1422,27 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     run(tryLocal);
     bool                     local = tryLocal;
     const unsigned long long fails = stats[2];
-    if (local && hist[kTableBins] > 0)
+    if (local && hist[kFailedTable] > 0)
     {
-        // a table did not fit: the same lists in the global layout, at the h the first run converged to
-        local      = false;
-        a.iterateH = 0;
-        ws->nbrs.reserve(globalWords);
-        a.nbrs = ws->nbrs.get();
-        run(false);
+        // tables that fit neither their place nor a region: again, at the h the first run converged to (without the
+        // rounds of the iteration the tables are smaller), with as many regions as were asked for ...
+        const uint64_t asked = stats[kStatRegions];
+        if (a.iterateH || (asked > a.regions && asked <= mostRegions))
+        {
+            ws->nbRegions = std::min(uint32_t(asked + asked / 4), mostRegions);
+            reserveTables(ws->nbRegions);
+            a.iterateH = 0;
+            run(true);
+        }
+        // ... or, and then the next 15 searches too, in the global layout
+        if (hist[kFailedTable] > 0)
+        {
+            local            = false;
+            ws->nbGlobalNext = 15, ws->nbGlobalNgmax = p->ngmax;
+            ws->nbrs.reserve(globalWords);
+            a.nbrs = ws->nbrs.get();
+            run(false);
+        }
     }
 
     ws->nbFirst      = first;

@@ -264,7 +264,7 @@ struct PairWalk
         , staged(false)
         , next(0)
     {
-        if (L.lists.tableCount != nullptr)
+        if (L.lists.info != nullptr)
         {
             bool     one;
             uint32_t b0;
@@ -281,14 +281,14 @@ struct PairWalk
                 b0                  = mask ? __builtin_amdgcn_readlane(b, __builtin_ctzll(mask)) : 0u;
                 one                 = ballot(some && b != b0) == 0 && mask != 0;
             }
-            const uint32_t count = L.lists.tableCount[b0];
-            if (one && count <= L.stage)
+            const TableInfo info = L.lists.info[b0];
+            if (one && info.count <= L.stage)
             {
                 staged = true;
                 if (firstSlot() < paddedNgmax8(L.ngmax)) { next = *reinterpret_cast<const uint64_t*>(listStart()); }
-                const uint32_t* tb = L.lists.table + size_t(b0) * kTableCap;
+                const uint32_t* tb = L.lists.tableAt(info);
                 uint32_t        at = 0;
-                ((stageRecords(tb, count, rec, ldsBytes() + at, kStride), at += uint32_t(sizeof(Rs))), ...);
+                ((stageRecords(tb, info.count, rec, ldsBytes() + at, kStride), at += uint32_t(sizeof(Rs))), ...);
             }
         }
         __syncthreads();
@@ -341,9 +341,10 @@ struct PairWalk
         }
         else
         {
-            constexpr int B = G ? G : 1;
-            uint32_t      ahead[4] = {};
-            if (G && k0 < t.n) { L.lists.quad(t.r, k0, ahead); }
+            constexpr int    B    = G ? G : 1;
+            const TargetList list = L.lists.list(t.r);
+            uint32_t         ahead[4] = {};
+            if (G && k0 < t.n) { list.quad(k0, ahead); }
 #pragma unroll
             for (int u = 0; u < 4; ++u)
                 asm volatile("" : "+v"(ahead[u])); // (else this load and the loop's become one at the top of each round)
@@ -353,9 +354,9 @@ struct PairWalk
                 if constexpr (G)
                 {
                     // the next quad's entries (the last one's again) load while this one's records do
-                    L.lists.quad(t.r, k + 4 * W < t.n ? k + 4 * W : k, ahead);
+                    list.quad(k + 4 * W < t.n ? k + 4 * W : k, ahead);
                 }
-                else { L.lists.quad(t.r, k, j); }
+                else { list.quad(k, j); }
 #pragma unroll 1
                 for (int u0 = 0; u0 < 4; u0 += B)
                 {
@@ -445,7 +446,7 @@ inline PairLaunch pairLaunch(const sphx_workspace* ws, size_t recBytes, int wave
     constexpr size_t kLds = 160 * 1024, kLdsUnit = 1280; // of a CU, and what it is given out in
     const size_t     part      = size_t(waves - 1) * sums * kWave * sizeof(double);
     uint64_t         blocks    = 0;
-    for (uint32_t b = 0; b < kTableBins; ++b)
+    for (uint32_t b = 0; b <= kLargeTable; ++b)
         blocks += ws->nbTableHist[b];
     if (!ws->nbLocal || blocks == 0) { return {0, part}; }
     const uint32_t each = stagedBytes(uint32_t(recBytes));
@@ -455,7 +456,7 @@ inline PairLaunch pairLaunch(const sphx_workspace* ws, size_t recBytes, int wave
     {
         const size_t room = kLds / kLdsUnit / perCu * kLdsUnit;
         if (part > room) { break; }
-        const uint32_t fit    = std::min(uint32_t(room / each), kTableCap);
+        const uint32_t fit    = std::min(uint32_t(room / each), kTableBins * kTableBin);
         uint64_t       staged = 0;
         uint32_t       stage  = 0; // the largest table among those that fit
         for (uint32_t b = 0; (b + 1) * kTableBin <= fit; ++b)
