@@ -58,8 +58,8 @@ __host__ __device__ inline size_t localOffset(uint32_t g, uint32_t ngmax8, uint3
  * needs more (particles far apart under long supports, or an h iteration, whose rounds add up) moves to one of a few regions
  * for tables of tableRegion() entries. With 2048 entries whatever ngmax, hits past ngmax among them, and no regions, one
  * such group made the search run twice and leave particle indices (ms, then and now, 250k particles, mixed): std
- * pass at ngmax = 1200 4.53 and 2.84; search with h 1.3 times too large 1.08 and 0.84; search of 1M clustered
- * particles from an estimate of h 69 and 53. */
+ * pass at ngmax = 1200 4.53 and 2.84; search with h 1.3 times too large 1.08 and 0.84; first std pass over
+ * 1M clustered particles, from an estimate of h, 69 and 53. */
 inline uint32_t tableCapacity(uint32_t ngmax)
 {
     const double n = ngmax, r = std::cbrt(3.0 * n / (4.0 * M_PI)), lattice = 27.0 + 54.0 * r + 9.0 * M_PI * r * r + n;

@@ -815,8 +815,10 @@ __device__ __forceinline__ void flushLeaves(const SearchArgs& a, const Target& t
     }
 }
 
-//! Sort the first n <= 128 entries of the found-leaf buffer by rank: an entry's place is the number of smaller
-//! ranks (the ranks of distinct leaves are distinct)
+/*! Sort the first n <= 128 entries of the found-leaf buffer by rank: an entry's place is the number of smaller
+ * ranks (the ranks of distinct leaves are distinct). Eight ranks at a time, past n the largest: a group whose box spans a
+ * dense cluster sorts some 300 buffers on an otherwise idle SIMD, where half of a plain loop is its branch (std pass
+ * over 250k particles, 90% in a ball of a thousandth of the box, mixed: 11.75 -> 11.42 ms; one over a lattice is unchanged). */
 template<class Lds>
 __device__ __forceinline__ void sortFoundLeaves(Lds& lds, int n)
 {
@@ -830,16 +832,19 @@ __device__ __forceinline__ void sortFoundLeaves(Lds& lds, int n)
     if (!ballot(inversion)) { return; }
     const int node0 = on0 ? lds.bufNode[lane] : 0, node1 = on1 ? lds.bufNode[lane + kWave] : 0;
     int       at0 = 0, at1 = 0;
-    for (int q = 0; q < min(n, kWave); ++q)
-    {
-        const int r = __builtin_amdgcn_readlane(r0, q);
-        at0 += r < r0 ? 1 : 0, at1 += r < r1 ? 1 : 0;
-    }
-    for (int q = kWave; q < n; ++q)
-    {
-        const int r = __builtin_amdgcn_readlane(r1, q - kWave);
-        at0 += r < r0 ? 1 : 0, at1 += r < r1 ? 1 : 0;
-    }
+    auto below = [&](int mine, int count) {
+        for (int q = 0; q < count; q += 8)
+        {
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+            {
+                const int r = __builtin_amdgcn_readlane(mine, q + u);
+                at0 += r < r0 ? 1 : 0, at1 += r < r1 ? 1 : 0;
+            }
+        }
+    };
+    below(r0, min(n, kWave));
+    below(r1, n - kWave);
     __builtin_amdgcn_wave_barrier();
     if (on0) { lds.bufRank[at0] = r0, lds.bufNode[at0] = node0; }
     if (on1) { lds.bufRank[at1] = r1, lds.bufNode[at1] = node1; }
@@ -1009,7 +1014,7 @@ __device__ __forceinline__ unsigned searchGroupInto(const SearchArgs& a, const T
         done         = top == 0;
         bool  sweep  = done;
         int32_t limit = INT32_MAX;
-        if (!done && (nBuf >= kLeafCap || nBuf > kBufCap - 8 - kWave))
+        if (!done && nBuf >= kLeafCap)
         {
             // the first pending node: the first visited child of the first pushed node, whose rank
             // is its parent's, or else the node left below the popped ones

@@ -1,6 +1,6 @@
 """The search's matrix tests against the oracle's lists, entry by entry: pairs at the very edge of the support (where
-the tile is tested again exactly), far offsets and scales of the coordinates, and smoothing lengths that differ
-widely within a group."""
+the tile is tested again exactly), far offsets and scales of the coordinates, smoothing lengths that differ
+widely within a group, and a dense cluster."""
 import numpy as np
 import pytest
 
@@ -10,7 +10,7 @@ from sphexa_amd.particles import STD_FIELDS, ParticleSet
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("case", ["lattice_edge", "spread_h", "far", "tiny", "huge", "coincident"])
+@pytest.mark.parametrize("case", ["lattice_edge", "spread_h", "far", "tiny", "huge", "coincident", "cluster"])
 def test_lists_equal_the_oracles(case):
     import torch
 
@@ -32,6 +32,13 @@ def test_lists_equal_the_oracles(case):
         x, y, z = (c + rng.uniform(-0.3, 0.3, n) / side for c in (x, y, z))
     if case == "spread_h":
         h = h * rng.choice([0.3, 0.6, 1.0, 1.2], n)
+    if case == "cluster":
+        # nine tenths in a small ball: groups around it reach hundreds of leaves, found by the batch and one at a time
+        ball = rng.permutation(n) < n * 9 // 10
+        x, y, z = (np.where(ball, 0.5 + 0.02 * rng.standard_normal(n), rng.uniform(0, 1, n)) for _ in range(3))
+        r2 = (x - 0.5) ** 2 + (y - 0.5) ** 2 + (z - 0.5) ** 2
+        density = 0.9 * n * np.exp(-r2 / (2 * 0.02**2)) / (2 * np.pi * 0.02**2) ** 1.5 + 0.1 * n
+        h = 0.5 * (300 / (4 * np.pi * density)) ** (1 / 3)
     if case == "far":
         x, y, z, lo, hi = x + 1e6, y + 1e6, z + 1e6, 1e6 - 0.1, 1e6 + 1.1
     if case in ("tiny", "huge"):
