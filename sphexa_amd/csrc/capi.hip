@@ -186,8 +186,7 @@ int sphx_workspace_destroy(sphx_workspace_t* ws)
         if (kv.second.stop) { (void)hipEventDestroy(kv.second.stop); }
     }
     ws->tree.releaseAll();
-    ws->nbrs.release(), ws->nbTable.release(), ws->nbTableInfo.release(), ws->nbOwner.release();
-    ws->nbGroupStats.release(), ws->scratch.release(), ws->keyTmp.release();
+    ws->nbrs.release(), ws->nbSide.release(), ws->scratch.release(), ws->keyTmp.release();
     ws->fieldTmp.release(), ws->order.release(), ws->records.release(), ws->counters.release(), ws->hostVisible.release(), ws->reduce64.release();
     ws->adj.pairStart.release(), ws->adj.rowStart.release(), ws->adj.js.release(), ws->adj.jsSorted.release();
     ws->adj.targetsByPair.release(), ws->adj.targets.release(), ws->adj.records.release();

@@ -279,10 +279,12 @@ struct sphx_workspace
 
     sphx::Tree tree;
 
-    // neighbour lists of the last search, and their groups' tables when they are local lists
-    sphx::DevBuf<uint32_t> nbrs, nbTable, nbOwner;
-    sphx::DevBuf<sphx::TableInfo> nbTableInfo;
-    sphx::DevBuf<char>     nbGroupStats; // the search's statistics per group
+    // neighbour lists of the last search, and in one allocation (a first search makes two, whatever its form, and one
+    // over a view after it none) the groups' statistics, tables' places, owners and tables
+    sphx::DevBuf<uint32_t> nbrs, nbSide;
+    uint32_t*              nbOwner = nullptr; // in nbSide
+    sphx::TableInfo*       nbTableInfo = nullptr;
+    uint32_t*              nbTable = nullptr;
     bool                   nbLocal = false, nbOwned = false; // nbOwned: nbOwner holds the search's groups
     bool                   nbPartial = false;                // the search's view left targets of its range out
     uint32_t               nbTableHist[sphx::kTableBins + 2] = {}; // groups by table size
@@ -676,8 +678,8 @@ inline DevBox pairBox(const sphx_workspace* ws, const sphx_box_t* b)
 //! host: the stored lists of the last search
 inline NeighborLists neighborLists(const sphx_workspace* ws)
 {
-    return NeighborLists{ws->nbrs.get(), ws->nbTable.get(), ws->nbLocal ? ws->nbTableInfo.get() : nullptr,
-                         ws->nbOwned && (ws->nbLocal || ws->nbPartial) ? ws->nbOwner.get() : nullptr, ws->nbNgmax};
+    return NeighborLists{ws->nbrs.get(), ws->nbTable, ws->nbLocal ? ws->nbTableInfo : nullptr,
+                         ws->nbOwned && (ws->nbLocal || ws->nbPartial) ? ws->nbOwner : nullptr, ws->nbNgmax};
 }
 
 /* ---------------------------------------------------------------------------------------------

@@ -1332,9 +1332,6 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     const size_t localWords  = blocks64 * paddedNgmax8(p->ngmax) * kGroup / 2;
     const size_t globalWords = blocks64 * paddedNgmax(p->ngmax) * kGroup;
     ws->nbrs.reserve(tryLocal ? localWords : globalWords);
-    if (tryLocal) { ws->nbTableInfo.reserve(std::max<size_t>(1, groups)); }
-    const size_t ownerPairs = owned ? (size_t(last - first) + 1) / 2 : 0; // two owners per 64-bit word
-    if (owned) { ws->nbOwner.reserve(2 * std::max<size_t>(1, ownerPairs)); }
     ws->counters.reserve(2 * kCounterSlots);
 
     double scale = 0;
@@ -1356,22 +1353,26 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
     a.groups = grp;
     a.iterateH = iterateH ? 1 : 0;
     a.nbrs       = ws->nbrs.get();
-    a.owner      = owned ? ws->nbOwner.get() : nullptr;
-    a.info       = ws->nbTableInfo.get();
     a.tableCap = tableCap, a.regionCap = regionCap, a.region0 = uint32_t(tables / 64);
     a.regionsTaken = reinterpret_cast<uint32_t*>(ws->counters.get()) + 2 * kStatRegions;
-    a.regions      = 0;
-    a.table        = nullptr;
-    auto reserveTables = [&](uint32_t wanted)
+    // nbSide: statistics (8 words a group), places (2), owners (with room for them also where this search has no view), then
+    // the tables and regions of local lists
+    static_assert(sizeof(GroupStat) == 32 && sizeof(TableInfo) == 8, "words per group");
+    const size_t statWords = 8 * std::max<size_t>(1, groups), infoWords = 2 * std::max<size_t>(1, groups);
+    const size_t ownerWords = (size_t(last - first) + 1) / 2 * 2, sideWords = (statWords + infoWords + ownerWords + 63) / 64 * 64;
+    auto         reserveSide = [&](bool local, uint32_t wanted)
     {
         a.regions = std::min(std::max(groups / 64 + 4, wanted), mostRegions);
-        ws->nbTable.reserve(tables + size_t(a.regions) * regionCap);
-        a.table = ws->nbTable.get();
+        ws->nbSide.reserve(sideWords + (local ? tables + size_t(a.regions) * regionCap : 0));
+        uint32_t* words = ws->nbSide.get();
+        a.groupStats    = reinterpret_cast<GroupStat*>(words);
+        a.info = ws->nbTableInfo = reinterpret_cast<TableInfo*>(words + statWords);
+        ws->nbOwner              = words + statWords + infoWords;
+        a.owner                  = owned ? ws->nbOwner : nullptr;
+        a.table = ws->nbTable = words + sideWords;
     };
-    if (tryLocal) { reserveTables(ws->nbRegions); }
+    reserveSide(tryLocal, ws->nbRegions);
     a.nc         = f->nc;
-    ws->nbGroupStats.reserve(std::max<size_t>(1, groups) * sizeof(GroupStat));
-    a.groupStats = reinterpret_cast<GroupStat*>(ws->nbGroupStats.get());
     a.minLen   = std::min(box.len[0], std::min(box.len[1], box.len[2]));
     a.m = nullptr, a.wh = nullptr, a.sincN = 0, a.sincInt = -1, a.K = 0, a.xmOut = nullptr, a.toRho = 0;
     const bool f32 = p->hydro_type == SPHX_F32;
@@ -1393,7 +1394,7 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
         clearStatsKernel<<<1, kClearThreads, 0, ws->stream>>>(reinterpret_cast<unsigned long long*>(ws->counters.get()));
         SPHX_CHECK_LAUNCH();
         static_assert(NeighborLists::kNoGroup == 0xffffffffu, "the fill value");
-        if (ownerPairs) { fill64(ws, reinterpret_cast<uint64_t*>(ws->nbOwner.get()), ~uint64_t(0), ownerPairs); }
+        if (owned && ownerWords) { fill64(ws, reinterpret_cast<uint64_t*>(ws->nbOwner), ~uint64_t(0), ownerWords / 2); }
         if (groups > 0)
         {
             unsigned    blocks = ceilDiv(groups, kWavesPerBlock);
@@ -1435,7 +1436,7 @@ int findNeighbors(sphx_workspace* ws, const DevBox& box, const sphx_fields_t* f,
         if (a.iterateH || (asked > a.regions && asked <= mostRegions))
         {
             ws->nbRegions = std::min(uint32_t(asked + asked / 4), mostRegions);
-            reserveTables(ws->nbRegions);
+            reserveSide(true, ws->nbRegions);
             a.iterateH = 0;
             run(true);
         }
