@@ -584,12 +584,14 @@ bool updateTree(sphx_workspace* ws, const Key* keys, size_t nParticles, unsigned
 
     // link the new leaf array (its leaf starts as the keys, one per leaf), then count the particles
     buildLinked(ws, s.nextLeaves.get(), size_t(newL), 1, box);
+    t.valid = false; // its layout is of leaves until the particles are counted
     SPHX_REQUIRE(t.numLeafNodes == newL, SPHX_ERR_STATE, "linking the updated leaves changed their number");
     const uint32_t n = uint32_t(nParticles);
     leafLayoutKernel<<<ceilDiv(size_t(newL) + 1, 256), 256, 0, st>>>(t.leaves.get(), uint32_t(newL), keys, n,
                                                                      t.layout.get(), t.counts.get());
     SPHX_CHECK_LAUNCH();
     t.numParticles = nParticles;
+    t.valid        = true;
     return unchanged;
 }
 
