@@ -257,6 +257,8 @@ __device__ __forceinline__ uint32_t waveOr(uint32_t v)
 
 enum class Fold
 {
+    none,    // all pairs of the tile use the direct image (the fused XMass, whose tiles are all tested exactly, without three
+             // subtractions a pair: 9.95 -> 9.35 ms at 8M particles, mixed, 12.2 -> 11.8 FP64)
     shifted, // one periodic image (shift a multiple of the box length, or 0) serves all pairs of the tile
     perPair  // box too small for a single image: rint fold per pair, as the reference
 };
@@ -279,7 +281,7 @@ __device__ __forceinline__ uint64_t exactMask(const SearchArgs& a, const Target&
         {
             double dx = tx[c0 + c] - t.x, dy = ty[c0 + c] - t.y, dz = tz[c0 + c] - t.z;
             if constexpr (mode == Fold::shifted) { dx = dx - shift[0], dy = dy - shift[1], dz = dz - shift[2]; }
-            else
+            if constexpr (mode == Fold::perPair)
             {
                 dx = dx - double(b.pbc[0]) * b.len[0] * rint(dx * b.ilen[0]);
                 dy = dy - double(b.pbc[1]) * b.len[1] * rint(dy * b.ilen[1]);
@@ -487,7 +489,8 @@ __device__ __forceinline__ void sweepTile(const SearchArgs& a, const Target& t, 
     {
         if (code != kPerPairImage && g.usable) { m = tileMask(a.box, lds, buf, n, g, shift, code == kEachImage, exact); }
     }
-    if (exact)
+    if (Sink::kStageMass && code == kNoShiftImage) { m = exactMask<Fold::none>(a, t, lds, buf, n, shift); }
+    else if (exact)
     {
         m = perPair ? exactMask<Fold::perPair>(a, t, lds, buf, n, shift)
                     : exactMask<Fold::shifted>(a, t, lds, buf, n, shift);
