@@ -23,7 +23,7 @@
 //
 // Measured (ms; with exact tests of every tile, hits appended tile by tile and statistics by atomics of every group, then
 // this): 8M turbulence, mixed 5.2 -> 3.6, 4.1M FP64 3.1 -> 2.2, 1M 0.79 -> 0.51, 4M Evrard sphere 3.7 -> 2.8; vector
-// instructions per group 21.2k -> 13.9k. Bound by the vector ALU (four fifths of its issue slots at 8M) and, at four waves
+// instructions per group 21.2k -> 13.9k. Bound by the vector ALU (0.8 instructions per SIMD and four cycles at 8M) and, at four waves
 // per SIMD (16 waves fill a CU's LDS and 128 registers a wave), by latency: the chains of a window's plan, loads and
 // filter, and of the appends.
 #include <cstring>

@@ -20,7 +20,8 @@
 // momentum-energy 4.92 -> 3.24; FP64 VE at 4.1M, 2.35 -> 1.02, 2.90 -> 1.70, 3.26 -> 1.74, 4.06 -> 1.77, 6.76 ->
 // 5.1-5.4 (with the kernel evaluated instead of gathered from its table; a card at its power limit runs
 // momentum slower when the loops before it are faster). What bounds them now: the FP32 form
-// the vector ALU (67-90% of its issue slots), the FP64 form the latency of a block's phases at 2-3 waves per SIMD.
+// the vector ALU (0.9 to 1.1 instructions per SIMD and four cycles; FP32 and FP64 multiply-adds by turns reach 1.1), the FP64
+// form (0.6 to 0.85) the latency of a block's phases at 2-3 waves per SIMD.
 //
 // Two arithmetic forms share each kernel template:
 //  * T = double ("plain" FP64): the reference JLoop formulas in FP64.
@@ -192,7 +193,8 @@ __device__ __forceinline__ T overDistance(T a, T d2)
 extern __shared__ Chunk16 pairLds[];
 
 //! bytes of a staged neighbour of `bytes` of records: an odd number of 16-byte chunks, so that the records of
-//! different neighbours start in all sixteen 16-byte bank groups
+//! different neighbours start in all sixteen 16-byte bank groups. The 64 lanes of a read still meet in them by chance:
+//! conflicts take 12 to 36% of a CU's cycles in the loops at 8M particles.
 __host__ __device__ constexpr uint32_t stagedBytes(uint32_t bytes) { return 16u * ((bytes / 16u) | 1u); }
 
 /*! copy the records of the group's table to LDS (all waves), record e at dst + e * stride. Each thread has B
