@@ -13,15 +13,28 @@ from sphexa_amd.particles import STD_FIELDS, ParticleSet
 pytestmark = pytest.mark.gpu
 
 
+def lattice():
+    arr, spec = ic.sedov_lattice(11, seed=2)
+    return arr, abi.Box.make(spec["lo"], spec["hi"], abi.PERIODIC)
+
+
+def spread_supports():
+    """supports from 50 to most of the particles: more tables outgrow their place, at ngmax = 300, than there is room for"""
+    n, rng = 12000, np.random.default_rng(2)
+    near = np.exp(rng.uniform(np.log(50), np.log(0.85 * n), n))
+    x, y, z = rng.uniform(0, 1, (3, n))
+    arr = dict(x=x, y=y, z=z, h=0.5 * (3 * near / (4 * np.pi * n)) ** (1 / 3), m=np.full(n, 1.0 / n), u=np.ones(n),
+               vx=0 * x, vy=0 * x, vz=0 * x)
+    return arr, abi.Box.make(0.0, 1.0, abi.OPEN)
+
+
 class Case:
-    def __init__(self, ngmax, side=11, h_factor=1.0):
+    def __init__(self, ngmax, particles=lattice):
         from sphexa_amd.lib import Workspace
 
-        arr, spec = ic.sedov_lattice(side, seed=2)
-        arr["h"] = arr["h"] * h_factor
+        arr, self.box = particles()
         self.ws = Workspace(0)
         self.params = abi.Params.defaults(self.ws.K, ngmax=ngmax, ng0=60)
-        self.box = abi.Box.make(spec["lo"], spec["hi"], abi.PERIODIC)
         self.ps = ParticleSet.from_host(arr, STD_FIELDS)
         self.n, self.ngmax = self.ps.n, ngmax
         self.ws.domain_sync(self.box, self.ps.sync_fields(), self.params, self.n)
@@ -76,14 +89,13 @@ class Case:
         self.ws.set_groups(view)
 
 
-@pytest.mark.parametrize("ngmax", [90, 150])
-@pytest.mark.parametrize("layout", ["tables", "many_groups", "overflow", "fused"])
+@pytest.mark.parametrize("layout,ngmax", [(kind, n) for kind in ("tables", "many_groups", "fused") for n in (90, 150)] +
+                         [("overflow", 300)])
 def test_left_out_targets_have_no_list(layout, ngmax):
     import torch
 
-    # groups of 4, every second: 8 per block of 64, more than whose tables are kept; 3.5 times the smoothing
-    # length: tables of thousands of particles
-    c = Case(ngmax, side=20, h_factor=3.5) if layout == "overflow" else Case(ngmax)
+    # (many groups: of 4, every second: 8 per block of 64, more than whose tables are kept)
+    c = Case(ngmax, spread_supports if layout == "overflow" else lattice)
     c.search()
     whole, stored = c.lists(0, c.n), np.minimum(c.ps.host("nc").astype(np.int64) - 1, ngmax)
     assert np.array_equal((whole >= 0).sum(1), stored) and np.all(whole[:, 0] >= 0)
