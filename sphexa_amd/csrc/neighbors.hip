@@ -1260,7 +1260,7 @@ constexpr unsigned kCopyRun   = 32; // entries of each row per round
 /*! row i - first of `out` = stored list of target i. A wave takes the 64 targets of one list block: it reads kCopyRun
  * entries of each (16-byte runs of the 64 lists lie side by side), turns the tile in LDS and writes 128 bytes per row and
  * half wave. One thread per row, each writing its own 4 bytes, took 349 us for 250k particles and 25M
- * entries; this takes 64. Bound by the table lookups and the writes (105 MB). */
+ * entries; this takes 62, and one row alone 23 us with its call (24 when each quad of a round waited for the last). Bound by the table lookups and the writes (105 MB). */
 __global__ void __launch_bounds__(kCopyWaves* kWave)
     copyListsKernel(NeighborLists lists, const uint32_t* __restrict__ nc, uint32_t* __restrict__ out,
                     uint32_t searchFirst, uint32_t first, uint32_t last)
@@ -1275,17 +1275,16 @@ __global__ void __launch_bounds__(kCopyWaves* kWave)
     const uint32_t      most  = waveMax(n);
     for (uint32_t k0 = 0; k0 < most; k0 += kCopyRun)
     {
-#pragma unroll
-        for (uint32_t k = 0; k < kCopyRun; k += 4)
+        if (k0 < n)
         {
-            uint32_t j[4];
-            if (k0 + k < n)
-            {
-                list.quad(k0 + k, j);
+            // (past the last quad it again, so that the round's loads go out together)
+            uint32_t j[kCopyRun / 4][4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    tile[w][lane][k + u] = j[u];
-            }
+            for (uint32_t q = 0; q < kCopyRun / 4; ++q)
+                list.quad(min(k0 + 4 * q, (n - 1) & ~3u), j[q]);
+#pragma unroll
+            for (uint32_t k = 0; k < kCopyRun; ++k)
+                tile[w][lane][k] = j[k / 4][k % 4];
         }
         __builtin_amdgcn_wave_barrier(); // a wave's LDS accesses complete in order
         const uint32_t k = lane % kCopyRun;
